@@ -108,6 +108,27 @@ def test_ple_gate_conv_hist(T, HC, D, dil):
     assert bits_equal(host(hd), O.ple_hist(x[:2], hist, D, dil))
 
 
+@pytest.mark.parametrize('T,HC,D', [(3, 8, 4), (5, 1, 252), (2, 3, 1280), (4, 2, 1284), (3, 4, 2560), (1, 5, 4092)])
+def test_ple_gate_wave_per_stream_equals_workgroup_per_token(T, HC, D):
+    """the 128-bit form (D % 4 == 0, ldv % 4 == 0) gives the bits of the general kernel, which an odd ldv selects: lengths around a wave's
+    step of 256 values and around a batch of five steps, and in place"""
+    rng = np.random.default_rng(D)
+    kn = outliers(rng, (T, HC, D)); q = outliers(rng, (T, HC, D)); val = rng.standard_normal((T, D + 5)).astype(f32)
+    qscl = (0.5 + rng.random(T * HC)).astype(f32); qw = (1 + 0.1 * rng.standard_normal((HC, D))).astype(f32)
+    for rec in (False, True):
+        res = []
+        for ldv in (D + 4, D + 5):
+            gated = dev(np.zeros((T, HC, D), f32)); gate = dev(np.zeros((T, HC), f32)); v = np.ascontiguousarray(val[:, :ldv])
+            call('camx_pf_ple_gate', ptr(dev(kn)), ptr(dev(q)), ptr(dev(qscl)) if rec else NULL, ptr(dev(qw)) if rec else NULL, ptr(dev(v)), I(ldv),
+                 ptr(gated), ptr(gate), I(HC), I(D), I(T))
+            res.append((host(gated), host(gate)))
+        assert bits_equal(res[0][0], res[1][0]) and bits_equal(res[0][1], res[1][1])
+        assert close_fp32(res[0][1], O.ple_gate(kn, q, val, qscl if rec else None, qw if rec else None)[1])
+    knd = dev(kn); gate = dev(np.zeros((T, HC), f32))
+    call('camx_pf_ple_gate', ptr(knd), ptr(dev(q)), NULL, NULL, ptr(dev(np.ascontiguousarray(val[:, :D + 4]))), I(D + 4), ptr(knd), ptr(gate), I(HC), I(D), I(T))
+    assert bits_equal(host(knd), (val[:, None, :D] * host(gate)[:, :, None]).astype(f32))
+
+
 def test_launcher_surface_of_the_new_symbols():
     """the reference's module and symbol names reach the entry points with the reference's argument lists"""
     import torch
