@@ -39,6 +39,16 @@ def check(err):
         raise RuntimeError(f'HIP error {err}: {_lib.load().camx_error_string(int(err)).decode()}')
 
 
+def stream_handle():
+    """the hipStream_t of torch's current stream on the current device, as an integer: 0.2 us, where building the Stream object
+    that torch.cuda.current_stream() returns takes 2.9 us of the 7.6 us a launch costs its caller (hipLaunchKernel itself: 3.6 us)"""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+
+
+def _dim3(d):
+    return (int(d[0]), 1, 1) if len(d) == 1 else (tuple(int(x) for x in d) + (1, 1))[:3]
+
+
 def _val(a):
     return a.value if hasattr(a, 'value') else a
 
@@ -201,8 +211,8 @@ class Kernel:
 
     def __call__(self, grid, block, *args, shmem=0, stream=None):
         vals = [ctypes.c_void_p(a.data_ptr()) if isinstance(a, torch.Tensor) else a for a in args]
-        grid, block = (tuple(int(x) for x in grid) + (1, 1))[:3], (tuple(int(x) for x in block) + (1, 1))[:3]
-        s = torch.cuda.current_stream().cuda_stream if stream is None else stream
+        grid, block = _dim3(grid), _dim3(block)
+        s = stream_handle() if stream is None else stream
         r = RECORD
         if r is not None and r.intercept(self, grid, block, vals, shmem, s):
             return

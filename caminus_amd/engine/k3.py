@@ -59,11 +59,11 @@ class TapeOps:
         reference's K3_Q35_KV_Q8 modules) and needs kv_error, the sticky int32 word"""
         import ctypes
         import torch
-        from ..device import lib as _lib
+        from ..device import hip as _hip, lib as _lib
         self.T, self.kv_q8_dense, self.kv_error = int(T), bool(kv_q8_dense), kv_error
         self.q35 = bool(q35)            # the dense line's modules: own_add_rms16 at any row length, one unweighted addend, the fp16 copy rounded once
         if self.kv_q8_dense and kv_error is None: raise ValueError('TapeOps: the dense Q8 KV line needs its error word (kv_error)')
-        self._C, self._torch, self._L, self._check = ctypes, torch, _lib.load(), _lib.check
+        self._C, self._torch, self._L, self._check, self._stream = ctypes, torch, _lib.load(), _lib.check, _hip.stream_handle
         self.params = None              # the pass parameters of gdn_conv (int32 [4] on the device; [1] = tokens of the previous pass to commit)
         self.n = 0
 
@@ -71,8 +71,8 @@ class TapeOps:
         return self._C.c_void_p(None if t is None else t.data_ptr())
 
     def _go(self, name, *args):
-        st = self._C.c_void_p(self._torch.cuda.current_stream().cuda_stream)
-        self._check(getattr(self._L, name)(*args, st))
+        err = getattr(self._L, name)(*args, self._C.c_void_p(self._stream()))
+        if err: self._check(err)
         self.n += 1
         return self.n - 1
 

@@ -353,3 +353,17 @@ def test_record_hook_and_loaded_list():
     sync()
     assert bits_equal(host(c, np.uint16), O.f2bf(x))
     assert hip.LOADED.index('core') >= 0 and len(set(hip.LOADED)) == len(hip.LOADED)
+
+
+def test_stream_handle_is_the_current_stream():
+    """launches go to the stream that torch.cuda.current_stream() names: default, a side stream, inside another thread"""
+    import threading
+    import torch
+    from caminus_amd.device import hip
+    side = torch.cuda.Stream()
+    assert hip.stream_handle() == torch.cuda.current_stream().cuda_stream
+    seen = []
+    with torch.cuda.stream(side):
+        assert hip.stream_handle() == side.cuda_stream
+        th = threading.Thread(target=lambda: seen.append((hip.stream_handle(), torch.cuda.current_stream().cuda_stream))); th.start(); th.join()
+    assert seen[0][0] == seen[0][1] and hip.stream_handle() == torch.cuda.current_stream().cuda_stream
