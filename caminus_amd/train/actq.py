@@ -66,6 +66,12 @@ def _backward(x2, gy, bits, clip):
     return dx
 
 
+def _given(gy, like, shape):
+    """the gradient of y, zeros where nothing upstream depends on y. The functions below turn autograd's own zero filling off: it
+    would write and never read one tensor per output without a gradient (codes and scales: 11 us of a 32768 x 1024 block entry)."""
+    return torch.zeros(shape, device=like.device, dtype=torch.bfloat16) if gy is None else gy
+
+
 class ActQ(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, bits, clip):
@@ -93,12 +99,13 @@ class ActQCodes(torch.autograd.Function):
         ctx.quant = (bits, clip)
         ctx.in_shape = x.shape
         ctx.mark_non_differentiable(c, s)
+        ctx.set_materialize_grads(False)
         return y.view(x.shape), c, s
 
     @staticmethod
     def backward(ctx, gy, _gc, _gs):
         (x2,) = ctx.saved_tensors
-        return _backward(x2, gy, *ctx.quant).view(ctx.in_shape), None, None
+        return _backward(x2, _given(gy, x2, x2.shape), *ctx.quant).view(ctx.in_shape), None, None
 
 
 class SiluMulActQ(torch.autograd.Function):
@@ -118,6 +125,7 @@ class SiluMulActQ(torch.autograd.Function):
         ctx.save_for_backward(gu)
         ctx.quant = (bits, clip)
         ctx.mark_non_differentiable(c, s)
+        ctx.set_materialize_grads(False)
         return y, c, s
 
     @staticmethod
@@ -125,7 +133,7 @@ class SiluMulActQ(torch.autograd.Function):
         (gu,) = ctx.saved_tensors
         M, F2 = gu.shape
         Fh = F2 // 2
-        g2 = gy.to(torch.bfloat16).contiguous()
+        g2 = _given(gy, gu, (M, Fh)).to(torch.bfloat16).contiguous()
         dgu = torch.empty(M, F2, device=gu.device, dtype=torch.bfloat16)
         if M:
             _, clipf, qmax = _scalars(Fh, ctx.quant[1], ctx.quant[0])
@@ -158,6 +166,7 @@ class BlockEntry(torch.autograd.Function):
         ctx.quant = (bits, clip)
         ctx.in_shape = x.shape
         ctx.mark_non_differentiable(c, s)
+        ctx.set_materialize_grads(False)
         return y.view(x.shape), c, s, ab.view(*x.shape[:-1], nab)
 
     @staticmethod
@@ -165,7 +174,7 @@ class BlockEntry(torch.autograd.Function):
         x2, nw, rstd, wab = ctx.saved_tensors
         M, d = x2.shape
         nab = 0 if wab is None else wab.shape[0]
-        dy2 = dy.reshape(M, d).to(torch.bfloat16).contiguous()
+        dy2 = _given(dy, x2, (M, d)).reshape(M, d).to(torch.bfloat16).contiguous()
         dab2 = None
         if nab:
             dab2 = (torch.zeros(M, nab, device=x2.device, dtype=torch.bfloat16) if dab is None

@@ -217,6 +217,23 @@ def test_actq_autograd_wrappers():
     assert gu.grad.shape == (M, 2048) and gu.grad.dtype == torch.bfloat16 and torch.isfinite(gu.grad.float()).all()
 
 
+def test_block_entry_gradient_of_one_output():
+    """an output nothing depends on has a zero gradient: y alone, ab alone"""
+    import torch
+    from caminus_amd.train import actq as A
+    rng = np.random.default_rng(8)
+    M, d, nab = 9, 256, 4
+    x = outliers(rng, (M, d)); nw = (0.5 + rng.random(d)).astype(np.float32); wab = O.f2bf((rng.standard_normal((nab, d)) / 30).astype(np.float32))
+    dy = O.f2bf(rng.standard_normal((M, d)).astype(np.float32)); dab = O.f2bf(rng.standard_normal((M, nab)).astype(np.float32))
+    rstd = O.block_entry_fwd(x, nw, wab, 1e-6)[4]
+    for use_y in (True, False):
+        xt = torch.from_numpy(x).to('cuda:0').requires_grad_()
+        y, c, s, ab = A.block_entry(xt, torch.from_numpy(nw).to('cuda:0'), dev(wab).view(torch.bfloat16), 1e-6)
+        if use_y: y.backward(dev(dy).view(torch.bfloat16))
+        else: ab.backward(dev(dab).view(torch.bfloat16))
+        assert bits_equal(host(xt.grad), O.block_entry_bwd(x, nw, rstd, wab, dy if use_y else np.zeros_like(dy), np.zeros_like(dab) if use_y else dab))
+
+
 @pytest.mark.parametrize('bf', [False, True])
 def test_actq_fwd_and_bwd_four_million_values(bf):
     """enough values that the forward's division-free rounding meets its fallback thousands of times"""
