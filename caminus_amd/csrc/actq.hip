@@ -152,26 +152,40 @@ CAMX_DEV float actq_rotate(Src src, int row, int l, int hw, int nch, f32x4 (&u)[
     return amax;
 }
 
-// rintf(u / s) for a lane's four values. p = u * rcp(s) is within 8e-5 of the exact quotient while |p| < 256 (rcp: 1 ulp; one
-// more rounding), the IEEE quotient within 1.6e-5 of it, and half-integers are floats: when p is farther than 3e-4 from every
-// half-integer, rintf of the two agree. Other lanes (about one value in 1600, and infinities / NaN) divide.
-CAMX_DEV f32x4 rint_div4(f32x4 u, float s, float s_rcp) {
-    f32x4 p = {u.x * s_rcp, u.y * s_rcp, u.z * s_rcp, u.w * s_rcp};
-    f32x4 r = {rintf(p.x), rintf(p.y), rintf(p.z), rintf(p.w)};
-    bool safe = true;
-#define S_(e) safe &= (fabsf(p.e - r.e) <= 0.4997f) & (fabsf(p.e) < 256.0f);
-    CAMX_EACH4(S_)
-#undef S_
-    if (!safe) { r.x = rintf(u.x / s); r.y = rintf(u.y / s); r.z = rintf(u.z / s); r.w = rintf(u.w / s); }
-    return r;
-}
+// The row's scale and what the lanes need to divide by it. p = u * rcp(s) is within 8e-5 of the exact quotient while |p| < 256 (rcp:
+// 1 ulp; one more rounding), the IEEE quotient within 1.6e-5 of it, and half-integers are floats: when p is farther than 3e-4 from
+// every half-integer, rintf of the two agree. A lane that holds a closer value (about one value in 1600) divides, and so does every
+// lane of a row whose largest quotient is not below 256 or not a number (an infinite amax). A NaN among the four values needs no
+// look of its own: its p is a NaN as its quotient is, and the maximum passes over it.
+struct RowScale {
+    float s, rcp, lo, hi; bool row_ok;
+    CAMX_DEV RowScale(float s_, float amax, int qmax) : s(s_), rcp(__builtin_amdgcn_rcpf(s_)), lo((float)(-qmax - 1)), hi((float)qmax) { row_ok = amax * rcp < 256.0f; }
+    // clamp(rintf(u / s), lo, hi) of four values; the median of a NaN and two numbers is the smaller number, lo, as fminf(fmaxf(NaN, lo), hi) is
+    CAMX_DEV f32x4 quant4(f32x4 u) const {
+        const f32x4 p = {u.x * rcp, u.y * rcp, u.z * rcp, u.w * rcp};
+        f32x4 r = {rintf(p.x), rintf(p.y), rintf(p.z), rintf(p.w)};
+        const float off = fmaxf(fmaxf(fabsf(p.x - r.x), fabsf(p.y - r.y)), fmaxf(fabsf(p.z - r.z), fabsf(p.w - r.w)));
+        if (!(row_ok && !(off > 0.4997f))) { r.x = rintf(u.x / s); r.y = rintf(u.y / s); r.z = rintf(u.z / s); r.w = rintf(u.w / s); }
+        return (f32x4){__builtin_amdgcn_fmed3f(r.x, lo, hi), __builtin_amdgcn_fmed3f(r.y, lo, hi), __builtin_amdgcn_fmed3f(r.z, lo, hi), __builtin_amdgcn_fmed3f(r.w, lo, hi)};
+    }
+    // the low four bits of four quantized values, packed. For values in [-8, 7]: q + 8 is the code with its top bit turned over, and
+    // the digits q + 8 of a base-16 number are summed exactly in fp32 (four multiply-adds and one conversion instead of eleven instructions)
+    CAMX_DEV uint32_t nibbles4(f32x4 q) const {
+        if (hi <= 7.0f) return (uint32_t)__builtin_fmaf(q.w, 4096.0f, __builtin_fmaf(q.z, 256.0f, __builtin_fmaf(q.y, 16.0f, q.x + 34952.0f))) ^ 0x8888u;
+        return ((uint32_t)(int)q.x & 0xfu) | (((uint32_t)(int)q.y & 0xfu) << 4) | (((uint32_t)(int)q.z & 0xfu) << 8) | (((uint32_t)(int)q.w & 0xfu) << 12);
+    }
+};
 
+// max over the wave (order-free) in row moves and four lane reads
+CAMX_DEV float wave_max64(float v) {
+    v = fmaxf(v, lane_xor1(v)); v = fmaxf(v, lane_xor2(v)); v = fmaxf(v, lane_xor4(v)); v = fmaxf(v, lane_xor8(v));
+    return fmaxf(fmaxf(lane_read(v, 0), lane_read(v, 16)), fmaxf(lane_read(v, 32), lane_read(v, 48)));
+}
 // row-wide max (order-free); lds: 4 floats
 template <int NHW = 8>
 CAMX_DEV float row_max(float amax, float * lds) {
     const int tid = threadIdx.x;
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1) amax = fmaxf(amax, __shfl_xor(amax, m, 64));
+    amax = wave_max64(amax);
     if (NHW == 2) return amax;                           // the row is this wave's
     __syncthreads();
     if ((tid & 63) == 0) lds[tid >> 6] = amax;
@@ -185,23 +199,16 @@ CAMX_DEV void actq_fwd_row(Src src, int row, uint16_t * __restrict__ y, float * 
     const int tid = threadIdx.x, l = slot_of(tid) & 31, hw = tid >> 5, nch = K / 128;
     f32x4 u[NR];
     const float amax = row_max<NHW>(actq_rotate<NR, Src, NHW>(src, row, l, hw, nch, u), lds);
-    const float s = fmaxf(amax * clip / (float)qmax, 1e-8f), s_rcp = __builtin_amdgcn_rcpf(s);
+    const float s = fmaxf(amax * clip / (float)qmax, 1e-8f);
+    const RowScale rs(s, amax, qmax);
     if (tid == 0 && s_out) s_out[row] = s;
-    const float lo = (float)(-qmax - 1), hi = (float)qmax;
 #pragma unroll
     for (int c = 0; c < NR; c++) {
         const int ch = hw + NHW * c;
         if (ch < nch) {
-            f32x4 q;
-            f32x4 r = rint_div4(u[c], s, s_rcp);
-#define Q_(e) q.e = fminf(fmaxf(r.e, lo), hi);
-            CAMX_EACH4(Q_)
-#undef Q_
+            const f32x4 q = rs.quant4(u[c]);
             if (y) { f32x4 d; d.x = q.x * s; d.y = q.y * s; d.z = q.z * s; d.w = q.w * s; *(u32x2 *)(y + (size_t)row * K + ch * 128 + 4 * l) = pack_f2bf_x4(d); }
-            if (codes) {
-                const uint32_t pk = ((uint32_t)(int)q.x & 0xfu) | (((uint32_t)(int)q.y & 0xfu) << 4) | (((uint32_t)(int)q.z & 0xfu) << 8) | (((uint32_t)(int)q.w & 0xfu) << 12);
-                codes[(size_t)row * (K / 4) + ch * 32 + l] = (uint16_t)pk;
-            }
+            if (codes) codes[(size_t)row * (K / 4) + ch * 32 + l] = (uint16_t)rs.nibbles4(q);
         }
     }
 }
@@ -246,14 +253,9 @@ CAMX_DEV void hadamard128_w32(float (&u)[4][8], int q) {
 #pragma unroll
     for (int k = 0; k < 8; k++) { bfly(u[0][k], u[2][k]); bfly(u[1][k], u[3][k]); }
 }
-CAMX_DEV float wave_max64(float v) {
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1) v = fmaxf(v, __shfl_xor(v, m, 64));
-    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
-}
-// u = bf16(H128 . bf16(source)) of the lane's 32 values from the fetched words; returns the row's max |u|
+// u = bf16(H128 . bf16(source)) of the lane's 32 values from the fetched words; gmax[j]: the lane's max |u| in group j; returns the row's
 template <typename Src>
-CAMX_DEV float actq_rotate_w(const Src & src, const u32x4 (&raw)[4][Src::NW], int q, float (&u)[4][8], u32x4 (&keep)[4]) {
+CAMX_DEV float actq_rotate_w(const Src & src, const u32x4 (&raw)[4][Src::NW], int q, float (&u)[4][8], u32x4 (&keep)[4], float (&gmax)[4]) {
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         f32x4 a, b;
@@ -262,16 +264,17 @@ CAMX_DEV float actq_rotate_w(const Src & src, const u32x4 (&raw)[4][Src::NW], in
         u[j][0] = a.x; u[j][1] = a.y; u[j][2] = a.z; u[j][3] = a.w; u[j][4] = b.x; u[j][5] = b.y; u[j][6] = b.z; u[j][7] = b.w;
     }
     hadamard128_w32(u, q);
-    float amax = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 4; j++)
+    for (int j = 0; j < 4; j++) {
+        gmax[j] = 0.0f;                                                            // (an absent chunk holds zeros)
 #pragma unroll
         for (int k = 0; k < 8; k += 4) {
             const f32x4 v = rbf4_any(scaled4((f32x4){u[j][k], u[j][k + 1], u[j][k + 2], u[j][k + 3]}));
             u[j][k] = v.x; u[j][k + 1] = v.y; u[j][k + 2] = v.z; u[j][k + 3] = v.w;
-            amax = fmaxf(amax, absmax4(v));                                        // (an absent chunk holds zeros)
+            gmax[j] = fmaxf(fmaxf(gmax[j], fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
         }
-    return wave_max64(amax);
+    }
+    return wave_max64(fmaxf(fmaxf(gmax[0], gmax[1]), fmaxf(gmax[2], gmax[3])));
 }
 template <typename Src>
 CAMX_DEV void fetch_row_w(const Src & src, int row, int c, int q, bool on, u32x4 (&raw)[4][Src::NW]) {
@@ -300,7 +303,6 @@ __global__ void __launch_bounds__(256) actq_fwd_wave_k(Src src, uint16_t * __res
     const bool on = c < nch;
     const int row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (!Src::lds_tables && row >= M) return;
-    const float lo = (float)(-qmax - 1), hi = (float)qmax;
     u32x4 raw[4][Src::NW];
     fetch_row_w(src, min(row, M - 1), c, q, on, raw);
     if (Src::lds_tables) {                               // the gates' table, shared by the workgroup's four rows
@@ -311,29 +313,22 @@ __global__ void __launch_bounds__(256) actq_fwd_wave_k(Src src, uint16_t * __res
         src.set_small(small);
         if (row >= M) return;
     }
-    float u[4][8];
+    float u[4][8], gmax[4];
     u32x4 keep[4];                                       // (only the backward uses it)
-    const float amax = actq_rotate_w(src, raw, q, u, keep);
-    const float s = fmaxf(amax * clip / (float)qmax, 1e-8f), s_rcp = __builtin_amdgcn_rcpf(s);
+    const float amax = actq_rotate_w(src, raw, q, u, keep, gmax);
+    const float s = fmaxf(amax * clip / (float)qmax, 1e-8f);
+    const RowScale rs(s, amax, qmax);
     if (lane == 0 && s_out) s_out[row] = s;
     if (!on) return;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        f32x4 qa = rint_div4((f32x4){u[j][0], u[j][1], u[j][2], u[j][3]}, s, s_rcp), qb = rint_div4((f32x4){u[j][4], u[j][5], u[j][6], u[j][7]}, s, s_rcp);
-#define Q_(e) qa.e = fminf(fmaxf(qa.e, lo), hi); qb.e = fminf(fmaxf(qb.e, lo), hi);
-        CAMX_EACH4(Q_)
-#undef Q_
+        const f32x4 qa = rs.quant4((f32x4){u[j][0], u[j][1], u[j][2], u[j][3]}), qb = rs.quant4((f32x4){u[j][4], u[j][5], u[j][6], u[j][7]});
         const size_t e0 = (size_t)row * K + c * 128 + 32 * j + 8 * q;
         if (y) {
             const u32x2 pa = pack_f2bf_x4((f32x4){qa.x * s, qa.y * s, qa.z * s, qa.w * s}), pb = pack_f2bf_x4((f32x4){qb.x * s, qb.y * s, qb.z * s, qb.w * s});
             *(u32x4 *)(y + e0) = (u32x4){pa.x, pa.y, pb.x, pb.y};
         }
-        if (codes) {
-#define N_(v, sh) (((uint32_t)(int)(v) & 0xfu) << (sh))
-            const uint32_t pk = N_(qa.x, 0) | N_(qa.y, 4) | N_(qa.z, 8) | N_(qa.w, 12) | N_(qb.x, 16) | N_(qb.y, 20) | N_(qb.z, 24) | N_(qb.w, 28);
-#undef N_
-            *(uint32_t *)(codes + (e0 >> 2)) = pk;
-        }
+        if (codes) *(uint32_t *)(codes + (e0 >> 2)) = rs.nibbles4(qa) | (rs.nibbles4(qb) << 16);
     }
 }
 
@@ -354,21 +349,16 @@ CAMX_DEV void block8_sum2(float & a, float & b, float * lds16) {
     for (int w = 1; w < 8; w++) { a += lds16[w]; b += lds16[8 + w]; }
 }
 
-// u / s for a row's values, s the row's scale: the IEEE quotient by the compiler's own expansion (reciprocal, one Newton step,
-// the product and two corrections, each an fma) without its scaling and fix-up steps, which only act when an exponent is
-// extreme. Taken when s and max |u| / s lie in [2^-60, 2^60] and the lane's four quotients are at least 2^-60 in magnitude:
-// every intermediate is then a normal number and both forms run the same arithmetic (an exhaustive-neighbourhood check on a CPU
-// over 10^8 (u, s) pairs, with every reciprocal within an ulp, found no difference). Other lanes divide.
+// u / s for a row's values (bf16 numbers), s the row's scale (>= 1e-8): with r1 = 1 / s correctly rounded, t0 = u r1, its residual
+// u - s t0 (exact) and t0 + residual r1 is the correctly rounded quotient for every pair of a bf16 and an fp32 significand (all 2^30
+// checked on a CPU). Taken when s and max |u| / s are at most 2^60 and the lane's four t0 are at least 2^-60 in magnitude, so that
+// nothing is out of range and no residual loses bits; other lanes divide (a zero among them: its quotient is the zero).
 struct RowDiv {
     float s, r1; bool row_ok;
-    CAMX_DEV RowDiv(float s_, float amax) : s(s_) {
-        const float r0 = __builtin_amdgcn_rcpf(s_);
-        r1 = __builtin_fmaf(__builtin_fmaf(-s_, r0, 1.0f), r0, r0);
-        row_ok = s_ >= 0x1p-60f && s_ <= 0x1p60f && amax * r1 <= 0x1p60f;
-    }
+    CAMX_DEV RowDiv(float s_, float amax) : s(s_), r1(1.0f / s_) { row_ok = s_ >= 0x1p-60f && s_ <= 0x1p60f && amax * r1 <= 0x1p60f; }
     CAMX_DEV f32x4 div4(f32x4 u, bool needed = true) const {       // needed: false in a lane whose values are padding
         f32x4 t, t0 = {u.x * r1, u.y * r1, u.z * r1, u.w * r1};
-#define T_(e) { const float rem = __builtin_fmaf(-s, t0.e, u.e), t1 = __builtin_fmaf(rem, r1, t0.e); t.e = __builtin_fmaf(__builtin_fmaf(-s, t1, u.e), r1, t1); }
+#define T_(e) t.e = __builtin_fmaf(__builtin_fmaf(-s, t0.e, u.e), r1, t0.e);
         CAMX_EACH4(T_)
 #undef T_
         const float least = fminf(fminf(fabsf(t0.x), fabsf(t0.y)), fminf(fabsf(t0.z), fabsf(t0.w)));     // (a NaN quotient is a NaN either way)
@@ -376,11 +366,24 @@ struct RowDiv {
         return t;
     }
 };
+// The straight-through step of one value: r = rintf(t), q its clamp to [lo, hi], m: r lies strictly inside. Gives the factor of g in
+// dL/ds, m ? q - t : q, and m as 1 or 0.
+struct Ste {
+    float lo, hi, lo1, hi1;
+    CAMX_DEV Ste(int qmax) : lo((float)(-qmax - 1)), hi((float)qmax), lo1((float)-qmax), hi1((float)(qmax - 1)) {}
+    CAMX_DEV float operator()(float t, float & m) const {
+        const float r = rintf(t), q = __builtin_amdgcn_fmed3f(r, lo, hi);              // (a NaN: lo, as fminf(fmaxf(NaN, lo), hi))
+        const bool in = __builtin_amdgcn_fmed3f(r, lo1, hi1) == r;                      // lo < r < hi of an integer; false for a NaN
+        m = in ? 1.0f : 0.0f;
+        return q - (in ? t : 0.0f);
+    }
+};
 
+// st8: eight values before their rounding to bf16, the wave-per-row kernel's form
 struct SinkF32 {
     float * dx; int K;
     CAMX_DEV void operator()(int row, int k, f32x4 v, u32x2) const { *(f32x4 *)(dx + (size_t)row * K + k) = v; }
-    CAMX_DEV void st8(int row, int k, f32x4 a, f32x4 b, u32x4) const { f32x4 * p = (f32x4 *)(dx + (size_t)row * K + k); p[0] = a; p[1] = b; }
+    CAMX_DEV void st8(int row, int k, f32x4 a, f32x4 b, u32x4) const { f32x4 * p = (f32x4 *)(dx + (size_t)row * K + k); p[0] = rbf4_canon(a); p[1] = rbf4_canon(b); }
     CAMX_DEV void set_small(const float *) {}
 };
 struct SinkBF16 {
@@ -448,8 +451,8 @@ struct SinkSiluMul {
         const uint16_t * r = gu + (size_t)row * ld + k;
         const u32x4 gw = *(const u32x4 *)r, uw = *(const u32x4 *)(r + F);
         u32x2 dg0, du0, dg1, du1;
-        grads4((u32x2){gw.x, gw.y}, (u32x2){uw.x, uw.y}, (u32x2){keep.x, keep.y}, a, dg0, du0);
-        grads4((u32x2){gw.z, gw.w}, (u32x2){uw.z, uw.w}, (u32x2){keep.z, keep.w}, b, dg1, du1);
+        grads4((u32x2){gw.x, gw.y}, (u32x2){uw.x, uw.y}, (u32x2){keep.x, keep.y}, rbf4_any(a), dg0, du0);      // (a NaN's bits are settled by the stores' rounding)
+        grads4((u32x2){gw.z, gw.w}, (u32x2){uw.z, uw.w}, (u32x2){keep.z, keep.w}, rbf4_any(b), dg1, du1);
         uint16_t * o = dgu + (size_t)row * (2 * F) + k;
         *(u32x4 *)o = (u32x4){dg0.x, dg0.y, dg1.x, dg1.y};
         *(u32x4 *)(o + F) = (u32x4){du0.x, du0.y, du1.x, du1.y};
@@ -473,7 +476,7 @@ CAMX_DEV void actq_bwd_row(Src src, int row, const uint16_t * __restrict__ g, Si
     u32x2 keep[NR];                                      // what the source hands to the sink (the fused SiLU form only)
     const float amax = row_max<NHW>(actq_rotate<NR, Src, NHW>(src, row, l, hw, nch, u, keep), lds16);
     const float s_raw = amax * clip / (float)qmax, s = fmaxf(s_raw, 1e-8f);
-    const float lo = (float)(-qmax - 1), hi = (float)qmax;
+    const Ste ste(qmax);
     // dL/ds = sum g (q - m t) and the number of max-|u| elements; m: the rounded value lies strictly inside (lo, hi). The
     // straight-through part g m is formed here (g is not needed afterwards); the ties are counted from the compares' lane masks
     // on the scalar unit, one counter per half-wave (a count is exact in any order).
@@ -487,8 +490,7 @@ CAMX_DEV void actq_bwd_row(Src src, int row, const uint16_t * __restrict__ g, Si
         if (hw + NHW * c < nch) {
             const f32x4 t4 = rd.div4(u[c]);
             uint64_t any = 0;
-#define D_(e) { const float t = t4.e, r = rintf(t), q = fminf(fmaxf(r, lo), hi); const bool m = r > lo && r < hi; \
-                dlds = __builtin_fmaf(gv[c].e, m ? q - t : q, dlds); gv[c].e = gv[c].e * (m ? 1.0f : 0.0f); \
+#define D_(e) { float m; const float x = ste(t4.e, m); dlds = __builtin_fmaf(gv[c].e, x, dlds); gv[c].e = gv[c].e * m; \
                 const uint64_t tie = __builtin_amdgcn_ballot_w64(fabsf(u[c].e) == amax); any |= tie; \
                 ties_lo += __builtin_popcount((uint32_t)tie); ties_hi += __builtin_popcount((uint32_t)(tie >> 32)); }
             CAMX_EACH4(D_)
@@ -570,13 +572,12 @@ __global__ void __launch_bounds__(256) actq_bwd_wave_k(Src src, const uint16_t *
         src.set_small(small); sink.set_small(dsmall);
         if (row_raw >= M) return;
     }
-    float u[4][8];
+    float u[4][8], gmax[4];
     u32x4 keep[4];
-    const float amax = actq_rotate_w(src, raw, q, u, keep);
+    const float amax = actq_rotate_w(src, raw, q, u, keep, gmax);
     const float s_raw = amax * clip / (float)qmax, s = fmaxf(s_raw, 1e-8f);
-    const float lo = (float)(-qmax - 1), hi = (float)qmax;
+    const Ste ste(qmax);
     const RowDiv rd(s, amax);
-    const uint64_t on_mask = __builtin_amdgcn_ballot_w64(on);
     float gm[4][8], part[4][2];                          // g m; the reference lanes' sums of dL/ds terms
     int ties_n = 0;
     uint32_t tied = 0;                                   // bit j: group j holds a max-|u| element in some lane
@@ -588,18 +589,14 @@ __global__ void __launch_bounds__(256) actq_bwd_wave_k(Src src, const uint16_t *
         const f32x4 ta = rd.div4((f32x4){u[j][0], u[j][1], u[j][2], u[j][3]}, on), tb = rd.div4((f32x4){u[j][4], u[j][5], u[j][6], u[j][7]}, on);
         const float t8[8] = {ta.x, ta.y, ta.z, ta.w, tb.x, tb.y, tb.z, tb.w};
         float x8[8];
-        uint64_t any = 0;
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-            const float t = t8[k], r = rintf(t), qv = fminf(fmaxf(r, lo), hi);
-            const bool m = r > lo && r < hi;
-            x8[k] = m ? qv - t : qv;
-            gm[j][k] = g8[k] * (m ? 1.0f : 0.0f);
-            const uint64_t tie = __builtin_amdgcn_ballot_w64(fabsf(u[j][k]) == amax) & on_mask;
-            any |= tie;
-            ties_n += __builtin_popcountll(tie);
+        for (int k = 0; k < 8; k++) { float m; x8[k] = ste(t8[k], m); gm[j][k] = g8[k] * m; }
+        // ties are looked for only in a group whose largest value in some lane is the row's (wave-uniform; a row has few such elements)
+        if (__builtin_amdgcn_ballot_w64(on && gmax[j] == amax) != 0) {
+            tied |= 1u << j;
+#pragma unroll
+            for (int k = 0; k < 8; k++) ties_n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(on && fabsf(u[j][k]) == amax));
         }
-        if (any) tied |= 1u << j;
 #pragma unroll
         for (int kk = 0; kk < 2; kk++) {
             float a = 0.0f;
@@ -643,7 +640,7 @@ __global__ void __launch_bounds__(256) actq_bwd_wave_k(Src src, const uint16_t *
     if (!on) return;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        const f32x4 a = rbf4_canon(scaled4((f32x4){gm[j][0], gm[j][1], gm[j][2], gm[j][3]})), b = rbf4_canon(scaled4((f32x4){gm[j][4], gm[j][5], gm[j][6], gm[j][7]}));
+        const f32x4 a = scaled4((f32x4){gm[j][0], gm[j][1], gm[j][2], gm[j][3]}), b = scaled4((f32x4){gm[j][4], gm[j][5], gm[j][6], gm[j][7]});
         sink.st8(row, c * 128 + 32 * j + 8 * q, a, b, keep[j]);
     }
 }

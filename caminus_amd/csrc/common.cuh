@@ -105,7 +105,7 @@ CAMX_DEV uint32_t hw_pk_bf16(float lo, float hi) {
     const f32x2 in = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(in, bf16x2));
 }
-CAMX_DEV bool any_nan4(f32x4 v) { return (v.x != v.x) | (v.y != v.y) | (v.z != v.z) | (v.w != v.w); }
+CAMX_DEV bool any_nan4(f32x4 v) { return __builtin_isunordered(v.x, v.y) | __builtin_isunordered(v.z, v.w); }       // (one compare looks at two values)
 CAMX_DEV u32x2 pack_bf16x4_rne(f32x4 v) {  // to_bf16 of four values, packed little-endian
     u32x2 r;
     if (__builtin_expect(any_nan4(v), 0)) {
