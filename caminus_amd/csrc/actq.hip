@@ -125,7 +125,7 @@ struct RmsRegSrc {
 template <typename S, typename = void> struct SrcByRound : std::false_type {};
 template <typename S> struct SrcByRound<S, std::void_t<decltype(S::by_round)>> : std::true_type {};
 
-// u = bf16(H128 . bf16(source)) for the NR rounds of this half-wave; returns the lane's max |u| over its active chunks
+// u = bf16(H128 . bf16(source)) for the NR rounds of this half-wave (NHW == 2: NR is ceil(K / 256), so only the last can be partial); returns the lane's max |u| over its active chunks
 // NHW: the half-waves that share a row (8: a 256-thread workgroup; 2: one wave); half-wave hw takes chunks hw, hw + NHW, ...
 template <int NR, typename Src, int NHW = 8>
 CAMX_DEV float actq_rotate(Src src, int row, int l, int hw, int nch, f32x4 (&u)[NR], u32x2 * keep = nullptr) {
@@ -134,7 +134,7 @@ CAMX_DEV float actq_rotate(Src src, int row, int l, int hw, int nch, f32x4 (&u)[
         const int ch = hw + NHW * c;
         f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
         u32x2 kp = {0u, 0u};
-        if (ch < nch) {
+        if ((NHW == 2 && c < NR - 1) || ch < nch) {
             if constexpr (SrcByRound<Src>::value) { static_assert(NHW == 2, "a wave per row"); v = src.at(c); }
             else v = src(row, ch * 128 + 4 * l, kp);
         }
@@ -147,25 +147,29 @@ CAMX_DEV float actq_rotate(Src src, int row, int l, int hw, int nch, f32x4 (&u)[
         const f32x4 in = Src::bf16_valued ? u[c] : rbf4_any(u[c]);                // autocast's bf16 input
         const f32x4 v = rbf4_any(scaled4(hadamard128_l4(in, l, false)));
         u[c] = v;
-        if (hw + NHW * c < nch) amax = fmaxf(amax, absmax4(v));
+        if ((NHW == 2 && c < NR - 1) || hw + NHW * c < nch) amax = fmaxf(amax, absmax4(v));
     }
     return amax;
 }
 
-// The row's scale and what the lanes need to divide by it. p = u * rcp(s) is within 8e-5 of the exact quotient while |p| < 256 (rcp:
-// 1 ulp; one more rounding), the IEEE quotient within 1.6e-5 of it, and half-integers are floats: when p is farther than 3e-4 from
-// every half-integer, rintf of the two agree. A lane that holds a closer value (about one value in 1600) divides, and so does every
-// lane of a row whose largest quotient is not below 256 or not a number (an infinite amax). A NaN among the four values needs no
-// look of its own: its p is a NaN as its quotient is, and the maximum passes over it.
+// The row's scale and what the lanes need to divide by it. For |p| < 2^k, p = u * rcp(s) (rcp: 1 ulp; one more rounding) is within
+// 2.5 * 2^(k - 23) of the exact quotient and the IEEE quotient within 2^(k - 24), and half-integers are floats: when p is farther than
+// their sum from every half-integer, rintf of the two agree. Rows whose quotients stay below 16 (every int4 row with clip near 1) ask
+// for 1e-5 (the sum: 5.8e-6), others below 256 for 3e-4. A lane that holds a closer value divides, and so does every lane of a row
+// whose largest quotient is not below 256 or not a number (an infinite amax). A NaN among the four values needs no look of its own: its
+// p is a NaN as its quotient is, and the maximum passes over it.
 struct RowScale {
-    float s, rcp, lo, hi; bool row_ok;
-    CAMX_DEV RowScale(float s_, float amax, int qmax) : s(s_), rcp(__builtin_amdgcn_rcpf(s_)), lo((float)(-qmax - 1)), hi((float)qmax) { row_ok = amax * rcp < 256.0f; }
+    float s, rcp, lo, hi, most;                          // most: how far p may lie from its integer
+    CAMX_DEV RowScale(float s_, float amax, int qmax) : s(s_), rcp(__builtin_amdgcn_rcpf(s_)), lo((float)(-qmax - 1)), hi((float)qmax) {
+        const float p = amax * rcp;
+        most = p < 16.0f ? 0.49999f : p < 256.0f ? 0.4997f : -1.0f;
+    }
     // clamp(rintf(u / s), lo, hi) of four values; the median of a NaN and two numbers is the smaller number, lo, as fminf(fmaxf(NaN, lo), hi) is
     CAMX_DEV f32x4 quant4(f32x4 u) const {
         const f32x4 p = {u.x * rcp, u.y * rcp, u.z * rcp, u.w * rcp};
         f32x4 r = {rintf(p.x), rintf(p.y), rintf(p.z), rintf(p.w)};
         const float off = fmaxf(fmaxf(fabsf(p.x - r.x), fabsf(p.y - r.y)), fmaxf(fabsf(p.z - r.z), fabsf(p.w - r.w)));
-        if (!(row_ok && !(off > 0.4997f))) { r.x = rintf(u.x / s); r.y = rintf(u.y / s); r.z = rintf(u.z / s); r.w = rintf(u.w / s); }
+        if (off > most || most < 0.0f) { r.x = rintf(u.x / s); r.y = rintf(u.y / s); r.z = rintf(u.z / s); r.w = rintf(u.w / s); }
         return (f32x4){__builtin_amdgcn_fmed3f(r.x, lo, hi), __builtin_amdgcn_fmed3f(r.y, lo, hi), __builtin_amdgcn_fmed3f(r.z, lo, hi), __builtin_amdgcn_fmed3f(r.w, lo, hi)};
     }
     // the low four bits of four quantized values, packed. For values in [-8, 7]: q + 8 is the code with its top bit turned over, and
@@ -196,7 +200,7 @@ CAMX_DEV float row_max(float amax, float * lds) {
 template <int NR, typename Src, int NHW = 8>
 CAMX_DEV void actq_fwd_row(Src src, int row, uint16_t * __restrict__ y, float * __restrict__ s_out, int K, float clip, int qmax,
                            uint16_t * __restrict__ codes, float * lds) {
-    const int tid = threadIdx.x, l = slot_of(tid) & 31, hw = tid >> 5, nch = K / 128;
+    const int tid = threadIdx.x, l = slot_of(tid) & 31, hw = (tid >> 5) & (NHW - 1), nch = K / 128;
     f32x4 u[NR];
     const float amax = row_max<NHW>(actq_rotate<NR, Src, NHW>(src, row, l, hw, nch, u), lds);
     const float s = fmaxf(amax * clip / (float)qmax, 1e-8f);
@@ -464,13 +468,13 @@ struct SinkSiluMul {
 // then one chunk's: round c holds chunks 2 c and 2 c + 1); out, when given, receives round c's result in place of the sink.
 template <int NR, typename Src, typename Sink, int NHW = 8>
 CAMX_DEV void actq_bwd_row(Src src, int row, const uint16_t * __restrict__ g, Sink sink, int K, float clip, int qmax, float * lds16, f32x4 * out = nullptr) {
-    const int tid = threadIdx.x, l = slot_of(tid) & 31, hw = tid >> 5, nch = K / 128;
+    const int tid = threadIdx.x, l = slot_of(tid) & 31, hw = (tid >> 5) & (NHW - 1), nch = K / 128;
     f32x4 u[NR], gv[NR];
 #pragma unroll
     for (int c = 0; c < NR; c++) {
         const int ch = hw + NHW * c;
         u32x2 raw = {0u, 0u};
-        if (ch < nch) raw = *(const u32x2 *)(g + (size_t)row * K + ch * 128 + 4 * l);
+        if ((NHW == 2 && c < NR - 1) || ch < nch) raw = *(const u32x2 *)(g + (size_t)row * K + ch * 128 + 4 * l);
         gv[c] = unpack_bf16x4(raw);
     }
     u32x2 keep[NR];                                      // what the source hands to the sink (the fused SiLU form only)
@@ -487,15 +491,19 @@ CAMX_DEV void actq_bwd_row(Src src, int row, const uint16_t * __restrict__ g, Si
 #pragma unroll
     for (int c = 0; c < NR; c++) {
         if (NHW == 2) dlds = 0.0f;
-        if (hw + NHW * c < nch) {
+        if ((NHW == 2 && c < NR - 1) || hw + NHW * c < nch) {
             const f32x4 t4 = rd.div4(u[c]);
-            uint64_t any = 0;
-#define D_(e) { float m; const float x = ste(t4.e, m); dlds = __builtin_fmaf(gv[c].e, x, dlds); gv[c].e = gv[c].e * m; \
-                const uint64_t tie = __builtin_amdgcn_ballot_w64(fabsf(u[c].e) == amax); any |= tie; \
-                ties_lo += __builtin_popcount((uint32_t)tie); ties_hi += __builtin_popcount((uint32_t)(tie >> 32)); }
+#define D_(e) { float m; const float x = ste(t4.e, m); dlds = __builtin_fmaf(gv[c].e, x, dlds); gv[c].e = gv[c].e * m; }
             CAMX_EACH4(D_)
 #undef D_
-            if (any) tied |= 1u << c;
+            const float most = fmaxf(fmaxf(fabsf(u[c].x), fabsf(u[c].y)), fmaxf(fabsf(u[c].z), fabsf(u[c].w)));
+            if (__builtin_amdgcn_ballot_w64(most == amax) != 0) {          // (few rounds hold such an element)
+                tied |= 1u << c;
+#define T_(e) { const uint64_t tie = __builtin_amdgcn_ballot_w64(fabsf(u[c].e) == amax); \
+                ties_lo += __builtin_popcount((uint32_t)tie); ties_hi += __builtin_popcount((uint32_t)(tie >> 32)); }
+                CAMX_EACH4(T_)
+#undef T_
+            }
         }
         if (NHW == 2) part[NHW == 2 ? c : 0] = dlds;
     }
@@ -519,7 +527,7 @@ CAMX_DEV void actq_bwd_row(Src src, int row, const uint16_t * __restrict__ g, Si
     for (int c = 0; c < NR; c++) {
         const int ch = hw + NHW * c;
         if (out) out[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-        if (ch < nch) {
+        if ((NHW == 2 && c < NR - 1) || ch < nch) {
             f32x4 d = gv[c];
             if (tied & (1u << c)) {                      // wave-uniform: a row has few such elements, most rounds skip this
 #define V_(e) if (fabsf(u[c].e) == amax && u[c].e != 0.0f) d.e += u[c].e > 0.0f ? coef : -coef;
@@ -677,8 +685,8 @@ struct AbTerm {
 };
 
 // NHW = 8: a 256-thread workgroup per row (NR rounds of 1024 values); NHW = 2: one wave per row for rows of at most 1024 values (NR
-// rounds of 256): a lane then holds 16 values instead of 4, and what every lane computes once per row (the square root, the
-// divisions, the reductions' tails, 900 instructions in all) is spread over four times as many values.
+// rounds of 256) without projections: a lane then holds 16 values instead of 4, and what every lane computes once per row (the square
+// root, the divisions, the reductions' tails) is spread over four times as many values.
 // The projections: wave w takes rows w, w + W, ... of wab (W waves per row), up to four of them at a time so that their loads fly together,
 // each under the 256-thread tree (a lane holds the logical threads 4 lane .. 4 lane + 3, which add their elements 256 apart in
 // order); rows of at most 2048 values keep bf16(h) in registers.
@@ -714,12 +722,7 @@ __global__ void __launch_bounds__(32 * NHW) block_entry_fwd_k(const float * x, c
         src.rstd = rstd;
         if (threadIdx.x == 0 && rstd_out) rstd_out[row] = rstd;
         actq_fwd_row<NR, RmsRegSrc<NR>, NHW>(src, row, y, s, d, clip, qmax, codes, lds);
-        if (nab == 0) return;
-#pragma unroll
-        for (int i = 0; i < NA; i++) {
-            const f32x4 a = src.at(i % NR);
-            hk[KEEP ? i : 0] = 256 * i + 4 * lane < d ? (f32x4){rbf(a.x), rbf(a.y), rbf(a.z), rbf(a.w)} : (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-        }
+        return;
     } else {
         const float ss = row_tree_sum(SqTerm{xr}, d, &slot);
         rstd = rsqrt_exact(ss / (float)d + eps);
@@ -728,7 +731,7 @@ __global__ void __launch_bounds__(32 * NHW) block_entry_fwd_k(const float * x, c
         if (nab == 0) return;
     }
     const AbTerm term{xr, nw, rstd, wab};
-    if (KEEP && NHW != 2) {
+    if (KEEP) {
 #pragma unroll
         for (int i = 0; i < NA; i++) { const int k = 256 * i + 4 * lane; hk[KEEP ? i : 0] = k < d ? term(k) : (f32x4){0.0f, 0.0f, 0.0f, 0.0f}; }
     }
@@ -765,14 +768,163 @@ __global__ void __launch_bounds__(32 * NHW) block_entry_fwd_k(const float * x, c
     }
 }
 
+// ---- block entry with projections, rows of at most 1024 values: a wave per row, four rows share the projections on the matrix cores ----
+// Bound by instruction issue: with the projections as vector multiply-adds of a row's own wave, they, the conversions of wab and sixteen
+// reductions of 256 logical threads were two thirds of a row's instructions (32768 rows x 1024 values, 16 projections: 114 us, this
+// kernel 84; 512 rows: 11.6 and 7.0. Four rows in the registers of one wave, wab as fp32 in LDS: 76 and 22). A K = 1 matrix instruction
+// (v_mfma_f32_4x4x1: 16 blocks of 4 x 4 single multiply-adds, each rounded like fmaf) computes for 16 logical threads t the terms of
+// 4 rows x 4 projections, so a thread's chain over its elements t, t + 256, .. is a chain of NR such instructions in the same order.
+// A workgroup's four waves own a row each and hand bf16(h) on through LDS; then wave w takes projections 4 w .. 4 w + 3 of all four rows.
+// Roles: block Q (lanes 4 Q .. 4 Q + 3) is the logical threads 16 Q + 4 n + k, for one (n, k) per instruction. A: lane 4 Q + i holds row
+// i's value there. B: lane 4 Q + j holds projection j's, from the caches; odd blocks hold their four
+// projections in reverse, so that the tree's first step (t ^ 16, the other block of a pair) is a row_half_mirror. The following steps
+// (t ^ 8, 4, 2, 1) pair n and k: registers. The eight group sums of a (row, projection) meet in LDS, where one lane adds them in order.
+CAMX_DEV f32x4 mirror4(f32x4 v) { return (f32x4){lane_xor4(v.x), lane_xor4(v.y), lane_xor4(v.z), lane_xor4(v.w)}; }      // row_half_mirror
+CAMX_DEV float bf_lo(uint32_t v) { return __builtin_bit_cast(float, v << 16); }
+CAMX_DEV float bf_hi(uint32_t v) { return __builtin_bit_cast(float, v & 0xffff0000u); }
+template <int NR>
+__global__ void __launch_bounds__(256, 4) block_entry_fwd_quad(const float * __restrict__ x, const float * __restrict__ nw, const uint16_t * __restrict__ wab, int nab, float eps,
+                                                               uint16_t * __restrict__ y, float * __restrict__ s_out, uint16_t * __restrict__ codes, uint16_t * __restrict__ ab,
+                                                               float * __restrict__ rstd_out, int d, float clip, int qmax, int M) {
+    constexpr int HS = 128 * NR + 4;                     // words of a row of packed pairs; + 4: the four rows of a read fall on different banks
+    __shared__ __attribute__((aligned(16))) uint32_t hbuf[4][HS];
+    __shared__ __attribute__((aligned(16))) float gsum[4][4 * 4 * 8];         // [wave][row][projection][group]
+    const int lraw = threadIdx.x & 63, lane = slot_of(lraw), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int Q = lraw >> 2, odd = Q & 1, jp = odd ? 3 - (lraw & 3) : lraw & 3;      // the lane's block and its projection of the wave's four
+    f32x4 xk[NR], wk[NR];
+    const int r0 = 4 * blockIdx.x, row = r0 + wave;
+#pragma unroll
+    for (int c = 0; c < NR; c++) {
+        const int k = 256 * c + 4 * lane;
+        xk[c] = wk[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+        if (c < NR - 1 || k < d) { xk[c] = __builtin_nontemporal_load((const f32x4 *)(x + (size_t)min(row, M - 1) * d + k)); wk[c] = *(const f32x4 *)(nw + k); }
+    }
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int c = 0; c < NR; c++) {                   // (padding adds +0 to a sum of squares)
+        const f32x4 v = xk[c];
+        acc.x = __builtin_fmaf(v.x, v.x, acc.x); acc.y = __builtin_fmaf(v.y, v.y, acc.y); acc.z = __builtin_fmaf(v.z, v.z, acc.z); acc.w = __builtin_fmaf(v.w, v.w, acc.w);
+    }
+    const float ss = wave_groups_in_order(group32_sum(acc));
+    const float rstd = rsqrt_exact(ss / (float)d + eps);
+    u32x2 hb[NR];
+#pragma unroll
+    for (int c = 0; c < NR; c++) {
+        const f32x4 v = xk[c], w = wk[c];
+        hb[c] = (u32x2){hw_pk_bf16(v.x * rstd * w.x, v.y * rstd * w.y), hw_pk_bf16(v.z * rstd * w.z, v.w * rstd * w.w)};
+        *(u32x2 *)&hbuf[wave][128 * c + 2 * lane] = hb[c];
+    }
+    f32x4 u[NR];
+    float amax = 0.0f;
+#pragma unroll
+    for (int c = 0; c < NR; c++) {
+        u[c] = rbf4_any(scaled4(hadamard128_l4(unpack_bf16x4(hb[c]), lane & 31, false)));
+        amax = fmaxf(fmaxf(amax, fmaxf(fabsf(u[c].x), fabsf(u[c].y))), fmaxf(fabsf(u[c].z), fabsf(u[c].w)));
+    }
+    amax = wave_max64(amax);
+    const float s = fmaxf(amax * clip / (float)qmax, 1e-8f);
+    const RowScale rs(s, amax, qmax);
+    if (row < M) {                                   // (wave-uniform)
+        if (lraw == 0) { if (s_out) s_out[row] = s; if (rstd_out) rstd_out[row] = rstd; }
+#pragma unroll
+        for (int c = 0; c < NR; c++) {
+            const int k = 256 * c + 4 * lane;
+            const f32x4 q = rs.quant4(u[c]);
+            if (c < NR - 1 || k < d) {
+                if (y) *(u32x2 *)(y + (size_t)row * d + k) = pack_f2bf_x4((f32x4){q.x * s, q.y * s, q.z * s, q.w * s});
+                if (codes) codes[((size_t)row * d + k) >> 2] = (uint16_t)rs.nibbles4(q);
+            }
+        }
+    }
+    u32x2 B[NR][4];                                      // (from the caches: 32 KiB for a workgroup)
+#pragma unroll
+    for (int c = 0; c < NR; c++)
+#pragma unroll
+        for (int n = 0; n < 4; n++) {
+            const int k = 256 * c + 16 * Q + 4 * n;
+            B[c][n] = (u32x2){0u, 0u};
+            if (4 * wave + jp < nab && (c < NR - 1 || k < d)) B[c][n] = *(const u32x2 *)(wab + (size_t)(4 * wave + jp) * d + k);
+        }
+    __syncthreads();
+    if (4 * wave < nab) {                            // (uniform in a wave)
+        u32x4 A[NR][2];                              // row (lane & 3): elements 256 c + 16 Q .. + 15, packed pairs
+#pragma unroll
+        for (int c = 0; c < NR; c++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) A[c][h] = *(const u32x4 *)&hbuf[lraw & 3][128 * c + 8 * Q + 4 * h];
+        f32x4 sum[2];                                // [k & 1]; a word per row
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++) {
+            const int k = kk == 1 ? 2 : kk == 2 ? 1 : kk;        // 0, 2, 1, 3: the pairs of t ^ 2
+            f32x4 a[4];
+#pragma unroll
+            for (int n = 0; n < 4; n++) a[n] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int c = 0; c < NR; c++)
+#pragma unroll
+                for (int n = 0; n < 4; n++) {
+                    const uint32_t av = A[c][n >> 1][2 * (n & 1) + (k >> 1)], bv = k >> 1 ? B[c][n].y : B[c][n].x;
+                    a[n] = __builtin_amdgcn_mfma_f32_4x4x1f32(k & 1 ? bf_hi(av) : bf_lo(av), k & 1 ? bf_hi(bv) : bf_lo(bv), a[n], 0, 0, 0);
+                }
+            const f32x4 t0 = a[0] + mirror4(a[0]), t1 = a[1] + mirror4(a[1]), t2 = a[2] + mirror4(a[2]), t3 = a[3] + mirror4(a[3]);      // t ^ 16
+            const f32x4 m0 = t0 + t2, m1 = t1 + t3;  // t ^ 8
+            const f32x4 w = m0 + m1;                 // t ^ 4
+            sum[k & 1] = k >> 1 ? sum[k & 1] + w : w;            // t ^ 2
+        }
+        const f32x4 g = sum[0] + sum[1];             // t ^ 1; a pair's blocks hold the same sums: the even one hands on rows 0 and 1, the odd one 2 and 3
+        float * o = gsum[wave] + ((odd ? 8 : 0) + jp) * 8 + (Q >> 1);
+        o[0] = odd ? g.z : g.x;
+        o[4 * 8] = odd ? g.w : g.y;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier();
+        const int rr = r0 + (lraw >> 2), j = 4 * wave + (lraw & 3);
+        if (lraw < 16 && j < nab && rr < M) {
+            const f32x4 a = *(const f32x4 *)(gsum[wave] + 8 * lraw), b = *(const f32x4 *)(gsum[wave] + 8 * lraw + 4);
+            float tot = 0.0f;
+            tot += a.x; tot += a.y; tot += a.z; tot += a.w; tot += b.x; tot += b.y; tot += b.z; tot += b.w;
+            ab[(size_t)rr * nab + j] = f2bf(tot);
+        }
+    }
+}
+
+// dx = rstd (dh w - xhat mean(dh w xhat)) of one row from the lane's registers
+template <int NR>
+CAMX_DEV void rms_bwd_row(const RmsRegSrc<NR> & src, const f32x4 (&dh)[NR], float * dx, int d, int la) {
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f}, gw[NR], xh[NR];
+#pragma unroll
+    for (int c = 0; c < NR; c++) {
+        const int k = 256 * c + 4 * la;
+        gw[c] = xh[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+        if (c < NR - 1 || k < d) {
+            const f32x4 w = src.wk[c], xv = src.xk[c];
+            gw[c] = (f32x4){dh[c].x * w.x, dh[c].y * w.y, dh[c].z * w.z, dh[c].w * w.w};
+            xh[c] = (f32x4){xv.x * src.rstd, xv.y * src.rstd, xv.z * src.rstd, xv.w * src.rstd};
+            acc.x = __builtin_fmaf(gw[c].x, xh[c].x, acc.x); acc.y = __builtin_fmaf(gw[c].y, xh[c].y, acc.y);
+            acc.z = __builtin_fmaf(gw[c].z, xh[c].z, acc.z); acc.w = __builtin_fmaf(gw[c].w, xh[c].w, acc.w);
+        }
+    }
+    const float gs = group32_sum(acc);                   // the 32 logical threads of a group, then the eight groups in order
+    float dot = lane_read(gs, 0);
+#pragma unroll
+    for (int q = 1; q < 8; q++) dot += lane_read(gs, 8 * q);
+    dot = dot / (float)d;
+#pragma unroll
+    for (int c = 0; c < NR; c++) {
+        const int k = 256 * c + 4 * la;
+        if (c < NR - 1 || k < d) {
+            f32x4 r;
+            r.x = src.rstd * (gw[c].x - xh[c].x * dot); r.y = src.rstd * (gw[c].y - xh[c].y * dot);
+            r.z = src.rstd * (gw[c].z - xh[c].z * dot); r.w = src.rstd * (gw[c].w - xh[c].w * dot);
+            *(f32x4 *)(dx + k) = r;
+        }
+    }
+}
 // dh = actq backward of dy, plus the two projection groups' input gradients (wab rows [0, nab / 2) and [nab / 2, nab), each
-// group's sum rounded to bf16); then the RMSNorm backward dx = rstd (dh w - xhat mean(dh w xhat)), xhat = x rstd. d <= 1024.
-// One wave per row, NR = ceil(d / 256) rounds: lane (slot la) holds elements 256 c + 4 la .. + 3 of round c through all three steps,
-// i.e. the logical threads 4 la .. 4 la + 3 of the 256-thread tree of the dot product (thread t owns elements t, t + 256, ...).
+// group's sum rounded to bf16); then the RMSNorm backward. d <= 1024. One wave per row, NR = ceil(d / 256) rounds: lane (slot la) holds
+// elements 256 c + 4 la .. + 3 of round c through all steps, i.e. the logical threads 4 la .. 4 la + 3 of the 256-thread tree of the dot
+// product (thread t owns elements t, t + 256, ...). This kernel: no projections.
 struct SinkNone { CAMX_DEV void operator()(int, int, f32x4, u32x2) const {} };
 template <int NR>
-__global__ void __launch_bounds__(64) block_entry_bwd_k(const float * x, const float * nw, const float * rstd_in, const uint16_t * wab, int nab,
-                                                        const uint16_t * dy, const uint16_t * dab, float * dx, int d, float clip, int qmax) {
+__global__ void __launch_bounds__(64) block_entry_bwd_k(const float * x, const float * nw, const float * rstd_in, const uint16_t * dy, float * dx, int d, float clip, int qmax) {
     const int row = blockIdx.x, la = slot_of(threadIdx.x);
     const float rstd = rstd_in[row];
     const float * xr = x + (size_t)row * d;
@@ -786,72 +938,75 @@ __global__ void __launch_bounds__(64) block_entry_bwd_k(const float * x, const f
     src.rstd = rstd;
     f32x4 dh[NR];
     actq_bwd_row<NR, RmsRegSrc<NR>, SinkNone, 2>(src, row, dy, SinkNone{}, d, clip, qmax, nullptr, dh);
-    if (nab) {                                           // the projections' part of dh
-        const int half = nab / 2;
-        float dabs[2][8];                                // the row's dab by group, the same in every lane: scalar registers
+    rms_bwd_row(src, dh, dx + (size_t)row * d, d, la);
+}
+
+// The same for nab > 0 with the projections' part on the matrix cores (as vector multiply-adds of the row's own wave 139 us at 32768 x
+// 1024 with 16 projections, this kernel 113; 512 rows: 12.3 and 8.7): a workgroup's four waves own a row each, and wave w first computes
+// that part for columns 256 w .. 256 w + 255 of all four rows. A K = 1 instruction adds one j's term dab[row][j] wab[j][column] (rounded
+// like fmaf) for 4 rows x 64 columns: block Q's four columns are its lanes' own, so with A = dab (lane 4 Q + i: row i) and B = a lane's
+// column of wab, D holds a lane's column with a word per row. The two groups' sums,
+// rounded to bf16, reach the rows' owners through LDS.
+template <int NR>
+__global__ void __launch_bounds__(256, 4) block_entry_bwd_quad(const float * x, const float * __restrict__ nw, const float * __restrict__ rstd_in, const uint16_t * __restrict__ wab,
+                                                               int nab, const uint16_t * __restrict__ dy, const uint16_t * __restrict__ dab, float * dx, int d, float clip, int qmax, int M) {
+    __shared__ __attribute__((aligned(16))) uint32_t pbuf[4][2][128 * NR];                // [row][group][pairs of columns]
+    const int lraw = threadIdx.x & 63, la = slot_of(lraw), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = nab / 2;
+    RmsRegSrc<NR> src;
+#pragma unroll
+    for (int c = 0; c < NR; c++) {
+        const int k = 256 * c + 4 * la;
+        src.wk[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+        if (c < NR - 1 || k < d) src.wk[c] = *(const f32x4 *)(nw + k);
+    }
+    const int r0 = 4 * blockIdx.x;
+    const int row = min(r0 + wave, M - 1);           // (a wave past the end repeats the last row and stores nothing)
+#pragma unroll
+    for (int c = 0; c < NR; c++) {
+        const int k = 256 * c + 4 * la;
+        src.xk[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+        if (c < NR - 1 || k < d) src.xk[c] = __builtin_nontemporal_load((const f32x4 *)(x + (size_t)row * d + k));
+    }
+    src.rstd = rstd_in[row];
+    if (wave < NR) {
+        u32x2 B[2][8];
 #pragma unroll
         for (int h = 0; h < 2; h++)
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-                const uint32_t w = j < half ? (uint32_t)__builtin_amdgcn_readfirstlane((int)dab[(size_t)row * nab + h * half + j]) : 0u;
-                dabs[h][j] = __builtin_bit_cast(float, w << 16);
+                const int k = 256 * wave + 4 * la;
+                B[h][j] = (u32x2){0u, 0u};
+                if (j < half && k < d) B[h][j] = *(const u32x2 *)(wab + (size_t)(h * half + j) * d + k);
             }
+        const uint16_t * ar = dab + (size_t)min(r0 + (lraw & 3), M - 1) * nab;
 #pragma unroll
-        for (int c = 0; c < NR; c++) {
-            const int k = 256 * c + 4 * la;
-            if (k < d) {
-                f32x4 p[2];                              // rows [0, half) of wab add into p[0], [half, nab) into p[1], each in order
+        for (int h = 0; h < 2; h++) {
+            f32x4 acc[4];
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    u32x2 wv[8];
+            for (int k = 0; k < 4; k++) acc[k] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                    for (int j = 0; j < 8; j++) { wv[j] = (u32x2){0u, 0u}; if (j < half) wv[j] = *(const u32x2 *)(wab + (size_t)(h * half + j) * d + k); }
-                    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                    for (int j = 0; j < 8; j++) {
-                        if (j < half) {                  // (uniform)
-                            const f32x4 w = unpack_bf16x4(wv[j]);
-                            const float cj = dabs[h][j];
-                            acc.x = __builtin_fmaf(cj, w.x, acc.x); acc.y = __builtin_fmaf(cj, w.y, acc.y); acc.z = __builtin_fmaf(cj, w.z, acc.z); acc.w = __builtin_fmaf(cj, w.w, acc.w);
-                        }
-                    }
-                    p[h] = acc;
+            for (int j = 0; j < 8; j++) {
+                if (j < half) {                      // (uniform)
+                    const float av = bf2f(ar[h * half + j]);
+                    acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(av, bf_lo(B[h][j].x), acc[0], 0, 0, 0);
+                    acc[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(av, bf_hi(B[h][j].x), acc[1], 0, 0, 0);
+                    acc[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(av, bf_lo(B[h][j].y), acc[2], 0, 0, 0);
+                    acc[3] = __builtin_amdgcn_mfma_f32_4x4x1f32(av, bf_hi(B[h][j].y), acc[3], 0, 0, 0);
                 }
-                const f32x4 ra = rbf4_canon(p[0]), rb = rbf4_canon(p[1]);
-                f32x4 g = dh[c];
-                g.x = (g.x + ra.x) + rb.x; g.y = (g.y + ra.y) + rb.y; g.z = (g.z + ra.z) + rb.z; g.w = (g.w + ra.w) + rb.w;
-                dh[c] = g;
             }
+#pragma unroll
+            for (int r = 0; r < 4; r++) *(u32x2 *)&pbuf[r][h][128 * wave + 2 * la] = pack_f2bf_x4((f32x4){acc[0][r], acc[1][r], acc[2][r], acc[3][r]});
         }
     }
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f}, gw[NR], xh[NR];
+    f32x4 dh[NR];
+    actq_bwd_row<NR, RmsRegSrc<NR>, SinkNone, 2>(src, row, dy, SinkNone{}, d, clip, qmax, nullptr, dh);
+    __syncthreads();
 #pragma unroll
     for (int c = 0; c < NR; c++) {
-        const int k = 256 * c + 4 * la;
-        gw[c] = xh[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-        if (k < d) {
-            const f32x4 w = src.wk[c], xv = src.xk[c];
-            gw[c] = (f32x4){dh[c].x * w.x, dh[c].y * w.y, dh[c].z * w.z, dh[c].w * w.w};
-            xh[c] = (f32x4){xv.x * rstd, xv.y * rstd, xv.z * rstd, xv.w * rstd};
-            acc.x = __builtin_fmaf(gw[c].x, xh[c].x, acc.x); acc.y = __builtin_fmaf(gw[c].y, xh[c].y, acc.y);
-            acc.z = __builtin_fmaf(gw[c].z, xh[c].z, acc.z); acc.w = __builtin_fmaf(gw[c].w, xh[c].w, acc.w);
-        }
+        const f32x4 ra = unpack_bf16x4(*(const u32x2 *)&pbuf[wave][0][128 * c + 2 * la]), rb = unpack_bf16x4(*(const u32x2 *)&pbuf[wave][1][128 * c + 2 * la]);
+        dh[c].x = (dh[c].x + ra.x) + rb.x; dh[c].y = (dh[c].y + ra.y) + rb.y; dh[c].z = (dh[c].z + ra.z) + rb.z; dh[c].w = (dh[c].w + ra.w) + rb.w;
     }
-    const float gs = group32_sum(acc);                   // the 32 logical threads of a group, then the eight groups in order
-    float dot = lane_read(gs, 0);
-#pragma unroll
-    for (int q = 1; q < 8; q++) dot += lane_read(gs, 8 * q);
-    dot = dot / (float)d;
-#pragma unroll
-    for (int c = 0; c < NR; c++) {
-        const int k = 256 * c + 4 * la;
-        if (k < d) {
-            f32x4 r;
-            r.x = rstd * (gw[c].x - xh[c].x * dot); r.y = rstd * (gw[c].y - xh[c].y * dot);
-            r.z = rstd * (gw[c].z - xh[c].z * dot); r.w = rstd * (gw[c].w - xh[c].w * dot);
-            *(f32x4 *)(dx + (size_t)row * d + k) = r;
-        }
-    }
+    if (r0 + wave < M) rms_bwd_row(src, dh, dx + (size_t)row * d, d, la);
 }
 
 __attribute__((visibility("hidden"))) int silu_luts_get(hipStream_t st, const uint16_t ** lut, const uint16_t ** small);       // quant.hip
@@ -935,6 +1090,16 @@ int camx_block_entry_fwd(const float * x, const float * nw, const uint16_t * wab
     if (!x || !nw || (!y && !codes) || actq_check(d, qmax, M) || nab < 0 || nab > 16 || (nab && (!wab || !ab)) || ((uintptr_t)x & 15) ||
         ((uintptr_t)nw & 15) || ((uintptr_t)wab & 7) || ((uintptr_t)y & 7) || ((uintptr_t)codes & 1)) return CAMX_EINVAL;
     if (M == 0) return CAMX_OK;
+    if (d <= 1024 && nab > 0) {                          // four rows share the projections on the matrix cores
+        const dim3 grid((unsigned)(((long)M + 3) / 4)), block(256);
+        switch ((d + 255) / 256) {
+            case 1: block_entry_fwd_quad<1><<<grid, block, 0, st>>>(x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax, M); break;
+            case 2: block_entry_fwd_quad<2><<<grid, block, 0, st>>>(x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax, M); break;
+            case 3: block_entry_fwd_quad<3><<<grid, block, 0, st>>>(x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax, M); break;
+            default: block_entry_fwd_quad<4><<<grid, block, 0, st>>>(x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax, M); break;
+        }
+        CAMX_LAUNCH_RET();
+    }
     if (d <= 1024) {                                     // one wave per row, rounds of 256 values
         switch ((d + 255) / 256) {
             case 1: block_entry_fwd_k<1, 2><<<dim3(M), dim3(64), 0, st>>>(x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax); break;
@@ -983,11 +1148,21 @@ int camx_block_entry_bwd(const float * x, const float * nw, const float * rstd, 
     if (!x || !nw || !rstd || !dy || !dx || actq_check(d, qmax, M) || d > 1024 || nab < 0 || nab > 16 || (nab & 1) || (nab && (!wab || !dab)) ||
         ((uintptr_t)x & 15) || ((uintptr_t)nw & 15) || ((uintptr_t)dy & 7) || ((uintptr_t)dx & 15) || ((uintptr_t)wab & 7)) return CAMX_EINVAL;
     if (M == 0) return CAMX_OK;
+    if (nab > 0) {                                       // four rows share the projections' part on the matrix cores
+        const dim3 grid((unsigned)(((long)M + 3) / 4)), block(256);
+        switch ((d + 255) / 256) {
+            case 1: block_entry_bwd_quad<1><<<grid, block, 0, st>>>(x, nw, rstd, wab, nab, dy, dab, dx, d, clip, qmax, M); break;
+            case 2: block_entry_bwd_quad<2><<<grid, block, 0, st>>>(x, nw, rstd, wab, nab, dy, dab, dx, d, clip, qmax, M); break;
+            case 3: block_entry_bwd_quad<3><<<grid, block, 0, st>>>(x, nw, rstd, wab, nab, dy, dab, dx, d, clip, qmax, M); break;
+            default: block_entry_bwd_quad<4><<<grid, block, 0, st>>>(x, nw, rstd, wab, nab, dy, dab, dx, d, clip, qmax, M); break;
+        }
+        CAMX_LAUNCH_RET();
+    }
     switch ((d + 255) / 256) {
-        case 1: block_entry_bwd_k<1><<<dim3(M), dim3(64), 0, st>>>(x, nw, rstd, wab, nab, dy, dab, dx, d, clip, qmax); break;
-        case 2: block_entry_bwd_k<2><<<dim3(M), dim3(64), 0, st>>>(x, nw, rstd, wab, nab, dy, dab, dx, d, clip, qmax); break;
-        case 3: block_entry_bwd_k<3><<<dim3(M), dim3(64), 0, st>>>(x, nw, rstd, wab, nab, dy, dab, dx, d, clip, qmax); break;
-        default: block_entry_bwd_k<4><<<dim3(M), dim3(64), 0, st>>>(x, nw, rstd, wab, nab, dy, dab, dx, d, clip, qmax); break;
+        case 1: block_entry_bwd_k<1><<<dim3(M), dim3(64), 0, st>>>(x, nw, rstd, dy, dx, d, clip, qmax); break;
+        case 2: block_entry_bwd_k<2><<<dim3(M), dim3(64), 0, st>>>(x, nw, rstd, dy, dx, d, clip, qmax); break;
+        case 3: block_entry_bwd_k<3><<<dim3(M), dim3(64), 0, st>>>(x, nw, rstd, dy, dx, d, clip, qmax); break;
+        default: block_entry_bwd_k<4><<<dim3(M), dim3(64), 0, st>>>(x, nw, rstd, dy, dx, d, clip, qmax); break;
     }
     CAMX_LAUNCH_RET();
 }

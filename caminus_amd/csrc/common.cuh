@@ -33,11 +33,11 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 // lane -> the logical slot it holds (and back: the map is an involution)
 CAMX_DEV int slot_of(int lane) { const int s = lane & 7; return (lane & ~7) | (s < 4 ? s : 11 - s); }
 
-// ---- slot exchanges (every lane of the exchanging group must be active) ---------------------------------------------------
-CAMX_DEV float lane_xor1(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, false)); }   // quad_perm [1,0,3,2]
-CAMX_DEV float lane_xor2(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x4E, 0xf, 0xf, false)); }   // quad_perm [2,3,0,1]
-CAMX_DEV float lane_xor4(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x141, 0xf, 0xf, false)); }  // row_half_mirror
-CAMX_DEV float lane_xor8(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x128, 0xf, 0xf, false)); }  // row_ror:8
+// ---- slot exchanges (every lane of the exchanging group must be active; in this form the compiler folds the move into its consumer) ---------------------------------------------------
+CAMX_DEV float lane_xor1(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, true)); }   // quad_perm [1,0,3,2]
+CAMX_DEV float lane_xor2(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xf, 0xf, true)); }   // quad_perm [2,3,0,1]
+CAMX_DEV float lane_xor4(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xf, 0xf, true)); }  // row_half_mirror
+CAMX_DEV float lane_xor8(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf, 0xf, true)); }  // row_ror:8
 CAMX_DEV float lane_xor16(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, v), 0x401f)); }              // swizzle SWAP,16
 CAMX_DEV float lane_read(float v, int lane) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane)); }
 
@@ -114,13 +114,12 @@ CAMX_DEV u32x2 pack_bf16x4_rne(f32x4 v) {  // to_bf16 of four values, packed lit
     } else { r.x = hw_pk_bf16(v.x, v.y); r.y = hw_pk_bf16(v.z, v.w); }
     return r;
 }
-CAMX_DEV u32x2 pack_f2bf_x4(f32x4 v) {     // f2bf of four values (NaN -> 0x7fc0), packed little-endian
-    u32x2 r;
+CAMX_DEV u32x2 pack_f2bf_x4(f32x4 v) {     // f2bf of four values (NaN -> 0x7fc0, the hardware's result for a NaN with those bits), packed little-endian
     if (__builtin_expect(any_nan4(v), 0)) {
-        r.x = (uint32_t)f2bf(v.x) | ((uint32_t)f2bf(v.y) << 16);
-        r.y = (uint32_t)f2bf(v.z) | ((uint32_t)f2bf(v.w) << 16);
-    } else { r.x = hw_pk_bf16(v.x, v.y); r.y = hw_pk_bf16(v.z, v.w); }
-    return r;
+        const float q = __builtin_bit_cast(float, 0x7fc00000u);
+        v.x = v.x != v.x ? q : v.x; v.y = v.y != v.y ? q : v.y; v.z = v.z != v.z ? q : v.z; v.w = v.w != v.w ? q : v.w;
+    }
+    return (u32x2){hw_pk_bf16(v.x, v.y), hw_pk_bf16(v.z, v.w)};
 }
 CAMX_DEV u32x2 pack_f16x4(f32x4 v) {
     u32x2 r;

@@ -217,6 +217,29 @@ def test_actq_autograd_wrappers():
     assert gu.grad.shape == (M, 2048) and gu.grad.dtype == torch.bfloat16 and torch.isfinite(gu.grad.float()).all()
 
 
+@pytest.mark.parametrize('M,d,nab', [(1, 1024, 16), (2, 384, 14), (3, 256, 2), (5, 128, 4), (4, 768, 12), (1023, 1024, 10)])
+def test_block_entry_rows_shared_by_a_workgroup(M, d, nab):
+    """four rows share the projections: row counts around multiples of four, projection counts around the waves' four, every round
+    count; a row of zeros, one with an infinity and one of subnormals (their products and sums round like fmaf)"""
+    rng = np.random.default_rng(77 + M + d)
+    x = outliers(rng, (M, d)); nw = (0.5 + rng.random(d)).astype(np.float32); wab = O.f2bf(rng.standard_normal((nab, d)) * 0.05)
+    if M > 1: x[1] = 0
+    if M > 2: x[2, 3] = np.inf
+    if M > 3: x[3] *= 1e-38
+    ry, rs, rc, rab, rstd = O.block_entry_fwd(x, nw, wab, 1e-6)
+    y = dev(np.zeros((M, d), np.uint16)); s = dev(np.zeros(M, np.float32)); c = dev(np.zeros((M, d // 2), np.uint8))
+    ab = dev(np.full((M + 4, nab), 0x1234, np.uint16)); rstd_d = dev(np.zeros(M, np.float32))
+    call('camx_block_entry_fwd', ptr(dev(x)), ptr(dev(nw)), ptr(dev(wab)), I(nab), F(1e-6), ptr(y), ptr(s), ptr(c), ptr(ab), ptr(rstd_d), I(d), F(1.0), I(7), I(M))
+    assert bits_equal(host(rstd_d), rstd) and bits_equal(host(s), rs) and bits_equal(host(c), rc) and bits_equal(host(y, np.uint16), ry)
+    assert bits_equal(host(ab, np.uint16)[:M], rab) and (host(ab, np.uint16)[M:] == 0x1234).all()
+    x[2 % M] = 1.0                                                             # (finite rows for the backward)
+    rstd = O.block_entry_fwd(x, nw, wab, 1e-6)[4]
+    dy = O.f2bf(rng.standard_normal((M, d)).astype(np.float32)); dab = O.f2bf(rng.standard_normal((M, nab)).astype(np.float32))
+    dx = dev(np.full((M + 4, d), 7.0, np.float32))
+    call('camx_block_entry_bwd', ptr(dev(x)), ptr(dev(nw)), ptr(dev(rstd)), ptr(dev(wab)), I(nab), ptr(dev(dy)), ptr(dev(dab)), ptr(dx), I(d), F(1.0), I(7), I(M))
+    assert bits_equal(host(dx)[:M], O.block_entry_bwd(x, nw, rstd, wab, dy, dab)) and (host(dx)[M:] == 7.0).all()
+
+
 def test_block_entry_gradient_of_one_output():
     """an output nothing depends on has a zero gradient: y alone, ab alone"""
     import torch
