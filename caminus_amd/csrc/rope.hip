@@ -1084,13 +1084,21 @@ static void launch_nr(const NrArgs & a, int io, hipStream_t st) {
     const int es = io ? 2 : 4;
     const bool vec = (a.D & 3) == 0 && (a.head_stride & 3) == 0 && ((uintptr_t)a.x & (4 * es - 1)) == 0 && ((uintptr_t)a.out & (4 * es - 1)) == 0;
     const bool vec8 = (a.head_stride & 7) == 0 && ((uintptr_t)a.x & 15) == 0 && ((uintptr_t)a.out & 15) == 0 && ((uintptr_t)a.w & 15) == 0;
-    if (vec8 && a.D == 256 && a.heads >= 8 && (long)a.T * a.heads >= 4096 && a.nrot >= 16 && (a.nrot & (a.nrot - 1)) == 0) {
+    // (from four heads a token: 2048 tokens x 4 heads of 256 took 10.0 us as a wave per head with a cos / sin of its own, 4 heads of 128 9.5
+    // and 5.2 as below; two heads of 256: 6.2, below 7.7)
+    if (vec8 && a.D == 256 && a.heads >= 4 && (long)a.T * a.heads >= 4096 && a.nrot >= 16 && (a.nrot & (a.nrot - 1)) == 0) {
 #define NR_W8(XL) (io ? qk_nr_tokens_w8<true, XL, 3><<<dim3(a.T), dim3(256), 0, st>>>(a) : qk_nr_tokens_w8<false, XL, 3><<<dim3(a.T), dim3(256), 0, st>>>(a))
+#define NR_W4(XL) (io ? qk_nr_tokens_w8<true, XL, 1><<<dim3(a.T), dim3(128), 0, st>>>(a) : qk_nr_tokens_w8<false, XL, 1><<<dim3(a.T), dim3(128), 0, st>>>(a))
+        if (a.heads <= 4) {                                            // (two waves hold the token's heads)
+            switch (a.nrot) { case 16: NR_W4(1); break; case 32: NR_W4(2); break; case 64: NR_W4(4); break; case 128: NR_W4(8); break; default: NR_W4(16); break; }
+            return;
+        }
+#undef NR_W4
         switch (a.nrot) { case 16: NR_W8(1); break; case 32: NR_W8(2); break; case 64: NR_W8(4); break; case 128: NR_W8(8); break; default: NR_W8(16); break; }
 #undef NR_W8
         return;
     }
-    if (vec && a.heads >= 8 && (long)a.T * a.heads >= 4096 && a.D <= 256 && a.nrot >= 8 && a.nrot <= a.D && (a.nrot & (a.nrot - 1)) == 0) {
+    if (vec && a.heads >= (((uintptr_t)a.w & 15) ? 8 : 4) && (long)a.T * a.heads >= 4096 && a.D <= 256 && a.nrot >= 8 && a.nrot <= a.D && (a.nrot & (a.nrot - 1)) == 0) {
 #define NR_FAST(XL) (io ? qk_nr_tokens_fast<true, XL><<<dim3(a.T), dim3(256), 0, st>>>(a) : qk_nr_tokens_fast<false, XL><<<dim3(a.T), dim3(256), 0, st>>>(a))
         switch (a.nrot) { case 8: NR_FAST(1); break; case 16: NR_FAST(2); break; case 32: NR_FAST(4); break; case 64: NR_FAST(8); break;
                           case 128: NR_FAST(16); break; default: NR_FAST(32); break; }

@@ -75,6 +75,25 @@ def test_qk_nr_chunks(io, D, n_rot):
     assert bits_equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize('io', [0, 1])
+@pytest.mark.parametrize('heads,D,n_rot', [(4, 256, 64), (4, 256, 256), (3, 256, 64), (5, 256, 16), (7, 256, 128), (4, 128, 128), (6, 64, 8)])
+def test_qk_nr_chunks_of_few_heads(io, heads, D, n_rot):
+    """fewer than eight heads a token: 1400 tokens at once (the per-token kernels from four heads) and in chunks of 100 (the per-head kernel)"""
+    rng = np.random.default_rng(9 + heads + D)
+    T, stride, pos0 = 1400, D, 14000
+    x = outliers(rng, (T * heads, stride)); w = (1 + 0.1 * rng.standard_normal(D)).astype(f32)
+    ts = float(f32(f32(1e7) ** f32(-2.0 / n_rot)))
+    xd, wd = dev(O.f2bf(x) if io else x), dev(w)
+    dt = np.uint16 if io else f32
+    outs = []
+    for chunk in (T, 100):
+        y = dev(np.zeros((T * heads, D), dt))
+        for t in range(0, T, chunk):
+            call('camx_pf_qk_nr', ptr(xd[t * heads:]), I(stride), I(heads), ptr(wd), I(D), I(n_rot), F(ts), F(1e-6), I(pos0 + t), ptr(y[t * heads:]), I(chunk), I(io))
+        outs.append(host(y, dt) if io else host(y))
+    assert bits_equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize('yarn', [False, True])
 def test_qk_rope_bf16_chunks(yarn):
     """2049 tokens of bf16 rows at once (four tokens per workgroup) and in chunks of 500 (one)"""
