@@ -203,16 +203,13 @@ static int launch_mmq(const MmqArgs & a, int layout, hipStream_t st) {
 }
 
 // ---- fused SwiGLU -> MMQ q8_1, the wide form ---------------------------------------------------------------------------------
-// bf16(silu(g)) of a bf16 g is a function of 16 bits: the whole table (65536 x 2 B = 128 KiB) fits in one CU's 160 KiB of
-// LDS. Persistent workgroups (one per CU, 16 waves) copy the table from a static device array once and then look every
-// gate value up with one 16-bit LDS read, which takes the two transcendentals, the divide and the first bf16 rounding
-// off the VALU. The table itself is computed once per device ((float)exp in double, then the reference's fp32 statement
-// g / (1 + e), then round-to-nearest-even to bf16).
+// bf16(silu(g)) of a bf16 g is a function of 16 bits: a table lookup takes the two transcendentals, the divide and the first
+// bf16 rounding off the VALU. The table (65536 entries, computed once per device: (float)exp in double, then the reference's fp32
+// statement g / (1 + e), then round-to-nearest-even to bf16) is read from LDS in a small form that covers the gates in use.
 //
 // A wave's work item is 8 tokens x one 128-value block column: lane l takes the 8 consecutive values 8 (l & 15) .. + 7 of
 // tokens (l >> 4) and (l >> 4) + 4 (load i = token half i), so that one 128-bit load instruction of g (and of u) fetches
-// four 256-byte row pieces. Items are numbered with the token group running fastest inside a band of four block columns,
-// so the waves that run together read different rows (1 KiB of each) and write four long runs of blocks. A 32-value
+// four 256-byte row pieces. A 32-value
 // quantization group is the 4 lanes of a quad (for each i), a 128-value block 16 lanes. The reference's
 // 8 threads of a group are (lane & 3, half): thread 2 (lane & 3) + h holds values 4h .. 4h + 3 of the lane, so its
 // xor 4 / 2 / 1 butterfly is lane ^ 2, lane ^ 1 (quad permutes) and the lane's two halves. Lane (l & 3) == i does
@@ -222,10 +219,8 @@ static int launch_mmq(const MmqArgs & a, int layout, hipStream_t st) {
 // Written straight from the lanes they would leave as 8-byte pieces that straddle 64-byte boundaries (3.3 write requests
 // per block instead of 2.25, each costing a full 64-byte slot on the way to HBM), so a wave stages its blocks in its own
 // 1152 bytes of LDS and writes them out as one aligned run of 16 bytes per lane. Nothing but the table is shared
-// between waves: no barrier after the table copy, every wave runs its own pipeline (two items of loads in flight).
+// between waves: no barrier after the table copy.
 #define SWM_TOK 8
-#define SWM_STAGE (16 * SWM_TOK * 144)           // 16 waves x 1152 bytes
-#define SWM_LDS (131072 + SWM_STAGE)
 
 __device__ uint16_t g_silu_lut[65536];
 __device__ __attribute__((aligned(16))) uint32_t g_zero16[4] = {0, 0, 0, 0};   // (not const: it must live in the global address space, or the selects below turn the loads into flat ones)
@@ -281,8 +276,8 @@ CAMX_DEV void swm_load(SwmItem & it, const void * __restrict__ src, const int32_
 // CANON: the activation is packed with f2bf (a NaN becomes 0x7fc0, as silu_mul_bf16 stores it) instead of the hardware convert, which
 // keeps a NaN's sign and payload. Returns whether a group sum of this lane's quad is a NaN: the callers run the item with the hardware
 // convert first and, in the rare wave that reports one (a NaN or infinite input), once more with CANON, which rewrites the same bytes.
-// LUTMODE: where bf16(silu g) comes from. LUT_FULL: the 65536-entry table (in LDS for the persistent kernel, in device memory for the
-// rare redo of the one-shot kernel). LUT_SMALL: the 8192-entry table of the one-shot kernel, which holds the gates a model produces
+// LUTMODE: where bf16(silu g) comes from. LUT_FULL: the 65536-entry table (in device memory, for the rare redo).
+// LUT_SMALL: the 8192-entry table in LDS, which holds the gates a model produces
 // (+-0 and 2^-24 <= |g| < 2^8 less two values); bit 1 of the result reports a gate outside it, and the caller redoes the item with the full table.
 enum { LUT_FULL = 0, LUT_SMALL = 1 };
 template <int LAYOUT, int SRC, bool CANON = false, int LUTMODE = LUT_FULL>
@@ -358,58 +353,7 @@ CAMX_DEV int swm_compute(const SwmItem & it, const uint16_t * lut, uint8_t * sta
     return flags;
 }
 
-// SRC_F32 (quantize_mmq_q8_1 without scatter): the same work split and copy-out on fp32 rows (column c = row ids[c] or c), no table
-template <int LAYOUT, int SRC>
-__global__ void __launch_bounds__(1024) swiglu_mmq_lut(const void * __restrict__ gu, const int32_t * __restrict__ ids, long ld, long F,
-                                                       uint8_t * __restrict__ y, uint16_t * __restrict__ act, int T, unsigned ncol, unsigned nitems) {
-    extern __shared__ __attribute__((aligned(16))) uint16_t lut[];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    uint8_t * stage = (uint8_t *)lut + (SRC == SRC_SWIGLU_BF16 ? 131072 : 0) + wave * (SWM_TOK * 144);
-    const unsigned stride = gridDim.x * 16;                                   // (ids stay below 2^31: checked by the launcher)
-    unsigned j = blockIdx.x * 16 + wave;
-    // item id -> 4 neighbouring block columns x token groups, token groups fastest: the four waves of a SIMD row read 1 KiB of each token row
-    // and the workgroups that run side by side write neighbouring runs of the same block rows (ncol is a multiple of 4: K is padded to 512)
-    const unsigned ntg = (unsigned)((T + SWM_TOK - 1) / SWM_TOK);
-#define SWM_TG(id) ((long)((((id) >> 2) % ntg)) * SWM_TOK)
-#define SWM_UNIT(id) ((long)(((((id) >> 2) / ntg) << 2) + ((id) & 3)))
-    SwmItem A, B, C;                                                          // three items in rotation: two steps of loads in flight
-    swm_load<SRC>(A, gu, ids, ld, F, T, SWM_TG(j), SWM_UNIT(j), lane, j < nitems);                  // in flight while the table is copied
-    swm_load<SRC>(B, gu, ids, ld, F, T, SWM_TG(j + stride), SWM_UNIT(j + stride), lane, j + stride < nitems);
-    if (SRC == SRC_SWIGLU_BF16) {
-        for (int i = threadIdx.x; i < 8192; i += 1024) ((u32x4 *)lut)[i] = ((const u32x4 *)g_silu_lut)[i];
-        __syncthreads();
-    }
-    // copy-out of a finished item: 1152 contiguous bytes = 72 lanes' worth of 16 B (lanes 0 .. 7 take a second unit)
-    auto flush = [&](unsigned id) {
-        const long tg = SWM_TG(id), unit = SWM_UNIT(id);
-        const int nunits = (int)min((long)SWM_TOK, T - tg) * 9;               // tokens of the group that exist
-        uint8_t * dst = y + ((size_t)unit * T + (size_t)tg) * 144;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier();       // the wave's own LDS writes, in order
-        if (lane < nunits) __builtin_nontemporal_store(*(const u32x4 *)(stage + 16 * lane), (u32x4 *)(dst + 16 * lane));
-        if (lane < 8 && 64 + lane < nunits) __builtin_nontemporal_store(*(const u32x4 *)(stage + 1024 + 16 * lane), (u32x4 *)(dst + 1024 + 16 * lane));
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier();
-    };
-#define SWM_STEP(CUR, NXT2, jc)                                                                                              \
-    {                                                                                                                        \
-        const unsigned jn = (jc) + 2 * stride;                                                                                  \
-        swm_load<SRC>(NXT2, gu, ids, ld, F, T, SWM_TG(jn), SWM_UNIT(jn), lane, jn < nitems);                                 \
-        if ((jc) < nitems) {                                                                                                 \
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(swm_compute<LAYOUT, SRC>(CUR, lut, stage, F, act, T, SWM_TG(jc), SWM_UNIT(jc), lane) & 1) != 0, 0))  \
-                swm_compute<LAYOUT, SRC, true>(CUR, lut, stage, F, act, T, SWM_TG(jc), SWM_UNIT(jc), lane);                  \
-            flush(jc);                                                                                                       \
-        }                                                                                                                    \
-    }
-    for (; j < nitems; j += 3 * stride) {
-        SWM_STEP(A, C, j)
-        SWM_STEP(B, A, j + stride)
-        SWM_STEP(C, B, j + 2 * stride)
-    }
-#undef SWM_STEP
-#undef SWM_TG
-#undef SWM_UNIT
-}
-
-// ---- the one-shot form for prefill chunks -----------------------------------------------------------------------------------------
+// ---- the one-shot form ------------------------------------------------------------------------------------------------------------
 // A workgroup of SWS_WAVES waves takes SWS_WAVES neighbouring token groups of one block column and ends; the hardware hands the next
 // workgroup to whichever CU is free, which keeps the chip's accesses inside a narrow moving window of the inputs and makes neighbouring
 // waves write neighbouring runs of one block row (measured with every launch on cold lines, the same access pattern runs 12 % faster
@@ -596,9 +540,7 @@ static int silu_lut_ready(hipStream_t st, int * ncu, const uint16_t ** lut = nul
         silu_small_fill<<<dim3((SWS_TAB + 255) / 256), dim3(256), 0, st>>>();
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
-        if (hipFuncSetAttribute((const void *)swiglu_mmq_lut<MMQ_DS4, SRC_SWIGLU_BF16>, hipFuncAttributeMaxDynamicSharedMemorySize, SWM_LDS) != hipSuccess ||
-            hipFuncSetAttribute((const void *)swiglu_mmq_lut<MMQ_D4, SRC_SWIGLU_BF16>, hipFuncAttributeMaxDynamicSharedMemorySize, SWM_LDS) != hipSuccess ||
-            hipFuncSetAttribute((const void *)silu_mul_lut, hipFuncAttributeMaxDynamicSharedMemorySize, 131072) != hipSuccess) return CAMX_EINVAL;
+        if (hipFuncSetAttribute((const void *)silu_mul_lut, hipFuncAttributeMaxDynamicSharedMemorySize, 131072) != hipSuccess) return CAMX_EINVAL;
         void * sym = nullptr, * sym_small = nullptr;
         if (hipGetSymbolAddress(&sym, HIP_SYMBOL(g_silu_lut)) != hipSuccess || !sym) return CAMX_EINVAL;
         if (hipGetSymbolAddress(&sym_small, HIP_SYMBOL(g_silu_small)) != hipSuccess || !sym_small) return CAMX_EINVAL;
@@ -669,18 +611,10 @@ int camx_quantize_mmq_q8_1(const float * x, const int32_t * ids, void * vy, long
     (void)s02; (void)s03; (void)n_expert_used;
     if (!x || !vy || ne00 < 4 || ne00 % 4 || s01 < ne00 || s01 % 4 || ne0 % 512 || ne0 < ne00 || ne0 >= ne00 + 512 || ne1 < 0 || ne2 != 1 ||
         (layout != MMQ_D4 && layout != MMQ_DS4) || ((uintptr_t)x & 15) || ((uintptr_t)vy & 15)) return CAMX_EINVAL;
-    if (ne1 >= 256 && (long)((ne1 + SWM_TOK - 1) / SWM_TOK) * (ne0 / 128) < 0x7ff00000L) {       // enough columns to fill the chip: persistent workgroups, block rows stored as whole aligned runs
-        int dev = 0, ncu = 256;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return CAMX_EINVAL;
-        const long ncol = ne0 / 128, nitems = (long)((ne1 + SWM_TOK - 1) / SWM_TOK) * ncol;
-        if (ne1 >= 2048 && ncol <= 65535) {                                   // a prefill chunk: the one-shot form (no table for fp32 rows)
-            launch_oneshot<SRC_F32>(x, ids, s01, ne00, vy, nullptr, ne1, ncol, layout, st);
-            CAMX_LAUNCH_RET();
-        }
-        const long nwg = (nitems + 15) / 16;                                  // a small batch does not start workgroups that would only copy the table
-        const dim3 grid((unsigned)(nwg < ncu ? nwg : ncu)), block(1024);
-        if (layout == MMQ_DS4) swiglu_mmq_lut<MMQ_DS4, SRC_F32><<<grid, block, SWM_STAGE, st>>>(x, ids, s01, ne00, (uint8_t *)vy, nullptr, ne1, (unsigned)ncol, (unsigned)nitems);
-        else swiglu_mmq_lut<MMQ_D4, SRC_F32><<<grid, block, SWM_STAGE, st>>>(x, ids, s01, ne00, (uint8_t *)vy, nullptr, ne1, (unsigned)ncol, (unsigned)nitems);
+    // from 256 columns the one-shot form (no table for fp32 rows): block rows stored as whole aligned runs. K = 2048 / 5120: 256 columns
+    // 4.9 / 4.8 us against 6.2 / 6.5 of the rows kernel, 2047 columns 6.4 / 11.9; below, the rows kernel's smaller workgroups (128: 4.4 against 4.8)
+    if (ne1 >= 256 && ne0 / 128 <= 65535 && (long)((ne1 + SWM_TOK - 1) / SWM_TOK) * (ne0 / 128) < 0x7ff00000L) {
+        launch_oneshot<SRC_F32>(x, ids, s01, ne00, vy, nullptr, ne1, ne0 / 128, layout, st);
         CAMX_LAUNCH_RET();
     }
     MmqArgs a = {x, ids, (uint8_t *)vy, nullptr, ne00, ne0, s01, ne1, ne1, 0, nullptr};
@@ -695,7 +629,9 @@ int camx_quantize_mmq_q8_1_scatter(const float * x, const int32_t * ids, void * 
     if (!x || !vy || !ids || ne00 < 4 || ne00 % 4 || s02 < ne00 || s02 % 4 || ne0 % 512 || ne0 < ne00 || ne0 >= ne00 + 512 || ne2 != 1 ||
         n_expert_used < 1 || ntok < 0 || ne1 != ntok * n_expert_used || (layout != MMQ_D4 && layout != MMQ_DS4) ||
         ((uintptr_t)x & 15) || ((uintptr_t)vy & 15)) return CAMX_EINVAL;
-    if (ntok >= 2048 && ne0 / 128 <= 65535 && (long)ntok * n_expert_used < 0x7fffffffL) {      // a prefill chunk: the one-shot form
+    // a prefill chunk takes the one-shot form. To 8 columns each: 1536 tokens x 5120 20.8 us against the rows kernel's 31.4, 1024 x 5120
+    // 15.0 and 15.2, 777 x 5120 13.6 and 12.5; 2047 x 2048 12.4 and 12.9, 1536 x 2048 10.8 and 10.7
+    if ((ntok >= 2048 || (long)ntok * ne00 >= 5 << 20) && ne0 / 128 <= 65535 && (long)ntok * n_expert_used < 0x7fffffffL) {
         launch_oneshot_scatter(x, ids, s02, ne00, vy, ntok, n_expert_used, ne1, ne0 / 128, layout, st);
         CAMX_LAUNCH_RET();
     }
@@ -709,21 +645,14 @@ int camx_swiglu_mmq_q8_1(const uint16_t * gu, long ld, long F, void * vy, uint16
     if (!gu || !vy || F < 4 || F % 4 || ld < 2 * F || ld % 4 || T < 0 || (layout != MMQ_D4 && layout != MMQ_DS4) ||
         ((uintptr_t)gu & 7) || ((uintptr_t)vy & 15) || ((uintptr_t)act & 7)) return CAMX_EINVAL;
     if (T == 0) return CAMX_OK;
-    if (F % 8 == 0 && ld % 8 == 0 && !((uintptr_t)gu & 15) && !((uintptr_t)act & 15) &&
+    if (F % 8 == 0 && ld % 8 == 0 && !((uintptr_t)gu & 15) && !((uintptr_t)act & 15) && (F + 511) / 512 * 4 <= 65535 &&
         (long)((T + SWM_TOK - 1) / SWM_TOK) * ((F + 511) / 512 * 4) < 0x7ff00000L) {
         int ncu = 0;
         const int rc = silu_lut_ready(st, &ncu);
         if (rc) return rc;
-        const long Kp = (F + 511) / 512 * 512;
-        const long ncol = Kp / 128, nitems = (long)((T + SWM_TOK - 1) / SWM_TOK) * ncol;
-        const long nwg = (nitems + 15) / 16;                                  // a small batch does not start workgroups that would only copy the table
-        const dim3 grid((unsigned)(nwg < ncu ? nwg : ncu)), block(1024);
-        if (T >= 2048 && ncol <= 65535) {                                     // a prefill chunk: the one-shot form
-            launch_oneshot<SRC_SWIGLU_BF16>(gu, nullptr, ld, F, vy, act, T, ncol, layout, st);
-            CAMX_LAUNCH_RET();
-        }
-        if (layout == MMQ_DS4) swiglu_mmq_lut<MMQ_DS4, SRC_SWIGLU_BF16><<<grid, block, SWM_LDS, st>>>(gu, nullptr, ld, F, (uint8_t *)vy, act, T, (unsigned)ncol, (unsigned)nitems);
-        else swiglu_mmq_lut<MMQ_D4, SRC_SWIGLU_BF16><<<grid, block, SWM_LDS, st>>>(gu, nullptr, ld, F, (uint8_t *)vy, act, T, (unsigned)ncol, (unsigned)nitems);
+        // every batch size: 17408 values, 16 tokens 4.3 us (persistent workgroups with the whole table in LDS: 6.5), 777 tokens 16.6 (18.6),
+        // 2047 tokens 34.0 (36.7); 768 values 3.9 - 5.6 us (6.5 - 8.2)
+        launch_oneshot<SRC_SWIGLU_BF16>(gu, nullptr, ld, F, vy, act, T, (F + 511) / 512 * 4, layout, st);
         CAMX_LAUNCH_RET();
     }
     const uint16_t * lut = nullptr;

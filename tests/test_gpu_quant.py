@@ -71,6 +71,18 @@ def test_mmq_quantize_scatter(K, ntok, k, pad):
         assert bits_equal(host(y), ref)
 
 
+@pytest.mark.parametrize('K,ntok,k', [(7492, 700, 2), (7488, 701, 1), (5120, 1024, 3), (5116, 1025, 1)])
+def test_mmq_quantize_scatter_by_values(K, ntok, k):
+    """fewer than 2048 tokens of wide rows: either side of the 5 Mi values from which the one-shot form takes them"""
+    test_mmq_quantize_scatter(K, ntok, k, 0)
+
+
+@pytest.mark.parametrize('T', [1, 7, 9, 63, 65, 129])
+def test_swiglu_mmq_small_batches(T):
+    """every batch size takes the one-shot form: token counts around a wave's eight, its two items and a workgroup's 64"""
+    test_swiglu_mmq(T, 776, 0, 1)
+
+
 @pytest.mark.parametrize('T,Fh,pad,layout', [(3, 17408, 0, 1), (8, 768, 0, 1), (5, 1024, 0, 1), (11, 1000, 0, 1), (17, 2056, 8, 0), (300, 392, 16, 1),
                                              (9, 8, 0, 0), (2048, 392, 0, 1), (2051, 264, 16, 0), (4100, 136, 8, 1)])
 def test_swiglu_mmq(T, Fh, pad, layout):
