@@ -240,6 +240,31 @@ def test_block_entry_rows_shared_by_a_workgroup(M, d, nab):
     assert bits_equal(host(dx)[:M], O.block_entry_bwd(x, nw, rstd, wab, dy, dab)) and (host(dx)[M:] == 7.0).all()
 
 
+@pytest.mark.parametrize('K', [128, 640, 2048])
+def test_actq_signs_of_zeros(K):
+    """rows whose chunks begin with -0: the sign of a zero result comes through the rotation of the wave-per-row kernels (all zeros of one
+    sign, of either at random, pairs that cancel behind a -0, and ordinary rows beside them), in x and in the gradient"""
+    rng = np.random.default_rng(K)
+    M = 24
+    x = outliers(rng, (M, K))
+    x[0] = -0.0; x[1] = 0.0
+    x[2] = np.where(rng.random(K) < 0.5, -0.0, 0.0); x[3, ::128] = -0.0; x[3, 1::128] = 0.0
+    x[4] = np.where(np.arange(K) % 2, 0.0, -0.0)
+    x[5] = -0.0; x[5, 64::128] = 3.0; x[5, 65::128] = -3.0; x[5, 96::128] = 3.0; x[5, 97::128] = 3.0
+    x[6, :128] = -0.0
+    g = rng.standard_normal((M, K)).astype(np.float32); g[7] = -0.0; g[8] = np.where(np.arange(K) % 3, 0.0, -0.0); g[9, ::128] = -0.0; g[9, 1::128] = -0.0; g[0] = -0.0
+    g = O.f2bf(g)
+    for bf in (False, True):
+        src = O.f2bf(x) if bf else x
+        ry, rs, rc = O.actq_fwd(src, clip=1.0, qmax=7, bf16=bf)
+        y = dev(np.zeros((M, K), np.uint16)); s = dev(np.zeros(M, np.float32)); c = dev(np.zeros((M, K // 2), np.uint8))
+        call('camx_actq_fwd', ptr(dev(src)), I(int(bf)), ptr(y), ptr(s), ptr(c), I(K), F(1.0), I(7), I(M))
+        assert bits_equal(host(s), rs) and bits_equal(host(c), rc) and bits_equal(host(y, np.uint16), ry)
+        dx = dev(np.zeros((M, K), np.uint16 if bf else np.float32))
+        call('camx_actq_bwd', ptr(dev(src)), I(int(bf)), ptr(dev(g)), ptr(dx), I(K), F(1.0), I(7), I(M))
+        assert bits_equal(host(dx, np.uint16) if bf else host(dx), O.actq_bwd(src, g, clip=1.0, qmax=7, bf16=bf))
+
+
 def test_block_entry_gradient_of_one_output():
     """an output nothing depends on has a zero gradient: y alone, ab alone"""
     import torch
