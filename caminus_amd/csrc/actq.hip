@@ -71,6 +71,19 @@ CAMX_DEV u32x2 silu_lookup4(u32x2 gw, const uint16_t * small, const uint16_t * l
     }
     return r;
 }
+// Byte offsets of two packed gates' entries in the 16-bit small table, for the wave-per-row kernels: the sign falls out of a shift that
+// also scales the magnitude to bytes. most: the largest magnitude offset so far; SWS_LAST in it says that a gate is a zero or outside the
+// table, which the caller then settles four gates at a time as above (a compare per eight gates instead of four per two).
+constexpr uint16_t SWS_LAST = 2 * SWS_SPAN;
+CAMX_DEV uint32_t small_offset2(uint32_t w, u16x2 & most) {
+    const u16x2 a = __builtin_bit_cast(u16x2, w) << (u16x2){1, 1};
+    const u16x2 i = __builtin_elementwise_min(a - (u16x2){(uint16_t)(2 * SWS_A0), (uint16_t)(2 * SWS_A0)}, (u16x2){SWS_LAST, SWS_LAST});      // below the table: wraps, clamps
+    most = __builtin_elementwise_max(most, i);
+    return ((w >> 2) & 0x20002000u) | __builtin_bit_cast(uint32_t, i);
+}
+CAMX_DEV uint32_t small_pair(const uint16_t * small, uint32_t o) {
+    return (uint32_t)*(const uint16_t *)((const uint8_t *)small + (o & 0xffffu)) | ((uint32_t)*(const uint16_t *)((const uint8_t *)small + (o >> 16)) << 16);
+}
 struct SiluMulSrc {
     static constexpr bool bf16_valued = true;      // the activation is rounded to bf16 as it is formed
     static constexpr bool lds_tables = true;       // the wave-per-row kernels hold the small tables in LDS
@@ -90,8 +103,13 @@ struct SiluMulSrc {
     static constexpr int NW = 2;                   // the wave-per-row form: eight gates, eight multipliers
     CAMX_DEV void fetch(int row, int k, u32x4 (&w)[NW]) const { const uint16_t * r = gu + (size_t)row * ld + k; w[0] = *(const u32x4 *)r; w[1] = *(const u32x4 *)(r + F); }
     CAMX_DEV void value8(const u32x4 (&w)[NW], f32x4 & a, f32x4 & b, u32x4 & keep) const {
-        const u32x2 k0 = silu_lookup4((u32x2){w[0].x, w[0].y}, small, lut), k1 = silu_lookup4((u32x2){w[0].z, w[0].w}, small, lut);
-        keep = (u32x4){k0.x, k0.y, k1.x, k1.y};
+        u16x2 most = {0, 0};
+        const uint32_t o0 = small_offset2(w[0].x, most), o1 = small_offset2(w[0].y, most), o2 = small_offset2(w[0].z, most), o3 = small_offset2(w[0].w, most);
+        if (most.x != SWS_LAST && most.y != SWS_LAST) keep = (u32x4){small_pair(small, o0), small_pair(small, o1), small_pair(small, o2), small_pair(small, o3)};
+        else {
+            const u32x2 k0 = silu_lookup4((u32x2){w[0].x, w[0].y}, small, lut), k1 = silu_lookup4((u32x2){w[0].z, w[0].w}, small, lut);
+            keep = (u32x4){k0.x, k0.y, k1.x, k1.y};
+        }
         f32x4 sa, sb, ua, ub;
         unpack_bf16x8(keep, sa, sb); unpack_bf16x8(w[1], ua, ub);
         a = rbf4_any((f32x4){sa.x * ua.x, sa.y * ua.y, sa.z * ua.z, sa.w * ua.w});
@@ -468,8 +486,8 @@ struct SinkSiluMul {
         *(u32x2 *)(o + F + k) = dup;
     }
     // four values' dg and du from their gates, multipliers, bf16(silu g) and dact
-    CAMX_DEV void grads4(u32x2 gw, u32x2 uw, u32x2 keep, f32x4 dact, u32x2 & dgp, u32x2 & dup) const {
-        const f32x4 g = unpack_bf16x4(gw), u = unpack_bf16x4(uw), sl4 = unpack_bf16x4(keep);
+    CAMX_DEV void grads4(u32x2 gw, u32x2 uw, u32x2 keep, f32x4 dact, u32x2 & dgp, u32x2 & dup) const { grads4(gw, uw, keep, dact, sigmoids4(gw), dgp, dup); }
+    CAMX_DEV f32x4 sigmoids4(u32x2 gw) const {
         bool outside = true;
         f32x4 sig;
         if (dsmall) {
@@ -478,6 +496,15 @@ struct SinkSiluMul {
             sig = (f32x4){dsmall[i01 & 0xffffu], dsmall[i01 >> 16], dsmall[i23 & 0xffffu], dsmall[i23 >> 16]};
         }
         if (outside) sig = (f32x4){dlut[gw.x & 0xffffu], dlut[gw.x >> 16], dlut[gw.y & 0xffffu], dlut[gw.y >> 16]};
+        return sig;
+    }
+    CAMX_DEV float small_at(uint32_t o) const { return *(const float *)((const uint8_t *)dsmall + o); }
+    CAMX_DEV f32x4 small4(uint32_t o0, uint32_t o1) const {               // from the byte offsets into the 16-bit table
+        const uint32_t a = o0 << 1, b = o1 << 1;                          // (the offsets use 14 bits of each half)
+        return (f32x4){small_at(a & 0xffffu), small_at(a >> 16), small_at(b & 0xffffu), small_at(b >> 16)};
+    }
+    CAMX_DEV void grads4(u32x2 gw, u32x2 uw, u32x2 keep, f32x4 dact, f32x4 sig, u32x2 & dgp, u32x2 & dup) const {
+        const f32x4 g = unpack_bf16x4(gw), u = unpack_bf16x4(uw), sl4 = unpack_bf16x4(keep);
         const f32x4 ds = rbf4_any((f32x4){dact.x * u.x, dact.y * u.y, dact.z * u.z, dact.w * u.w});       // (a NaN's bits are settled by the store's rounding)
         f32x4 dg, du;
 #define S_(e) { du.e = dact.e * sl4.e; dg.e = ds.e * sig.e * __builtin_fmaf(g.e, 1.0f - sig.e, 1.0f); }
@@ -491,8 +518,13 @@ struct SinkSiluMul {
         const uint16_t * r = gu + (size_t)row * ld + k;
         const u32x4 gw = *(const u32x4 *)r, uw = *(const u32x4 *)(r + F);
         u32x2 dg0, du0, dg1, du1;
-        grads4((u32x2){gw.x, gw.y}, (u32x2){uw.x, uw.y}, (u32x2){keep.x, keep.y}, rbf4_any(a), dg0, du0);      // (a NaN's bits are settled by the stores' rounding)
-        grads4((u32x2){gw.z, gw.w}, (u32x2){uw.z, uw.w}, (u32x2){keep.z, keep.w}, rbf4_any(b), dg1, du1);
+        u16x2 most = {0, 0};
+        const uint32_t o0 = small_offset2(gw.x, most), o1 = small_offset2(gw.y, most), o2 = small_offset2(gw.z, most), o3 = small_offset2(gw.w, most);
+        f32x4 s0, s1;
+        if (most.x != SWS_LAST && most.y != SWS_LAST) { s0 = small4(o0, o1); s1 = small4(o2, o3); }
+        else { s0 = sigmoids4((u32x2){gw.x, gw.y}); s1 = sigmoids4((u32x2){gw.z, gw.w}); }
+        grads4((u32x2){gw.x, gw.y}, (u32x2){uw.x, uw.y}, (u32x2){keep.x, keep.y}, rbf4_any(a), s0, dg0, du0);      // (a NaN's bits are settled by the stores' rounding)
+        grads4((u32x2){gw.z, gw.w}, (u32x2){uw.z, uw.w}, (u32x2){keep.z, keep.w}, rbf4_any(b), s1, dg1, du1);
         uint16_t * o = dgu + (size_t)row * (2 * F) + k;
         *(u32x4 *)o = (u32x4){dg0.x, dg0.y, dg1.x, dg1.y};
         *(u32x4 *)(o + F) = (u32x4){du0.x, du0.y, du1.x, du1.y};
