@@ -149,13 +149,14 @@ __global__ void __launch_bounds__(256) kv_q8_read_rows(const uint8_t * __restric
     }
 }
 
-// The same reader for a chunk of rows with at most 32 blocks per row (M <= 512; row bytes a multiple of 16, 16-byte aligned cache): a
-// wave per row, four rows per workgroup; the row comes in as 16-byte pieces straight to the wave's LDS (two requests per wave instead
-// of three 2-byte loads per lane and block) and is decoded from there.
-template <bool F16>
+// The same reader for a chunk of rows with at most NB = 32 or 64 blocks per row (M <= 512 or 1024; row bytes a multiple of 16, 16-byte
+// aligned cache): a wave per row, four rows per workgroup; the row comes in as 16-byte pieces straight to the wave's LDS (two or three
+// requests per wave instead of three 2-byte loads per lane and block) and is decoded from there. 16384 rows of M = 1024 to fp16, 103 MB:
+// 19.7 us, a workgroup per row as above 26.0 (2048 rows: 5.1 and 5.0, so wider rows come here from there on).
+template <bool F16, int NB>
 __global__ void __launch_bounds__(256) kv_q8_read_wave_rows(const uint8_t * __restrict__ cache, const int32_t * __restrict__ row_ids, int pos0, int rows, int M,
                                                             void * __restrict__ k, int ldk, void * __restrict__ v, int ldv, int T, int * __restrict__ err) {
-    __shared__ __attribute__((aligned(16))) uint8_t stage_all[4][2 * 16 * 34];
+    __shared__ __attribute__((aligned(16))) uint8_t stage_all[4][NB * 34];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, sub = lane & 7;
     const int tt = blockIdx.x * 4 + wave;
     if (tt >= T) return;
@@ -168,7 +169,7 @@ __global__ void __launch_bounds__(256) kv_q8_read_wave_rows(const uint8_t * __re
     const uint8_t * src = cache + (size_t)pos * rb;
     uint8_t * stage = stage_all[wave];
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
+    for (int i = 0; i < (NB * 34 + 1023) / 1024; i++) {
         const int p = 64 * i + lane;
         const uint8_t * q = src + 16 * (size_t)p;
         if (p < n16)
@@ -176,7 +177,7 @@ __global__ void __launch_bounds__(256) kv_q8_read_wave_rows(const uint8_t * __re
     }
     __builtin_amdgcn_s_waitcnt(0x0f70);                                    // vmcnt(0): the wave's own row has landed
 #pragma unroll
-    for (int it = 0; it < 4; it++) {
+    for (int it = 0; it < NB / 8; it++) {
         const int b = it * 8 + (lane >> 3);
         if (b >= 2 * nb) continue;
         const uint8_t * blk = stage + (size_t)b * 34;
@@ -316,11 +317,15 @@ int camx_own_kv_q8_read(const uint8_t * cache, const int32_t * row_ids, int pos0
     if (!cache || !k || !v || !err || T < 0 || ((uintptr_t)cache & 1) || ((uintptr_t)k & (f16 ? 7 : 3)) || ((uintptr_t)v & (f16 ? 7 : 3)) ||
         (f16 && ((ldk | ldv) & 3))) return CAMX_EINVAL;
     if (T == 0) return CAMX_OK;
-    const bool chunk = T >= 1024 && M >= 32 && M % 32 == 0 && M <= 512 && (2 * (M / 32) * 34) % 16 == 0 && ldk >= M && ldv >= M && rows >= 1 &&
+    const bool chunk = T >= 1024 && M >= 32 && M % 32 == 0 && (M <= 512 || (M <= 1024 && T >= 2048)) && (2 * (M / 32) * 34) % 16 == 0 && ldk >= M && ldv >= M && rows >= 1 &&
                        ((uintptr_t)cache & 15) == 0 && (f16 || ((((uintptr_t)k | (uintptr_t)v) & 15) == 0 && ((ldk | ldv) & 3) == 0));
     if (chunk) {
-        if (f16) kv_q8_read_wave_rows<true><<<dim3((T + 3) / 4), dim3(256), 0, st>>>(cache, row_ids, pos0, rows, M, k, ldk, v, ldv, T, err);
-        else kv_q8_read_wave_rows<false><<<dim3((T + 3) / 4), dim3(256), 0, st>>>(cache, row_ids, pos0, rows, M, k, ldk, v, ldv, T, err);
+        const dim3 grid((T + 3) / 4), block(256);
+        if (M <= 512) {
+            if (f16) kv_q8_read_wave_rows<true, 32><<<grid, block, 0, st>>>(cache, row_ids, pos0, rows, M, k, ldk, v, ldv, T, err);
+            else kv_q8_read_wave_rows<false, 32><<<grid, block, 0, st>>>(cache, row_ids, pos0, rows, M, k, ldk, v, ldv, T, err);
+        } else if (f16) kv_q8_read_wave_rows<true, 64><<<grid, block, 0, st>>>(cache, row_ids, pos0, rows, M, k, ldk, v, ldv, T, err);
+        else kv_q8_read_wave_rows<false, 64><<<grid, block, 0, st>>>(cache, row_ids, pos0, rows, M, k, ldk, v, ldv, T, err);
     }
     else if (f16) kv_q8_read_rows<true><<<dim3(T), dim3(256), 0, st>>>(cache, row_ids, pos0, rows, M, k, ldk, v, ldv, err);
     else kv_q8_read_rows<false><<<dim3(T), dim3(256), 0, st>>>(cache, row_ids, pos0, rows, M, k, ldk, v, ldv, err);

@@ -145,3 +145,9 @@ def test_kv_q8_read_round_trip(M, T, f16):
     ok, ov, oerr = O.kv_q8_read(cache, M, len(ids), row_ids=ids, f16=f16, fill=7)
     assert int(host(err2)[0]) == oerr == 1 and bits_equal(host(k2, dt), ok) and bits_equal(host(v2, dt), ov)
     assert (host(k2, dt)[1] == 7).all()
+
+
+@pytest.mark.parametrize('M,T,f16', [(1024, 2048, True), (1024, 2051, False), (640, 2049, True), (896, 2048, False), (672, 2050, True)])
+def test_kv_q8_read_wave_per_wide_row(M, T, f16):
+    """rows of 33 to 64 blocks from 2048 rows on: a wave per row where a row is whole 16-byte pieces (672 is not)"""
+    test_kv_q8_read_round_trip(M, T, f16)
