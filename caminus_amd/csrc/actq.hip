@@ -4,8 +4,9 @@
 // 96-218, 247-333).
 //
 // Rows of at most 2048 values with 16-byte aligned operands, forward and backward, plain and SiLU-fused: one wave per row
-// (actq_fwd_wave_k, actq_bwd_wave_k; 30 vector instructions per value against 44 forward, 63 against 78 backward), the fused
-// forms with the gates' tables in LDS. Everything else (longer rows, the RMSNorm-fused block entry, unaligned operands):
+// (actq_fwd_wave_k, actq_bwd_wave_k; 26 vector instructions per value against 44 forward, 49 against 78 backward), the fused
+// forms with the gates' tables in LDS (38 and 76). The RMSNorm-fused block entry of rows of at most 1024 values: a wave per row as well,
+// four rows sharing the projections (block_entry_fwd_quad, block_entry_bwd_quad). Everything else (longer rows, unaligned operands):
 // One 256-thread workgroup per row. A half-wave (32 lanes) transforms one 128-chunk: lane l holds elements 4l .. 4l + 3,
 // butterfly stages 1-2 in registers, 4 .. 64 across lanes; half-wave h takes chunks h, h + 8, ... (the reference's wave h of
 // 32), NR = ceil(K / 1024) rounds of them stay in registers across the row-wide reductions. Kernels are instantiated per
