@@ -309,7 +309,7 @@ __global__ void __launch_bounds__(512) ple_gate_rows(const float * kn, const flo
         for (int u = 0; u < PLE_UNR; u++) {
             const int i = min(b + 256 * u + 4 * p, D - 4);            // (past the row: its last values, not added below)
             kv[u] = __builtin_nontemporal_load((const f32x4 *)(k_ + i));
-            qv[u] = *(const f32x4 *)(q_ + i);
+            qv[u] = __builtin_nontemporal_load((const f32x4 *)(q_ + i));
             if (REC) wv[u] = *(const f32x4 *)(w_ + i);
         }
 #pragma unroll
