@@ -291,7 +291,7 @@ __global__ void __launch_bounds__(256) ple_gate_k(const float * kn, const float 
 // The same with one wave per (token, stream) and 128-bit accesses, for D % 4 == 0 and 16-byte aligned rows: lane p holds the
 // logical threads 4 p .. 4 p + 3 of the tree, so a stream's dot product needs no LDS and no barrier, and the HC waves of a token's
 // workgroup share its val row through the caches. Memory bound: with 4-byte loads, two barriers and an integer division per stored
-// value the kernel above takes 80 us for the 273 MB of 2048 tokens x 4 streams x 2560, this one 54; PLE_UNR steps of loads are issued ahead of their sums.
+// value the kernel above takes 80 us for the 273 MB of 2048 tokens x 4 streams x 2560, this one 51 (53 with plain loads of q); PLE_UNR steps of loads are issued ahead of their sums.
 // (gated may alias kn: a wave stores its own row only, after the dot product that consumed it)
 constexpr int PLE_UNR = 5;                               // 2560 values: two batches, 40 registers of loads in flight
 CAMX_DEV void ple_dot4(f32x4 & acc, f32x4 k, f32x4 q) { acc.x = acc.x + k.x * q.x; acc.y = acc.y + k.y * q.y; acc.z = acc.z + k.z * q.z; acc.w = acc.w + k.w * q.w; }
