@@ -881,6 +881,7 @@ __global__ void __launch_bounds__(256, 4) block_entry_fwd_quad(const float * __r
     for (int c = 0; c < NR; c++) {
         const f32x4 v = xk[c], w = wk[c];
         hb[c] = (u32x2){hw_pk_bf16(v.x * rstd * w.x, v.y * rstd * w.y), hw_pk_bf16(v.z * rstd * w.z, v.w * rstd * w.w)};
+        if (c == NR - 1 && 256 * c + 4 * lane >= d) hb[c] = (u32x2){0u, 0u};            // (0 x an infinite rstd is a NaN, and the projections add the padding's products)
         *(u32x2 *)&hbuf[wave][128 * c + 2 * lane] = hb[c];
     }
     f32x4 u[NR];

@@ -240,6 +240,22 @@ def test_block_entry_rows_shared_by_a_workgroup(M, d, nab):
     assert bits_equal(host(dx)[:M], O.block_entry_bwd(x, nw, rstd, wab, dy, dab)) and (host(dx)[M:] == 7.0).all()
 
 
+@pytest.mark.parametrize('M,d,nab', [(5, 384, 4), (2, 128, 16), (4, 896, 10), (3, 512, 2), (3, 1152, 3)])
+def test_block_entry_infinite_rstd(M, d, nab):
+    """eps = 0 and rows whose squares underflow: rstd is infinite, the projections of the row's own elements are +inf or NaN as the signs
+    have it, and rows that end inside a round of 256 add nothing for the padding behind them"""
+    rng = np.random.default_rng(d + nab)
+    x = (1e-30 * (0.5 + rng.random((M, d)))).astype(np.float32); x[1] *= np.where(rng.random(d) < 0.5, -1, 1)
+    nw = (0.5 + rng.random(d)).astype(np.float32); wab = O.f2bf((0.01 + rng.random((nab, d))).astype(np.float32))
+    ry, rs, rc, rab, rstd = O.block_entry_fwd(x, nw, wab, 0.0)
+    assert np.isinf(rstd).all() and np.isinf(O.bf2f(rab)[0]).all() and np.isnan(O.bf2f(rab)[1]).all()
+    y = dev(np.zeros((M, d), np.uint16)); s = dev(np.zeros(M, np.float32)); c = dev(np.zeros((M, d // 2), np.uint8))
+    ab = dev(np.zeros((M, nab), np.uint16)); rstd_d = dev(np.zeros(M, np.float32))
+    call('camx_block_entry_fwd', ptr(dev(x)), ptr(dev(nw)), ptr(dev(wab)), I(nab), F(0.0), ptr(y), ptr(s), ptr(c), ptr(ab), ptr(rstd_d), I(d), F(1.0), I(7), I(M))
+    assert bits_equal(host(rstd_d), rstd) and bits_equal(host(s), rs) and bits_equal(host(c), rc) and bits_equal(host(y, np.uint16), ry)
+    assert bits_equal(host(ab, np.uint16), rab)
+
+
 @pytest.mark.parametrize('K', [128, 640, 2048])
 def test_actq_signs_of_zeros(K):
     """rows whose chunks begin with -0: the sign of a zero result comes through the rotation of the wave-per-row kernels (all zeros of one
