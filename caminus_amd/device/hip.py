@@ -46,6 +46,7 @@ def stream_handle():
 
 
 def _dim3(d):
+    d = tuple(d)                                                # (any iterable)
     return (int(d[0]), 1, 1) if len(d) == 1 else (tuple(int(x) for x in d) + (1, 1))[:3]
 
 

@@ -96,6 +96,19 @@ def _refused(c, exc=(ValueError, ContextBoundsError), **changes):
     assert c.rec.calls == [] and c.loads == [] and c.entered == []
 
 
+@pytest.mark.parametrize('form', [tuple, list, iter, np.array, lambda d: (v for v in d)])
+def test_kernel_takes_any_iterable_as_a_grid(form):
+    """grid and block of one to three (or more, ignored) dimensions: sequences, arrays and iterators, as integers to the adapter"""
+    from caminus_amd.device import hip
+    seen = []
+    k = hip.Kernel(lambda *a: seen.append(a) or 0, 'probe', lambda grid, block, vals: [grid, block] + vals)
+    for d in ((5,), (5, 2), (5, 2, 3), (5, 2, 3, 4)):
+        k(form(d), form((64,)), 7, stream=0)
+        grid, block, v = seen.pop()[:3]
+        assert grid == (tuple(d) + (1, 1))[:3] and block == (64, 1, 1) and v == 7
+        assert all(type(x) is int for x in grid + block)
+
+
 def test_codec_needs_an_indexed_gpu():
     K.Q8KVCodec(torch.device('cuda:1'))
     for dev in ('cpu', 'cuda', 0, None):
