@@ -174,14 +174,17 @@ CAMX_DEV float actq_rotate(Src src, int row, int l, int hw, int nch, f32x4 (&u)[
 // The row's scale and what the lanes need to divide by it. For |p| < 2^k, p = u * rcp(s) (rcp: 1 ulp; one more rounding) is within
 // 2.5 * 2^(k - 23) of the exact quotient and the IEEE quotient within 2^(k - 24), and half-integers are floats: when p is farther than
 // their sum from every half-integer, rintf of the two agree. Rows whose quotients stay below 16 (every int4 row with clip near 1) ask
-// for 1e-5 (the sum: 5.8e-6), others below 256 for 3e-4. A lane that holds a closer value divides, and so does every lane of a row
-// whose largest quotient is not below 256 or not a number (an infinite amax). A NaN among the four values needs no look of its own: its
-// p is a NaN as its quotient is, and the maximum passes over it.
+// for 1e-5 (the sum: 5.8e-6), others below 256 for 3e-4 (9.2e-5), below 4096 for 2e-3 (1.5e-3; more than eight bits, or a clip far below
+// 1: 4096 x 4096 fp32 values at qmax 127 and clip 0.4 take 20.9 us, 23.9 with every lane of such a row dividing, 22.1 with the lanes
+// that hold a quotient above 256). A lane that holds a closer value divides, and so does every lane of a row whose largest quotient is not
+// below 4096 or not a number (an infinite amax). A NaN among the four values needs no look of its own: its p is a NaN as its quotient
+// is, and the maximum passes over it. (A scale above 2^126 has a subnormal reciprocal, which may be taken as zero: |u| is at most
+// HSCALE times the largest float or infinite, so the quotients of such a row are below 0.36 and round to the same zeros.)
 struct RowScale {
     float s, rcp, lo, hi, most;                          // most: how far p may lie from its integer
     CAMX_DEV RowScale(float s_, float amax, int qmax) : s(s_), rcp(__builtin_amdgcn_rcpf(s_)), lo((float)(-qmax - 1)), hi((float)qmax) {
         const float p = amax * rcp;
-        most = p < 16.0f ? 0.49999f : p < 256.0f ? 0.4997f : -1.0f;
+        most = p < 16.0f ? 0.49999f : p < 256.0f ? 0.4997f : p < 4096.0f ? 0.498f : -1.0f;
     }
     // clamp(rintf(u / s), lo, hi) of four values; the median of a NaN and two numbers is the smaller number, lo, as fminf(fmaxf(NaN, lo), hi) is
     CAMX_DEV f32x4 quant4(f32x4 u) const {

@@ -29,6 +29,22 @@ def test_actq_fwd(M, K, qmax):
             if qmax <= 7: assert bits_equal(host(c)[2 * shift:2 * shift + M * K // 2].reshape(M, K // 2), rc)
 
 
+@pytest.mark.parametrize('K', [1024, 2304])
+@pytest.mark.parametrize('qmax,clip', [(127, 0.51), (127, 0.4), (511, 1.0), (2047, 0.55), (2047, 0.45), (32767, 1.0), (7, 0.02), (7, 1e-3)])
+def test_actq_fwd_large_quotients(K, qmax, clip):
+    """row maxima of 249 to 32767 scales: either side of the limits up to which a lane may round u * rcp(s)"""
+    rng = np.random.default_rng(K + qmax)
+    M = 64
+    x = outliers(rng, (M, K))
+    x[1] = 0; x[1, ::128] = np.arange(K // 128) + 1                        # (chunks of one value each: equal quotients, half-integers among them)
+    for bf in (False, True):
+        src = O.f2bf(x) if bf else x
+        ry, rs, rc = O.actq_fwd(src, clip=clip, qmax=qmax, bf16=bf)
+        y = dev(np.zeros((M, K), np.uint16)); s = dev(np.zeros(M, np.float32))
+        call('camx_actq_fwd', ptr(dev(src)), I(int(bf)), ptr(y), ptr(s), NULL, I(K), F(clip), I(qmax), I(M))
+        assert bits_equal(host(s), rs) and bits_equal(host(y, np.uint16), ry)
+
+
 @pytest.mark.parametrize('M,d,nab', [(6, 896, 8), (5, 1024, 16), (3, 2048, 5), (2, 4096, 2), (130, 1024, 14), (4, 128, 1), (3, 8192, 3), (7, 768, 0),
                                      (9, 512, 6), (5, 256, 16), (300, 640, 3), (4, 1152, 9)])
 def test_block_entry_fwd(M, d, nab):
