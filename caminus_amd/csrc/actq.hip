@@ -39,6 +39,7 @@ CAMX_DEV f32x4 scaled4(f32x4 v) { v.x *= HSCALE; v.y *= HSCALE; v.z *= HSCALE; v
 CAMX_DEV void unpack_bf16x8(u32x4 w, f32x4 & a, f32x4 & b) { a = unpack_bf16x4((u32x2){w.x, w.y}); b = unpack_bf16x4((u32x2){w.z, w.w}); }
 struct PlainF32 {
     static constexpr bool bf16_valued = false, lds_tables = false; static constexpr int NW = 2;
+    static CAMX_DEV u32x4 absent(int) { return (u32x4){0u, 0u, 0u, 0u}; }           // what stands for the words of a chunk behind the row
     CAMX_DEV void set_small(const uint16_t *) {}
     const float * x; int K;
     CAMX_DEV f32x4 operator()(int row, int k) const { return *(const f32x4 *)(x + (size_t)row * K + k); }
@@ -48,6 +49,7 @@ struct PlainF32 {
 };
 struct PlainBF16 {
     static constexpr bool bf16_valued = true, lds_tables = false; static constexpr int NW = 1;
+    static CAMX_DEV u32x4 absent(int) { return (u32x4){0u, 0u, 0u, 0u}; }           // what stands for the words of a chunk behind the row
     CAMX_DEV void set_small(const uint16_t *) {}
     const uint16_t * x; int K;
     CAMX_DEV f32x4 operator()(int row, int k) const { return unpack_bf16x4(*(const u32x2 *)(x + (size_t)row * K + k)); }
@@ -55,32 +57,32 @@ struct PlainBF16 {
     CAMX_DEV void fetch(int row, int k, u32x4 (&w)[NW]) const { w[0] = *(const u32x4 *)(x + (size_t)row * K + k); }
     CAMX_DEV void value8(const u32x4 (&w)[NW], f32x4 & a, f32x4 & b, u32x4 &) const { unpack_bf16x8(w[0], a, b); }
 };
-// the bf16 words {t[g0], t[g1]} and {t[g2], t[g3]} of four packed bf16 gates: from the small table in LDS when there is one and it
-// holds all four, else from the full table in device memory
-CAMX_DEV u32x2 silu_lookup4(u32x2 gw, const uint16_t * small, const uint16_t * lut) {
-    u32x2 r;
-    bool outside = true;
-    if (small) {                                                           // (the index of a gate outside the table is a valid entry too)
-        outside = false;
-        const uint32_t i01 = small_index2(gw.x, outside), i23 = small_index2(gw.y, outside);
-        r.x = (uint32_t)small[i01 & 0xffffu] | ((uint32_t)small[i01 >> 16] << 16);
-        r.y = (uint32_t)small[i23 & 0xffffu] | ((uint32_t)small[i23 >> 16] << 16);
-    }
-    if (outside) {
-        r.x = (uint32_t)lut[gw.x & 0xffffu] | ((uint32_t)lut[gw.x >> 16] << 16);
-        r.y = (uint32_t)lut[gw.y & 0xffffu] | ((uint32_t)lut[gw.y >> 16] << 16);
-    }
-    return r;
+// the bf16 words {t[g0], t[g1]} and {t[g2], t[g3]} of four packed bf16 gates from the full table in device memory
+CAMX_DEV u32x2 silu_lookup4(u32x2 gw, const uint16_t * lut) {
+    return (u32x2){(uint32_t)lut[gw.x & 0xffffu] | ((uint32_t)lut[gw.x >> 16] << 16), (uint32_t)lut[gw.y & 0xffffu] | ((uint32_t)lut[gw.y >> 16] << 16)};
 }
 // Byte offsets of two packed gates' entries in the 16-bit small table, for the wave-per-row kernels: the sign falls out of a shift that
-// also scales the magnitude to bytes. most: the largest magnitude offset so far; SWS_LAST in it says that a gate is a zero or outside the
-// table, which the caller then settles four gates at a time as above (a compare per eight gates instead of four per two).
+// also scales the magnitude to bytes. most: the largest magnitude offset so far; SWS_LAST in it says that a gate is a zero, whose entry
+// that is, or outside the table: small_outside8 then tells which (a compare per eight gates instead of four per two). 16384 x 2048 with
+// half the gates zeros: forward 43.8 us, backward 96.2; 45.5 and 100.3 with zeros on the full tables' path. Chunks behind the row stand
+// as gates of 1 for the same reason: 16384 x 512 32.3 and 68.5 us, as zeros 38.9 and 75.4.
 constexpr uint16_t SWS_LAST = 2 * SWS_SPAN;
 CAMX_DEV uint32_t small_offset2(uint32_t w, u16x2 & most) {
     const u16x2 a = __builtin_bit_cast(u16x2, w) << (u16x2){1, 1};
     const u16x2 i = __builtin_elementwise_min(a - (u16x2){(uint16_t)(2 * SWS_A0), (uint16_t)(2 * SWS_A0)}, (u16x2){SWS_LAST, SWS_LAST});      // below the table: wraps, clamps
     most = __builtin_elementwise_max(most, i);
     return ((w >> 2) & 0x20002000u) | __builtin_bit_cast(uint32_t, i);
+}
+// whether one of eight packed gates is not in the small table (zeros are: less one they wrap to the largest number)
+CAMX_DEV bool small_outside8(u32x4 w) {
+    u16x2 low = {0xffff, 0xffff}, high = {0, 0};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t wi = w[i];
+        const u16x2 a = __builtin_bit_cast(u16x2, wi & 0x7fff7fffu);
+        low = __builtin_elementwise_min(low, a - (u16x2){1, 1}); high = __builtin_elementwise_max(high, a);
+    }
+    return (low.x < SWS_A0 - 1) | (low.y < SWS_A0 - 1) | (high.x >= SWS_A0 + SWS_SPAN) | (high.y >= SWS_A0 + SWS_SPAN);
 }
 CAMX_DEV uint32_t small_pair(const uint16_t * small, uint32_t o) {
     return (uint32_t)*(const uint16_t *)((const uint8_t *)small + (o & 0xffffu)) | ((uint32_t)*(const uint16_t *)((const uint8_t *)small + (o >> 16)) << 16);
@@ -96,21 +98,21 @@ struct SiluMulSrc {
         const uint16_t * r = gu + (size_t)row * ld;
         const u32x2 gw = *(const u32x2 *)(r + k);
         const f32x4 u = unpack_bf16x4(*(const u32x2 *)(r + F + k));
-        keep = silu_lookup4(gw, small, lut);
+        keep = silu_lookup4(gw, lut);
         const f32x4 sl = unpack_bf16x4(keep);
         return rbf4_any((f32x4){sl.x * u.x, sl.y * u.y, sl.z * u.z, sl.w * u.w});      // (feeds the rotation: of a NaN only its NaN-ness survives)
     }
     CAMX_DEV f32x4 operator()(int row, int k) const { u32x2 keep; return (*this)(row, k, keep); }
+    static CAMX_DEV u32x4 absent(int w) { return w ? (u32x4){0u, 0u, 0u, 0u} : (u32x4){0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u}; }      // gates of 1, multipliers of 0: +0 without a zero gate's check
     static constexpr int NW = 2;                   // the wave-per-row form: eight gates, eight multipliers
     CAMX_DEV void fetch(int row, int k, u32x4 (&w)[NW]) const { const uint16_t * r = gu + (size_t)row * ld + k; w[0] = *(const u32x4 *)r; w[1] = *(const u32x4 *)(r + F); }
     CAMX_DEV void value8(const u32x4 (&w)[NW], f32x4 & a, f32x4 & b, u32x4 & keep) const {
         u16x2 most = {0, 0};
         const uint32_t o0 = small_offset2(w[0].x, most), o1 = small_offset2(w[0].y, most), o2 = small_offset2(w[0].z, most), o3 = small_offset2(w[0].w, most);
-        if (most.x != SWS_LAST && most.y != SWS_LAST) keep = (u32x4){small_pair(small, o0), small_pair(small, o1), small_pair(small, o2), small_pair(small, o3)};
-        else {
-            const u32x2 k0 = silu_lookup4((u32x2){w[0].x, w[0].y}, small, lut), k1 = silu_lookup4((u32x2){w[0].z, w[0].w}, small, lut);
+        if (__builtin_expect(most.x == SWS_LAST || most.y == SWS_LAST, 0) && __builtin_expect(small_outside8(w[0]), 0)) {
+            const u32x2 k0 = silu_lookup4((u32x2){w[0].x, w[0].y}, lut), k1 = silu_lookup4((u32x2){w[0].z, w[0].w}, lut);
             keep = (u32x4){k0.x, k0.y, k1.x, k1.y};
-        }
+        } else keep = (u32x4){small_pair(small, o0), small_pair(small, o1), small_pair(small, o2), small_pair(small, o3)};
         f32x4 sa, sb, ua, ub;
         unpack_bf16x8(keep, sa, sb); unpack_bf16x8(w[1], ua, ub);
         a = rbf4_any((f32x4){sa.x * ua.x, sa.y * ua.y, sa.z * ua.z, sa.w * ua.w});
@@ -343,7 +345,7 @@ CAMX_DEV void fetch_row_w(const Src & src, int row, int c, int q, bool on, u32x4
 #pragma unroll
     for (int j = 0; j < 4; j++) {
 #pragma unroll
-        for (int w = 0; w < Src::NW; w++) raw[j][w] = (u32x4){0u, 0u, 0u, 0u};
+        for (int w = 0; w < Src::NW; w++) raw[j][w] = Src::absent(w);
         if (on) src.fetch(row, c * 128 + 32 * j + 8 * q, raw[j]);
     }
 }
@@ -491,17 +493,7 @@ struct SinkSiluMul {
     }
     // four values' dg and du from their gates, multipliers, bf16(silu g) and dact
     CAMX_DEV void grads4(u32x2 gw, u32x2 uw, u32x2 keep, f32x4 dact, u32x2 & dgp, u32x2 & dup) const { grads4(gw, uw, keep, dact, sigmoids4(gw), dgp, dup); }
-    CAMX_DEV f32x4 sigmoids4(u32x2 gw) const {
-        bool outside = true;
-        f32x4 sig;
-        if (dsmall) {
-            outside = false;
-            const uint32_t i01 = small_index2(gw.x, outside), i23 = small_index2(gw.y, outside);
-            sig = (f32x4){dsmall[i01 & 0xffffu], dsmall[i01 >> 16], dsmall[i23 & 0xffffu], dsmall[i23 >> 16]};
-        }
-        if (outside) sig = (f32x4){dlut[gw.x & 0xffffu], dlut[gw.x >> 16], dlut[gw.y & 0xffffu], dlut[gw.y >> 16]};
-        return sig;
-    }
+    CAMX_DEV f32x4 sigmoids4(u32x2 gw) const { return (f32x4){dlut[gw.x & 0xffffu], dlut[gw.x >> 16], dlut[gw.y & 0xffffu], dlut[gw.y >> 16]}; }
     CAMX_DEV float small_at(uint32_t o) const { return *(const float *)((const uint8_t *)dsmall + o); }
     CAMX_DEV f32x4 small4(uint32_t o0, uint32_t o1) const {               // from the byte offsets into the 16-bit table
         const uint32_t a = o0 << 1, b = o1 << 1;                          // (the offsets use 14 bits of each half)
@@ -525,8 +517,8 @@ struct SinkSiluMul {
         u16x2 most = {0, 0};
         const uint32_t o0 = small_offset2(gw.x, most), o1 = small_offset2(gw.y, most), o2 = small_offset2(gw.z, most), o3 = small_offset2(gw.w, most);
         f32x4 s0, s1;
-        if (most.x != SWS_LAST && most.y != SWS_LAST) { s0 = small4(o0, o1); s1 = small4(o2, o3); }
-        else { s0 = sigmoids4((u32x2){gw.x, gw.y}); s1 = sigmoids4((u32x2){gw.z, gw.w}); }
+        if (__builtin_expect(most.x == SWS_LAST || most.y == SWS_LAST, 0) && __builtin_expect(small_outside8(gw), 0)) { s0 = sigmoids4((u32x2){gw.x, gw.y}); s1 = sigmoids4((u32x2){gw.z, gw.w}); }
+        else { s0 = small4(o0, o1); s1 = small4(o2, o3); }
         grads4((u32x2){gw.x, gw.y}, (u32x2){uw.x, uw.y}, (u32x2){keep.x, keep.y}, rbf4_any(a), s0, dg0, du0);      // (a NaN's bits are settled by the stores' rounding)
         grads4((u32x2){gw.z, gw.w}, (u32x2){uw.z, uw.w}, (u32x2){keep.z, keep.w}, rbf4_any(b), s1, dg1, du1);
         uint16_t * o = dgu + (size_t)row * (2 * F) + k;

@@ -166,6 +166,25 @@ def test_silu_mul_actq_bwd(M, Fh, ld):
     assert bits_equal(got, O.silu_mul_actq_bwd(gu, g, table=True))        # bit for bit against the table's own definition (every gate here is finite)
 
 
+@pytest.mark.parametrize('Fh', [128, 1152, 1920, 2048, 2304])
+def test_silu_mul_actq_zero_gates(Fh):
+    """zeros of both signs are inside the small tables: rows of nothing else, half zeros, one zero among eight gates, zeros beside gates
+    outside the tables, and zero multipliers; row widths that leave lanes of a wave without a chunk. Forward and backward bit for bit"""
+    rng = np.random.default_rng(40 + Fh)
+    M = 9
+    gate = (rng.standard_normal((M, Fh)) * 2).astype(np.float32); up = rng.standard_normal((M, Fh)).astype(np.float32)
+    gate[0] = 0.0; gate[1] = -0.0; gate[2] = np.where(rng.random(Fh) < 0.5, 0.0, gate[2]); gate[3, 3::8] = -0.0
+    gate[4, ::8] = 0.0; gate[4, 1::16] = 300.0; gate[4, 2::32] = -2.0 ** -26; gate[5, ::8] = 2.0 ** -24; gate[5, 1::8] = -0.0; gate[6] = 0.0; gate[6, 9] = 1e-30
+    up[7] = 0.0; up[8, ::2] = -0.0
+    gu = O.f2bf(np.concatenate([gate, up], axis=1)); g = O.f2bf(rng.standard_normal((M, Fh)).astype(np.float32))
+    y = dev(np.zeros((M, Fh), np.uint16)); s = dev(np.zeros(M, np.float32)); c = dev(np.zeros((M, Fh // 2), np.uint8)); dgu = dev(np.zeros((M, 2 * Fh), np.uint16))
+    call('camx_silu_mul_actq_fwd', ptr(dev(gu)), I(2 * Fh), I(Fh), ptr(y), ptr(s), ptr(c), F(1.0), I(7), I(M))
+    fy, fs, fc = O.silu_mul_actq_fwd(gu)
+    assert bits_equal(host(s), fs) and bits_equal(host(c), fc) and bits_equal(host(y, np.uint16), fy)
+    call('camx_silu_mul_actq_bwd', ptr(dev(gu)), I(2 * Fh), I(Fh), ptr(dev(g)), ptr(dgu), F(1.0), I(7), I(M))
+    assert bits_equal(host(dgu, np.uint16), O.silu_mul_actq_bwd(gu, g, table=True))
+
+
 @pytest.mark.parametrize('M,Fh', [(6, 1024), (1200, 256), (5, 2304)])
 def test_silu_mul_actq_gates_of_every_magnitude(M, Fh):
     """gates and multipliers over the whole bf16 exponent range (most gates outside the small tables the wave-per-row kernels hold in
