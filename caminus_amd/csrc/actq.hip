@@ -560,14 +560,18 @@ CAMX_DEV void actq_bwd_row(Src src, int row, const uint16_t * __restrict__ g, Si
 #define D_(e) { float m; const float x = ste(t4.e, m); dlds = __builtin_fmaf(gv[c].e, x, dlds); gv[c].e = gv[c].e * m; }
             CAMX_EACH4(D_)
 #undef D_
-            const float most = fmaxf(fmaxf(fabsf(u[c].x), fabsf(u[c].y)), fmaxf(fabsf(u[c].z), fabsf(u[c].w)));
-            if (__builtin_amdgcn_ballot_w64(most == amax) != 0) {          // (few rounds hold such an element)
-                tied |= 1u << c;
-#define T_(e) { const uint64_t tie = __builtin_amdgcn_ballot_w64(fabsf(u[c].e) == amax); \
+#define T_(e) { const uint64_t tie = __builtin_amdgcn_ballot_w64(fabsf(u[c].e) == amax); any |= tie; \
                 ties_lo += __builtin_popcount((uint32_t)tie); ties_hi += __builtin_popcount((uint32_t)(tie >> 32)); }
-                CAMX_EACH4(T_)
-#undef T_
+            uint64_t any = 0;
+            // a wave per row: few rounds hold such an element, so they are looked for first. (In the workgroup form that look costs up to five
+            // registers, a wave per SIMD at several widths: 8192 rows of 7168 bf16 values 102.6 us with it, 94.2 without, fused 8192 x 6144 186 and 173)
+            if (NHW == 8) { CAMX_EACH4(T_) }
+            else {
+                const float most = fmaxf(fmaxf(fabsf(u[c].x), fabsf(u[c].y)), fmaxf(fabsf(u[c].z), fabsf(u[c].w)));
+                if (__builtin_amdgcn_ballot_w64(most == amax) != 0) { CAMX_EACH4(T_) }
             }
+#undef T_
+            if (any) tied |= 1u << c;
         }
         if (NHW == 2) part[NHW == 2 ? c : 0] = dlds;
     }

@@ -82,7 +82,7 @@ def test_silu_mul_actq_fwd(M, Fh):
 # ---- backward ----------------------------------------------------------------------------------------------------------------
 
 @pytest.mark.parametrize('M,K,qmax', [(5, 896, 7), (3, 2048, 7), (2, 8192, 7), (4, 128, 3), (3, 768, 127), (300, 1024, 7), (7, 5120, 7), (9, 1152, 7), (6, 1920, 7),
-                                      (5, 1536, 15)])
+                                      (5, 1536, 15), (4, 4096, 7), (4, 6144, 7), (3, 7168, 7)])
 def test_actq_bwd(M, K, qmax):
     rng = np.random.default_rng(100 + K + qmax)
     x = outliers(rng, (M, K)); x[0] = 0
