@@ -629,9 +629,10 @@ int camx_quantize_mmq_q8_1_scatter(const float * x, const int32_t * ids, void * 
     if (!x || !vy || !ids || ne00 < 4 || ne00 % 4 || s02 < ne00 || s02 % 4 || ne0 % 512 || ne0 < ne00 || ne0 >= ne00 + 512 || ne2 != 1 ||
         n_expert_used < 1 || ntok < 0 || ne1 != ntok * n_expert_used || (layout != MMQ_D4 && layout != MMQ_DS4) ||
         ((uintptr_t)x & 15) || ((uintptr_t)vy & 15)) return CAMX_EINVAL;
-    // a prefill chunk takes the one-shot form. To 8 columns each: 1536 tokens x 5120 20.8 us against the rows kernel's 31.4, 1024 x 5120
-    // 15.0 and 15.2, 777 x 5120 13.6 and 12.5; 2047 x 2048 12.4 and 12.9, 1536 x 2048 10.8 and 10.7
-    if ((ntok >= 2048 || (long)ntok * ne00 >= 5 << 20) && ne0 / 128 <= 65535 && (long)ntok * n_expert_used < 0x7fffffffL) {
+    // a prefill chunk takes the one-shot form. Fewer tokens of wide rows gain by it only where the rows come from memory: 1500 x 5120 to
+    // one column each 11.8 us against the rows kernel's 13.8, to eight 30.6 and 37.2; where the launch before has just written them
+    // (21 - 58 MB, the Infinity Cache) it loses: 10.8 and 10.0 us, 1280 x 7168 13.9 and 11.5, to eight 40.6 and 36.5
+    if (ntok >= 2048 && ne0 / 128 <= 65535 && (long)ntok * n_expert_used < 0x7fffffffL) {
         launch_oneshot_scatter(x, ids, s02, ne00, vy, ntok, n_expert_used, ne1, ne0 / 128, layout, st);
         CAMX_LAUNCH_RET();
     }

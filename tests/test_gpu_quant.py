@@ -71,9 +71,9 @@ def test_mmq_quantize_scatter(K, ntok, k, pad):
         assert bits_equal(host(y), ref)
 
 
-@pytest.mark.parametrize('K,ntok,k', [(7492, 700, 2), (7488, 701, 1), (5120, 1024, 3), (5116, 1025, 1)])
-def test_mmq_quantize_scatter_by_values(K, ntok, k):
-    """fewer than 2048 tokens of wide rows: either side of the 5 Mi values from which the one-shot form takes them"""
+@pytest.mark.parametrize('K,ntok,k', [(7492, 700, 2), (7488, 701, 1), (5120, 1024, 3), (5116, 1025, 1), (2052, 2047, 2), (2052, 2048, 2)])
+def test_mmq_quantize_scatter_wide_rows(K, ntok, k):
+    """wide rows on either side of the 2048 tokens from which the one-shot form takes them"""
     test_mmq_quantize_scatter(K, ntok, k, 0)
 
 
