@@ -293,9 +293,10 @@ __global__ void __launch_bounds__(256) ple_gate_k(const float * kn, const float 
 // workgroup share its val row through the caches. Memory bound: with 4-byte loads, two barriers and an integer division per stored
 // value the kernel above takes 80 us for the 273 MB of 2048 tokens x 4 streams x 2560, this one 51 (53 with plain loads of q); PLE_UNR steps of loads are issued ahead of their sums.
 // (gated may alias kn: a wave stores its own row only, after the dot product that consumed it)
-constexpr int PLE_UNR = 5;                               // 2560 values: two batches, 40 registers of loads in flight
+// PLE_UNR: 256-value steps of a batch of loads, at most five (2560 values: two batches, 40 registers of loads in flight), chosen for equal
+// batches: steps behind the row repeat its last values (2048 x 8 x 128 with five steps a batch 12.4 us, with one 8.1; the kernel above: 9.2).
 CAMX_DEV void ple_dot4(f32x4 & acc, f32x4 k, f32x4 q) { acc.x = acc.x + k.x * q.x; acc.y = acc.y + k.y * q.y; acc.z = acc.z + k.z * q.z; acc.w = acc.w + k.w * q.w; }
-template <bool REC>
+template <bool REC, int PLE_UNR>
 __global__ void __launch_bounds__(512) ple_gate_rows(const float * kn, const float * q, const float * __restrict__ qscl, const float * __restrict__ qw,
                                                      const float * __restrict__ val, int ldv, float * gated, float * gate_out, int HC, int D) {
     const int p = slot_of(threadIdx.x & 63), st = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -571,8 +572,13 @@ int camx_pf_ple_gate(const float * kn, const float * q, const float * qscl, cons
     if (!kn || !q || !val || !gated || !gate_out || HC < 1 || HC > 8 || D < 1 || ldv < D || T < 0 || ((qscl == nullptr) != (qw == nullptr))) return CAMX_EINVAL;
     if (T == 0) return CAMX_OK;
     if (D % 4 == 0 && ldv % 4 == 0 && !(((uintptr_t)kn | (uintptr_t)q | (uintptr_t)qw | (uintptr_t)val | (uintptr_t)gated) & 15)) {      // 128-bit accesses
-        if (qscl) ple_gate_rows<true><<<dim3(T), dim3(64 * HC), 0, st>>>(kn, q, qscl, qw, val, ldv, gated, gate_out, HC, D);
-        else ple_gate_rows<false><<<dim3(T), dim3(64 * HC), 0, st>>>(kn, q, qscl, qw, val, ldv, gated, gate_out, HC, D);
+        const int steps = (D + 255) / 256, batches = (steps + 4) / 5;
+#define PLE_ROWS(U) { if (qscl) ple_gate_rows<true, U><<<dim3(T), dim3(64 * HC), 0, st>>>(kn, q, qscl, qw, val, ldv, gated, gate_out, HC, D); \
+                      else ple_gate_rows<false, U><<<dim3(T), dim3(64 * HC), 0, st>>>(kn, q, qscl, qw, val, ldv, gated, gate_out, HC, D); }
+        switch ((steps + batches - 1) / batches) {
+            case 1: PLE_ROWS(1) break; case 2: PLE_ROWS(2) break; case 3: PLE_ROWS(3) break; case 4: PLE_ROWS(4) break; default: PLE_ROWS(5) break;
+        }
+#undef PLE_ROWS
         CAMX_LAUNCH_RET();
     }
     ple_gate_k<<<dim3(T), dim3(256), 0, st>>>(kn, q, qscl, qw, val, ldv, gated, gate_out, HC, D);

@@ -108,10 +108,11 @@ def test_ple_gate_conv_hist(T, HC, D, dil):
     assert bits_equal(host(hd), O.ple_hist(x[:2], hist, D, dil))
 
 
-@pytest.mark.parametrize('T,HC,D', [(3, 8, 4), (5, 1, 252), (2, 3, 1280), (4, 2, 1284), (3, 4, 2560), (1, 5, 4092)])
+@pytest.mark.parametrize('T,HC,D', [(3, 8, 4), (5, 1, 252), (2, 3, 1280), (4, 2, 1284), (3, 4, 2560), (1, 5, 4092),
+                                   (3, 2, 260), (2, 8, 764), (5, 3, 1024), (2, 2, 1536), (3, 1, 2044)])
 def test_ple_gate_wave_per_stream_equals_workgroup_per_token(T, HC, D):
     """the 128-bit form (D % 4 == 0, ldv % 4 == 0) gives the bits of the general kernel, which an odd ldv selects: lengths around a wave's
-    step of 256 values and around a batch of five steps, and in place"""
+    step of 256 values and around batches of one to five steps, and in place"""
     rng = np.random.default_rng(D)
     kn = outliers(rng, (T, HC, D)); q = outliers(rng, (T, HC, D)); val = rng.standard_normal((T, D + 5)).astype(f32)
     qscl = (0.5 + rng.random(T * HC)).astype(f32); qw = (1 + 0.1 * rng.standard_normal((HC, D))).astype(f32)
