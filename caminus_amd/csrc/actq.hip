@@ -1010,12 +1010,13 @@ __global__ void __launch_bounds__(64) block_entry_bwd_k(const float * x, const f
     rms_bwd_row(src, dh, dx + (size_t)row * d, d, la);
 }
 
-// The same for nab > 0 with the projections' part on the matrix cores (as vector multiply-adds of the row's own wave 139 us at 32768 x
-// 1024 with 16 projections, this kernel 113; 512 rows: 12.3 and 8.7): a workgroup's four waves own a row each, and wave w first computes
-// that part for columns 256 w .. 256 w + 255 of all four rows. A K = 1 instruction adds one j's term dab[row][j] wab[j][column] (rounded
-// like fmaf) for 4 rows x 64 columns: block Q's four columns are its lanes' own, so with A = dab (lane 4 Q + i: row i) and B = a lane's
-// column of wab, D holds a lane's column with a word per row. The two groups' sums,
-// rounded to bf16, reach the rows' owners through LDS.
+// The same for nab > 0 with the projections' part on the matrix cores (as vector multiply-adds of the row's own wave 143 us at 32768 x
+// 1024 with 16 projections, this kernel 115; 512 rows: 13.1 and 9.6): a workgroup's four waves own a row each and first compute a quarter
+// of that part for all four rows, one of the two groups for half of the column blocks of 256 (32768 x 256 with 4 projections 31.8 us, as
+// one wave per column block 36.4, with vector multiply-adds 34.3). A K = 1 instruction adds one j's term dab[row][j] wab[j][column]
+// (rounded like fmaf) for 4 rows x 64 columns: block Q's four columns are its lanes' own, so with A = dab (lane 4 Q + i: row i) and B = a
+// lane's column of wab, D holds a lane's column with a word per row. The two groups' sums, rounded to bf16, reach the rows' owners
+// through LDS.
 template <int NR>
 __global__ void __launch_bounds__(256, 4) block_entry_bwd_quad(const float * x, const float * __restrict__ nw, const float * __restrict__ rstd_in, const uint16_t * __restrict__ wab,
                                                                int nab, const uint16_t * __restrict__ dy, const uint16_t * __restrict__ dab, float * dx, int d, float clip, int qmax, int M) {
@@ -1037,34 +1038,40 @@ __global__ void __launch_bounds__(256, 4) block_entry_bwd_quad(const float * x, 
         if (c < NR - 1 || k < d) src.xk[c] = __builtin_nontemporal_load((const f32x4 *)(x + (size_t)row * d + k));
     }
     src.rstd = rstd_in[row];
-    if (wave < NR) {
-        u32x2 B[2][8];
+    // wave w: group w & 1 of column blocks (w >> 1) and (w >> 1) + 2; of a single block words w >> 1 of each lane's two
+    constexpr int NT = (2 * NR + 3) / 4, NP = NR == 1 ? 1 : 2;
+    const int h = wave & 1, c0 = NR == 1 ? 0 : wave >> 1, p0 = NR == 1 ? wave >> 1 : 0;
+    uint32_t B[NT][8][NP];
 #pragma unroll
-        for (int h = 0; h < 2; h++)
+    for (int t = 0; t < NT; t++)
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int k = 256 * wave + 4 * la;
-                B[h][j] = (u32x2){0u, 0u};
-                if (j < half && k < d) B[h][j] = *(const u32x2 *)(wab + (size_t)(h * half + j) * d + k);
+        for (int j = 0; j < 8; j++) {
+            const int k = 256 * (c0 + 2 * t) + 4 * la;
+            const uint16_t * b = wab + (size_t)(h * half + j) * d + k;
+            const bool on = j < half && k < d;
+            if (NP == 1) B[t][j][0] = on ? ((const uint32_t *)b)[p0] : 0u;
+            else { u32x2 v = {0u, 0u}; if (on) v = *(const u32x2 *)b; B[t][j][0] = v.x; B[t][j][NP - 1] = v.y; }
+        }
+    const uint16_t * ar = dab + (size_t)min(r0 + (lraw & 3), M - 1) * nab + h * half;
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const int cb = c0 + 2 * t;
+        if (cb >= NR) break;                             // (uniform)
+        f32x4 acc[2 * NP];
+#pragma unroll
+        for (int k = 0; k < 2 * NP; k++) acc[k] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            if (j < half) {                              // (uniform)
+                const float av = bf2f(ar[j]);
+#pragma unroll
+                for (int k = 0; k < 2 * NP; k++) acc[k] = __builtin_amdgcn_mfma_f32_4x4x1f32(av, k & 1 ? bf_hi(B[t][j][k >> 1]) : bf_lo(B[t][j][k >> 1]), acc[k], 0, 0, 0);
             }
-        const uint16_t * ar = dab + (size_t)min(r0 + (lraw & 3), M - 1) * nab;
+        }
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            f32x4 acc[4];
-#pragma unroll
-            for (int k = 0; k < 4; k++) acc[k] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                if (j < half) {                      // (uniform)
-                    const float av = bf2f(ar[h * half + j]);
-                    acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(av, bf_lo(B[h][j].x), acc[0], 0, 0, 0);
-                    acc[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(av, bf_hi(B[h][j].x), acc[1], 0, 0, 0);
-                    acc[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(av, bf_lo(B[h][j].y), acc[2], 0, 0, 0);
-                    acc[3] = __builtin_amdgcn_mfma_f32_4x4x1f32(av, bf_hi(B[h][j].y), acc[3], 0, 0, 0);
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < 4; r++) *(u32x2 *)&pbuf[r][h][128 * wave + 2 * la] = pack_f2bf_x4((f32x4){acc[0][r], acc[1][r], acc[2][r], acc[3][r]});
+        for (int r = 0; r < 4; r++) {
+            if (NP == 1) pbuf[r][h][2 * la + p0] = pack_f2bf_x4((f32x4){acc[0][r], acc[1][r], 0.0f, 0.0f}).x;
+            else *(u32x2 *)&pbuf[r][h][128 * cb + 2 * la] = pack_f2bf_x4((f32x4){acc[0][r], acc[1][r], acc[2 * NP - 2][r], acc[2 * NP - 1][r]});
         }
     }
     f32x4 dh[NR];

@@ -122,7 +122,8 @@ def test_actq_bwd_quotients_at_the_exponent_limits(K):
             assert np.array_equal(nan_w, nan_g) and bits_equal(np.where(nan_w, 0, got), np.where(nan_w, 0, want))
 
 
-@pytest.mark.parametrize('M,d,nab', [(6, 896, 14), (5, 1024, 0), (9, 256, 2), (130, 896, 16), (7, 1024, 16), (3, 128, 4), (171, 896, 8), (12, 640, 6), (9, 384, 0)])
+@pytest.mark.parametrize('M,d,nab', [(6, 896, 14), (5, 1024, 0), (9, 256, 2), (130, 896, 16), (7, 1024, 16), (3, 128, 4), (171, 896, 8), (12, 640, 6), (9, 384, 0),
+                                     (10, 256, 14), (6, 128, 16), (5, 512, 10), (6, 768, 16)])
 def test_block_entry_bwd(M, d, nab):
     """every round count of the wave-per-row kernel; row 1 has one value in the row's last chunk and one in chunk 1 with the same
     |h|: their chunks rotate to constants, so 256 elements tie for the row's maximum across rounds that not all lanes take part in"""
