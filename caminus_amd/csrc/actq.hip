@@ -752,58 +752,59 @@ struct AbTerm {
     CAMX_DEV f32x4 other(int k) const { return unpack_bf16x4(*(const u32x2 *)(wab + k)); }
 };
 
-// NHW = 8: a 256-thread workgroup per row (NR rounds of 1024 values); NHW = 2: one wave per row for rows of at most 1024 values (NR
-// rounds of 256) without projections: a lane then holds 16 values instead of 4, and what every lane computes once per row (the square
-// root, the divisions, the reductions' tails) is spread over four times as many values.
-// The projections: wave w takes rows w, w + W, ... of wab (W waves per row), up to four of them at a time so that their loads fly together,
-// each under the 256-thread tree (a lane holds the logical threads 4 lane .. 4 lane + 3, which add their elements 256 apart in
-// order); rows of at most 2048 values keep bf16(h) in registers.
-template <int NR, int NHW>
-__global__ void __launch_bounds__(32 * NHW) block_entry_fwd_k(const float * x, const float * nw, const uint16_t * wab, int nab, float eps, uint16_t * y,
-                                                              float * s, uint16_t * codes, uint16_t * ab, float * rstd_out, int d, float clip, int qmax) {
+// One wave per row for rows of at most 1024 values (NR rounds of 256) without projections: a lane holds 16 values instead of the
+// workgroup form's 4, and what every lane computes once per row (the square root, the divisions, the reductions' tails) is spread over
+// four times as many values.
+template <int NR>
+__global__ void __launch_bounds__(64) block_entry_fwd_wave(const float * x, const float * nw, float eps, uint16_t * y, float * s, uint16_t * codes, float * rstd_out,
+                                                           int d, float clip, int qmax) {
+    const int row = blockIdx.x, lane = slot_of(threadIdx.x);
+    const float * xr = x + (size_t)row * d;
+    RmsRegSrc<NR> src;                                   // the row and the norm weights in registers: every HBM byte of x crosses once
+#pragma unroll
+    for (int c = 0; c < NR; c++) {
+        const int k = 256 * c + 4 * lane;
+        src.xk[c] = src.wk[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+        if (k < d) { src.xk[c] = __builtin_nontemporal_load((const f32x4 *)(xr + k)); src.wk[c] = *(const f32x4 *)(nw + k); }
+    }
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int c = 0; c < NR; c++)
+        if (256 * c + 4 * lane < d) {
+            acc.x = __builtin_fmaf(src.xk[c].x, src.xk[c].x, acc.x); acc.y = __builtin_fmaf(src.xk[c].y, src.xk[c].y, acc.y);
+            acc.z = __builtin_fmaf(src.xk[c].z, src.xk[c].z, acc.z); acc.w = __builtin_fmaf(src.xk[c].w, src.xk[c].w, acc.w);
+        }
+    const float ss = wave_groups_in_order(group32_sum(acc));
+    src.rstd = rsqrt_exact(ss / (float)d + eps);
+    if (threadIdx.x == 0 && rstd_out) rstd_out[row] = src.rstd;
+    actq_fwd_row<NR, RmsRegSrc<NR>, 2>(src, row, y, s, d, clip, qmax, codes, nullptr);
+}
+
+// Longer rows: a 256-thread workgroup per row (NR rounds of 1024 values). The projections: wave w takes rows w, w + 4, ... of wab, up to
+// two of them at a time so that their loads fly together, each under the 256-thread tree (a lane holds the logical threads 4 lane ..
+// 4 lane + 3, which add their elements 256 apart in order); rows of at most 2048 values keep bf16(h) in registers.
+template <int NR>
+__global__ void __launch_bounds__(256) block_entry_fwd_k(const float * x, const float * nw, const uint16_t * wab, int nab, float eps, uint16_t * y,
+                                                         float * s, uint16_t * codes, uint16_t * ab, float * rstd_out, int d, float clip, int qmax) {
     __shared__ float lds[4];
     __shared__ float slot;
     const int row = blockIdx.x;
     const float * xr = x + (size_t)row * d;
-    constexpr int NW = NHW / 2, NA = NR * NHW / 2;       // waves per row; 256-element steps of a row
+    constexpr int NW = 4, NA = 4 * NR;                   // waves per row; 256-element steps of a row
     constexpr bool KEEP = NA <= 8;
     const int lane = slot_of(threadIdx.x & 63), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     f32x4 hk[KEEP ? NA : 1];
-    float rstd;
-    if constexpr (NHW == 2) {                            // the row and the norm weights in registers: every HBM byte of x crosses once
-        RmsRegSrc<NR> src;
-#pragma unroll
-        for (int c = 0; c < NR; c++) {
-            const int k = 256 * c + 4 * lane;
-            src.xk[c] = src.wk[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-            if (k < d) { src.xk[c] = __builtin_nontemporal_load((const f32x4 *)(xr + k)); src.wk[c] = *(const f32x4 *)(nw + k); }
-        }
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int c = 0; c < NR; c++)
-            if (256 * c + 4 * lane < d) {
-                acc.x = __builtin_fmaf(src.xk[c].x, src.xk[c].x, acc.x); acc.y = __builtin_fmaf(src.xk[c].y, src.xk[c].y, acc.y);
-                acc.z = __builtin_fmaf(src.xk[c].z, src.xk[c].z, acc.z); acc.w = __builtin_fmaf(src.xk[c].w, src.xk[c].w, acc.w);
-            }
-        const float ss = wave_groups_in_order(group32_sum(acc));
-        rstd = rsqrt_exact(ss / (float)d + eps);
-        src.rstd = rstd;
-        if (threadIdx.x == 0 && rstd_out) rstd_out[row] = rstd;
-        actq_fwd_row<NR, RmsRegSrc<NR>, NHW>(src, row, y, s, d, clip, qmax, codes, lds);
-        return;
-    } else {
-        const float ss = row_tree_sum(SqTerm{xr}, d, &slot);
-        rstd = rsqrt_exact(ss / (float)d + eps);
-        if (threadIdx.x == 0 && rstd_out) rstd_out[row] = rstd;
-        actq_fwd_row<NR, RmsSrc, NHW>(RmsSrc{x, nw, rstd, d}, row, y, s, d, clip, qmax, codes, lds);
-        if (nab == 0) return;
-    }
+    const float ss = row_tree_sum(SqTerm{xr}, d, &slot);
+    const float rstd = rsqrt_exact(ss / (float)d + eps);
+    if (threadIdx.x == 0 && rstd_out) rstd_out[row] = rstd;
+    actq_fwd_row<NR, RmsSrc>(RmsSrc{x, nw, rstd, d}, row, y, s, d, clip, qmax, codes, lds);
+    if (nab == 0) return;
     const AbTerm term{xr, nw, rstd, wab};
     if (KEEP) {
 #pragma unroll
         for (int i = 0; i < NA; i++) { const int k = 256 * i + 4 * lane; hk[KEEP ? i : 0] = k < d ? term(k) : (f32x4){0.0f, 0.0f, 0.0f, 0.0f}; }
     }
-    constexpr int JB = NA <= 4 ? 4 : NA <= 8 ? 2 : 1;   // rows of wab whose loads fly together
+    constexpr int JB = NA <= 8 ? 2 : 1;                  // rows of wab whose loads fly together
     for (int j0 = wave; j0 < nab; j0 += JB * NW) {
         u32x2 wv[JB][NA];
 #pragma unroll
@@ -1178,14 +1179,14 @@ int camx_block_entry_fwd(const float * x, const float * nw, const uint16_t * wab
     }
     if (d <= 1024) {                                     // one wave per row, rounds of 256 values
         switch ((d + 255) / 256) {
-            case 1: block_entry_fwd_k<1, 2><<<dim3(M), dim3(64), 0, st>>>(x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax); break;
-            case 2: block_entry_fwd_k<2, 2><<<dim3(M), dim3(64), 0, st>>>(x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax); break;
-            case 3: block_entry_fwd_k<3, 2><<<dim3(M), dim3(64), 0, st>>>(x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax); break;
-            default: block_entry_fwd_k<4, 2><<<dim3(M), dim3(64), 0, st>>>(x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax); break;
+            case 1: block_entry_fwd_wave<1><<<dim3(M), dim3(64), 0, st>>>(x, nw, eps, y, s, codes, rstd_out, d, clip, qmax); break;
+            case 2: block_entry_fwd_wave<2><<<dim3(M), dim3(64), 0, st>>>(x, nw, eps, y, s, codes, rstd_out, d, clip, qmax); break;
+            case 3: block_entry_fwd_wave<3><<<dim3(M), dim3(64), 0, st>>>(x, nw, eps, y, s, codes, rstd_out, d, clip, qmax); break;
+            default: block_entry_fwd_wave<4><<<dim3(M), dim3(64), 0, st>>>(x, nw, eps, y, s, codes, rstd_out, d, clip, qmax); break;
         }
         CAMX_LAUNCH_RET();
     }
-    ACTQ_ROUNDS(d, (block_entry_fwd_k<NR, 8><<<dim3(M), dim3(256), 0, st>>>(x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax)))
+    ACTQ_ROUNDS(d, (block_entry_fwd_k<NR><<<dim3(M), dim3(256), 0, st>>>(x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax)))
     CAMX_LAUNCH_RET();
 }
 

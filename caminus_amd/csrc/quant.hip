@@ -244,31 +244,18 @@ CAMX_DEV float max3_abs(float a, float b, float c) { return fmaxf(fmaxf(fabsf(a)
 
 struct SwmItem { u32x4 gw[2], uw[2]; };
 
-// issue the four 128-bit loads of work item (tokens tg .. tg + 7, block column unit). Every lane always issues all four
-// (a lane past the row's end or past the last token, or a whole wave without work, reads 16 zero bytes instead): with a
-// fixed number of loads in flight the compiler can wait for exactly the older item's data and leave this item's loads
-// outstanding across the other item's arithmetic.
-template <int SRC>
-CAMX_DEV void swm_load(SwmItem & it, const void * __restrict__ src, const int32_t * __restrict__ ids, long ld, long F, int T, long tg, long unit,
-                       int lane, bool valid) {
+// issue the four 128-bit loads of work item (tokens tg .. tg + 7, block column unit) of bf16 rows [g | u]; a lane past the row's end or
+// past the last token reads 16 zero bytes instead
+CAMX_DEV void swm_load(SwmItem & it, const uint16_t * __restrict__ gu, long ld, long F, int T, long tg, long unit, int lane) {
     const long e0 = unit * 128 + 8 * (lane & 15);
 #pragma unroll
     for (int i = 0; i < 2; i++) {
         const long t = tg + (lane >> 4) + 4 * i;
-        const bool tok = valid && t < T;
-        if (SRC == SRC_SWIGLU_BF16) {
-            const bool ok = tok && e0 < F;
-            const uint16_t * r = (const uint16_t *)src + (size_t)(ok ? t : 0) * ld + e0;
-            const u32x4 * pg = ok ? (const u32x4 *)r : (const u32x4 *)g_zero16;
-            const u32x4 * pu = ok ? (const u32x4 *)(r + F) : (const u32x4 *)g_zero16;
-            it.gw[i] = __builtin_nontemporal_load(pg); it.uw[i] = __builtin_nontemporal_load(pu);     // read once, never written: +15 % over plain loads
-        } else {                                                // fp32 rows: gw[i] = values 0 .. 3, uw[i] = values 4 .. 7 of the lane's eight
-            const long row = tok ? (ids ? ids[t] : t) : 0;
-            const float * r = (const float *)src + (size_t)row * ld + e0;
-            const u32x4 * p0 = tok && e0 < F ? (const u32x4 *)r : (const u32x4 *)g_zero16;
-            const u32x4 * p1 = tok && e0 + 4 < F ? (const u32x4 *)(r + 4) : (const u32x4 *)g_zero16;
-            it.gw[i] = __builtin_nontemporal_load(p0); it.uw[i] = __builtin_nontemporal_load(p1);
-        }
+        const bool ok = t < T && e0 < F;
+        const uint16_t * r = gu + (size_t)(ok ? t : 0) * ld + e0;
+        const u32x4 * pg = ok ? (const u32x4 *)r : (const u32x4 *)g_zero16;
+        const u32x4 * pu = ok ? (const u32x4 *)(r + F) : (const u32x4 *)g_zero16;
+        it.gw[i] = __builtin_nontemporal_load(pg); it.uw[i] = __builtin_nontemporal_load(pu);     // read once, never written: +15 % over plain loads
     }
 }
 
@@ -427,7 +414,7 @@ __global__ void __launch_bounds__(SWS_WAVES * 64) swiglu_mmq_oneshot(const void 
             }
     } else {
 #pragma unroll
-        for (int k = 0; k < SWS_IPW; k++) swm_load<SRC>(it[k], gu, ids, ld, F, T, tg0 + SWM_TOK * k, unit, lraw, tg0 + SWM_TOK * k < T);
+        for (int k = 0; k < SWS_IPW; k++) swm_load(it[k], (const uint16_t *)gu, ld, F, T, tg0 + SWM_TOK * k, unit, lraw);
         __builtin_amdgcn_s_waitcnt(0x0f70);                               // vmcnt(0): this wave's part of the table has landed (and its items)
         __syncthreads();
     }
