@@ -60,7 +60,7 @@ extern "C" __attribute__((visibility("default"))) int cpp_caller_run(char * msg,
         if (!rc && !(same(dx.download<float>(), x) && same(dh.download<float>(), h) && same(dh16.download<uint16_t>(), h16) && same(dq8.download<uint8_t>(), q8)))
             rc = fail(msg, len, "add + RMSNorm + q8_1 differs from the oracle");
     }
-    if (!rc) {   // fp32 rows -> q8_1 blocks in the MMQ layout, through the persistent kernel (>= 256 columns)
+    if (!rc) {   // fp32 rows -> q8_1 blocks in the MMQ layout, through the one-shot kernel (>= 256 columns)
         const int ncols = 300; const long K = 900, Kp = 1024;
         std::vector<float> x((size_t)ncols * K);
         for (auto & v : x) v = normal(rng);

@@ -147,7 +147,8 @@ def test_kv_q8_read_round_trip(M, T, f16):
     assert (host(k2, dt)[1] == 7).all()
 
 
-@pytest.mark.parametrize('M,T,f16', [(1024, 2048, True), (1024, 2051, False), (640, 2049, True), (896, 2048, False), (672, 2050, True)])
+@pytest.mark.parametrize('M,T,f16', [(1024, 2048, True), (1024, 2051, False), (640, 2049, True), (896, 2048, False), (672, 2050, True), (1024, 4100, True), (768, 4097, False)])
 def test_kv_q8_read_wave_per_wide_row(M, T, f16):
-    """rows of 33 to 64 blocks from 2048 rows on: a wave per row where a row is whole 16-byte pieces (672 is not)"""
+    """rows of 33 to 64 blocks from 2048 rows on: a wave per row where a row is whole 16-byte pieces (672 is not); from 4096 rows on the
+    half that is read by id, a row outside the cache among it, takes that kernel too"""
     test_kv_q8_read_round_trip(M, T, f16)

@@ -105,7 +105,7 @@ def test_swiglu_mmq(T, Fh, pad, layout):
 @pytest.mark.parametrize('T,Fh', [(32, 2048), (2048, 32), (4096, 16)])
 def test_swiglu_mmq_every_bf16_gate_value(T, Fh):
     """all 65536 bf16 gate bit patterns against the oracle's bf16(silu(g)) (u = 1 keeps the second rounding exact), NaN and infinite gates
-    included (the canonical NaN), through the persistent kernel (32 tokens) and the one-shot kernel of prefill chunks, whose small table
+    included (the canonical NaN), in a small batch and in prefill chunks: the one-shot kernel, whose small table
     holds 8190 of the gates and hands the others to the full table"""
     g = np.arange(65536, dtype=np.uint16).reshape(-1, Fh)
     g = np.concatenate([g] * (T // g.shape[0]), axis=0)[np.random.default_rng(5).permutation(T)]       # (4096 x 16: every value twice)
@@ -206,7 +206,7 @@ def test_q8_blocks_whose_scale_underflows():
     y = dev(np.zeros(nblk * 36, np.uint8))
     call('camx_gg_quantize_q8_1', ptr(dev(flat)), ptr(y), L64(flat.size), I(0), F(0), NULL)
     assert bits_equal(host(y), O.q8_1(flat).reshape(-1))
-    for ncols, K in ((16, 4096), (512, 128)):                                # the row kernel and the persistent one
+    for ncols, K in ((16, 4096), (512, 128)):                                # the row kernel and the one-shot one
         xm = flat.reshape(ncols, K)
         for layout in (0, 1):
             ym = dev(np.zeros((O.k_pad(K) // 128, ncols, 144), np.uint8))
