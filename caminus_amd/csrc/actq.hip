@@ -516,9 +516,8 @@ struct SinkSiluMul {
         u32x2 dg0, du0, dg1, du1;
         u16x2 most = {0, 0};
         const uint32_t o0 = small_offset2(gw.x, most), o1 = small_offset2(gw.y, most), o2 = small_offset2(gw.z, most), o3 = small_offset2(gw.w, most);
-        f32x4 s0, s1;
-        if (__builtin_expect(most.x == SWS_LAST || most.y == SWS_LAST, 0) && __builtin_expect(small_outside8(gw), 0)) { s0 = sigmoids4((u32x2){gw.x, gw.y}); s1 = sigmoids4((u32x2){gw.z, gw.w}); }
-        else { s0 = small4(o0, o1); s1 = small4(o2, o3); }
+        f32x4 s0 = small4(o0, o1), s1 = small4(o2, o3);
+        if (__builtin_expect(most.x == SWS_LAST || most.y == SWS_LAST, 0) && small_outside8(gw)) { s0 = sigmoids4((u32x2){gw.x, gw.y}); s1 = sigmoids4((u32x2){gw.z, gw.w}); }
         grads4((u32x2){gw.x, gw.y}, (u32x2){uw.x, uw.y}, (u32x2){keep.x, keep.y}, rbf4_any(a), s0, dg0, du0);      // (a NaN's bits are settled by the stores' rounding)
         grads4((u32x2){gw.z, gw.w}, (u32x2){uw.z, uw.w}, (u32x2){keep.z, keep.w}, rbf4_any(b), s1, dg1, du1);
         uint16_t * o = dgu + (size_t)row * (2 * F) + k;
