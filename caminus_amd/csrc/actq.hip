@@ -3,10 +3,10 @@
 // actq_fwd_codes_{f32,bf16}, actq_bwd_{f32,bf16}, silu_mul_actq_{fwd,bwd} and block_entry_{fwd,bwd} (kernels/actq.hip:40-53,
 // 96-218, 247-333).
 //
-// Rows of at most 2048 values with 16-byte aligned operands, forward and backward, plain and SiLU-fused: one wave per row
-// (actq_fwd_wave_k, actq_bwd_wave_k; 26 vector instructions per value against 44 forward, 49 against 78 backward), the fused
-// forms with the gates' tables in LDS (38 and 76). The RMSNorm-fused block entry of rows of at most 1024 values: a wave per row as well,
-// four rows sharing the projections (block_entry_fwd_quad, block_entry_bwd_quad). Everything else (longer rows, unaligned operands):
+// Rows of at most 4096 values with 16-byte aligned operands, forward and backward, plain and SiLU-fused: one wave per row, two above 2048
+// (actq_fwd_wave_k, actq_bwd_wave_k), the fused forms with the gates' tables in LDS. The RMSNorm-fused block entry of rows of at most
+// 1024 values: a wave per row as well, four rows sharing the projections (block_entry_fwd_quad, block_entry_bwd_quad). Everything else
+// (longer rows, unaligned operands):
 // One 256-thread workgroup per row. A half-wave (32 lanes) transforms one 128-chunk: lane l holds elements 4l .. 4l + 3,
 // butterfly stages 1-2 in registers, 4 .. 64 across lanes; half-wave h takes chunks h, h + 8, ... (the reference's wave h of
 // 32), NR = ceil(K / 1024) rounds of them stay in registers across the row-wide reductions. Kernels are instantiated per
@@ -45,7 +45,10 @@ struct PlainF32 {
     CAMX_DEV f32x4 operator()(int row, int k) const { return *(const f32x4 *)(x + (size_t)row * K + k); }
     CAMX_DEV f32x4 operator()(int row, int k, u32x2 &) const { return (*this)(row, k); }
     CAMX_DEV void fetch(int row, int k, u32x4 (&w)[NW]) const { const u32x4 * p = (const u32x4 *)(x + (size_t)row * K + k); w[0] = p[0]; w[1] = p[1]; }
-    CAMX_DEV void value8(const u32x4 (&w)[NW], f32x4 & a, f32x4 & b, u32x4 &) const { a = __builtin_bit_cast(f32x4, w[0]); b = __builtin_bit_cast(f32x4, w[1]); }
+    CAMX_DEV u32x4 packed8(const u32x4 (&w)[NW], u32x4 &) const {                   // autocast's bf16 input
+        const f32x4 a = __builtin_bit_cast(f32x4, w[0]), b = __builtin_bit_cast(f32x4, w[1]);
+        return (u32x4){hw_pk_bf16(a.x, a.y), hw_pk_bf16(a.z, a.w), hw_pk_bf16(b.x, b.y), hw_pk_bf16(b.z, b.w)};
+    }
 };
 struct PlainBF16 {
     static constexpr bool bf16_valued = true, lds_tables = false; static constexpr int NW = 1;
@@ -55,7 +58,7 @@ struct PlainBF16 {
     CAMX_DEV f32x4 operator()(int row, int k) const { return unpack_bf16x4(*(const u32x2 *)(x + (size_t)row * K + k)); }
     CAMX_DEV f32x4 operator()(int row, int k, u32x2 &) const { return (*this)(row, k); }
     CAMX_DEV void fetch(int row, int k, u32x4 (&w)[NW]) const { w[0] = *(const u32x4 *)(x + (size_t)row * K + k); }
-    CAMX_DEV void value8(const u32x4 (&w)[NW], f32x4 & a, f32x4 & b, u32x4 &) const { unpack_bf16x8(w[0], a, b); }
+    CAMX_DEV u32x4 packed8(const u32x4 (&w)[NW], u32x4 &) const { return w[0]; }
 };
 // the bf16 words {t[g0], t[g1]} and {t[g2], t[g3]} of four packed bf16 gates from the full table in device memory
 CAMX_DEV u32x2 silu_lookup4(u32x2 gw, const uint16_t * lut) {
@@ -106,7 +109,7 @@ struct SiluMulSrc {
     static CAMX_DEV u32x4 absent(int w) { return w ? (u32x4){0u, 0u, 0u, 0u} : (u32x4){0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u}; }      // gates of 1, multipliers of 0: +0 without a zero gate's check
     static constexpr int NW = 2;                   // the wave-per-row form: eight gates, eight multipliers
     CAMX_DEV void fetch(int row, int k, u32x4 (&w)[NW]) const { const uint16_t * r = gu + (size_t)row * ld + k; w[0] = *(const u32x4 *)r; w[1] = *(const u32x4 *)(r + F); }
-    CAMX_DEV void value8(const u32x4 (&w)[NW], f32x4 & a, f32x4 & b, u32x4 & keep) const {
+    CAMX_DEV u32x4 packed8(const u32x4 (&w)[NW], u32x4 & keep) const {              // (feeds the rotation: of a NaN only its NaN-ness survives)
         u16x2 most = {0, 0};
         const uint32_t o0 = small_offset2(w[0].x, most), o1 = small_offset2(w[0].y, most), o2 = small_offset2(w[0].z, most), o3 = small_offset2(w[0].w, most);
         if (__builtin_expect(most.x == SWS_LAST || most.y == SWS_LAST, 0) && __builtin_expect(small_outside8(w[0]), 0)) {
@@ -115,8 +118,7 @@ struct SiluMulSrc {
         } else keep = (u32x4){small_pair(small, o0), small_pair(small, o1), small_pair(small, o2), small_pair(small, o3)};
         f32x4 sa, sb, ua, ub;
         unpack_bf16x8(keep, sa, sb); unpack_bf16x8(w[1], ua, ub);
-        a = rbf4_any((f32x4){sa.x * ua.x, sa.y * ua.y, sa.z * ua.z, sa.w * ua.w});
-        b = rbf4_any((f32x4){sb.x * ub.x, sb.y * ub.y, sb.z * ub.z, sb.w * ub.w});
+        return (u32x4){hw_pk_bf16(sa.x * ua.x, sa.y * ua.y), hw_pk_bf16(sa.z * ua.z, sa.w * ua.w), hw_pk_bf16(sb.x * ub.x, sb.y * ub.y), hw_pk_bf16(sb.z * ub.z, sb.w * ub.w)};
     }
 };
 struct RmsSrc {
@@ -247,106 +249,156 @@ __global__ void __launch_bounds__(256) actq_fwd_k(Src src, uint16_t * y, float *
     actq_fwd_row<NR>(src, blockIdx.x, y, s, K, clip, qmax, codes, lds);
 }
 
-// ---- rows of at most 2048 values: one wave per row, no LDS, no barrier ------------------------------------------------------
-// Lane (c = lane >> 2, q = lane & 3) holds 32 values of chunk c: element 32 j + 8 q + k of the chunk is u[j][k]. Butterfly
-// stages 1, 2, 4 pair registers k, stages 8 and 16 pair lanes q ^ 1 and q ^ 2, stages 32 and 64 pair registers j: the same
-// pairs in the same order as above, five of the seven stages without a lane exchange.
+// ---- rows of at most 4096 values: one wave per row, two above 2048 ----------------------------------------------------------
+// Lane (g = lane >> 4, slot s of its 16) holds elements 8 s .. 8 s + 7 of one chunk per round: round j of part p of W is chunk
+// 4 W j + 4 p + g, so a wave's round is 512 consecutive values and all chunks of one residue mod 8, whose dL/ds terms the backward adds
+// in chunk order, sit in one lane. Butterfly stages 1, 2, 4 pair registers, 8 .. 64 pair slots s ^ 1, 2, 4, 8: the same pairs in the same
+// order as above. What a value costs is counted in issue cycles, measured on the card: an add, subtract, multiply, bit operation or
+// multiply-add that reads at most two vector registers takes 2.3 per wave and SIMD, everything else (shifts, converts, maxima,
+// compares, row moves, an operand in a scalar register) 4.2. Hence rounds of eight values that live as packed bf16 words between the
+// passes, maxima of packed words, and checks that a row settles once. bf16 rows, forward / backward, against four lanes a chunk with 32
+// values each (up to 2048) and a workgroup per row: 32768 x 512 35.6 -> 20.1 / 65.4 -> 27.2 us, 32768 x 1024 38.6 -> 29.4 / 69.4 -> 44.0,
+// 16384 x 2048 27.6 -> 26.5 / 44.5 -> 37.0 (floor 20.6 / 31.0: bytes at 6.5 TB/s), 8192 x 4096 30.9 -> 25.5 / 50.8 -> 38.6; at 32768 x 2048
+// the forward is bound by its bytes either way (49 us for 268 MB).
 CAMX_DEV void bfly(float & a, float & b) { const float s = a + b, d = a - b; a = s; b = d; }
-
-template <int CTRL>
-CAMX_DEV void lane_stage_w(float (&u)[4][8], uint32_t sign) {      // (own + partner) in the lower lane, (partner - own) in the upper one
+CAMX_DEV float bf_lo(uint32_t v) { return __builtin_bit_cast(float, v << 16); }
+CAMX_DEV float bf_hi(uint32_t v) { return __builtin_bit_cast(float, v & 0xffff0000u); }
+CAMX_DEV void unpack8(u32x4 w, float (&v)[8]) {
 #pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            const float own = u[j][k];
-            const float p = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, own), CTRL, 0xf, 0xf, true));
-            u[j][k] = p + __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, own) ^ sign);
-        }
+    for (int i = 0; i < 4; i++) { const uint32_t p = w[i]; v[2 * i] = bf_lo(p); v[2 * i + 1] = bf_hi(p); }
 }
-// The rotation of the wave-per-row kernels, one instruction per value and cross-lane stage.
+// the same words, unknown to the compiler: it would hold their unpacked values from one pass to the next (two registers for one)
+CAMX_DEV u32x4 unknown_words(u32x4 w) {
+    uint32_t a = w.x, b = w.y, c = w.z, d = w.w;
+    asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
+    return (u32x4){a, b, c, d};
+}
+// eight values to packed bf16 by the hardware convert: a NaN stays one (see rbf4_any)
+CAMX_DEV u32x4 pack8_any(const float (&v)[8]) { return (u32x4){hw_pk_bf16(v[0], v[1]), hw_pk_bf16(v[2], v[3]), hw_pk_bf16(v[4], v[5]), hw_pk_bf16(v[6], v[7])}; }
+// A batch of 2^20 values or more streams: its bf16 outputs leave past the caches as whole lines (the wave's round is 1 KiB without a gap:
+// 16384 x 2048 forward 31.4 -> 26.3 us, backward 40.1 -> 36.3 with g read past them too). fp32 gradients stay plain: a lane's eight values
+// are two half lines, which only the cache puts together (61 -> 85 us).
+CAMX_DEV void store16(u32x4 v, void * p, bool stream) {
+    if (stream) {                                        // (between two empty asm statements: the compiler makes one plain store of the two otherwise)
+        asm volatile("" ::: "memory");
+        __builtin_nontemporal_store(v, (u32x4 *)p);
+        asm volatile("" ::: "memory");
+    }
+    else *(u32x4 *)p = v;
+}
+CAMX_DEV u32x4 pack8_canon(const float (&v)[8]) {                     // f2bf of eight values (NaN -> 0x7fc0)
+    const u32x2 a = pack_f2bf_x4((f32x4){v[0], v[1], v[2], v[3]}), b = pack_f2bf_x4((f32x4){v[4], v[5], v[6], v[7]});
+    return (u32x4){a.x, a.y, b.x, b.y};
+}
 // A cross-lane stage gives own + partner in the lower lane and partner - own in the upper one: a sign flip and an add per value. Here the
 // upper lane keeps own - partner, the negative of its value: one multiply-add by +1 or -1 whose first operand comes from the partner
-// (v_fmac_f32 with a row move; the compiler does not fold the move into a multiply-add, and the s_nop gives the move the two wait
+// (v_fmac_f32 with a row move; the compiler does not fold the move into a multiply-add, and the s_nop gives the first move the two wait
 // states it needs behind the instructions before). Negation commutes with every later sum and difference and its rounding, so after
-// all stages a lane's values carry the sign of its index's parity, which the factor HSCALE takes along. Only a zero's sign is lost:
+// all stages a lane's values carry the sign of its slot's parity, which the factor HSCALE takes along. Only a zero's sign is lost:
 // sums that cancel are +0 in either form, so the last multiply adds +0; a sum is -0 only if the chunk's first element is -0 and its
-// second a zero, and a wave that holds such a chunk runs the plain form. (32768 x 2048, forward + backward: 136.2 -> 131.7 us. The
-// four-values-per-lane form of the other kernels gains nothing by it.)
-#define CAMX_FMAC4(CTRL, a, b, c, d, sg)                                                                                  \
-    asm("s_nop 1\n\tv_fmac_f32_dpp %0, %0, %4 " CTRL " row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %1, %1, %4 " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
-        "v_fmac_f32_dpp %2, %2, %4 " CTRL " row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %3, %3, %4 " CTRL " row_mask:0xf bank_mask:0xf"               \
-        : "+v"(a), "+v"(b), "+v"(c), "+v"(d) : "v"(sg))
-CAMX_DEV bool first_is_negative_zero(float x0, float x1) { return __builtin_bit_cast(uint32_t, x0) == 0x80000000u && x1 == 0.0f; }
-CAMX_DEV float parity_scale(int l) { return (__builtin_popcount(l) & 1) ? -HSCALE : HSCALE; }
-// u = HSCALE . H128 u
-CAMX_DEV void rotate128_w32(float (&u)[4][8], int q) {
-    const bool plain = __builtin_amdgcn_ballot_w64(q == 0 && first_is_negative_zero(u[0][0], u[0][1])) != 0;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-#pragma unroll
-        for (int k = 0; k < 8; k += 2) bfly(u[j][k], u[j][k + 1]);
-#pragma unroll
-        for (int k = 0; k < 8; k += 4) { bfly(u[j][k], u[j][k + 2]); bfly(u[j][k + 1], u[j][k + 3]); }
-#pragma unroll
-        for (int k = 0; k < 4; k++) bfly(u[j][k], u[j][k + 4]);
+// second a zero, and a wave that holds such a chunk runs the plain form.
+struct Lanes16 {
+    float s1, s2, s4, s8, h;                             // a stage's factor of the partner, HSCALE with the parity's sign
+    bool first;                                          // the lane holds its chunk's first elements
+    CAMX_DEV explicit Lanes16(int s) {
+        s1 = s & 1 ? -1.0f : 1.0f; s2 = s & 2 ? -1.0f : 1.0f; s4 = s & 4 ? -1.0f : 1.0f; s8 = s & 8 ? -1.0f : 1.0f;
+        h = (__builtin_popcount(s) & 1) ? -HSCALE : HSCALE;
+        first = s == 0;
     }
-    float h = HSCALE;
-    if (plain) {
-        lane_stage_w<0xB1>(u, (q & 1) ? 0x80000000u : 0u);
-        lane_stage_w<0x4E>(u, (q & 2) ? 0x80000000u : 0u);
-    } else {
-        const float s1 = q & 1 ? -1.0f : 1.0f, s2 = q & 2 ? -1.0f : 1.0f;
-        h = parity_scale(q);
+    CAMX_DEV bool plain(uint32_t w0) const { return first && (w0 & 0x7fffffffu) == 0x00008000u; }          // elements 0 and 1: -0 and a zero
+};
+template <int CTRL>
+CAMX_DEV void lane_stage8(float (&u)[8], float sg) {      // (own + partner) in the lower lane, (partner - own) in the upper one
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-            for (int k = 0; k < 8; k += 4) CAMX_FMAC4("quad_perm:[1,0,3,2]", u[j][k], u[j][k + 1], u[j][k + 2], u[j][k + 3], s1);
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-            for (int k = 0; k < 8; k += 4) CAMX_FMAC4("quad_perm:[2,3,0,1]", u[j][k], u[j][k + 1], u[j][k + 2], u[j][k + 3], s2);
+    for (int k = 0; k < 8; k++) {
+        const float own = u[k];
+        const float p = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, own), CTRL, 0xf, 0xf, true));
+        u[k] = p + __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, own) ^ (__builtin_bit_cast(uint32_t, sg) & 0x80000000u));
     }
-#pragma unroll
-    for (int k = 0; k < 8; k++) { bfly(u[0][k], u[1][k]); bfly(u[2][k], u[3][k]); }
-#pragma unroll
-    for (int k = 0; k < 8; k++) { bfly(u[0][k], u[2][k]); bfly(u[1][k], u[3][k]); }
-    const float z = plain ? -0.0f : 0.0f;                              // (x + -0 is x)
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int k = 0; k < 8; k++) u[j][k] = __builtin_fmaf(u[j][k], h, z);
 }
-// u = bf16(H128 . bf16(source)) of the lane's 32 values from the fetched words; gmax[j]: the lane's max |u| in group j; returns the row's
-template <typename Src>
-CAMX_DEV float actq_rotate_w(const Src & src, const u32x4 (&raw)[4][Src::NW], int q, float (&u)[4][8], u32x4 (&keep)[4], float (&gmax)[4]) {
+#define CAMX_FMAC8(CTRL, SG) \
+    "v_fmac_f32_dpp %0, %0, " SG " " CTRL " row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %1, %1, " SG " " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %2, %2, " SG " " CTRL " row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %3, %3, " SG " " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %4, %4, " SG " " CTRL " row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %5, %5, " SG " " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %6, %6, " SG " " CTRL " row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %7, %7, " SG " " CTRL " row_mask:0xf bank_mask:0xf\n\t"
+// v = HSCALE . H128 of the chunk's packed bf16 values; plain: wave-uniform
+CAMX_DEV void rotate128_w16(u32x4 w, float (&v)[8], const Lanes16 & ln, bool plain) {
+    unpack8(w, v);
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        f32x4 a, b;
-        src.value8(raw[j], a, b, keep[j]);
-        if (!Src::bf16_valued) { a = rbf4_any(a); b = rbf4_any(b); }              // autocast's bf16 input
-        u[j][0] = a.x; u[j][1] = a.y; u[j][2] = a.z; u[j][3] = a.w; u[j][4] = b.x; u[j][5] = b.y; u[j][6] = b.z; u[j][7] = b.w;
+    for (int k = 0; k < 8; k += 2) bfly(v[k], v[k + 1]);
+#pragma unroll
+    for (int k = 0; k < 8; k += 4) { bfly(v[k], v[k + 2]); bfly(v[k + 1], v[k + 3]); }
+#pragma unroll
+    for (int k = 0; k < 4; k++) bfly(v[k], v[k + 4]);
+    if (__builtin_expect(plain, 0)) {
+        lane_stage8<0xB1>(v, ln.s1); lane_stage8<0x4E>(v, ln.s2); lane_stage8<0x141>(v, ln.s4); lane_stage8<0x128>(v, ln.s8);
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] *= HSCALE;
+    } else {
+        asm("s_nop 1\n\t" CAMX_FMAC8("quad_perm:[1,0,3,2]", "%8") CAMX_FMAC8("quad_perm:[2,3,0,1]", "%9") CAMX_FMAC8("row_half_mirror", "%10") CAMX_FMAC8("row_ror:8", "%11")
+            : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]) : "v"(ln.s1), "v"(ln.s2), "v"(ln.s4), "v"(ln.s8));
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] = __builtin_fmaf(v[k], ln.h, 0.0f);
     }
-    rotate128_w32(u, q);
+}
+// the larger magnitude of two packed bf16 pairs, per half (a NaN's is the largest of all)
+CAMX_DEV u16x2 absmax_pk(u16x2 m, uint32_t w) { return __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, w & 0x7fff7fffu)); }
+CAMX_DEV u16x2 absmax_pk8(u32x4 w) { return absmax_pk(absmax_pk(absmax_pk(__builtin_bit_cast(u16x2, w.x & 0x7fff7fffu), w.y), w.z), w.w); }
+CAMX_DEV float absmax_of(u16x2 m) { const uint32_t a = m.x, b = m.y; return __builtin_bit_cast(float, (a > b ? a : b) << 16); }
+// max |u| of a row's packed words without its NaNs, and whether it holds one (wave-uniform)
+template <int R>
+CAMX_DEV float row_absmax_w(const u32x4 (&uw)[R], u16x2 most, bool & nan) {
+    float m = absmax_of(most);
+    nan = __builtin_amdgcn_ballot_w64(m != m) != 0;
+    if (__builtin_expect(nan, 0)) {
+        m = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        gmax[j] = 0.0f;                                                            // (an absent chunk holds zeros)
+        for (int j = 0; j < R; j++) {
+            float v[8];
+            unpack8(unknown_words(uw[j]), v);
 #pragma unroll
-        for (int k = 0; k < 8; k += 4) {
-            const f32x4 v = rbf4_any((f32x4){u[j][k], u[j][k + 1], u[j][k + 2], u[j][k + 3]});
-            u[j][k] = v.x; u[j][k + 1] = v.y; u[j][k + 2] = v.z; u[j][k + 3] = v.w;
-            gmax[j] = fmaxf(fmaxf(gmax[j], fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+            for (int k = 0; k < 8; k++) m = fmaxf(m, fabsf(v[k]));
         }
     }
-    return wave_max64(fmaxf(fmaxf(gmax[0], gmax[1]), fmaxf(gmax[2], gmax[3])));
+    return wave_max64(m);
 }
-template <typename Src>
-CAMX_DEV void fetch_row_w(const Src & src, int row, int c, int q, bool on, u32x4 (&raw)[4][Src::NW]) {
+// the same over the two waves of a row, whose signs carry the NaNs; xch: four floats
+template <int W>
+CAMX_DEV float share_absmax(float amax, bool & nan, float * xch, int wave) {
+    if (W == 1) return amax;
+    if ((threadIdx.x & 63) == 0) xch[wave] = nan ? -amax : amax;         // (-0 for a row of NaNs)
+    __syncthreads();
+    const float a = xch[wave & ~1], b = xch[wave | 1];
+    nan = __builtin_signbit(a) || __builtin_signbit(b);
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, fmaxf(fabsf(a), fabsf(b)))));
+}
+// u = bf16(H128 . bf16(source)) of the lane's rounds as packed words, from the fetched words; returns the lane's largest magnitudes
+template <int R, typename Src>
+CAMX_DEV u16x2 actq_rotate_w(const Src & src, const u32x4 (&raw)[R][Src::NW], const Lanes16 & ln, u32x4 (&uw)[R], u32x4 (&keep)[R]) {
+    u16x2 most = {0, 0};
+    bool zero = false;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < R; j++) { uw[j] = src.packed8(raw[j], keep[j]); zero |= ln.plain(uw[j].x); }
+    const bool plain = __builtin_amdgcn_ballot_w64(zero) != 0;
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        float v[8];
+        rotate128_w16(uw[j], v, ln, plain);
+        uw[j] = pack8_any(v);
+        uw[j] = unknown_words(uw[j]);
+        const u16x2 m = absmax_pk8(uw[j]);               // (an absent chunk holds zeros)
+        most = __builtin_elementwise_max(most, m);
+        __builtin_amdgcn_sched_barrier(0);               // (round by round: side by side they cost a wave per SIMD in registers)
+    }
+    return most;
+}
+template <int R, int W, typename Src>
+CAMX_DEV void fetch_row_w(const Src & src, int row, int e0, bool last_on, u32x4 (&raw)[R][Src::NW]) {
+#pragma unroll
+    for (int j = 0; j < R; j++) {
 #pragma unroll
         for (int w = 0; w < Src::NW; w++) raw[j][w] = Src::absent(w);
-        if (on) src.fetch(row, c * 128 + 32 * j + 8 * q, raw[j]);
+        if (j < R - 1 || last_on) src.fetch(row, e0 + 512 * W * j, raw[j]);
     }
 }
 
@@ -357,42 +409,68 @@ CAMX_DEV void lds_table_copy(const void * src, void * dst, int bytes) {         
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)((const uint8_t *)src + 1024 * j + 16 * lane),
                                          (__attribute__((address_space(3))) void *)((uint8_t *)dst + 1024 * j), 16, 0, 0);
 }
-// One row per wave, four rows per workgroup. The kernel's time at 8192 rows is its arithmetic plus the launch's ramp, the first
-// loads and the last stores, whatever the number of waves in flight (3 to 8 per SIMD measured alike); a wave that walks several
+// Whether rintf(u * rcp) is the row's quantizer for every value: no NaN, the largest quotient below 16 and not rounding above qmax (so
+// nothing is clamped), and no bf16 value whose quotient lies within 2e-5 of a half-integer (see RowScale: 1e-5 would do). The bf16
+// values next to the half-integers' products with s are few enough to be looked at once per row, a half-integer per lane (1 to 2 % of
+// rows hold one), in place of a subtraction and a maximum per value.
+CAMX_DEV bool row_is_tame(const RowScale & rs, float amax, bool nan) {
+    const float p = amax * rs.rcp;
+    if (nan || !(p < 16.0f && p < rs.hi + 0.499f && rs.s < 0x1p100f)) return false;            // (uniform; an infinite amax gives a NaN)
+    const int lane = threadIdx.x & 63;
+    const float hs = ((float)lane + 0.5f) * rs.s, near = bf_lo(hw_pk_bf16(hs, 0.0f));
+    return __builtin_amdgcn_ballot_w64((float)lane < rs.hi && fabsf(near - hs) < 2e-5f * rs.s) == 0;
+}
+// The kernel's time at 8192 rows and more is the larger of its arithmetic and its bytes, plus the launch's ramp; a wave that walks several
 // rows with the next row's loads in flight measured 5 to 15 % slower.
-template <typename Src>
+template <typename Src, int R, int W>
 __global__ void __launch_bounds__(256) actq_fwd_wave_k(Src src, uint16_t * __restrict__ y, float * __restrict__ s_out, uint16_t * __restrict__ codes,
-                                                       int K, float clip, int qmax, int M, const uint16_t * small_g = nullptr) {
-    const int lane = threadIdx.x & 63, nch = K / 128, c = lane >> 2, q = lane & 3;
-    const bool on = c < nch;
-    const int row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (!Src::lds_tables && row >= M) return;
-    u32x4 raw[4][Src::NW];
-    fetch_row_w(src, min(row, M - 1), c, q, on, raw);
-    if (Src::lds_tables) {                               // the gates' table, shared by the workgroup's four rows
+                                                       int K, float clip, int qmax, int M, bool stream, const uint16_t * small_g = nullptr) {
+    const int lane = threadIdx.x & 63, slot = slot_of(lane) & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), part = wave % W;
+    const int c0 = 4 * part + (lane >> 4), e0 = 128 * c0 + 8 * slot;     // round j: + 512 W j
+    const bool last_on = c0 + 4 * W * (R - 1) < K / 128;
+    const int row = blockIdx.x * (4 / W) + wave / W;
+    if (!Src::lds_tables && W == 1 && row >= M) return;
+    u32x4 raw[R][Src::NW];
+    fetch_row_w<R, W>(src, min(row, M - 1), e0, last_on, raw);
+    if (Src::lds_tables) {                               // the gates' table, shared by the workgroup's rows
         __shared__ __attribute__((aligned(16))) uint16_t small[SWS_TAB];
         lds_table_copy(small_g, small, 2 * SWS_TAB);
         __builtin_amdgcn_s_waitcnt(0x0f70);              // vmcnt(0): this wave's part of the table (and its row)
         __syncthreads();
         src.set_small(small);
-        if (row >= M) return;
+        if (W == 1 && row >= M) return;
     }
-    float u[4][8], gmax[4];
-    u32x4 keep[4];                                       // (only the backward uses it)
-    const float amax = actq_rotate_w(src, raw, q, u, keep, gmax);
+    __shared__ float xch[4];
+    const Lanes16 ln(slot);
+    u32x4 uw[R], keep[R];                                // (keep: only the backward uses it)
+    const u16x2 most = actq_rotate_w<R>(src, raw, ln, uw, keep);
+    bool nan;
+    float amax = row_absmax_w<R>(uw, most, nan);
+    amax = share_absmax<W>(amax, nan, xch, wave);
+    if (W > 1 && row >= M) return;
     const float s = fmaxf(amax * clip / (float)qmax, 1e-8f);
     const RowScale rs(s, amax, qmax);
-    if (lane == 0 && s_out) s_out[row] = s;
-    if (!on) return;
+    if (lane == 0 && part == 0 && s_out) s_out[row] = s;
+    const bool tame = row_is_tame(rs, amax, nan);
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const f32x4 qa = rs.quant4((f32x4){u[j][0], u[j][1], u[j][2], u[j][3]}), qb = rs.quant4((f32x4){u[j][4], u[j][5], u[j][6], u[j][7]});
-        const size_t e0 = (size_t)row * K + c * 128 + 32 * j + 8 * q;
-        if (y) {
-            const u32x2 pa = pack_f2bf_x4((f32x4){qa.x * s, qa.y * s, qa.z * s, qa.w * s}), pb = pack_f2bf_x4((f32x4){qb.x * s, qb.y * s, qb.z * s, qb.w * s});
-            *(u32x4 *)(y + e0) = (u32x4){pa.x, pa.y, pb.x, pb.y};
+    for (int j = 0; j < R; j++) {
+        if (j == R - 1 && !last_on) break;
+        float q[8];
+        unpack8(uw[j], q);
+        if (__builtin_expect(tame, 1)) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) q[k] = rintf(q[k] * rs.rcp);
+        } else {
+            const f32x4 a = rs.quant4((f32x4){q[0], q[1], q[2], q[3]}), b = rs.quant4((f32x4){q[4], q[5], q[6], q[7]});
+            q[0] = a.x; q[1] = a.y; q[2] = a.z; q[3] = a.w; q[4] = b.x; q[5] = b.y; q[6] = b.z; q[7] = b.w;
         }
-        if (codes) *(uint32_t *)(codes + (e0 >> 2)) = rs.nibbles4(qa) | (rs.nibbles4(qb) << 16);
+        const size_t e = (size_t)row * K + e0 + 512 * W * j;
+        if (codes) *(uint32_t *)(codes + (e >> 2)) = rs.nibbles4((f32x4){q[0], q[1], q[2], q[3]}) | (rs.nibbles4((f32x4){q[4], q[5], q[6], q[7]}) << 16);
+        if (y) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) q[k] *= s;
+            store16(__builtin_expect(tame, 1) ? pack8_any(q) : pack8_canon(q), y + e, stream);   // (a tame row's products are numbers)
+        }
     }
 }
 
@@ -429,6 +507,25 @@ struct RowDiv {
         if (needed && !(row_ok && least >= 0x1p-60f)) { t.x = u.x / s; t.y = u.y / s; t.z = u.z / s; t.w = u.w / s; }
         return t;
     }
+    // the same of eight values, but for the sign of a zero quotient, which u = 0 does not ask to be divided for
+    CAMX_DEV void div8(const float (&u)[8], float (&t)[8], bool needed) const {
+        float least = 0x1p60f;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const float t0 = u[k] * r1;
+            t[k] = __builtin_fmaf(__builtin_fmaf(-s, t0, u[k]), r1, t0);
+            least = fminf(least, fabsf(t0));
+        }
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(needed && !(row_ok && least >= 0x1p-60f)) != 0, 0)) {
+            bool divide = !row_ok;
+#pragma unroll
+            for (int k = 0; k < 8; k++) divide |= u[k] != 0.0f && fabsf(u[k] * r1) < 0x1p-60f;
+            if (__builtin_amdgcn_ballot_w64(needed && divide) != 0) {
+#pragma unroll
+                for (int k = 0; k < 8; k++) { const float d = u[k] / s; t[k] = divide ? d : t[k]; }
+            }
+        }
+    }
 };
 // The straight-through step of one value: r = rintf(t), q its clamp to [lo, hi], m: r lies strictly inside. Gives the factor of g in
 // dL/ds, m ? q - t : q, and m as 1 or 0.
@@ -447,16 +544,16 @@ struct Ste {
 struct SinkF32 {
     float * dx; int K;
     CAMX_DEV void operator()(int row, int k, f32x4 v, u32x2) const { *(f32x4 *)(dx + (size_t)row * K + k) = v; }
-    CAMX_DEV void st8(int row, int k, f32x4 a, f32x4 b, u32x4) const { f32x4 * p = (f32x4 *)(dx + (size_t)row * K + k); p[0] = rbf4_canon(a); p[1] = rbf4_canon(b); }
+    CAMX_DEV void st8(int row, int k, const float (&v)[8], u32x4, bool) const {
+        f32x4 * p = (f32x4 *)(dx + (size_t)row * K + k);
+        p[0] = rbf4_canon((f32x4){v[0], v[1], v[2], v[3]}); p[1] = rbf4_canon((f32x4){v[4], v[5], v[6], v[7]});
+    }
     CAMX_DEV void set_small(const float *) {}
 };
 struct SinkBF16 {
     uint16_t * dx; int K;
     CAMX_DEV void operator()(int row, int k, f32x4 v, u32x2) const { *(u32x2 *)(dx + (size_t)row * K + k) = pack_f2bf_x4(v); }
-    CAMX_DEV void st8(int row, int k, f32x4 a, f32x4 b, u32x4) const {
-        const u32x2 pa = pack_f2bf_x4(a), pb = pack_f2bf_x4(b);
-        *(u32x4 *)(dx + (size_t)row * K + k) = (u32x4){pa.x, pa.y, pb.x, pb.y};
-    }
+    CAMX_DEV void st8(int row, int k, const float (&v)[8], u32x4, bool stream) const { store16(pack8_canon(v), dx + (size_t)row * K + k, stream); }
     CAMX_DEV void set_small(const float *) {}
 };
 struct SinkLds { float * buf; CAMX_DEV void operator()(int, int k, f32x4 v, u32x2) const { *(f32x4 *)(buf + k) = v; } };
@@ -510,7 +607,8 @@ struct SinkSiluMul {
     }
     // (the gates and multipliers are read a second time here: held in registers since the source fetched them they cost 48 more,
     // two waves per SIMD instead of three, and 8192 x 2048 takes 65 us instead of 62)
-    CAMX_DEV void st8(int row, int k, f32x4 a, f32x4 b, u32x4 keep) const {
+    CAMX_DEV void st8(int row, int k, const float (&v)[8], u32x4 keep, bool stream) const {
+        const f32x4 a = {v[0], v[1], v[2], v[3]}, b = {v[4], v[5], v[6], v[7]};
         const uint16_t * r = gu + (size_t)row * ld + k;
         const u32x4 gw = *(const u32x4 *)r, uw = *(const u32x4 *)(r + F);
         u32x2 dg0, du0, dg1, du1;
@@ -521,8 +619,8 @@ struct SinkSiluMul {
         grads4((u32x2){gw.x, gw.y}, (u32x2){uw.x, uw.y}, (u32x2){keep.x, keep.y}, rbf4_any(a), s0, dg0, du0);      // (a NaN's bits are settled by the stores' rounding)
         grads4((u32x2){gw.z, gw.w}, (u32x2){uw.z, uw.w}, (u32x2){keep.z, keep.w}, rbf4_any(b), s1, dg1, du1);
         uint16_t * o = dgu + (size_t)row * (2 * F) + k;
-        *(u32x4 *)o = (u32x4){dg0.x, dg0.y, dg1.x, dg1.y};
-        *(u32x4 *)(o + F) = (u32x4){du0.x, du0.y, du1.x, du1.y};
+        store16((u32x4){dg0.x, dg0.y, dg1.x, dg1.y}, o, stream);
+        store16((u32x4){du0.x, du0.y, du1.x, du1.y}, o + F, stream);
     }
 };
 
@@ -613,31 +711,30 @@ __global__ void __launch_bounds__(256) actq_bwd_k(Src src, const uint16_t * g, S
     actq_bwd_row<NR>(src, blockIdx.x, g, sink, K, clip, qmax, lds);
 }
 
-// ---- backward of rows of at most 2048 values: one wave per row, in the layout of actq_fwd_wave_k ------------------------------------
+// ---- backward of rows of at most 4096 values: a wave or two per row, in the layout of actq_fwd_wave_k --------------------------------
 // The sum of dL/ds keeps the tree of the workgroup form. There, the lane of half-wave h with index l adds the terms of elements
-// 4 l .. 4 l + 3 of chunk h, then of chunk h + 8, in order; here those eight terms sit in two lanes (c = h and c = h + 8, 32 lanes
-// apart) as registers 4 kk .. 4 kk + 3 of group j, with l = 8 j + 2 q + kk. Every lane runs the four-term chain from zero, the upper
-// 32 lanes fetch the lower lanes' results and run theirs again from there. The 32 sums of a half-wave then combine by
-// l ^ 16, 8 (registers j), 4, 2 (lanes q), 1 (registers kk), and the eight half-wave sums, held by lanes 32 + 4 h, are added in order.
-CAMX_DEV float from_other_half(float v, int lane) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (lane ^ 32), __builtin_bit_cast(int, v)));
-}
-template <typename Src, typename Sink>
-__global__ void __launch_bounds__(256) actq_bwd_wave_k(Src src, const uint16_t * __restrict__ g, Sink sink, int K, float clip, int qmax, int M,
+// 4 l .. 4 l + 3 of chunks h, h + 8, .. in order; here those sit in one lane (slot l >> 1) as registers 4 (l & 1) .. + 3 of its rounds: of every
+// second round in a row of one wave, whose other rounds are chunks h + 4, of every round in a row of two. The 32 sums of a half-wave
+// then combine by l ^ 16, 8, 4, 2 (slots) and 1 (registers), and the eight half-wave sums are added in order.
+// Eight values at a time, as packed words between the passes: a group in which no lane's quotient can round to qmax (or below -qmax) and no
+// lane holds the row's maximum needs no clamp, no mask and no look for ties, and its part of the gradient is g itself.
+template <typename Src, typename Sink, int R, int W>
+__global__ void __launch_bounds__(256) actq_bwd_wave_k(Src src, const uint16_t * __restrict__ g, Sink sink, int K, float clip, int qmax, int M, bool stream,
                                                        const uint16_t * small_g = nullptr, const float * dsmall_g = nullptr) {
-    const int lane = threadIdx.x & 63, nch = K / 128, c = lane >> 2, q = lane & 3;
-    const bool on = c < nch, upper = lane >= 32;
-    const int row_raw = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (!Src::lds_tables && row_raw >= M) return;
+    const int lane = threadIdx.x & 63, slot = slot_of(lane) & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), part = wave % W;
+    const int c0 = 4 * part + (lane >> 4), e0 = 128 * c0 + 8 * slot;     // round j: + 512 W j
+    const bool last_on = c0 + 4 * W * (R - 1) < K / 128;
+    const int row_raw = blockIdx.x * (4 / W) + wave / W;
+    if (!Src::lds_tables && W == 1 && row_raw >= M) return;
     const int row = min(row_raw, M - 1);
-    u32x4 raw[4][Src::NW], graw[4];
-    fetch_row_w(src, row, c, q, on, raw);
+    u32x4 raw[R][Src::NW], gw[R];
+    fetch_row_w<R, W>(src, row, e0, last_on, raw);
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        graw[j] = (u32x4){0u, 0u, 0u, 0u};
-        if (on) graw[j] = *(const u32x4 *)(g + (size_t)row * K + c * 128 + 32 * j + 8 * q);
+    for (int j = 0; j < R; j++) {
+        gw[j] = (u32x4){0u, 0u, 0u, 0u};
+        if (j < R - 1 || last_on) gw[j] = __builtin_nontemporal_load((const u32x4 *)(g + (size_t)row * K + e0 + 512 * W * j));
     }
-    if (Src::lds_tables) {                               // the gates' tables, shared by the workgroup's four rows
+    if (Src::lds_tables) {                               // the gates' tables, shared by the workgroup's rows
         __shared__ __attribute__((aligned(16))) uint16_t small[SWS_TAB];
         __shared__ __attribute__((aligned(16))) float dsmall[SWS_TAB];
         lds_table_copy(small_g, small, 2 * SWS_TAB);
@@ -645,78 +742,110 @@ __global__ void __launch_bounds__(256) actq_bwd_wave_k(Src src, const uint16_t *
         __builtin_amdgcn_s_waitcnt(0x0f70);              // vmcnt(0): this wave's part of the tables (and its row)
         __syncthreads();
         src.set_small(small); sink.set_small(dsmall);
-        if (row_raw >= M) return;
+        if (W == 1 && row_raw >= M) return;
     }
-    float u[4][8], gmax[4];
-    u32x4 keep[4];
-    const float amax = actq_rotate_w(src, raw, q, u, keep, gmax);
+    __shared__ float xch[4];
+    __shared__ float sums[4][4];
+    __shared__ int counts[4];
+    const Lanes16 ln(slot);
+    u32x4 uw[R], keep[R];
+    const u16x2 most = actq_rotate_w<R>(src, raw, ln, uw, keep);
+    bool nan;
+    float amax = row_absmax_w<R>(uw, most, nan);
+    amax = share_absmax<W>(amax, nan, xch, wave);
     const float s_raw = amax * clip / (float)qmax, s = fmaxf(s_raw, 1e-8f);
     const Ste ste(qmax);
     const RowDiv rd(s, amax);
-    float gm[4][8], part[4][2];                          // g m; the reference lanes' sums of dL/ds terms
+    // a group's largest quotient that leaves it alone: below qmax - 1/2 by more than its rounding (qmax up to 1024); none in a row with a NaN
+    const float calm = nan || qmax > 1024 ? -1.0f : ste.hi - 0.51f;
+    constexpr int NC = W == 1 && R > 1 ? 2 : 1;          // chains of rounds
+    float acc[NC][2];                                    // the reference lanes' sums of dL/ds terms
+#pragma unroll
+    for (int c = 0; c < NC; c++) acc[c][0] = acc[c][1] = 0.0f;
     int ties_n = 0;
     uint32_t tied = 0;                                   // bit j: group j holds a max-|u| element in some lane
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        f32x4 ga, gb;
-        unpack_bf16x8(graw[j], ga, gb);
-        const float g8[8] = {ga.x, ga.y, ga.z, ga.w, gb.x, gb.y, gb.z, gb.w};
-        const f32x4 ta = rd.div4((f32x4){u[j][0], u[j][1], u[j][2], u[j][3]}, on), tb = rd.div4((f32x4){u[j][4], u[j][5], u[j][6], u[j][7]}, on);
-        const float t8[8] = {ta.x, ta.y, ta.z, ta.w, tb.x, tb.y, tb.z, tb.w};
-        float x8[8];
+    for (int j = 0; j < R; j++) {
+        const bool on = j < R - 1 || last_on;
+        float u[8], gv[8], t[8], x[8];
+        unpack8(unknown_words(uw[j]), u); unpack8(unknown_words(gw[j]), gv);
+        rd.div8(u, t, on);
 #pragma unroll
-        for (int k = 0; k < 8; k++) { float m; x8[k] = ste(t8[k], m); gm[j][k] = g8[k] * m; }
-        // ties are looked for only in a group whose largest value in some lane is the row's (wave-uniform; a row has few such elements)
-        if (__builtin_amdgcn_ballot_w64(on && gmax[j] == amax) != 0) {
-            tied |= 1u << j;
+        for (int k = 0; k < 8; k++) x[k] = rintf(t[k]) - t[k];
+        const float gm = absmax_of(absmax_pk8(uw[j]));
+        if (__builtin_amdgcn_ballot_w64(on && (!(gm * rd.r1 < calm) || gm == amax)) != 0) {
+            float m[8];
 #pragma unroll
-            for (int k = 0; k < 8; k++) ties_n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(on && fabsf(u[j][k]) == amax));
+            for (int k = 0; k < 8; k++) { x[k] = ste(t[k], m[k]); m[k] *= gv[k]; }
+            gw[j] = pack8_any(m);                        // (the products are bf16 values)
+            int n = 0;
+#pragma unroll
+            for (int k = 0; k < 8; k++) n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(on && fabsf(u[k]) == amax));
+            ties_n += n;
+            if (n) tied |= 1u << j;
         }
 #pragma unroll
         for (int kk = 0; kk < 2; kk++) {
-            float a = 0.0f;
+            float a = acc[j % NC][kk];
 #pragma unroll
-            for (int e = 0; e < 4; e++) a = __builtin_fmaf(g8[4 * kk + e], x8[4 * kk + e], a);
-            const float below = from_other_half(a, lane);
-            float b = below;
-#pragma unroll
-            for (int e = 0; e < 4; e++) b = __builtin_fmaf(g8[4 * kk + e], x8[4 * kk + e], b);
-            part[j][kk] = upper ? (on ? b : below) : a;
+            for (int e = 0; e < 4; e++) a = __builtin_fmaf(gv[4 * kk + e], x[4 * kk + e], a);
+            a = on ? a : acc[j % NC][kk];
+            asm volatile("" : "+v"(a));                  // (here, not behind the last group with every group's values kept until then)
+            acc[j % NC][kk] = a;
         }
+        __builtin_amdgcn_sched_barrier(0);
     }
     float dlds;
     {
-        const float b00 = part[0][0] + part[2][0], b01 = part[0][1] + part[2][1], b10 = part[1][0] + part[3][0], b11 = part[1][1] + part[3][1];   // l ^ 16
-        float c0 = b00 + b10, c1 = b01 + b11;                                                                                                      // l ^ 8
-        c0 += lane_xor2(c0); c1 += lane_xor2(c1);                                                                                                  // l ^ 4
-        c0 += lane_xor1(c0); c1 += lane_xor1(c1);                                                                                                  // l ^ 2
-        const float d = c0 + c1;                                                                                                                   // l ^ 1
-        dlds = lane_read(d, 32);
+        float d[NC];
 #pragma unroll
-        for (int h = 1; h < 8; h++) dlds += lane_read(d, 32 + 4 * h);
+        for (int c = 0; c < NC; c++) {
+            float a = acc[c][0], b = acc[c][1];
+            a += lane_xor8(a); b += lane_xor8(b);                        // l ^ 16
+            a += lane_xor4(a); b += lane_xor4(b);                        // l ^ 8
+            a += lane_xor2(a); b += lane_xor2(b);                        // l ^ 4
+            a += lane_xor1(a); b += lane_xor1(b);                        // l ^ 2
+            d[c] = a + b;                                                // l ^ 1
+        }
+        if (W == 1) {                                    // half-wave h: chain h >> 2, lanes 16 (h & 3) .. + 15
+            dlds = lane_read(d[0], 0);
+#pragma unroll
+            for (int h = 1; h < 4 * NC; h++) dlds += lane_read(d[h >> 2], 16 * (h & 3));
+            if (NC == 1) dlds += 0.0f;                   // (the absent half-waves' sums)
+        } else {                                         // half-wave h: part h >> 2
+            if ((lane & 15) == 0) sums[wave][lane >> 4] = d[0];
+            if (lane == 0) counts[wave] = ties_n;
+            __syncthreads();
+            const float * sp = sums[wave & ~1];
+            dlds = sp[0];
+#pragma unroll
+            for (int h = 1; h < 8; h++) dlds += sp[h];
+            ties_n = counts[wave & ~1] + counts[wave | 1];
+        }
     }
+    if (W > 1 && row_raw >= M) return;
     const float coef = s_raw >= 1e-8f ? dlds * clip / (float)qmax / (float)ties_n : 0.0f;
+    bool zero = false;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        if (tied & (1u << j)) {                          // wave-uniform: a row has few such elements
+    for (int j = 0; j < R; j++) {
+        if (__builtin_expect(tied & (1u << j), 0)) {     // wave-uniform: a row has few such elements
+            float u[8], d[8];
+            unpack8(unknown_words(uw[j]), u); unpack8(unknown_words(gw[j]), d);
 #pragma unroll
             for (int k = 0; k < 8; k++)
-                if (on && fabsf(u[j][k]) == amax && u[j][k] != 0.0f) gm[j][k] += u[j][k] > 0.0f ? coef : -coef;
+                if ((j < R - 1 || last_on) && fabsf(u[k]) == amax && u[k] != 0.0f) d[k] += u[k] > 0.0f ? coef : -coef;
+            gw[j] = pack8_any(d);                        // the gradient of the bf16 tensor u
         }
+        zero |= ln.plain(gw[j].x);
     }
+    const bool plain = __builtin_amdgcn_ballot_w64(zero) != 0;
 #pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int k = 0; k < 8; k += 4) {
-            const f32x4 v = rbf4_any((f32x4){gm[j][k], gm[j][k + 1], gm[j][k + 2], gm[j][k + 3]});      // the gradient of the bf16 tensor u
-            gm[j][k] = v.x; gm[j][k + 1] = v.y; gm[j][k + 2] = v.z; gm[j][k + 3] = v.w;
-        }
-    rotate128_w32(gm, q);
-    if (!on) return;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const f32x4 a = {gm[j][0], gm[j][1], gm[j][2], gm[j][3]}, b = {gm[j][4], gm[j][5], gm[j][6], gm[j][7]};
-        sink.st8(row, c * 128 + 32 * j + 8 * q, a, b, keep[j]);
+    for (int j = 0; j < R; j++) {
+        float d[8];
+        rotate128_w16(gw[j], d, ln, plain);
+        if (j == R - 1 && !last_on) break;
+        sink.st8(row, e0 + 512 * W * j, d, keep[j], stream);
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -848,8 +977,6 @@ __global__ void __launch_bounds__(256) block_entry_fwd_k(const float * x, const 
 // projections in reverse, so that the tree's first step (t ^ 16, the other block of a pair) is a row_half_mirror. The following steps
 // (t ^ 8, 4, 2, 1) pair n and k: registers. The eight group sums of a (row, projection) meet in LDS, where one lane adds them in order.
 CAMX_DEV f32x4 mirror4(f32x4 v) { return (f32x4){lane_xor4(v.x), lane_xor4(v.y), lane_xor4(v.z), lane_xor4(v.w)}; }      // row_half_mirror
-CAMX_DEV float bf_lo(uint32_t v) { return __builtin_bit_cast(float, v << 16); }
-CAMX_DEV float bf_hi(uint32_t v) { return __builtin_bit_cast(float, v & 0xffff0000u); }
 template <int NR>
 __global__ void __launch_bounds__(256, 4) block_entry_fwd_quad(const float * __restrict__ x, const float * __restrict__ nw, const uint16_t * __restrict__ wab, int nab, float eps,
                                                                uint16_t * __restrict__ y, float * __restrict__ s_out, uint16_t * __restrict__ codes, uint16_t * __restrict__ ab,
@@ -1118,8 +1245,20 @@ __attribute__((visibility("hidden"))) int dsilu_luts_init(hipStream_t st) {     
     return dsilu_luts_get(st, &lut, &small);
 }
 
-// the wave-per-row forward kernel: rows of at most 2048 values, operands aligned for its 16-byte loads and 16- / 4-byte stores
-static bool actq_wave_ok(int K, const void * x, const void * y, const void * codes) { return K <= 2048 && !((uintptr_t)x & 15) && !((uintptr_t)y & 15) && !((uintptr_t)codes & 3); }
+// the wave-per-row kernels: rows of at most 4096 values (longer ones would need more registers than a wave has, or sums handed from wave
+// to wave), operands aligned for 16-byte loads and 16- / 4-byte stores
+static bool actq_wave_ok(int K, uintptr_t x, uintptr_t y, uintptr_t codes) { return K <= 4096 && !((x | y) & 15) && !(codes & 3); }
+// one instance per number of rounds of 512 values, from 2048 on two waves a row
+#define ACTQ_WAVES(K, M, CALL)                                                                                          \
+    {                                                                                                                   \
+        const bool stream = (long)(M) * (K) >= (1L << 20);                                                              \
+        const dim3 grid((unsigned)((K) > 2048 ? ((long)(M) + 1) / 2 : ((long)(M) + 3) / 4)), block(256);                \
+        switch (((K) + 511) / 512) {                                                                                    \
+            case 1: { constexpr int R = 1, W = 1; CALL; } break; case 2: { constexpr int R = 2, W = 1; CALL; } break;   \
+            case 3: { constexpr int R = 3, W = 1; CALL; } break; case 4: { constexpr int R = 4, W = 1; CALL; } break;   \
+            case 5: case 6: { constexpr int R = 3, W = 2; CALL; } break; default: { constexpr int R = 4, W = 2; CALL; } break; \
+        }                                                                                                               \
+    }
 
 static int actq_check(int K, int qmax, int M) { return (K < 128 || K % 128 || K > 8192 || qmax < 1 || M < 0) ? CAMX_EINVAL : CAMX_OK; }
 
@@ -1139,9 +1278,9 @@ extern "C" {
 int camx_actq_fwd(const void * x, int is_bf16, uint16_t * y, float * s, uint16_t * codes, int K, float clip, int qmax, int M, hipStream_t st) {
     if (!x || (!y && !codes) || actq_check(K, qmax, M) || ((uintptr_t)x & (is_bf16 ? 7 : 15)) || ((uintptr_t)y & 7) || ((uintptr_t)codes & 1)) return CAMX_EINVAL;
     if (M == 0) return CAMX_OK;
-    if (actq_wave_ok(K, x, y, codes)) {
-        if (is_bf16) actq_fwd_wave_k<<<dim3((M + 3) / 4), dim3(256), 0, st>>>(PlainBF16{(const uint16_t *)x, K}, y, s, codes, K, clip, qmax, M);
-        else actq_fwd_wave_k<<<dim3((M + 3) / 4), dim3(256), 0, st>>>(PlainF32{(const float *)x, K}, y, s, codes, K, clip, qmax, M);
+    if (actq_wave_ok(K, (uintptr_t)x, (uintptr_t)y, (uintptr_t)codes)) {
+        if (is_bf16) ACTQ_WAVES(K, M, (actq_fwd_wave_k<PlainBF16, R, W><<<grid, block, 0, st>>>(PlainBF16{(const uint16_t *)x, K}, y, s, codes, K, clip, qmax, M, stream)))
+        else ACTQ_WAVES(K, M, (actq_fwd_wave_k<PlainF32, R, W><<<grid, block, 0, st>>>(PlainF32{(const float *)x, K}, y, s, codes, K, clip, qmax, M, stream)))
         CAMX_LAUNCH_RET();
     }
     if (is_bf16) { ACTQ_ROUNDS(K, (actq_fwd_k<NR><<<dim3(M), dim3(256), 0, st>>>(PlainBF16{(const uint16_t *)x, K}, y, s, codes, K, clip, qmax))) }
@@ -1154,8 +1293,8 @@ int camx_silu_mul_actq_fwd(const uint16_t * gu, int ld, int F, uint16_t * y, flo
     const uint16_t * lut = nullptr, * small = nullptr;
     const int rc = silu_luts_get(st, &lut, &small);
     if (rc) return rc;
-    if (F <= 2048 && !(ld & 7) && !((uintptr_t)gu & 15) && actq_wave_ok(F, gu, y, codes)) {       // one wave per row
-        actq_fwd_wave_k<<<dim3((M + 3) / 4), dim3(256), 0, st>>>(SiluMulSrc{gu, ld, F, lut, nullptr}, y, s, codes, F, clip, qmax, M, small);
+    if (!(ld & 7) && actq_wave_ok(F, (uintptr_t)gu, (uintptr_t)y, (uintptr_t)codes)) {
+        ACTQ_WAVES(F, M, (actq_fwd_wave_k<SiluMulSrc, R, W><<<grid, block, 0, st>>>(SiluMulSrc{gu, ld, F, lut, nullptr}, y, s, codes, F, clip, qmax, M, stream, small)))
         CAMX_LAUNCH_RET();
     }
     ACTQ_ROUNDS(F, (actq_fwd_k<NR><<<dim3(M), dim3(256), 0, st>>>(SiluMulSrc{gu, ld, F, lut, nullptr}, y, s, codes, F, clip, qmax)))
@@ -1193,9 +1332,9 @@ int camx_block_entry_fwd(const float * x, const float * nw, const uint16_t * wab
 int camx_actq_bwd(const void * x, int is_bf16, const uint16_t * g, void * dx, int K, float clip, int qmax, int M, hipStream_t st) {
     if (!x || !g || !dx || actq_check(K, qmax, M) || ((uintptr_t)x & (is_bf16 ? 7 : 15)) || ((uintptr_t)dx & (is_bf16 ? 7 : 15)) || ((uintptr_t)g & 7)) return CAMX_EINVAL;
     if (M == 0) return CAMX_OK;
-    if (K <= 2048 && !(((uintptr_t)x | (uintptr_t)g | (uintptr_t)dx) & 15)) {                  // one wave per row
-        if (is_bf16) actq_bwd_wave_k<<<dim3((M + 3) / 4), dim3(256), 0, st>>>(PlainBF16{(const uint16_t *)x, K}, g, SinkBF16{(uint16_t *)dx, K}, K, clip, qmax, M);
-        else actq_bwd_wave_k<<<dim3((M + 3) / 4), dim3(256), 0, st>>>(PlainF32{(const float *)x, K}, g, SinkF32{(float *)dx, K}, K, clip, qmax, M);
+    if (actq_wave_ok(K, (uintptr_t)x | (uintptr_t)g, (uintptr_t)dx, 0)) {
+        if (is_bf16) ACTQ_WAVES(K, M, (actq_bwd_wave_k<PlainBF16, SinkBF16, R, W><<<grid, block, 0, st>>>(PlainBF16{(const uint16_t *)x, K}, g, SinkBF16{(uint16_t *)dx, K}, K, clip, qmax, M, stream)))
+        else ACTQ_WAVES(K, M, (actq_bwd_wave_k<PlainF32, SinkF32, R, W><<<grid, block, 0, st>>>(PlainF32{(const float *)x, K}, g, SinkF32{(float *)dx, K}, K, clip, qmax, M, stream)))
         CAMX_LAUNCH_RET();
     }
     if (is_bf16) { ACTQ_ROUNDS(K, (actq_bwd_k<NR><<<dim3(M), dim3(256), 0, st>>>(PlainBF16{(const uint16_t *)x, K}, g, SinkBF16{(uint16_t *)dx, K}, K, clip, qmax))) }
@@ -1211,8 +1350,8 @@ int camx_silu_mul_actq_bwd(const uint16_t * gu, int ld, int F, const uint16_t * 
     int rc = silu_luts_get(st, &lut, &small);
     if (!rc) rc = dsilu_luts_get(st, &dlut, &dsmall);
     if (rc) return rc;
-    if (F <= 2048 && !(ld & 7) && !(((uintptr_t)gu | (uintptr_t)g | (uintptr_t)dgu) & 15)) {      // one wave per row
-        actq_bwd_wave_k<<<dim3((M + 3) / 4), dim3(256), 0, st>>>(SiluMulSrc{gu, ld, F, lut, nullptr}, g, SinkSiluMul{gu, ld, F, dgu, dlut, nullptr}, F, clip, qmax, M, small, dsmall);
+    if (!(ld & 7) && actq_wave_ok(F, (uintptr_t)gu | (uintptr_t)g, (uintptr_t)dgu, 0)) {
+        ACTQ_WAVES(F, M, (actq_bwd_wave_k<SiluMulSrc, SinkSiluMul, R, W><<<grid, block, 0, st>>>(SiluMulSrc{gu, ld, F, lut, nullptr}, g, SinkSiluMul{gu, ld, F, dgu, dlut, nullptr}, F, clip, qmax, M, stream, small, dsmall)))
         CAMX_LAUNCH_RET();
     }
     ACTQ_ROUNDS(F, (actq_bwd_k<NR><<<dim3(M), dim3(256), 0, st>>>(SiluMulSrc{gu, ld, F, lut, nullptr}, g, SinkSiluMul{gu, ld, F, dgu, dlut, nullptr}, F, clip, qmax)))

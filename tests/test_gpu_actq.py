@@ -292,6 +292,32 @@ def test_block_entry_infinite_rstd(M, d, nab):
     assert bits_equal(host(ab, np.uint16), rab)
 
 
+@pytest.mark.parametrize('K', [128, 512, 640, 1024, 1536, 1664, 2048, 2176, 3072, 3200, 4096])
+@pytest.mark.parametrize('streams', [False, True])
+def test_actq_rounds_and_waves_of_a_row(K, streams):
+    """every number of rounds of 512 values and of waves a row, whole and with a partial last round, below and from the batch size on
+    whose outputs pass by the caches: rows with a NaN, an infinity, nothing but zeros, negative zeros, one value per chunk whose quotients
+    are half-integers (3.5 = 7 / (14 / 7)), and a row whose maximum is everywhere"""
+    rng = np.random.default_rng(700 + K)
+    M = (1 << 20) // K + 3 if streams else 7
+    x = outliers(rng, (M, K))
+    x[0, K // 2] = np.nan; x[1, K - 1] = np.inf; x[2] = 0; x[3, :] = -0.0; x[3, 64] = 0.5
+    x[4] = 0; x[4, 0::128] = 14.0 * 0.5 ** (np.arange(K // 128) % 4)
+    x[5] = 0; x[5, ::128] = 3.0
+    g = O.f2bf(rng.standard_normal((M, K)).astype(np.float32)); g[6, :4] = 0x8000
+    for bf in (False, True):
+        src = O.f2bf(x) if bf else x
+        srcd = dev(src)
+        ry, rs, rc = O.actq_fwd(src, bf16=bf)
+        y = dev(np.zeros((M, K), np.uint16)); s = dev(np.zeros(M, np.float32)); c = dev(np.zeros((M, K // 2), np.uint8))
+        call('camx_actq_fwd', ptr(srcd), I(int(bf)), ptr(y), ptr(s), ptr(c), I(K), F(1.0), I(7), I(M))
+        assert bits_equal(host(s), rs) and bits_equal(host(y, np.uint16), ry) and bits_equal(host(c), rc)
+        want = O.actq_bwd(src, g, bf16=bf)
+        dx = dev(np.zeros((M, K), np.uint16 if bf else np.float32))
+        call('camx_actq_bwd', ptr(srcd), I(int(bf)), ptr(dev(g)), ptr(dx), I(K), F(1.0), I(7), I(M))
+        assert bits_equal(host(dx, np.uint16) if bf else host(dx), want)
+
+
 @pytest.mark.parametrize('K', [128, 640, 2048])
 def test_actq_signs_of_zeros(K):
     """rows whose chunks begin with -0: the sign of a zero result comes through the rotation of the wave-per-row kernels (all zeros of one
