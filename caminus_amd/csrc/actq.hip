@@ -5,7 +5,8 @@
 //
 // Rows of at most 4096 values with 16-byte aligned operands, forward and backward, plain and SiLU-fused: one wave per row, two above 2048
 // (actq_fwd_wave_k, actq_bwd_wave_k), the fused forms with the gates' tables in LDS. The RMSNorm-fused block entry of rows of at most
-// 1024 values: a wave per row as well, four rows sharing the projections (block_entry_fwd_quad, block_entry_bwd_quad). Everything else
+// 1024 values: a wave per row as well, four or sixteen rows sharing the projections (block_entry_fwd_quad, block_entry_fwd_rows16,
+// block_entry_bwd_quad). Everything else
 // (longer rows, unaligned operands):
 // One 256-thread workgroup per row. A half-wave (32 lanes) transforms one 128-chunk: lane l holds elements 4l .. 4l + 3,
 // butterfly stages 1-2 in registers, 4 .. 64 across lanes; half-wave h takes chunks h, h + 8, ... (the reference's wave h of
@@ -131,36 +132,15 @@ struct RmsSrc {
     }
     CAMX_DEV f32x4 operator()(int row, int k, u32x2 &) const { return (*this)(row, k); }
 };
-// The same source for a row that one wave holds in registers (rows of at most 256 NR values): round c of the lane is elements
-// 256 c + 4 slot .. + 3, the elements the lane holds in the row's sum of squares and in the projections, so x and the norm
-// weights are read once.
-template <int NR>
-struct RmsRegSrc {
-    static constexpr bool bf16_valued = false;
-    static constexpr bool by_round = true;
-    f32x4 xk[NR], wk[NR]; float rstd;
-    CAMX_DEV f32x4 at(int c) const {
-        f32x4 a; a.x = xk[c].x * rstd * wk[c].x; a.y = xk[c].y * rstd * wk[c].y; a.z = xk[c].z * rstd * wk[c].z; a.w = xk[c].w * rstd * wk[c].w;
-        return a;
-    }
-    CAMX_DEV f32x4 operator()(int, int k, u32x2 &) const { return at(k >> 8); }
-};
-template <typename S, typename = void> struct SrcByRound : std::false_type {};
-template <typename S> struct SrcByRound<S, std::void_t<decltype(S::by_round)>> : std::true_type {};
-
-// u = bf16(H128 . bf16(source)) for the NR rounds of this half-wave (NHW == 2: NR is ceil(K / 256), so only the last can be partial); returns the lane's max |u| over its active chunks
-// NHW: the half-waves that share a row (8: a 256-thread workgroup; 2: one wave); half-wave hw takes chunks hw, hw + NHW, ...
-template <int NR, typename Src, int NHW = 8>
+// u = bf16(H128 . bf16(source)) for the NR rounds of this half-wave, which takes chunks hw, hw + 8, ..; returns the lane's max |u| over its active chunks
+template <int NR, typename Src>
 CAMX_DEV float actq_rotate(Src src, int row, int l, int hw, int nch, f32x4 (&u)[NR], u32x2 * keep = nullptr) {
 #pragma unroll
     for (int c = 0; c < NR; c++) {
-        const int ch = hw + NHW * c;
+        const int ch = hw + 8 * c;
         f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
         u32x2 kp = {0u, 0u};
-        if ((NHW == 2 && c < NR - 1) || ch < nch) {
-            if constexpr (SrcByRound<Src>::value) { static_assert(NHW == 2, "a wave per row"); v = src.at(c); }
-            else v = src(row, ch * 128 + 4 * l, kp);
-        }
+        if (ch < nch) v = src(row, ch * 128 + 4 * l, kp);
         if (keep) keep[c] = kp;
         u[c] = v;
     }
@@ -170,7 +150,7 @@ CAMX_DEV float actq_rotate(Src src, int row, int l, int hw, int nch, f32x4 (&u)[
         const f32x4 in = Src::bf16_valued ? u[c] : rbf4_any(u[c]);                // autocast's bf16 input
         const f32x4 v = rbf4_any(scaled4(hadamard128_l4(in, l, false)));
         u[c] = v;
-        if ((NHW == 2 && c < NR - 1) || hw + NHW * c < nch) amax = fmaxf(amax, absmax4(v));
+        if (hw + 8 * c < nch) amax = fmaxf(amax, absmax4(v));
     }
     return amax;
 }
@@ -212,29 +192,27 @@ CAMX_DEV float wave_max64(float v) {
     return fmaxf(fmaxf(lane_read(v, 0), lane_read(v, 16)), fmaxf(lane_read(v, 32), lane_read(v, 48)));
 }
 // row-wide max (order-free); lds: 4 floats
-template <int NHW = 8>
 CAMX_DEV float row_max(float amax, float * lds) {
     const int tid = threadIdx.x;
     amax = wave_max64(amax);
-    if (NHW == 2) return amax;                           // the row is this wave's
     __syncthreads();
     if ((tid & 63) == 0) lds[tid >> 6] = amax;
     __syncthreads();
     return fmaxf(fmaxf(lds[0], lds[1]), fmaxf(lds[2], lds[3]));
 }
 
-template <int NR, typename Src, int NHW = 8>
+template <int NR, typename Src>
 CAMX_DEV void actq_fwd_row(Src src, int row, uint16_t * __restrict__ y, float * __restrict__ s_out, int K, float clip, int qmax,
                            uint16_t * __restrict__ codes, float * lds) {
-    const int tid = threadIdx.x, l = slot_of(tid) & 31, hw = (tid >> 5) & (NHW - 1), nch = K / 128;
+    const int tid = threadIdx.x, l = slot_of(tid) & 31, hw = tid >> 5, nch = K / 128;
     f32x4 u[NR];
-    const float amax = row_max<NHW>(actq_rotate<NR, Src, NHW>(src, row, l, hw, nch, u), lds);
+    const float amax = row_max(actq_rotate<NR, Src>(src, row, l, hw, nch, u), lds);
     const float s = fmaxf(amax * clip / (float)qmax, 1e-8f);
     const RowScale rs(s, amax, qmax);
     if (tid == 0 && s_out) s_out[row] = s;
 #pragma unroll
     for (int c = 0; c < NR; c++) {
-        const int ch = hw + NHW * c;
+        const int ch = hw + 8 * c;
         if (ch < nch) {
             const f32x4 q = rs.quant4(u[c]);
             if (y) { f32x4 d; d.x = q.x * s; d.y = q.y * s; d.z = q.z * s; d.w = q.w * s; *(u32x2 *)(y + (size_t)row * K + ch * 128 + 4 * l) = pack_f2bf_x4(d); }
@@ -278,13 +256,19 @@ CAMX_DEV u32x4 pack8_any(const float (&v)[8]) { return (u32x4){hw_pk_bf16(v[0], 
 // A batch of 2^20 values or more streams: its bf16 outputs leave past the caches as whole lines (the wave's round is 1 KiB without a gap:
 // 16384 x 2048 forward 31.4 -> 26.3 us, backward 40.1 -> 36.3 with g read past them too). fp32 gradients stay plain: a lane's eight values
 // are two half lines, which only the cache puts together (61 -> 85 us).
+typedef u32x4 u32x4_a8 __attribute__((aligned(8)));                      // (the block entry's operands are 8-byte aligned, its codes 2)
+typedef uint32_t u32_a2 __attribute__((aligned(2)));
+CAMX_DEV void store8(u32x2 v, void * p, bool stream) {
+    if (stream) { asm volatile("" ::: "memory"); __builtin_nontemporal_store(v, (u32x2 *)p); asm volatile("" ::: "memory"); }
+    else *(u32x2 *)p = v;
+}
 CAMX_DEV void store16(u32x4 v, void * p, bool stream) {
     if (stream) {                                        // (between two empty asm statements: the compiler makes one plain store of the two otherwise)
         asm volatile("" ::: "memory");
-        __builtin_nontemporal_store(v, (u32x4 *)p);
+        __builtin_nontemporal_store(v, (u32x4_a8 *)p);
         asm volatile("" ::: "memory");
     }
-    else *(u32x4 *)p = v;
+    else *(u32x4_a8 *)p = v;
 }
 CAMX_DEV u32x4 pack8_canon(const float (&v)[8]) {                     // f2bf of eight values (NaN -> 0x7fc0)
     const u32x2 a = pack_f2bf_x4((f32x4){v[0], v[1], v[2], v[3]}), b = pack_f2bf_x4((f32x4){v[4], v[5], v[6], v[7]});
@@ -420,6 +404,32 @@ CAMX_DEV bool row_is_tame(const RowScale & rs, float amax, bool nan) {
     const float hs = ((float)lane + 0.5f) * rs.s, near = bf_lo(hw_pk_bf16(hs, 0.0f));
     return __builtin_amdgcn_ballot_w64((float)lane < rs.hi && fabsf(near - hs) < 2e-5f * rs.s) == 0;
 }
+// the values and codes of a row (or a wave's part of it) from its packed rotated words; y, codes: the row's, or null
+template <int R, int W>
+CAMX_DEV void quantize_row_w(const u32x4 (&uw)[R], float amax, bool nan, float s, int qmax, int e0, bool last_on, uint16_t * y, uint16_t * codes, bool stream) {
+    const RowScale rs(s, amax, qmax);
+    const bool tame = row_is_tame(rs, amax, nan);
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        if (j == R - 1 && !last_on) break;
+        float q[8];
+        unpack8(uw[j], q);
+        if (__builtin_expect(tame, 1)) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) q[k] = rintf(q[k] * rs.rcp);
+        } else {
+            const f32x4 a = rs.quant4((f32x4){q[0], q[1], q[2], q[3]}), b = rs.quant4((f32x4){q[4], q[5], q[6], q[7]});
+            q[0] = a.x; q[1] = a.y; q[2] = a.z; q[3] = a.w; q[4] = b.x; q[5] = b.y; q[6] = b.z; q[7] = b.w;
+        }
+        const int e = e0 + 512 * W * j;
+        if (codes) *(u32_a2 *)(codes + (e >> 2)) = rs.nibbles4((f32x4){q[0], q[1], q[2], q[3]}) | (rs.nibbles4((f32x4){q[4], q[5], q[6], q[7]}) << 16);
+        if (y) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) q[k] *= s;
+            store16(__builtin_expect(tame, 1) ? pack8_any(q) : pack8_canon(q), y + e, stream);   // (a tame row's products are numbers)
+        }
+    }
+}
 // The kernel's time at 8192 rows and more is the larger of its arithmetic and its bytes, plus the launch's ramp; a wave that walks several
 // rows with the next row's loads in flight measured 5 to 15 % slower.
 template <typename Src, int R, int W>
@@ -449,29 +459,8 @@ __global__ void __launch_bounds__(256) actq_fwd_wave_k(Src src, uint16_t * __res
     amax = share_absmax<W>(amax, nan, xch, wave);
     if (W > 1 && row >= M) return;
     const float s = fmaxf(amax * clip / (float)qmax, 1e-8f);
-    const RowScale rs(s, amax, qmax);
     if (lane == 0 && part == 0 && s_out) s_out[row] = s;
-    const bool tame = row_is_tame(rs, amax, nan);
-#pragma unroll
-    for (int j = 0; j < R; j++) {
-        if (j == R - 1 && !last_on) break;
-        float q[8];
-        unpack8(uw[j], q);
-        if (__builtin_expect(tame, 1)) {
-#pragma unroll
-            for (int k = 0; k < 8; k++) q[k] = rintf(q[k] * rs.rcp);
-        } else {
-            const f32x4 a = rs.quant4((f32x4){q[0], q[1], q[2], q[3]}), b = rs.quant4((f32x4){q[4], q[5], q[6], q[7]});
-            q[0] = a.x; q[1] = a.y; q[2] = a.z; q[3] = a.w; q[4] = b.x; q[5] = b.y; q[6] = b.z; q[7] = b.w;
-        }
-        const size_t e = (size_t)row * K + e0 + 512 * W * j;
-        if (codes) *(uint32_t *)(codes + (e >> 2)) = rs.nibbles4((f32x4){q[0], q[1], q[2], q[3]}) | (rs.nibbles4((f32x4){q[4], q[5], q[6], q[7]}) << 16);
-        if (y) {
-#pragma unroll
-            for (int k = 0; k < 8; k++) q[k] *= s;
-            store16(__builtin_expect(tame, 1) ? pack8_any(q) : pack8_canon(q), y + e, stream);   // (a tame row's products are numbers)
-        }
-    }
+    quantize_row_w<R, W>(uw, amax, nan, s, qmax, e0, last_on, y ? y + (size_t)row * K : nullptr, codes ? codes + (size_t)row * (K / 4) : nullptr, stream);
 }
 
 // ---- backward ----------------------------------------------------------------------------------------------------------------
@@ -625,34 +614,31 @@ struct SinkSiluMul {
 };
 
 // lds16: 16 floats. sink receives bf16-valued floats: the gradient of the bf16 source, before any widening store.
-// NHW = 8: a 256-thread workgroup per row. NHW = 2: one wave per row of at most 1024 values (each half-wave sum of the tree is
-// then one chunk's: round c holds chunks 2 c and 2 c + 1); out, when given, receives round c's result in place of the sink.
-template <int NR, typename Src, typename Sink, int NHW = 8>
-CAMX_DEV void actq_bwd_row(Src src, int row, const uint16_t * __restrict__ g, Sink sink, int K, float clip, int qmax, float * lds16, f32x4 * out = nullptr) {
-    const int tid = threadIdx.x, l = slot_of(tid) & 31, hw = (tid >> 5) & (NHW - 1), nch = K / 128;
+template <int NR, typename Src, typename Sink>
+CAMX_DEV void actq_bwd_row(Src src, int row, const uint16_t * __restrict__ g, Sink sink, int K, float clip, int qmax, float * lds16) {
+    const int tid = threadIdx.x, l = slot_of(tid) & 31, hw = tid >> 5, nch = K / 128;
     f32x4 u[NR], gv[NR];
 #pragma unroll
     for (int c = 0; c < NR; c++) {
-        const int ch = hw + NHW * c;
+        const int ch = hw + 8 * c;
         u32x2 raw = {0u, 0u};
-        if ((NHW == 2 && c < NR - 1) || ch < nch) raw = *(const u32x2 *)(g + (size_t)row * K + ch * 128 + 4 * l);
+        if (ch < nch) raw = *(const u32x2 *)(g + (size_t)row * K + ch * 128 + 4 * l);
         gv[c] = unpack_bf16x4(raw);
     }
     u32x2 keep[NR];                                      // what the source hands to the sink (the fused SiLU form only)
-    const float amax = row_max<NHW>(actq_rotate<NR, Src, NHW>(src, row, l, hw, nch, u, keep), lds16);
+    const float amax = row_max(actq_rotate<NR, Src>(src, row, l, hw, nch, u, keep), lds16);
     const float s_raw = amax * clip / (float)qmax, s = fmaxf(s_raw, 1e-8f);
     const Ste ste(qmax);
     // dL/ds = sum g (q - m t) and the number of max-|u| elements; m: the rounded value lies strictly inside (lo, hi). The
     // straight-through part g m is formed here (g is not needed afterwards); the ties are counted from the compares' lane masks
     // on the scalar unit, one counter per half-wave (a count is exact in any order).
     const RowDiv rd(s, amax);
-    float dlds = 0.0f, part[NHW == 2 ? NR : 1];           // NHW == 2: a sum per round (a reference lane's terms are one chunk's)
+    float dlds = 0.0f;
     int ties_lo = 0, ties_hi = 0;
     uint32_t tied = 0;                                   // bit c: some lane of this wave holds a max-|u| element in round c
 #pragma unroll
     for (int c = 0; c < NR; c++) {
-        if (NHW == 2) dlds = 0.0f;
-        if ((NHW == 2 && c < NR - 1) || hw + NHW * c < nch) {
+        if (hw + 8 * c < nch) {
             const f32x4 t4 = rd.div4(u[c]);
 #define D_(e) { float m; const float x = ste(t4.e, m); dlds = __builtin_fmaf(gv[c].e, x, dlds); gv[c].e = gv[c].e * m; }
             CAMX_EACH4(D_)
@@ -660,39 +646,20 @@ CAMX_DEV void actq_bwd_row(Src src, int row, const uint16_t * __restrict__ g, Si
 #define T_(e) { const uint64_t tie = __builtin_amdgcn_ballot_w64(fabsf(u[c].e) == amax); any |= tie; \
                 ties_lo += __builtin_popcount((uint32_t)tie); ties_hi += __builtin_popcount((uint32_t)(tie >> 32)); }
             uint64_t any = 0;
-            // a wave per row: few rounds hold such an element, so they are looked for first. (In the workgroup form that look costs up to five
-            // registers, a wave per SIMD at several widths: 8192 rows of 7168 bf16 values 102.6 us with it, 94.2 without, fused 8192 x 6144 186 and 173)
-            if (NHW == 8) { CAMX_EACH4(T_) }
-            else {
-                const float most = fmaxf(fmaxf(fabsf(u[c].x), fabsf(u[c].y)), fmaxf(fabsf(u[c].z), fabsf(u[c].w)));
-                if (__builtin_amdgcn_ballot_w64(most == amax) != 0) { CAMX_EACH4(T_) }
-            }
+            // (a look whether the round holds such an element at all costs up to five registers here, a wave per SIMD at several widths: 8192 rows
+            // of 7168 bf16 values 102.6 us with it, 94.2 without, fused 8192 x 6144 186 and 173)
+            CAMX_EACH4(T_)
 #undef T_
             if (any) tied |= 1u << c;
         }
-        if (NHW == 2) part[NHW == 2 ? c : 0] = dlds;
     }
-    float ties;
-    if (NHW == 2) {                                      // the eight chunk sums in order (absent chunks add +0, as idle half-waves do)
-        ties = lane_read((float)(ties_lo + ties_hi), 0);          // lane 0's count: its half-wave is in every round that any lane is in (the counters of a lane that sits out a round miss that round)
-#pragma unroll
-        for (int c = 0; c < NR; c++) {
-            const float hs = half32_sum(part[NHW == 2 ? c : 0]);
-            const float even = lane_read(hs, 0), odd = lane_read(hs, 32);
-            dlds = c == 0 ? even : dlds + even;
-            dlds += odd;
-        }
-        if (2 * NR < 8) dlds += 0.0f;
-    } else {
-        ties = (tid & 31) == 0 ? (float)((tid & 32) ? ties_hi : ties_lo) : 0.0f;
-        block8_sum2(dlds, ties, lds16);
-    }
+    float ties = (tid & 31) == 0 ? (float)((tid & 32) ? ties_hi : ties_lo) : 0.0f;
+    block8_sum2(dlds, ties, lds16);
     const float coef = s_raw >= 1e-8f ? dlds * clip / (float)qmax / ties : 0.0f;
 #pragma unroll
     for (int c = 0; c < NR; c++) {
-        const int ch = hw + NHW * c;
-        if (out) out[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-        if ((NHW == 2 && c < NR - 1) || ch < nch) {
+        const int ch = hw + 8 * c;
+        if (ch < nch) {
             f32x4 d = gv[c];
             if (tied & (1u << c)) {                      // wave-uniform: a row has few such elements, most rounds skip this
 #define V_(e) if (fabsf(u[c].e) == amax && u[c].e != 0.0f) d.e += u[c].e > 0.0f ? coef : -coef;
@@ -700,7 +667,7 @@ CAMX_DEV void actq_bwd_row(Src src, int row, const uint16_t * __restrict__ g, Si
 #undef V_
             }
             const f32x4 r = rbf4_canon(scaled4(hadamard128_l4(rbf4_any(d), l, false)));      // rbf4_any: the gradient of the bf16 tensor u
-            if (out) out[c] = r; else sink(row, ch * 128 + 4 * l, r, keep[c]);
+            sink(row, ch * 128 + 4 * l, r, keep[c]);
         }
     }
 }
@@ -718,6 +685,98 @@ __global__ void __launch_bounds__(256) actq_bwd_k(Src src, const uint16_t * g, S
 // then combine by l ^ 16, 8, 4, 2 (slots) and 1 (registers), and the eight half-wave sums are added in order.
 // Eight values at a time, as packed words between the passes: a group in which no lane's quotient can round to qmax (or below -qmax) and no
 // lane holds the row's maximum needs no clamp, no mask and no look for ties, and its part of the gradient is g itself.
+struct PairShare { float amax[4], sums[4][4]; int counts[4]; };          // what the two waves of a row hand each other
+// g (packed, the gradient of the quantized values) becomes the gradient of the rotated values u (packed); returns whether a chunk's rotation
+// has to keep a negative zero (see Lanes16)
+template <int R, int W>
+CAMX_DEV bool quantize_bwd_w(const u32x4 (&uw)[R], u32x4 (&gw)[R], float amax, bool nan, float clip, int qmax, const Lanes16 & ln, bool last_on, int wave, PairShare & x) {
+    const int lane = threadIdx.x & 63;
+    const float s_raw = amax * clip / (float)qmax, s = fmaxf(s_raw, 1e-8f);
+    const Ste ste(qmax);
+    const RowDiv rd(s, amax);
+    // a group's largest quotient that leaves it alone: below qmax - 1/2 by more than its rounding (qmax up to 1024); none in a row with a NaN
+    const float calm = nan || qmax > 1024 ? -1.0f : ste.hi - 0.51f;
+    constexpr int NC = W == 1 && R > 1 ? 2 : 1;          // chains of rounds
+    float acc[NC][2];                                    // the reference lanes' sums of dL/ds terms
+#pragma unroll
+    for (int c = 0; c < NC; c++) acc[c][0] = acc[c][1] = 0.0f;
+    int ties_n = 0;
+    uint32_t tied = 0;                                   // bit j: group j holds a max-|u| element in some lane
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        const bool on = j < R - 1 || last_on;
+        float u[8], gv[8], t[8], v[8];
+        unpack8(unknown_words(uw[j]), u); unpack8(unknown_words(gw[j]), gv);
+        rd.div8(u, t, on);
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] = rintf(t[k]) - t[k];
+        const float gm = absmax_of(absmax_pk8(uw[j]));
+        if (__builtin_amdgcn_ballot_w64(on && (!(gm * rd.r1 < calm) || gm == amax)) != 0) {
+            float m[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) { v[k] = ste(t[k], m[k]); m[k] *= gv[k]; }
+            gw[j] = pack8_any(m);                        // (the products are bf16 values)
+            int n = 0;
+#pragma unroll
+            for (int k = 0; k < 8; k++) n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(on && fabsf(u[k]) == amax));
+            ties_n += n;
+            if (n) tied |= 1u << j;
+        }
+#pragma unroll
+        for (int kk = 0; kk < 2; kk++) {
+            float a = acc[j % NC][kk];
+#pragma unroll
+            for (int e = 0; e < 4; e++) a = __builtin_fmaf(gv[4 * kk + e], v[4 * kk + e], a);
+            a = on ? a : acc[j % NC][kk];
+            asm volatile("" : "+v"(a));                  // (here, not behind the last group with every group's values kept until then)
+            acc[j % NC][kk] = a;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    float dlds;
+    {
+        float d[NC];
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            float a = acc[c][0], b = acc[c][1];
+            a += lane_xor8(a); b += lane_xor8(b);                        // l ^ 16
+            a += lane_xor4(a); b += lane_xor4(b);                        // l ^ 8
+            a += lane_xor2(a); b += lane_xor2(b);                        // l ^ 4
+            a += lane_xor1(a); b += lane_xor1(b);                        // l ^ 2
+            d[c] = a + b;                                                // l ^ 1
+        }
+        if (W == 1) {                                    // half-wave h: chain h >> 2, lanes 16 (h & 3) .. + 15
+            dlds = lane_read(d[0], 0);
+#pragma unroll
+            for (int h = 1; h < 4 * NC; h++) dlds += lane_read(d[h >> 2], 16 * (h & 3));
+            if (NC == 1) dlds += 0.0f;                   // (the absent half-waves' sums)
+        } else {                                         // half-wave h: part h >> 2
+            if ((lane & 15) == 0) x.sums[wave][lane >> 4] = d[0];
+            if (lane == 0) x.counts[wave] = ties_n;
+            __syncthreads();
+            const float * sp = x.sums[wave & ~1];
+            dlds = sp[0];
+#pragma unroll
+            for (int h = 1; h < 8; h++) dlds += sp[h];
+            ties_n = x.counts[wave & ~1] + x.counts[wave | 1];
+        }
+    }
+    const float coef = s_raw >= 1e-8f ? dlds * clip / (float)qmax / (float)ties_n : 0.0f;
+    bool zero = false;
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        if (__builtin_expect(tied & (1u << j), 0)) {     // wave-uniform: a row has few such elements
+            float u[8], d[8];
+            unpack8(unknown_words(uw[j]), u); unpack8(unknown_words(gw[j]), d);
+#pragma unroll
+            for (int k = 0; k < 8; k++)
+                if ((j < R - 1 || last_on) && fabsf(u[k]) == amax && u[k] != 0.0f) d[k] += u[k] > 0.0f ? coef : -coef;
+            gw[j] = pack8_any(d);                        // the gradient of the bf16 tensor u
+        }
+        zero |= ln.plain(gw[j].x);
+    }
+    return __builtin_amdgcn_ballot_w64(zero) != 0;
+}
 template <typename Src, typename Sink, int R, int W>
 __global__ void __launch_bounds__(256) actq_bwd_wave_k(Src src, const uint16_t * __restrict__ g, Sink sink, int K, float clip, int qmax, int M, bool stream,
                                                        const uint16_t * small_g = nullptr, const float * dsmall_g = nullptr) {
@@ -744,101 +803,15 @@ __global__ void __launch_bounds__(256) actq_bwd_wave_k(Src src, const uint16_t *
         src.set_small(small); sink.set_small(dsmall);
         if (W == 1 && row_raw >= M) return;
     }
-    __shared__ float xch[4];
-    __shared__ float sums[4][4];
-    __shared__ int counts[4];
+    __shared__ PairShare share;
     const Lanes16 ln(slot);
     u32x4 uw[R], keep[R];
     const u16x2 most = actq_rotate_w<R>(src, raw, ln, uw, keep);
     bool nan;
     float amax = row_absmax_w<R>(uw, most, nan);
-    amax = share_absmax<W>(amax, nan, xch, wave);
-    const float s_raw = amax * clip / (float)qmax, s = fmaxf(s_raw, 1e-8f);
-    const Ste ste(qmax);
-    const RowDiv rd(s, amax);
-    // a group's largest quotient that leaves it alone: below qmax - 1/2 by more than its rounding (qmax up to 1024); none in a row with a NaN
-    const float calm = nan || qmax > 1024 ? -1.0f : ste.hi - 0.51f;
-    constexpr int NC = W == 1 && R > 1 ? 2 : 1;          // chains of rounds
-    float acc[NC][2];                                    // the reference lanes' sums of dL/ds terms
-#pragma unroll
-    for (int c = 0; c < NC; c++) acc[c][0] = acc[c][1] = 0.0f;
-    int ties_n = 0;
-    uint32_t tied = 0;                                   // bit j: group j holds a max-|u| element in some lane
-#pragma unroll
-    for (int j = 0; j < R; j++) {
-        const bool on = j < R - 1 || last_on;
-        float u[8], gv[8], t[8], x[8];
-        unpack8(unknown_words(uw[j]), u); unpack8(unknown_words(gw[j]), gv);
-        rd.div8(u, t, on);
-#pragma unroll
-        for (int k = 0; k < 8; k++) x[k] = rintf(t[k]) - t[k];
-        const float gm = absmax_of(absmax_pk8(uw[j]));
-        if (__builtin_amdgcn_ballot_w64(on && (!(gm * rd.r1 < calm) || gm == amax)) != 0) {
-            float m[8];
-#pragma unroll
-            for (int k = 0; k < 8; k++) { x[k] = ste(t[k], m[k]); m[k] *= gv[k]; }
-            gw[j] = pack8_any(m);                        // (the products are bf16 values)
-            int n = 0;
-#pragma unroll
-            for (int k = 0; k < 8; k++) n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(on && fabsf(u[k]) == amax));
-            ties_n += n;
-            if (n) tied |= 1u << j;
-        }
-#pragma unroll
-        for (int kk = 0; kk < 2; kk++) {
-            float a = acc[j % NC][kk];
-#pragma unroll
-            for (int e = 0; e < 4; e++) a = __builtin_fmaf(gv[4 * kk + e], x[4 * kk + e], a);
-            a = on ? a : acc[j % NC][kk];
-            asm volatile("" : "+v"(a));                  // (here, not behind the last group with every group's values kept until then)
-            acc[j % NC][kk] = a;
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    float dlds;
-    {
-        float d[NC];
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            float a = acc[c][0], b = acc[c][1];
-            a += lane_xor8(a); b += lane_xor8(b);                        // l ^ 16
-            a += lane_xor4(a); b += lane_xor4(b);                        // l ^ 8
-            a += lane_xor2(a); b += lane_xor2(b);                        // l ^ 4
-            a += lane_xor1(a); b += lane_xor1(b);                        // l ^ 2
-            d[c] = a + b;                                                // l ^ 1
-        }
-        if (W == 1) {                                    // half-wave h: chain h >> 2, lanes 16 (h & 3) .. + 15
-            dlds = lane_read(d[0], 0);
-#pragma unroll
-            for (int h = 1; h < 4 * NC; h++) dlds += lane_read(d[h >> 2], 16 * (h & 3));
-            if (NC == 1) dlds += 0.0f;                   // (the absent half-waves' sums)
-        } else {                                         // half-wave h: part h >> 2
-            if ((lane & 15) == 0) sums[wave][lane >> 4] = d[0];
-            if (lane == 0) counts[wave] = ties_n;
-            __syncthreads();
-            const float * sp = sums[wave & ~1];
-            dlds = sp[0];
-#pragma unroll
-            for (int h = 1; h < 8; h++) dlds += sp[h];
-            ties_n = counts[wave & ~1] + counts[wave | 1];
-        }
-    }
+    amax = share_absmax<W>(amax, nan, share.amax, wave);
+    const bool plain = quantize_bwd_w<R, W>(uw, gw, amax, nan, clip, qmax, ln, last_on, wave, share);
     if (W > 1 && row_raw >= M) return;
-    const float coef = s_raw >= 1e-8f ? dlds * clip / (float)qmax / (float)ties_n : 0.0f;
-    bool zero = false;
-#pragma unroll
-    for (int j = 0; j < R; j++) {
-        if (__builtin_expect(tied & (1u << j), 0)) {     // wave-uniform: a row has few such elements
-            float u[8], d[8];
-            unpack8(unknown_words(uw[j]), u); unpack8(unknown_words(gw[j]), d);
-#pragma unroll
-            for (int k = 0; k < 8; k++)
-                if ((j < R - 1 || last_on) && fabsf(u[k]) == amax && u[k] != 0.0f) d[k] += u[k] > 0.0f ? coef : -coef;
-            gw[j] = pack8_any(d);                        // the gradient of the bf16 tensor u
-        }
-        zero |= ln.plain(gw[j].x);
-    }
-    const bool plain = __builtin_amdgcn_ballot_w64(zero) != 0;
 #pragma unroll
     for (int j = 0; j < R; j++) {
         float d[8];
@@ -880,32 +853,157 @@ struct AbTerm {
     CAMX_DEV f32x4 other(int k) const { return unpack_bf16x4(*(const u32x2 *)(wab + k)); }
 };
 
-// One wave per row for rows of at most 1024 values (NR rounds of 256) without projections: a lane holds 16 values instead of the
-// workgroup form's 4, and what every lane computes once per row (the square root, the divisions, the reductions' tails) is spread over
-// four times as many values.
+// ---- block entry, rows of at most 1024 values: a wave per row, four values a lane -----------------------------------------------------
+// Round c of the lane is elements 256 c + 4 slot .. + 3: the elements (the logical threads 4 slot .. + 3) it holds in the RMSNorm's sums, in the
+// quantizer and in the projections, so x and the norm weights are read once and nothing crosses lanes but the rotation. hb: bf16(h), packed,
+// zeros behind the row.
+// u = bf16(H128 . bf16(h)), the row's max |u| without its NaNs, and whether it holds one
 template <int NR>
-__global__ void __launch_bounds__(64) block_entry_fwd_wave(const float * x, const float * nw, float eps, uint16_t * y, float * s, uint16_t * codes, float * rstd_out,
-                                                           int d, float clip, int qmax) {
-    const int row = blockIdx.x, lane = slot_of(threadIdx.x);
-    const float * xr = x + (size_t)row * d;
-    RmsRegSrc<NR> src;                                   // the row and the norm weights in registers: every HBM byte of x crosses once
+CAMX_DEV float entry_rotate(const u32x2 (&hb)[NR], int lane, f32x4 (&u)[NR], bool & nan) {
+    u16x2 most = {0, 0};
+#pragma unroll
+    for (int c = 0; c < NR; c++) {
+        const f32x4 v = scaled4(hadamard128_l4(unpack_bf16x4(hb[c]), lane & 31, false));
+        const u32x2 w = {hw_pk_bf16(v.x, v.y), hw_pk_bf16(v.z, v.w)};
+        u[c] = unpack_bf16x4(w);
+        most = absmax_pk(absmax_pk(most, w.x), w.y);
+    }
+    float m = absmax_of(most);
+    nan = __builtin_amdgcn_ballot_w64(m != m) != 0;
+    if (__builtin_expect(nan, 0)) {
+        m = 0.0f;
+#pragma unroll
+        for (int c = 0; c < NR; c++) m = fmaxf(m, absmax4(u[c]));
+    }
+    return wave_max64(m);
+}
+// values, codes, scale and rstd of a row
+template <int NR>
+CAMX_DEV void entry_row_fwd(const u32x2 (&hb)[NR], int lane, int row, bool stored, uint16_t * y, float * s_out, uint16_t * codes, float rstd, float * rstd_out, int d, float clip, int qmax, bool stream) {
+    f32x4 u[NR];
+    bool nan;
+    const float amax = entry_rotate<NR>(hb, lane, u, nan);
+    const float s = fmaxf(amax * clip / (float)qmax, 1e-8f);
+    const RowScale rs(s, amax, qmax);
+    const bool tame = row_is_tame(rs, amax, nan);
+    if (!stored) return;                                 // (wave-uniform)
+    if (__builtin_expect(tame, 1)) {
+#pragma unroll
+        for (int c = 0; c < NR; c++) u[c] = (f32x4){rintf(u[c].x * rs.rcp), rintf(u[c].y * rs.rcp), rintf(u[c].z * rs.rcp), rintf(u[c].w * rs.rcp)};
+    } else {
+#pragma unroll
+        for (int c = 0; c < NR; c++) u[c] = rs.quant4(u[c]);
+    }
 #pragma unroll
     for (int c = 0; c < NR; c++) {
         const int k = 256 * c + 4 * lane;
-        src.xk[c] = src.wk[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-        if (k < d) { src.xk[c] = __builtin_nontemporal_load((const f32x4 *)(xr + k)); src.wk[c] = *(const f32x4 *)(nw + k); }
+        if (c < NR - 1 || k < d) {
+            if (y) store8(pack_f2bf_x4((f32x4){u[c].x * s, u[c].y * s, u[c].z * s, u[c].w * s}), y + (size_t)row * d + k, stream);
+            if (codes) codes[((size_t)row * d + k) >> 2] = (uint16_t)rs.nibbles4(u[c]);
+        }
     }
+    if (lane == 0) { if (s_out) s_out[row] = s; if (rstd_out) rstd_out[row] = rstd; }          // (last: a wait for later loads waits for these stores too)
+}
+// dh, the gradient of bf16(h), from the packed gradient of the quantized values. The sum of dL/ds keeps the tree of the workgroup form (each
+// of its half-wave sums is one chunk's here: round c holds chunks 2 c and 2 c + 1); a round in which no lane's quotient can round to qmax or holds
+// the row's maximum needs no clamp, no mask and no look for ties (see actq_bwd_wave_k).
+template <int NR>
+CAMX_DEV void entry_row_bwd(const u32x2 (&hb)[NR], const u32x2 (&gy)[NR], int lane, f32x4 (&dh)[NR], int d, float clip, int qmax) {
+    f32x4 u[NR], gv[NR];
+    bool nan;
+    const float amax = entry_rotate<NR>(hb, lane, u, nan);
+    const float s_raw = amax * clip / (float)qmax, s = fmaxf(s_raw, 1e-8f);
+    const Ste ste(qmax);
+    const RowDiv rd(s, amax);
+    const float calm = nan || qmax > 1024 ? -1.0f : ste.hi - 0.51f;
+    float part[NR];
+    int ties_n = 0;
+    uint32_t tied = 0;                                   // bit c: some lane holds a max-|u| element in round c
+#pragma unroll
+    for (int c = 0; c < NR; c++) {
+        const bool on = c < NR - 1 || 256 * c + 4 * lane < d;
+        gv[c] = unpack_bf16x4(gy[c]);
+        const f32x4 t = rd.div4(u[c], on);
+        f32x4 v = {rintf(t.x) - t.x, rintf(t.y) - t.y, rintf(t.z) - t.z, rintf(t.w) - t.w};
+        const float most = fmaxf(fmaxf(fabsf(u[c].x), fabsf(u[c].y)), fmaxf(fabsf(u[c].z), fabsf(u[c].w)));
+        f32x4 g = gv[c];
+        if (__builtin_amdgcn_ballot_w64(on && (!(most * rd.r1 < calm) || most == amax)) != 0) {
+            int n = 0;
+#define D_(e) { float m; v.e = ste(t.e, m); g.e = gv[c].e * m; n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(on && fabsf(u[c].e) == amax)); }
+            CAMX_EACH4(D_)
+#undef D_
+            ties_n += n;
+            if (n) tied |= 1u << c;
+        }
+        float a = 0.0f;
+        a = __builtin_fmaf(gv[c].x, v.x, a); a = __builtin_fmaf(gv[c].y, v.y, a); a = __builtin_fmaf(gv[c].z, v.z, a); a = __builtin_fmaf(gv[c].w, v.w, a);
+        part[c] = on ? a : 0.0f;
+        gv[c] = g;
+    }
+    float dlds = 0.0f;                                   // the eight chunk sums in order (absent chunks add +0, as idle half-waves do)
+#pragma unroll
+    for (int c = 0; c < NR; c++) {
+        const float hs = half32_sum(part[c]);
+        const float even = lane_read(hs, 0), odd = lane_read(hs, 32);
+        dlds = c == 0 ? even : dlds + even;
+        dlds += odd;
+    }
+    if (2 * NR < 8) dlds += 0.0f;
+    const float coef = s_raw >= 1e-8f ? dlds * clip / (float)qmax / (float)ties_n : 0.0f;
+#pragma unroll
+    for (int c = 0; c < NR; c++) {
+        f32x4 e = gv[c];
+        if (__builtin_expect(tied & (1u << c), 0)) {     // wave-uniform: a row has few such elements, most rounds skip this
+#define V_(x) if ((c < NR - 1 || 256 * c + 4 * lane < d) && fabsf(u[c].x) == amax && u[c].x != 0.0f) e.x += u[c].x > 0.0f ? coef : -coef;
+            CAMX_EACH4(V_)
+#undef V_
+        }
+        dh[c] = rbf4_canon(scaled4(hadamard128_l4(rbf4_any(e), lane & 31, false)));      // rbf4_any: the gradient of the bf16 tensor u
+    }
+}
+// bf16(h) of four values, packed
+CAMX_DEV u32x2 rms_pack4(f32x4 v, float rstd, f32x4 w) { return (u32x2){hw_pk_bf16(v.x * rstd * w.x, v.y * rstd * w.y), hw_pk_bf16(v.z * rstd * w.z, v.w * rstd * w.w)}; }
+// sum of squares of the row under the 256-thread tree, from the lane's rounds (padding adds +0)
+template <int NR>
+CAMX_DEV float entry_rstd(const f32x4 (&xk)[NR], int d, float eps) {
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int c = 0; c < NR; c++)
-        if (256 * c + 4 * lane < d) {
-            acc.x = __builtin_fmaf(src.xk[c].x, src.xk[c].x, acc.x); acc.y = __builtin_fmaf(src.xk[c].y, src.xk[c].y, acc.y);
-            acc.z = __builtin_fmaf(src.xk[c].z, src.xk[c].z, acc.z); acc.w = __builtin_fmaf(src.xk[c].w, src.xk[c].w, acc.w);
-        }
-    const float ss = wave_groups_in_order(group32_sum(acc));
-    src.rstd = rsqrt_exact(ss / (float)d + eps);
-    if (threadIdx.x == 0 && rstd_out) rstd_out[row] = src.rstd;
-    actq_fwd_row<NR, RmsRegSrc<NR>, 2>(src, row, y, s, d, clip, qmax, codes, nullptr);
+    for (int c = 0; c < NR; c++) {
+        const f32x4 v = xk[c];
+        acc.x = __builtin_fmaf(v.x, v.x, acc.x); acc.y = __builtin_fmaf(v.y, v.y, acc.y); acc.z = __builtin_fmaf(v.z, v.z, acc.z); acc.w = __builtin_fmaf(v.w, v.w, acc.w);
+    }
+    return rsqrt_exact(wave_groups_in_order(group32_sum(acc)) / (float)d + eps);
+}
+// a lane's rounds of an fp32 row, zeros behind it
+template <int NR>
+CAMX_DEV void entry_load(const float * row, int d, int lane, bool stream, f32x4 (&v)[NR]) {
+#pragma unroll
+    for (int c = 0; c < NR; c++) {
+        const int k = 256 * c + 4 * lane;
+        v[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+        if (c < NR - 1 || k < d) v[c] = stream ? __builtin_nontemporal_load((const f32x4 *)(row + k)) : *(const f32x4 *)(row + k);
+    }
+}
+template <int NR>
+CAMX_DEV void entry_pack(const f32x4 (&xk)[NR], const f32x4 (&wk)[NR], float rstd, int d, int lane, u32x2 (&hb)[NR]) {
+#pragma unroll
+    for (int c = 0; c < NR; c++) {
+        hb[c] = rms_pack4(xk[c], rstd, wk[c]);
+        if (c == NR - 1 && 256 * c + 4 * lane >= d) hb[c] = (u32x2){0u, 0u};            // (0 x an infinite rstd is a NaN, and the projections add the padding's products)
+    }
+}
+// without projections
+template <int NR>
+__global__ void __launch_bounds__(64) block_entry_fwd_wave(const float * x, const float * nw, float eps, uint16_t * y, float * s, uint16_t * codes, float * rstd_out,
+                                                           int d, float clip, int qmax, bool stream) {
+    const int row = blockIdx.x, lane = slot_of(threadIdx.x);
+    f32x4 xk[NR], wk[NR];
+    entry_load<NR>(x + (size_t)row * d, d, lane, true, xk);
+    entry_load<NR>(nw, d, lane, false, wk);
+    const float rstd = entry_rstd<NR>(xk, d, eps);
+    u32x2 hb[NR];
+    entry_pack<NR>(xk, wk, rstd, d, lane, hb);
+    entry_row_fwd<NR>(hb, lane, row, true, y, s, codes, rstd, rstd_out, d, clip, qmax, stream);
 }
 
 // Longer rows: a 256-thread workgroup per row (NR rounds of 1024 values). The projections: wave w takes rows w, w + 4, ... of wab, up to
@@ -968,7 +1066,7 @@ __global__ void __launch_bounds__(256) block_entry_fwd_k(const float * x, const 
 // ---- block entry with projections, rows of at most 1024 values: a wave per row, four rows share the projections on the matrix cores ----
 // Bound by instruction issue: with the projections as vector multiply-adds of a row's own wave, they, the conversions of wab and sixteen
 // reductions of 256 logical threads were two thirds of a row's instructions (32768 rows x 1024 values, 16 projections: 114 us, this
-// kernel 84; 512 rows: 11.6 and 7.0. Four rows in the registers of one wave, wab as fp32 in LDS: 76 and 22). A K = 1 matrix instruction
+// kernel 84; 512 rows: 11.6 and 7.0; large batches with more than four projections: block_entry_fwd_rows16). A K = 1 matrix instruction
 // (v_mfma_f32_4x4x1: 16 blocks of 4 x 4 single multiply-adds, each rounded like fmaf) computes for 16 logical threads t the terms of
 // 4 rows x 4 projections, so a thread's chain over its elements t, t + 256, .. is a chain of NR such instructions in the same order.
 // A workgroup's four waves own a row each and hand bf16(h) on through LDS; then wave w takes projections 4 w .. 4 w + 3 of all four rows.
@@ -980,58 +1078,22 @@ CAMX_DEV f32x4 mirror4(f32x4 v) { return (f32x4){lane_xor4(v.x), lane_xor4(v.y),
 template <int NR>
 __global__ void __launch_bounds__(256, 4) block_entry_fwd_quad(const float * __restrict__ x, const float * __restrict__ nw, const uint16_t * __restrict__ wab, int nab, float eps,
                                                                uint16_t * __restrict__ y, float * __restrict__ s_out, uint16_t * __restrict__ codes, uint16_t * __restrict__ ab,
-                                                               float * __restrict__ rstd_out, int d, float clip, int qmax, int M) {
+                                                               float * __restrict__ rstd_out, int d, float clip, int qmax, int M, bool stream) {
     constexpr int HS = 128 * NR + 4;                     // words of a row of packed pairs; + 4: the four rows of a read fall on different banks
     __shared__ __attribute__((aligned(16))) uint32_t hbuf[4][HS];
     __shared__ __attribute__((aligned(16))) float gsum[4][4 * 4 * 8];         // [wave][row][projection][group]
     const int lraw = threadIdx.x & 63, lane = slot_of(lraw), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int Q = lraw >> 2, odd = Q & 1, jp = odd ? 3 - (lraw & 3) : lraw & 3;      // the lane's block and its projection of the wave's four
-    f32x4 xk[NR], wk[NR];
     const int r0 = 4 * blockIdx.x, row = r0 + wave;
-#pragma unroll
-    for (int c = 0; c < NR; c++) {
-        const int k = 256 * c + 4 * lane;
-        xk[c] = wk[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-        if (c < NR - 1 || k < d) { xk[c] = __builtin_nontemporal_load((const f32x4 *)(x + (size_t)min(row, M - 1) * d + k)); wk[c] = *(const f32x4 *)(nw + k); }
-    }
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int c = 0; c < NR; c++) {                   // (padding adds +0 to a sum of squares)
-        const f32x4 v = xk[c];
-        acc.x = __builtin_fmaf(v.x, v.x, acc.x); acc.y = __builtin_fmaf(v.y, v.y, acc.y); acc.z = __builtin_fmaf(v.z, v.z, acc.z); acc.w = __builtin_fmaf(v.w, v.w, acc.w);
-    }
-    const float ss = wave_groups_in_order(group32_sum(acc));
-    const float rstd = rsqrt_exact(ss / (float)d + eps);
+    f32x4 xk[NR], wk[NR];
+    entry_load<NR>(x + (size_t)min(row, M - 1) * d, d, lane, true, xk);
+    entry_load<NR>(nw, d, lane, false, wk);
+    const float rstd = entry_rstd<NR>(xk, d, eps);
     u32x2 hb[NR];
+    entry_pack<NR>(xk, wk, rstd, d, lane, hb);
 #pragma unroll
-    for (int c = 0; c < NR; c++) {
-        const f32x4 v = xk[c], w = wk[c];
-        hb[c] = (u32x2){hw_pk_bf16(v.x * rstd * w.x, v.y * rstd * w.y), hw_pk_bf16(v.z * rstd * w.z, v.w * rstd * w.w)};
-        if (c == NR - 1 && 256 * c + 4 * lane >= d) hb[c] = (u32x2){0u, 0u};            // (0 x an infinite rstd is a NaN, and the projections add the padding's products)
-        *(u32x2 *)&hbuf[wave][128 * c + 2 * lane] = hb[c];
-    }
-    f32x4 u[NR];
-    float amax = 0.0f;
-#pragma unroll
-    for (int c = 0; c < NR; c++) {
-        u[c] = rbf4_any(scaled4(hadamard128_l4(unpack_bf16x4(hb[c]), lane & 31, false)));
-        amax = fmaxf(fmaxf(amax, fmaxf(fabsf(u[c].x), fabsf(u[c].y))), fmaxf(fabsf(u[c].z), fabsf(u[c].w)));
-    }
-    amax = wave_max64(amax);
-    const float s = fmaxf(amax * clip / (float)qmax, 1e-8f);
-    const RowScale rs(s, amax, qmax);
-    if (row < M) {                                   // (wave-uniform)
-        if (lraw == 0) { if (s_out) s_out[row] = s; if (rstd_out) rstd_out[row] = rstd; }
-#pragma unroll
-        for (int c = 0; c < NR; c++) {
-            const int k = 256 * c + 4 * lane;
-            const f32x4 q = rs.quant4(u[c]);
-            if (c < NR - 1 || k < d) {
-                if (y) *(u32x2 *)(y + (size_t)row * d + k) = pack_f2bf_x4((f32x4){q.x * s, q.y * s, q.z * s, q.w * s});
-                if (codes) codes[((size_t)row * d + k) >> 2] = (uint16_t)rs.nibbles4(q);
-            }
-        }
-    }
+    for (int c = 0; c < NR; c++) *(u32x2 *)&hbuf[wave][128 * c + 2 * lane] = hb[c];
+    entry_row_fwd<NR>(hb, lane, row, row < M, y, s_out, codes, rstd, rstd_out, d, clip, qmax, stream);
     u32x2 B[NR][4];                                      // (from the caches: 32 KiB for a workgroup)
 #pragma unroll
     for (int c = 0; c < NR; c++)
@@ -1082,18 +1144,122 @@ __global__ void __launch_bounds__(256, 4) block_entry_fwd_quad(const float * __r
     }
 }
 
+// ---- block entry, rows of at most 1024 values: two rows a wave, sixteen a workgroup, the projections on the matrix cores ----------------
+// Bound by instruction issue (see actq_fwd_wave_k). A wave reads its rows four values a lane (element 256 c + 4 slot + k: the logical
+// threads of the RMSNorm's sum), hands bf16(h) through LDS to the 16-lane layout of the quantizer, and after a barrier computes one
+// group of 32 logical threads of the projections for all sixteen rows. A K = 1 matrix instruction (v_mfma_f32_16x16x1: four blocks of
+// 16 rows x 16 projections of single multiply-adds, each rounded like fmaf) adds one element of four logical threads, so a thread's chain
+// over its elements t, t + 256, .. is a chain of NR such instructions in the same order: wave w, instruction e, block b is thread
+// 32 w + 8 b + e. A lane's eight elements of a step are 16 bytes of LDS (rows) and of device memory (projections), converted once for
+// sixteen rows. The tree's first steps (t ^ 16, 8) pair blocks, which are registers of the result, the others (t ^ 4, 2, 1) instructions;
+// the eight group sums meet in LDS, where a thread adds them in order.
+// 32768 x 1024 with 16 projections 56.0 us, with 8 54.8; as four rows and four projections a wave 84 and 64. A barrier for the whole
+// workgroup costs what the matrix instructions save where there are four projections (57 us either way) and few workgroups
+// (512 rows: 10.2 us, four rows a workgroup 7.0).
+CAMX_DEV float bf_half(uint32_t v, int odd) { return odd ? bf_hi(v) : bf_lo(v); }
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+CAMX_DEV void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier(); __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront"); }
+// the packed words of a row's rounds of 512 from its words in LDS; chunks behind the row as zeros
+template <int R>
+CAMX_DEV void words_from_lds(const uint32_t * row, int lane, int slot, bool last_on, u32x4 (&w)[R][1]) {
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        w[j][0] = (u32x4){0u, 0u, 0u, 0u};
+        if (j < R - 1 || last_on) w[j][0] = *(const u32x4 *)(row + 256 * j + 64 * (lane >> 4) + 4 * slot);
+    }
+}
+template <int NR>
+__global__ void __launch_bounds__(512, 6) block_entry_fwd_rows16(const float * __restrict__ x, const float * __restrict__ nw, const uint16_t * __restrict__ wab, int nab, float eps,
+                                                              uint16_t * __restrict__ y, float * __restrict__ s_out, uint16_t * __restrict__ codes, uint16_t * __restrict__ ab,
+                                                              float * __restrict__ rstd_out, int d, float clip, int qmax, int M, bool stream) {
+    constexpr int HS = 128 * NR + 4, R = (NR + 1) / 2;   // words of a row of packed pairs; + 4: the sixteen rows of a read fall on different banks
+    __shared__ __attribute__((aligned(16))) uint32_t hbuf[16][HS];
+    __shared__ float gsum[8][16][16];         // [group][row][projection]
+    const int lraw = threadIdx.x & 63, la = slot_of(lraw), slot = la & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r0 = 16 * blockIdx.x;
+    f32x4 xk[2][NR], wk[NR];
+#pragma unroll
+    for (int i = 0; i < 2; i++) entry_load<NR>(x + (size_t)min(r0 + 2 * wave + i, M - 1) * d, d, la, true, xk[i]);
+    entry_load<NR>(nw, d, la, false, wk);
+    float rstd[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        rstd[i] = entry_rstd<NR>(xk[i], d, eps);
+        u32x2 hb[NR];
+        entry_pack<NR>(xk[i], wk, rstd[i], d, la, hb);
+#pragma unroll
+        for (int c = 0; c < NR; c++) *(u32x2 *)&hbuf[2 * wave + i][128 * c + 2 * la] = hb[c];
+    }
+    wave_lds_fence();
+    const Lanes16 ln(slot);
+    const int e0 = 128 * (lraw >> 4) + 8 * slot;
+    const bool last_on = e0 + 512 * (R - 1) < d;
+#pragma unroll 1
+    for (int i = 0; i < 2; i++) {
+        const int row = r0 + 2 * wave + i;
+        u32x4 raw[R][1], uw[R], keep[R];
+        words_from_lds<R>(hbuf[2 * wave + i], lraw, slot, last_on, raw);
+        const u16x2 most = actq_rotate_w<R>(PlainBF16{}, raw, ln, uw, keep);
+        bool nan;
+        const float amax = row_absmax_w<R>(uw, most, nan);
+        const float s = fmaxf(amax * clip / (float)qmax, 1e-8f);
+        if (row < M) {                                   // (wave-uniform)
+            quantize_row_w<R, 1>(uw, amax, nan, s, qmax, e0, last_on, y ? y + (size_t)row * d : nullptr, codes ? codes + (size_t)row * (d / 4) : nullptr, stream);
+            if (lraw == 0) { if (s_out) s_out[row] = s; if (rstd_out) rstd_out[row] = i ? rstd[1] : rstd[0]; }
+        }
+    }
+    const int i16 = lraw & 15, b = lraw >> 4;            // A: row, B: projection; block
+    u32x4 A[NR], B[NR];
+#pragma unroll
+    for (int c = 0; c < NR; c++) {                       // (from the caches: 32 KiB for a workgroup)
+        const int k = 256 * c + 32 * wave + 8 * b;
+        B[c] = (u32x4){0u, 0u, 0u, 0u};
+        if (i16 < nab && (c < NR - 1 || k < d)) B[c] = *(const u32x4_a8 *)(wab + (size_t)i16 * d + k);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < NR; c++) A[c] = *(const u32x4 *)&hbuf[i16][128 * c + 16 * wave + 4 * b];
+    f32x4 t[8];                                          // of instruction e: rows 4 b .. 4 b + 3 of projection i16
+#pragma unroll
+    for (int ee = 0; ee < 8; ee++) {
+        const int e = (ee & 1) * 4 + (ee >> 1 & 1) * 2 + (ee >> 2);          // 0, 4, 2, 6, 1, 5, 3, 7: the pairs of t ^ 4, then of t ^ 2
+        f32x16 a = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int c = 0; c < NR; c++) {
+            const uint32_t av = A[c][e >> 1], bv = B[c][e >> 1];
+            a = __builtin_amdgcn_mfma_f32_16x16x1f32(bf_half(av, e & 1), bf_half(bv, e & 1), a, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);           // (one chain at a time: 80 registers, six waves per SIMD; 110 and 63.4 us otherwise)
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) t[e][r] = (a[r] + a[8 + r]) + (a[4 + r] + a[12 + r]);            // t ^ 16, t ^ 8
+        if (ee & 1) t[e - 4] += t[e];                    // t ^ 4
+        if ((ee & 3) == 3) t[e & 1] += t[(e & 1) + 2];   // t ^ 2
+    }
+    const f32x4 sum = t[0] + t[1];                       // t ^ 1
+#pragma unroll
+    for (int r = 0; r < 4; r++) gsum[wave][4 * b + r][i16] = sum[r];
+    __syncthreads();
+    const int rr = threadIdx.x >> 4, j = threadIdx.x & 15;
+    if (rr < 16 && r0 + rr < M && j < nab) {
+        float tot = 0.0f;
+#pragma unroll
+        for (int g = 0; g < 8; g++) tot += gsum[g][rr][j];
+        ab[(size_t)(r0 + rr) * nab + j] = f2bf(tot);
+    }
+}
+
 // dx = rstd (dh w - xhat mean(dh w xhat)) of one row from the lane's registers
 template <int NR>
-CAMX_DEV void rms_bwd_row(const RmsRegSrc<NR> & src, const f32x4 (&dh)[NR], float * dx, int d, int la) {
+CAMX_DEV void rms_bwd_row(const f32x4 (&xk)[NR], const f32x4 (&wk)[NR], float rstd, const f32x4 (&dh)[NR], float * dx, int d, int la, bool stream) {
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f}, gw[NR], xh[NR];
 #pragma unroll
     for (int c = 0; c < NR; c++) {
         const int k = 256 * c + 4 * la;
         gw[c] = xh[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
         if (c < NR - 1 || k < d) {
-            const f32x4 w = src.wk[c], xv = src.xk[c];
+            const f32x4 w = wk[c], xv = xk[c];
             gw[c] = (f32x4){dh[c].x * w.x, dh[c].y * w.y, dh[c].z * w.z, dh[c].w * w.w};
-            xh[c] = (f32x4){xv.x * src.rstd, xv.y * src.rstd, xv.z * src.rstd, xv.w * src.rstd};
+            xh[c] = (f32x4){xv.x * rstd, xv.y * rstd, xv.z * rstd, xv.w * rstd};
             acc.x = __builtin_fmaf(gw[c].x, xh[c].x, acc.x); acc.y = __builtin_fmaf(gw[c].y, xh[c].y, acc.y);
             acc.z = __builtin_fmaf(gw[c].z, xh[c].z, acc.z); acc.w = __builtin_fmaf(gw[c].w, xh[c].w, acc.w);
         }
@@ -1108,108 +1274,117 @@ CAMX_DEV void rms_bwd_row(const RmsRegSrc<NR> & src, const f32x4 (&dh)[NR], floa
         const int k = 256 * c + 4 * la;
         if (c < NR - 1 || k < d) {
             f32x4 r;
-            r.x = src.rstd * (gw[c].x - xh[c].x * dot); r.y = src.rstd * (gw[c].y - xh[c].y * dot);
-            r.z = src.rstd * (gw[c].z - xh[c].z * dot); r.w = src.rstd * (gw[c].w - xh[c].w * dot);
-            *(f32x4 *)(dx + k) = r;
+            r.x = rstd * (gw[c].x - xh[c].x * dot); r.y = rstd * (gw[c].y - xh[c].y * dot);
+            r.z = rstd * (gw[c].z - xh[c].z * dot); r.w = rstd * (gw[c].w - xh[c].w * dot);
+            store16(__builtin_bit_cast(u32x4, r), dx + k, stream);
         }
     }
 }
-// dh = actq backward of dy, plus the two projection groups' input gradients (wab rows [0, nab / 2) and [nab / 2, nab), each
-// group's sum rounded to bf16); then the RMSNorm backward. d <= 1024. One wave per row, NR = ceil(d / 256) rounds: lane (slot la) holds
-// elements 256 c + 4 la .. + 3 of round c through all steps, i.e. the logical threads 4 la .. 4 la + 3 of the 256-thread tree of the dot
-// product (thread t owns elements t, t + 256, ...). This kernel: no projections.
-struct SinkNone { CAMX_DEV void operator()(int, int, f32x4, u32x2) const {} };
+// a lane's rounds of a bf16 row, zeros behind it
 template <int NR>
-__global__ void __launch_bounds__(64) block_entry_bwd_k(const float * x, const float * nw, const float * rstd_in, const uint16_t * dy, float * dx, int d, float clip, int qmax) {
-    const int row = blockIdx.x, la = slot_of(threadIdx.x);
-    const float rstd = rstd_in[row];
-    const float * xr = x + (size_t)row * d;
-    RmsRegSrc<NR> src;                                   // x and the norm weights once, for the quantizer's source and the RMSNorm backward
+CAMX_DEV void entry_load16(const uint16_t * row, int d, int lane, u32x2 (&v)[NR]) {
 #pragma unroll
     for (int c = 0; c < NR; c++) {
-        const int k = 256 * c + 4 * la;
-        src.xk[c] = src.wk[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-        if (k < d) { src.xk[c] = __builtin_nontemporal_load((const f32x4 *)(xr + k)); src.wk[c] = *(const f32x4 *)(nw + k); }
+        const int k = 256 * c + 4 * lane;
+        v[c] = (u32x2){0u, 0u};
+        if (c < NR - 1 || k < d) v[c] = __builtin_nontemporal_load((const u32x2 *)(row + k));
     }
-    src.rstd = rstd;
-    f32x4 dh[NR];
-    actq_bwd_row<NR, RmsRegSrc<NR>, SinkNone, 2>(src, row, dy, SinkNone{}, d, clip, qmax, nullptr, dh);
-    rms_bwd_row(src, dh, dx + (size_t)row * d, d, la);
+}
+// dh = actq backward of dy, plus the two projection groups' input gradients (wab rows [0, nab / 2) and [nab / 2, nab), each
+// group's sum rounded to bf16); then the RMSNorm backward. d <= 1024. One wave per row, NR = ceil(d / 256) rounds: the lane's elements are
+// the logical threads 4 slot .. 4 slot + 3 of the 256-thread tree of the dot product. This kernel: no projections.
+template <int NR>
+__global__ void __launch_bounds__(64) block_entry_bwd_k(const float * x, const float * nw, const float * rstd_in, const uint16_t * dy, float * dx, int d, float clip, int qmax, bool stream) {
+    const int row = blockIdx.x, la = slot_of(threadIdx.x);
+    const float rstd = rstd_in[row];
+    f32x4 xk[NR], wk[NR], dh[NR];
+    u32x2 gy[NR], hb[NR];
+    entry_load<NR>(x + (size_t)row * d, d, la, true, xk);
+    entry_load<NR>(nw, d, la, false, wk);
+    entry_load16<NR>(dy + (size_t)row * d, d, la, gy);
+    entry_pack<NR>(xk, wk, rstd, d, la, hb);
+    entry_row_bwd<NR>(hb, gy, la, dh, d, clip, qmax);
+    rms_bwd_row<NR>(xk, wk, rstd, dh, dx + (size_t)row * d, d, la, stream);
 }
 
 // The same for nab > 0 with the projections' part on the matrix cores (as vector multiply-adds of the row's own wave 143 us at 32768 x
-// 1024 with 16 projections, this kernel 115; 512 rows: 13.1 and 9.6): a workgroup's four waves own a row each and first compute a quarter
+// 1024 with 16 projections, 90): a workgroup's four waves own a row each and first compute a quarter
 // of that part for all four rows, one of the two groups for half of the column blocks of 256 (32768 x 256 with 4 projections 31.8 us, as
 // one wave per column block 36.4, with vector multiply-adds 34.3). A K = 1 instruction adds one j's term dab[row][j] wab[j][column]
 // (rounded like fmaf) for 4 rows x 64 columns: block Q's four columns are its lanes' own, so with A = dab (lane 4 Q + i: row i) and B = a
 // lane's column of wab, D holds a lane's column with a word per row. The two groups' sums, rounded to bf16, reach the rows' owners
-// through LDS.
+// through LDS. Loads return in order: rows of more than 512 values ask for what the projections need first (it comes from the caches) and for
+// the row and its gradient behind it, so that the projections run while those are on their way (115 -> 101 us at 32768 x 1024; 49.6 -> 52.2 at 32768 x 512); shorter
+// rows have too little to do meanwhile and ask for the row first.
 template <int NR>
 __global__ void __launch_bounds__(256, 4) block_entry_bwd_quad(const float * x, const float * __restrict__ nw, const float * __restrict__ rstd_in, const uint16_t * __restrict__ wab,
-                                                               int nab, const uint16_t * __restrict__ dy, const uint16_t * __restrict__ dab, float * dx, int d, float clip, int qmax, int M) {
+                                                               int nab, const uint16_t * __restrict__ dy, const uint16_t * __restrict__ dab, float * dx, int d, float clip, int qmax, int M, bool stream) {
     __shared__ __attribute__((aligned(16))) uint32_t pbuf[4][2][128 * NR];                // [row][group][pairs of columns]
     const int lraw = threadIdx.x & 63, la = slot_of(lraw), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = nab / 2;
-    RmsRegSrc<NR> src;
-#pragma unroll
-    for (int c = 0; c < NR; c++) {
-        const int k = 256 * c + 4 * la;
-        src.wk[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-        if (c < NR - 1 || k < d) src.wk[c] = *(const f32x4 *)(nw + k);
-    }
     const int r0 = 4 * blockIdx.x;
-    const int row = min(r0 + wave, M - 1);           // (a wave past the end repeats the last row and stores nothing)
-#pragma unroll
-    for (int c = 0; c < NR; c++) {
-        const int k = 256 * c + 4 * la;
-        src.xk[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-        if (c < NR - 1 || k < d) src.xk[c] = __builtin_nontemporal_load((const f32x4 *)(x + (size_t)row * d + k));
-    }
-    src.rstd = rstd_in[row];
+    const int row = min(r0 + wave, M - 1);               // (a wave past the end repeats the last row and stores nothing)
+    constexpr bool LATE = NR >= 3;
+    f32x4 xk[NR], wk[NR];
+    u32x2 gy[NR];
+    if (!LATE) { entry_load<NR>(nw, d, la, false, wk); entry_load<NR>(x + (size_t)row * d, d, la, true, xk); }
     // wave w: group w & 1 of column blocks (w >> 1) and (w >> 1) + 2; of a single block words w >> 1 of each lane's two
     constexpr int NT = (2 * NR + 3) / 4, NP = NR == 1 ? 1 : 2;
     const int h = wave & 1, c0 = NR == 1 ? 0 : wave >> 1, p0 = NR == 1 ? wave >> 1 : 0;
     uint32_t B[NT][8][NP];
+    float av[8];
+    const uint16_t * ar = dab + (size_t)min(r0 + (lraw & 3), M - 1) * nab + h * half;
 #pragma unroll
-    for (int t = 0; t < NT; t++)
+    for (int j = 0; j < 8; j++) {
+        av[j] = 0.0f;
+        if (j < half) av[j] = bf2f(ar[j]);               // (uniform)
+    }
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
+    for (int j = 0; j < 8; j++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
             const int k = 256 * (c0 + 2 * t) + 4 * la;
             const uint16_t * b = wab + (size_t)(h * half + j) * d + k;
             const bool on = j < half && k < d;
             if (NP == 1) B[t][j][0] = on ? ((const uint32_t *)b)[p0] : 0u;
             else { u32x2 v = {0u, 0u}; if (on) v = *(const u32x2 *)b; B[t][j][0] = v.x; B[t][j][NP - 1] = v.y; }
         }
-    const uint16_t * ar = dab + (size_t)min(r0 + (lraw & 3), M - 1) * nab + h * half;
+    if (LATE) { entry_load<NR>(x + (size_t)row * d, d, la, true, xk); entry_load<NR>(nw, d, la, false, wk); entry_load16<NR>(dy + (size_t)row * d, d, la, gy); }
+    const float rstd = rstd_in[row];
+    f32x4 acc[NT][2 * NP];                               // (half >= 1: the first term opens the sums)
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        if (j == 0 || j < half) {                        // (uniform)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int k = 0; k < 2 * NP; k++) {
+                    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                    acc[t][k] = __builtin_amdgcn_mfma_f32_4x4x1f32(av[j], k & 1 ? bf_hi(B[t][j][k >> 1]) : bf_lo(B[t][j][k >> 1]), j ? acc[t][k] : zero, 0, 0, 0);
+                }
+        }
+    }
 #pragma unroll
     for (int t = 0; t < NT; t++) {
         const int cb = c0 + 2 * t;
         if (cb >= NR) break;                             // (uniform)
-        f32x4 acc[2 * NP];
-#pragma unroll
-        for (int k = 0; k < 2 * NP; k++) acc[k] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            if (j < half) {                              // (uniform)
-                const float av = bf2f(ar[j]);
-#pragma unroll
-                for (int k = 0; k < 2 * NP; k++) acc[k] = __builtin_amdgcn_mfma_f32_4x4x1f32(av, k & 1 ? bf_hi(B[t][j][k >> 1]) : bf_lo(B[t][j][k >> 1]), acc[k], 0, 0, 0);
-            }
-        }
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            if (NP == 1) pbuf[r][h][2 * la + p0] = pack_f2bf_x4((f32x4){acc[0][r], acc[1][r], 0.0f, 0.0f}).x;
-            else *(u32x2 *)&pbuf[r][h][128 * cb + 2 * la] = pack_f2bf_x4((f32x4){acc[0][r], acc[1][r], acc[2 * NP - 2][r], acc[2 * NP - 1][r]});
+            if (NP == 1) pbuf[r][h][2 * la + p0] = pack_f2bf_x4((f32x4){acc[t][0][r], acc[t][1][r], 0.0f, 0.0f}).x;
+            else *(u32x2 *)&pbuf[r][h][128 * cb + 2 * la] = pack_f2bf_x4((f32x4){acc[t][0][r], acc[t][1][r], acc[t][2 * NP - 2][r], acc[t][2 * NP - 1][r]});
         }
     }
+    if (!LATE) entry_load16<NR>(dy + (size_t)row * d, d, la, gy);
+    u32x2 hb[NR];
+    entry_pack<NR>(xk, wk, rstd, d, la, hb);
     f32x4 dh[NR];
-    actq_bwd_row<NR, RmsRegSrc<NR>, SinkNone, 2>(src, row, dy, SinkNone{}, d, clip, qmax, nullptr, dh);
+    entry_row_bwd<NR>(hb, gy, la, dh, d, clip, qmax);
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < NR; c++) {
         const f32x4 ra = unpack_bf16x4(*(const u32x2 *)&pbuf[wave][0][128 * c + 2 * la]), rb = unpack_bf16x4(*(const u32x2 *)&pbuf[wave][1][128 * c + 2 * la]);
         dh[c].x = (dh[c].x + ra.x) + rb.x; dh[c].y = (dh[c].y + ra.y) + rb.y; dh[c].z = (dh[c].z + ra.z) + rb.z; dh[c].w = (dh[c].w + ra.w) + rb.w;
     }
-    if (r0 + wave < M) rms_bwd_row(src, dh, dx + (size_t)row * d, d, la);
+    if (r0 + wave < M) rms_bwd_row<NR>(xk, wk, rstd, dh, dx + (size_t)row * d, d, la, stream);
 }
 
 __attribute__((visibility("hidden"))) int silu_luts_get(hipStream_t st, const uint16_t ** lut, const uint16_t ** small);       // quant.hip
@@ -1305,23 +1480,21 @@ int camx_block_entry_fwd(const float * x, const float * nw, const uint16_t * wab
     if (!x || !nw || (!y && !codes) || actq_check(d, qmax, M) || nab < 0 || nab > 16 || (nab && (!wab || !ab)) || ((uintptr_t)x & 15) ||
         ((uintptr_t)nw & 15) || ((uintptr_t)wab & 7) || ((uintptr_t)y & 7) || ((uintptr_t)codes & 1)) return CAMX_EINVAL;
     if (M == 0) return CAMX_OK;
-    if (d <= 1024 && nab > 0) {                          // four rows share the projections on the matrix cores
-        const dim3 grid((unsigned)(((long)M + 3) / 4)), block(256);
-        switch ((d + 255) / 256) {
-            case 1: block_entry_fwd_quad<1><<<grid, block, 0, st>>>(x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax, M); break;
-            case 2: block_entry_fwd_quad<2><<<grid, block, 0, st>>>(x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax, M); break;
-            case 3: block_entry_fwd_quad<3><<<grid, block, 0, st>>>(x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax, M); break;
-            default: block_entry_fwd_quad<4><<<grid, block, 0, st>>>(x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax, M); break;
+    if (d <= 1024) {                                     // rounds of 256 values
+        const bool stream = (long)M * d >= (1L << 20);
+#define ENTRY_ROUNDS(KERNEL, GRID, BLOCK, ...)                                                                          \
+        switch ((d + 255) / 256) {                                                                                      \
+            case 1: KERNEL<1><<<dim3((unsigned)(GRID)), dim3(BLOCK), 0, st>>>(__VA_ARGS__); break;                      \
+            case 2: KERNEL<2><<<dim3((unsigned)(GRID)), dim3(BLOCK), 0, st>>>(__VA_ARGS__); break;                      \
+            case 3: KERNEL<3><<<dim3((unsigned)(GRID)), dim3(BLOCK), 0, st>>>(__VA_ARGS__); break;                      \
+            default: KERNEL<4><<<dim3((unsigned)(GRID)), dim3(BLOCK), 0, st>>>(__VA_ARGS__); break;                     \
         }
-        CAMX_LAUNCH_RET();
-    }
-    if (d <= 1024) {                                     // one wave per row, rounds of 256 values
-        switch ((d + 255) / 256) {
-            case 1: block_entry_fwd_wave<1><<<dim3(M), dim3(64), 0, st>>>(x, nw, eps, y, s, codes, rstd_out, d, clip, qmax); break;
-            case 2: block_entry_fwd_wave<2><<<dim3(M), dim3(64), 0, st>>>(x, nw, eps, y, s, codes, rstd_out, d, clip, qmax); break;
-            case 3: block_entry_fwd_wave<3><<<dim3(M), dim3(64), 0, st>>>(x, nw, eps, y, s, codes, rstd_out, d, clip, qmax); break;
-            default: block_entry_fwd_wave<4><<<dim3(M), dim3(64), 0, st>>>(x, nw, eps, y, s, codes, rstd_out, d, clip, qmax); break;
-        }
+        // sixteen rows share the projections, whatever their number, or four rows in steps of four projections; a sixteen-row workgroup has to
+        // come often enough to fill the chip. 16 projections at 4096 x 1024: 12.5 us, four rows a workgroup 14.5, at 2048 rows 10.9 and 9.6; 8 at
+        // 8192 x 1024 19.6 and 20.9, at 4096 x 640 10.4 and 9.9; 4 at 32768 x 1024 58 and 57
+        if (nab > 4 && M >= (nab > 8 ? 4096 : 8192)) { ENTRY_ROUNDS(block_entry_fwd_rows16, ((long)M + 15) / 16, 512, x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax, M, stream) }
+        else if (nab > 0) { ENTRY_ROUNDS(block_entry_fwd_quad, ((long)M + 3) / 4, 256, x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax, M, stream) }
+        else { ENTRY_ROUNDS(block_entry_fwd_wave, M, 64, x, nw, eps, y, s, codes, rstd_out, d, clip, qmax, stream) }
         CAMX_LAUNCH_RET();
     }
     ACTQ_ROUNDS(d, (block_entry_fwd_k<NR><<<dim3(M), dim3(256), 0, st>>>(x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax)))
@@ -1363,22 +1536,10 @@ int camx_block_entry_bwd(const float * x, const float * nw, const float * rstd, 
     if (!x || !nw || !rstd || !dy || !dx || actq_check(d, qmax, M) || d > 1024 || nab < 0 || nab > 16 || (nab & 1) || (nab && (!wab || !dab)) ||
         ((uintptr_t)x & 15) || ((uintptr_t)nw & 15) || ((uintptr_t)dy & 7) || ((uintptr_t)dx & 15) || ((uintptr_t)wab & 7)) return CAMX_EINVAL;
     if (M == 0) return CAMX_OK;
-    if (nab > 0) {                                       // four rows share the projections' part on the matrix cores
-        const dim3 grid((unsigned)(((long)M + 3) / 4)), block(256);
-        switch ((d + 255) / 256) {
-            case 1: block_entry_bwd_quad<1><<<grid, block, 0, st>>>(x, nw, rstd, wab, nab, dy, dab, dx, d, clip, qmax, M); break;
-            case 2: block_entry_bwd_quad<2><<<grid, block, 0, st>>>(x, nw, rstd, wab, nab, dy, dab, dx, d, clip, qmax, M); break;
-            case 3: block_entry_bwd_quad<3><<<grid, block, 0, st>>>(x, nw, rstd, wab, nab, dy, dab, dx, d, clip, qmax, M); break;
-            default: block_entry_bwd_quad<4><<<grid, block, 0, st>>>(x, nw, rstd, wab, nab, dy, dab, dx, d, clip, qmax, M); break;
-        }
-        CAMX_LAUNCH_RET();
-    }
-    switch ((d + 255) / 256) {
-        case 1: block_entry_bwd_k<1><<<dim3(M), dim3(64), 0, st>>>(x, nw, rstd, dy, dx, d, clip, qmax); break;
-        case 2: block_entry_bwd_k<2><<<dim3(M), dim3(64), 0, st>>>(x, nw, rstd, dy, dx, d, clip, qmax); break;
-        case 3: block_entry_bwd_k<3><<<dim3(M), dim3(64), 0, st>>>(x, nw, rstd, dy, dx, d, clip, qmax); break;
-        default: block_entry_bwd_k<4><<<dim3(M), dim3(64), 0, st>>>(x, nw, rstd, dy, dx, d, clip, qmax); break;
-    }
+    const bool stream = (long)M * d >= (1L << 20);
+    if (nab > 0) { ENTRY_ROUNDS(block_entry_bwd_quad, ((long)M + 3) / 4, 256, x, nw, rstd, wab, nab, dy, dab, dx, d, clip, qmax, M, stream) }       // four rows share the projections' part
+    else { ENTRY_ROUNDS(block_entry_bwd_k, M, 64, x, nw, rstd, dy, dx, d, clip, qmax, stream) }
+#undef ENTRY_ROUNDS
     CAMX_LAUNCH_RET();
 }
 

@@ -318,6 +318,21 @@ def test_actq_rounds_and_waves_of_a_row(K, streams):
         assert bits_equal(host(dx, np.uint16) if bf else host(dx), want)
 
 
+@pytest.mark.parametrize('M,d,nab,eps', [(4097, 1024, 16, 1e-6), (4111, 384, 10, 0.0), (4096, 128, 9, 1e-6), (8193, 640, 6, 0.0), (8207, 512, 8, 1e-6), (4100, 896, 13, 0.0)])
+def test_block_entry_fwd_sixteen_rows_a_workgroup(M, d, nab, eps):
+    """batches whose projections are shared by sixteen rows: last workgroups of 1, 15, 0, 1, 15 and 4 rows, every number of rounds, and rows of
+    zeros (with eps = 0 an infinite rstd), an infinity and a NaN beside ordinary ones"""
+    rng = np.random.default_rng(900 + d + nab)
+    x = outliers(rng, (M, d)); x[M - 2] = 0; x[5] = 0; x[17, 3] = np.inf; x[40, d - 1] = np.nan
+    nw = (1 + 0.1 * rng.standard_normal(d)).astype(np.float32); wab = O.f2bf(rng.standard_normal((nab, d)) * 0.05)
+    with np.errstate(all='ignore'): ry, rs, rc, rab, rstd = O.block_entry_fwd(x, nw, wab, eps)
+    y = dev(np.zeros((M, d), np.uint16)); s = dev(np.zeros(M, np.float32)); c = dev(np.zeros((M, d // 2), np.uint8))
+    ab = dev(np.zeros((M, nab), np.uint16)); rstd_d = dev(np.zeros(M, np.float32))
+    call('camx_block_entry_fwd', ptr(dev(x)), ptr(dev(nw)), ptr(dev(wab)), I(nab), F(eps), ptr(y), ptr(s), ptr(c), ptr(ab), ptr(rstd_d), I(d), F(1.0), I(7), I(M))
+    assert bits_equal(host(rstd_d), rstd) and bits_equal(host(s), rs) and bits_equal(host(c), rc) and bits_equal(host(y, np.uint16), ry)
+    assert bits_equal(host(ab, np.uint16), rab)
+
+
 @pytest.mark.parametrize('K', [128, 640, 2048])
 def test_actq_signs_of_zeros(K):
     """rows whose chunks begin with -0: the sign of a zero result comes through the rotation of the wave-per-row kernels (all zeros of one
