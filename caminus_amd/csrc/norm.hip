@@ -28,7 +28,6 @@ struct NormArgs {
     float * scl;             // optional row scale [rows]
     int N, rows;
     const float * inj; int HC; float rs;   // ADD_HC only
-    int row0;                // set by the launcher: first row of this launch (a batch may be split into a bulk launch and a tail)
     int stream;              // set by the launcher for large batches: h / h16 leave as non-temporal stores (the consumer of a decode-sized batch finds them in cache instead)
 };
 
@@ -38,7 +37,8 @@ struct NormArgs {
 // OUT != 0 is the chunk form for batches that stream from HBM: the set of copies is fixed at compile time (NORM_* bits, so
 // no branch stands in the store loop either), every access is non-temporal, the requests of a row leave a short pause apart,
 // and gamma waits in LDS instead of registers: GL == 1 one copy per workgroup (one gamma row for all), GL == 2 one row per
-// wave (row r uses gamma row r % wr). The launcher gives these forms whole workgroups only.
+// wave (row r uses gamma row r % wr). A wave past the last row repeats it and stores nothing (as a launch of its own the last rows
+// cost 4 to 10 us: 777 x 5120 14.3 us in two launches).
 enum { NORM_H = 1, NORM_H16 = 2, NORM_HBF = 4, NORM_Q8 = 8, NORM_SCL = 16 };
 #define CAMX_ISSUE_GAP() do { if (OUT) { __builtin_amdgcn_sched_barrier(0); __builtin_amdgcn_s_sleep(1); __builtin_amdgcn_sched_barrier(0); } } while (0)
 // SPLIT (a batch too small to fill the chip, with a q8_1 copy): a workgroup per row. Every wave loads the row and walks the same
@@ -49,8 +49,10 @@ __global__ void __launch_bounds__(256) add_rms_rows(NormArgs a) {
     static_assert(OUT == 0 ? GL == 0 : (EXACT && !SPLIT), "the chunk form is straight-line code");
     extern __shared__ __attribute__((aligned(16))) float gsh[];
     const int lraw = threadIdx.x & 63, lane = slot_of(lraw), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int row = a.row0 + (SPLIT ? blockIdx.x : blockIdx.x * 4 + wave);
-    if (!OUT && row >= a.rows) return;
+    const int row_raw = SPLIT ? blockIdx.x : blockIdx.x * 4 + wave;
+    if (!OUT && row_raw >= a.rows) return;
+    const bool live = !OUT || row_raw < a.rows;              // (wave-uniform)
+    const int row = live ? row_raw : a.rows - 1;
     auto mine = [&](int j) { return !SPLIT || (j & 3) == wave; };
     const int N = EXACT ? NI_MAX * 256 : a.N, ni = EXACT ? NI_MAX : N >> 8;
     if (GL == 1) {
@@ -155,7 +157,7 @@ __global__ void __launch_bounds__(256) add_rms_rows(NormArgs a) {
             if (j < ni && mine(j)) g[j] = *(const f32x4 *)(gw + 256 * j + 4 * lane);
     }
     if (SPLIT) __syncthreads();                   // every wave of the row has its loads back before any of them writes (x in place; h may be x)
-    if (ADD == ADD_HC || (ADD == ADD_F32_SLOTS && a.S > 0) || ((ADD == ADD_F32_DIRECT || ADD == ADD_BF16) && a.d)) {
+    if (live && (ADD == ADD_HC || (ADD == ADD_F32_SLOTS && a.S > 0) || ((ADD == ADD_F32_DIRECT || ADD == ADD_BF16) && a.d))) {
         // the updated residual goes back to the lines it was read from
 #pragma unroll
         for (int j = 0; j < NI_MAX; j++)
@@ -171,11 +173,12 @@ __global__ void __launch_bounds__(256) add_rms_rows(NormArgs a) {
         }
     const float tot = wave_groups_in_order(group32_sum(ss));
     const float scale = rsqrt_exact(tot / (float)N + a.eps);
-    if ((OUT ? (OUT & NORM_SCL) != 0 : a.scl != nullptr) && lane == 0 && (!SPLIT || wave == 0)) a.scl[row] = scale;
+    if (live && (OUT ? (OUT & NORM_SCL) != 0 : a.scl != nullptr) && lane == 0 && (!SPLIT || wave == 0)) a.scl[row] = scale;
     if (GL) {
         __builtin_amdgcn_s_waitcnt(0x0f70);       // vmcnt(0): this wave's gamma pieces have landed in LDS (they were first in the queue)
         if (GL == 1) __syncthreads();
     }
+    if (OUT && !live) return;
     const float * gl = gsh + (GL == 2 ? wave * N : 0);
     // (two copies of the loop, chosen once: with the choice inside it the stores of a long row were no longer issued back to back)
     auto emit = [&](auto nt, auto redo) {
@@ -221,7 +224,7 @@ __global__ void __launch_bounds__(256) add_rms_rows(NormArgs a) {
 template <int ADD>
 __global__ void __launch_bounds__(256) add_rms_rows_any(NormArgs a) {
     const int lane = slot_of(threadIdx.x & 63);
-    const int row = a.row0 + blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (row >= a.rows) return;
     const int N = a.N;
     float * xr = a.x + (size_t)row * N;
@@ -283,13 +286,14 @@ __global__ void __launch_bounds__(256) add_rms_rows_any(NormArgs a) {
 // and the last part forms the row's total with the same tree. Gamma comes straight into registers (a wave needs NS slabs of it).
 template <int NS, int W, int ADD, int OUT>
 __global__ void __launch_bounds__(256) add_rms_rows_div(NormArgs a) {
-    static_assert(ADD == ADD_NONE || ADD == ADD_F32_SLOTS || ADD == ADD_F32_DIRECT, "the addends of the row kernels");
+    static_assert(ADD != ADD_HC, "the addends of the row kernels");
     constexpr int N = NS * W * 256, RPW = 4 / W;
     __shared__ __attribute__((aligned(16))) float chain[RPW][256];
     __shared__ float totsh[RPW];
     const int lraw = threadIdx.x & 63, lane = slot_of(lraw), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int rw = wave / W, part = wave % W;
-    const int row = a.row0 + blockIdx.x * RPW + rw;
+    const bool live = (int)(blockIdx.x * RPW) + rw < a.rows;     // (wave-uniform)
+    const int row = live ? blockIdx.x * RPW + rw : a.rows - 1;
     const int e0 = part * (NS * 256) + 4 * lane;                        // this lane's first element of the row
     float * xr = a.x + (size_t)row * N + e0;
     f32x4 xv[NS];
@@ -328,11 +332,20 @@ __global__ void __launch_bounds__(256) add_rms_rows_div(NormArgs a) {
         for (int j = 0; j < NS; j++) xv[j] = xv[j] + dv[j];
         added = true;
     }
+    if (ADD == ADD_BF16 && a.d) {
+        const uint16_t * dr = (const uint16_t *)a.d + (size_t)row * N + e0;
+        u32x2 dv[NS];
+#pragma unroll
+        for (int j = 0; j < NS; j++) dv[j] = __builtin_nontemporal_load((const u32x2 *)(dr + 256 * j));
+#pragma unroll
+        for (int j = 0; j < NS; j++) xv[j] = xv[j] + unpack_bf16x4(dv[j]);
+        added = true;
+    }
     const float * gw = a.nw + (size_t)(row % a.wr) * N + e0;
     f32x4 g[NS];
 #pragma unroll
     for (int j = 0; j < NS; j++) g[j] = *(const f32x4 *)(gw + 256 * j);
-    if (added) {
+    if (added && live) {
 #pragma unroll
         for (int j = 0; j < NS; j++) __builtin_nontemporal_store(xv[j], (f32x4 *)(xr + 256 * j));
     }
@@ -351,6 +364,7 @@ __global__ void __launch_bounds__(256) add_rms_rows_div(NormArgs a) {
         }
         __syncthreads();
     }
+    if (!live) return;
     const float scale = rsqrt_exact(totsh[rw] / (float)N + a.eps);
     if ((OUT & NORM_SCL) && part == 0 && lane == 0) a.scl[row] = scale;
     auto emit = [&](auto redo) {
@@ -383,46 +397,46 @@ __global__ void __launch_bounds__(256) add_rms_rows_div(NormArgs a) {
     if ((OUT & NORM_HBF) && __builtin_expect(__builtin_amdgcn_ballot_w64(nan) != 0, 0)) emit(std::true_type{});
 }
 template <int ADD, int OUT>
-static int launch_norm_div(const NormArgs & a, hipStream_t st) {
-    if constexpr (ADD == ADD_NONE || ADD == ADD_F32_SLOTS || ADD == ADD_F32_DIRECT) {
+static bool launch_norm_div(const NormArgs & a, hipStream_t st) {
+    if constexpr (ADD != ADD_HC) {
         // Measured against the wave-per-row chunk form (cold lines): with a q8_1 copy 23.1 -> 22.2 us at 4096 x 2048 (the encode behind the
         // reduction is a quarter as long per wave), 2560-wide rows over two waves 24.3 -> 23.4 us at 8192 rows, and 1.5 - 2 % from 16384 rows on;
-        // q3p_add_rms16 at 4096 x 2048 is slower this way (26.7 -> 28.3 us) and keeps the wave per row.
+        // q3p_add_rms16 at 4096 x 2048 is slower this way (26.7 -> 28.3 us) and keeps the wave per row. Batches whose rows as a wave each
+        // leave the chip half empty: 5120-wide rows with a bf16 addend 512 rows 6.4 us (a wave per row: chunk form 7.7, general form 9.9), 640 rows 8.9
+        // (8.2, 10.8); with fp32 addend and copies 8.0 (9.7, 10.9) and 12.3 (10.6, 12.0); eight slots of 2048 512 rows 9.7 (15.2, 11.8), 1023 rows
+        // 16.4 (-, 17.6), 1024 rows 17.0 (19.8, -), 2048 rows 33.6 (32.6).
         const int ni = a.N >> 8;
-        if (!((OUT & NORM_Q8) || ni == 10 || a.rows >= 16384)) return 0;
-        const int w = ni == 10 ? 2 : 4, rpw = 4 / w, rows = a.rows - a.rows % rpw;
-        if (rows == 0) return 0;
-        NormArgs b = a; b.rows = rows;
-        const dim3 grid(rows / rpw), block(256);
+        if (!((OUT & NORM_Q8) || ni == 10 || a.rows >= 16384 || a.rows < (ADD == ADD_F32_SLOTS ? 2048 : 600))) return false;
+        const int w = ni == 10 ? 2 : 4, rpw = 4 / w;
+        const dim3 grid((a.rows + rpw - 1) / rpw), block(256);
         switch (ni) {
-        case 4: add_rms_rows_div<1, 4, ADD, OUT><<<grid, block, 0, st>>>(b); return rows;
-        case 8: add_rms_rows_div<2, 4, ADD, OUT><<<grid, block, 0, st>>>(b); return rows;
-        case 10: add_rms_rows_div<5, 2, ADD, OUT><<<grid, block, 0, st>>>(b); return rows;
-        case 16: add_rms_rows_div<4, 4, ADD, OUT><<<grid, block, 0, st>>>(b); return rows;
-        case 20: add_rms_rows_div<5, 4, ADD, OUT><<<grid, block, 0, st>>>(b); return rows;
+        case 4: add_rms_rows_div<1, 4, ADD, OUT><<<grid, block, 0, st>>>(a); return true;
+        case 8: add_rms_rows_div<2, 4, ADD, OUT><<<grid, block, 0, st>>>(a); return true;
+        case 10: add_rms_rows_div<5, 2, ADD, OUT><<<grid, block, 0, st>>>(a); return true;
+        case 16: add_rms_rows_div<4, 4, ADD, OUT><<<grid, block, 0, st>>>(a); return true;
+        case 20: add_rms_rows_div<5, 4, ADD, OUT><<<grid, block, 0, st>>>(a); return true;
         }
     }
-    return 0;
+    return false;
 }
 
-// The chunk form of add_rms_rows for one set of copies, if the launch fits it: returns the rows it took (whole workgroups).
+// The chunk form of add_rms_rows for one set of copies, if the launch fits it
 template <int ADD, int OUT>
-static int launch_norm_chunk(const NormArgs & a, hipStream_t st) {
-    const int rows = a.rows & ~3, ni = a.N >> 8, gl = a.wr == 1 ? 1 : 2;
-    if (gl == 2 && a.N > 2560) return 0;          // (a gamma row per wave: 4 N floats of LDS per workgroup)
-    const dim3 grid(rows / 4), block(256);
+static bool launch_norm_chunk(const NormArgs & a, hipStream_t st) {
+    const int ni = a.N >> 8, gl = a.wr == 1 ? 1 : 2;
+    if (gl == 2 && a.N > 2560) return false;      // (a gamma row per wave: 4 N floats of LDS per workgroup)
+    const dim3 grid((a.rows + 3) / 4), block(256);
     const size_t lds = (size_t)(gl == 1 ? 1 : 4) * a.N * sizeof(float);
-    NormArgs b = a; b.rows = rows;
     switch (ni) {
 #define CAMX_NORM_CHUNK(NI) case NI: \
-        if (gl == 1) add_rms_rows<NI, ADD, true, OUT, 1><<<grid, block, lds, st>>>(b); \
-        else if constexpr (ADD == ADD_NONE || ADD == ADD_HC) { if constexpr (NI <= 10) add_rms_rows<NI, ADD, true, OUT, 2><<<grid, block, lds, st>>>(b); } \
-        else return 0; \
-        return rows;
+        if (gl == 1) add_rms_rows<NI, ADD, true, OUT, 1><<<grid, block, lds, st>>>(a); \
+        else if constexpr (ADD == ADD_NONE || ADD == ADD_HC) { if constexpr (NI <= 10) add_rms_rows<NI, ADD, true, OUT, 2><<<grid, block, lds, st>>>(a); } \
+        else return false; \
+        return true;
         CAMX_NORM_CHUNK(4) CAMX_NORM_CHUNK(8) CAMX_NORM_CHUNK(10) CAMX_NORM_CHUNK(16) CAMX_NORM_CHUNK(20)
 #undef CAMX_NORM_CHUNK
     }
-    return 0;
+    return false;
 }
 
 // CHUNK_OUTS: the sets of copies (NORM_* masks) this entry point's prefill callers ask for; a batch that streams from HBM
@@ -431,21 +445,17 @@ template <int ADD, int... CHUNK_OUTS>
 static int launch_norm(const NormArgs & a0, hipStream_t st) {
     if (a0.rows <= 0) return CAMX_OK;
     NormArgs a = a0;
-    a.row0 = 0;
     a.stream = (long)a.rows * a.N >= (1L << 20);
     const int ni = a.N >> 8;
     const bool vec = (a.N & 255) == 0 && ni <= 32 && (a.ld16 & 3) == 0 &&
                      ((uintptr_t)a.x & 15) == 0 && ((uintptr_t)a.nw & 15) == 0 && ((uintptr_t)a.d & 15) == 0 && ((uintptr_t)a.h & 15) == 0 &&
                      ((uintptr_t)a.h16 & 7) == 0 && ((uintptr_t)a.hbf & 7) == 0 && ((uintptr_t)a.q8 & 3) == 0;
-    if (vec && a.stream && a.rows >= 1024 && (ADD == ADD_NONE || ADD == ADD_HC || a.d)) {
+    // (257 to 1023 rows with a q8_1 copy, and without an addend: the forms below)
+    if (vec && a.stream && a.rows > 256 && (a.rows >= 1024 || (a.d && !a.q8)) && (ADD == ADD_NONE || ADD == ADD_HC || a.d)) {
         const int mask = (a.h ? NORM_H : 0) | (a.h16 ? NORM_H16 : 0) | (a.hbf ? NORM_HBF : 0) | (a.q8 ? NORM_Q8 : 0) | (a.scl ? NORM_SCL : 0);
-        int done = 0;
-        (void)((mask == CHUNK_OUTS && ((done = launch_norm_div<ADD, CHUNK_OUTS>(a, st)) || (done = launch_norm_chunk<ADD, CHUNK_OUTS>(a, st)), true)) || ...);
-        if (done) {
-            const hipError_t e = hipGetLastError();
-            if (e != hipSuccess || done == a.rows) return (int)e;
-            a.row0 = done;                        // the last rows % 4 rows
-        }
+        bool done = false;
+        (void)((mask == CHUNK_OUTS && (done = launch_norm_div<ADD, CHUNK_OUTS>(a, st) || launch_norm_chunk<ADD, CHUNK_OUTS>(a, st), true)) || ...);
+        if (done) CAMX_LAUNCH_RET();
     }
     const dim3 block(256);
     // a workgroup per row: up to 1024 rows when a q8_1 copy follows the reduction, else up to 256 (5120-wide rows: 7.3 us against 8.7 for
@@ -458,7 +468,7 @@ static int launch_norm(const NormArgs & a0, hipStream_t st) {
 #undef CAMX_NORM_SPLIT
         }
     }
-    const dim3 grid((a.rows - a.row0 + 3) / 4);
+    const dim3 grid((a.rows + 3) / 4);
     if (!vec) add_rms_rows_any<ADD><<<grid, block, 0, st>>>(a);
     else switch (ni) {
 #define CAMX_NORM_EXACT(NI) case NI: add_rms_rows<NI, ADD, true><<<grid, block, 0, st>>>(a); break;
@@ -480,14 +490,15 @@ static int launch_norm(const NormArgs & a0, hipStream_t st) {
 // pause apart, before the first dependent instruction; the residual goes back as soon as it is summed, and the bf16 rows are
 // packed by the hardware convert and stored without a branch in the loop (a row that produced a NaN is redone with the
 // reference's integer rounding, which has no NaN case). A wave's reads and writes are two separate bursts: HBM serves a read
-// burst and a write burst faster than an interleaved stream. rows % 4 == 0 (no partial workgroup).
+// burst and a write burst faster than an interleaved stream. A wave past the last row repeats it and stores nothing.
 template <int NI>
 __global__ void __launch_bounds__(256) add_rms_bf16_chunk(float * __restrict__ x, const uint16_t * __restrict__ d, const float * __restrict__ nw, float eps,
-                                                          uint16_t * __restrict__ hbf) {
+                                                          uint16_t * __restrict__ hbf, int rows) {
     extern __shared__ __attribute__((aligned(16))) float gsh[];
     constexpr int N = NI * 256;
     const int lraw = threadIdx.x & 63, lane = slot_of(lraw), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const size_t row = (size_t)blockIdx.x * 4 + wave;
+    const bool live = (int)blockIdx.x * 4 + wave < rows;                 // (wave-uniform)
+    const size_t row = live ? (int)blockIdx.x * 4 + wave : rows - 1;
 #pragma unroll
     for (int j = wave; j < NI; j += 4)      // gamma piece j (1 KiB) -> LDS in lane order; read back in slot order below
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(nw + 256 * j + 4 * lraw), (__attribute__((address_space(3))) void *)(gsh + 256 * j), 16, 0, 0);
@@ -509,8 +520,10 @@ __global__ void __launch_bounds__(256) add_rms_bf16_chunk(float * __restrict__ x
         if (HB < NI) __builtin_amdgcn_sched_barrier(0);
     }
 #undef CAMX_ISSUE_GAP
+    if (live) {
 #pragma unroll
-    for (int j = 0; j < NI; j++) __builtin_nontemporal_store(xv[j], (f32x4 *)(xr + 256 * j + 4 * lane));
+        for (int j = 0; j < NI; j++) __builtin_nontemporal_store(xv[j], (f32x4 *)(xr + 256 * j + 4 * lane));
+    }
     f32x4 ss = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int j = 0; j < NI; j++) {
@@ -521,6 +534,7 @@ __global__ void __launch_bounds__(256) add_rms_bf16_chunk(float * __restrict__ x
     const float scale = rsqrt_exact(tot / (float)N + eps);
     __builtin_amdgcn_s_waitcnt(0x0f70);       // vmcnt(0): this wave's gamma pieces have landed in LDS (they were first in the queue)
     __syncthreads();
+    if (!live) return;
     uint16_t * hr = hbf + row * N;
     bool nan = false;
 #pragma unroll
@@ -542,18 +556,17 @@ __global__ void __launch_bounds__(256) add_rms_bf16_chunk(float * __restrict__ x
         }
     }
 }
-// Takes the first n - n % 4 rows when the chunk form applies (an addend, a bf16 copy and no fp32 copy, a chunk of at least 1024
-// rows of 256 NI values for the NI below, 16-byte aligned) and returns how many rows it took.
-static int launch_add_rms_bf16_chunk(float * x, const uint16_t * d, const float * nw, float eps, uint16_t * hbf, int N, int n, hipStream_t st) {
-    if (!d || !hbf || n < 1024 || (N & 255) || (((uintptr_t)x | (uintptr_t)d | (uintptr_t)nw | (uintptr_t)hbf) & 15)) return 0;
-    const int rows = n & ~3;
-    const dim3 grid(rows / 4), block(256);
+// Whether the chunk form applies: an addend, a bf16 copy and no fp32 copy, at least 600 rows (below, a row is divided over four waves:
+// launch_norm_div) of 256 NI values for the NI below, 16-byte aligned. A batch of less than 2^20 values stays in the caches.
+static bool launch_add_rms_bf16_chunk(float * x, const uint16_t * d, const float * nw, float eps, uint16_t * hbf, int N, int n, hipStream_t st) {
+    if (!d || !hbf || n < 600 || (n < 1024 && (long)n * N < (1L << 20)) || (N & 255) || (((uintptr_t)x | (uintptr_t)d | (uintptr_t)nw | (uintptr_t)hbf) & 15)) return false;
+    const dim3 grid((n + 3) / 4), block(256);
     switch (N >> 8) {
-#define CAMX_CHUNK(NI) case NI: add_rms_bf16_chunk<NI><<<grid, block, NI * 1024, st>>>(x, d, nw, eps, hbf); return rows;
+#define CAMX_CHUNK(NI) case NI: add_rms_bf16_chunk<NI><<<grid, block, NI * 1024, st>>>(x, d, nw, eps, hbf, n); return true;
         CAMX_CHUNK(4) CAMX_CHUNK(6) CAMX_CHUNK(8) CAMX_CHUNK(10) CAMX_CHUNK(12) CAMX_CHUNK(14) CAMX_CHUNK(16) CAMX_CHUNK(20) CAMX_CHUNK(24) CAMX_CHUNK(28) CAMX_CHUNK(32)
 #undef CAMX_CHUNK
     }
-    return 0;
+    return false;
 }
 
 extern "C" {
@@ -597,16 +610,9 @@ int camx_add_rms_q8_1(float * x, const float * d, const float * w, int S, const 
 
 int camx_add_rms_bf16(float * x, const uint16_t * d, const float * nw, float eps, float * h, uint16_t * hbf, int N, int n, hipStream_t st) {
     if (N < 1 || n < 0 || !x || !nw) return CAMX_EINVAL;
-    if (!h) {
-        const int done = launch_add_rms_bf16_chunk(x, d, nw, eps, hbf, N, n, st);
-        if (done) {
-            const hipError_t e = hipGetLastError();
-            if (e != hipSuccess || done == n) return (int)e;
-            x += (size_t)done * N; d += (size_t)done * N; hbf += (size_t)done * N; n -= done;     // the last n % 4 rows
-        }
-    }
+    if (!h && launch_add_rms_bf16_chunk(x, d, nw, eps, hbf, N, n, st)) CAMX_LAUNCH_RET();
     NormArgs a = {x, d, nullptr, 0, nw, 1, eps, h, nullptr, N, hbf, nullptr, nullptr, N, n, nullptr, 1, 0.0f};
-    return launch_norm<ADD_BF16>(a, st);
+    return launch_norm<ADD_BF16, NORM_HBF>(a, st);
 }
 
 int camx_pf_rms_mul(const float * x, const float * w, float * y, uint16_t * ybf, float * scl, int R, int wr, float eps, int K, hipStream_t st) {

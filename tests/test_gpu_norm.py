@@ -90,6 +90,35 @@ def test_add_rms_bf16(n, N):
     assert bits_equal(host(xd), ref['x']) and bits_equal(host(h), ref['h']) and bits_equal(host(hbf, np.uint16), ref['hbf'])
 
 
+@pytest.mark.parametrize('n,N', [(257, 5120), (599, 5120), (600, 5120), (777, 5120), (1026, 5120), (1027, 2048), (1031, 1536), (515, 2048), (2049, 1024), (603, 4096), (1025, 2560)])
+def test_norm_forms_between_256_and_chunk_rows(n, N):
+    """either side of the row counts at which a row is divided over waves, taken by a wave of the chunk form, or by the general form, with
+    last workgroups of one to four rows; the rows behind the batch keep their bytes. A NaN row takes the integer rounding of the bf16 copy"""
+    rng = np.random.default_rng(n + N)
+    x = outliers(rng, (n, N)); x[n - 1, 3] = np.nan; x[0, 0] = np.inf
+    d = outliers(rng, (n, N)); nw = (1 + 0.1 * rng.standard_normal(N)).astype(np.float32); nwd = dev(nw)
+    def padded(a):
+        return dev(np.concatenate([a, np.full((4, N), 77, a.dtype)]))
+    def tail_ok(t, like): return bits_equal(host(t, like)[n:], np.full((4, N), 77, like))
+    db = O.f2bf(d)
+    with np.errstate(all='ignore'): ref = O.add_rms_bf16(x, db, nw, 1e-6)
+    xd = padded(x); hbf = padded(np.zeros((n, N), np.uint16))
+    call('camx_add_rms_bf16', ptr(xd), ptr(dev(db)), ptr(nwd), F(1e-6), NULL, ptr(hbf), I(N), I(n))
+    assert bits_equal(host(xd)[:n], ref['x']) and bits_equal(host(hbf, np.uint16)[:n], ref['hbf']) and tail_ok(xd, np.float32) and tail_ok(hbf, np.uint16)
+    with np.errstate(all='ignore'): ref = O.add_rms16_q35(x, nw, 1e-6, d=d)
+    xd = padded(x); h = padded(np.zeros((n, N), np.float32)); h16 = padded(np.zeros((n, N), np.uint16))
+    call('camx_q35p_add_rms16', ptr(xd), ptr(dev(d)), ptr(nwd), F(1e-6), ptr(h), ptr(h16), I(N), I(n))
+    assert bits_equal(host(xd)[:n], ref['x']) and bits_equal(host(h)[:n], ref['h']) and bits_equal(host(h16, np.uint16)[:n], ref['h16'])
+    assert tail_ok(xd, np.float32) and tail_ok(h, np.float32) and tail_ok(h16, np.uint16)
+    if N > 2048: return
+    d3 = outliers(rng, (n, 3, N)); w3 = rng.random((n, 3)).astype(np.float32)
+    with np.errstate(all='ignore'): ref = O.add_rms16(x, nw, 1e-6, d=d3, w=w3, S=3)
+    xd = padded(x); h = padded(np.zeros((n, N), np.float32)); h16 = padded(np.zeros((n, N), np.uint16))
+    call('camx_q3p_add_rms16', ptr(xd), ptr(dev(d3)), ptr(dev(w3)), I(3), ptr(nwd), F(1e-6), ptr(h), ptr(h16), I(N), I(n))
+    assert bits_equal(host(xd)[:n], ref['x']) and bits_equal(host(h)[:n], ref['h']) and bits_equal(host(h16, np.uint16)[:n], ref['h16'])
+    assert tail_ok(xd, np.float32) and tail_ok(h, np.float32) and tail_ok(h16, np.uint16)
+
+
 @pytest.mark.parametrize('R,K,wr', [(8, 2560, 4), (3, 2048, 1), (5, 100, 1), (2, 896, 2), (516, 3072, 4), (512, 5120, 1), (1028, 2560, 4), (1029, 2560, 1), (1026, 2048, 1), (1024, 5120, 4), (16388, 2048, 4)])
 def test_rms_mul_and_rmsnorm(R, K, wr):
     rng = np.random.default_rng(R * K)
