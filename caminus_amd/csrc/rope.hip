@@ -1251,19 +1251,24 @@ static int rope_launch(const RopeArgs & a, int yarn, bool q8, hipStream_t st, bo
     if (a.n == 0) return CAMX_OK;
     const bool aligned = (a.ldq & (bf16in ? 7 : 3)) == 0 && ((uintptr_t)a.qkv & 15) == 0 && ((uintptr_t)a.q16 & 15) == 0 && ((uintptr_t)a.cache & 15) == 0;
     const bool wide = (!q8 || !bf16in) && !a.page_table && aligned;
-    // a batch of 2048 and more sequences through a page table: the chunk kernel with the token kernels' addressing and refusals
-    if (a.page_table && !bf16in && aligned && a.n >= 2048 &&
+    // A token per workgroup with all its loads first, from a batch that covers the chip (80 bf16 heads, 300 tokens 5.2 us, 777 tokens 7.6, 1500 tokens
+    // 10.5: the token kernel 6.2, 8.7, 14.6; 40 fp32 heads 5.0, 6.9, 9.2 and 5.7, 8.1, 12.1). The Q8 rows are bound by their arithmetic, which
+    // the token kernel spreads over more waves: 777 tokens 9.5 us, chunk 9.9, 1800 tokens 15.9 and 16.4, 2048 tokens 20.5 and 17.6; through a page table, where a token's row
+    // address is a chain of loads that the chunk kernel starts early, 512 tokens 7.5 and 8.0, 777 tokens 10.4 and 10.1, 1500 tokens 15.5 and 13.6.
+    const bool chunk = a.n > 256, chunk_q8 = a.n >= 2048, chunk_paged = a.n >= 700;
+    // sequences through a page table: the chunk kernel with the token kernels' addressing and refusals
+    if (a.page_table && !bf16in && aligned && chunk_paged &&
         (q8 ? (yarn ? rope_chunk_launch_f32<true, 1, true>(a, st) : rope_chunk_launch_f32<false, 1, true>(a, st))
             : (yarn ? rope_chunk_launch_f32<true, 1, false>(a, st) : rope_chunk_launch_f32<false, 1, false>(a, st)))) CAMX_LAUNCH_RET();
     // one token per workgroup: 29.9 us for 4096 tokens x 80 heads on cold lines (two tokens: 32.4, four: 34.9; the general kernel below: 32.3)
-    if (wide && bf16in && a.n >= 2048 && (yarn ? rope_chunk_launch<true, 1>(a, st) : rope_chunk_launch<false, 1>(a, st))) {}
+    if (wide && bf16in && chunk && (yarn ? rope_chunk_launch<true, 1>(a, st) : rope_chunk_launch<false, 1>(a, st))) {}
     else if (wide && bf16in && a.n >= 2048) {          // enough tokens to fill the chip two to a workgroup (4096 tokens, every launch on cold lines: 32.2 us; four: 34.0, one: 33.7)
         const dim3 g2((a.n + 1) / 2);
         if (yarn) qk_rope_wide_tokens<true, 2, false, 5, false><<<g2, dim3(256), 0, st>>>(a); else qk_rope_wide_tokens<false, 2, false, 5, false><<<g2, dim3(256), 0, st>>>(a);
     }
     else if (wide && bf16in) { if (yarn) qk_rope_wide_tokens<true, 1, false, 5, false><<<dim3(a.n), dim3(256), 0, st>>>(a); else qk_rope_wide_tokens<false, 1, false, 5, false><<<dim3(a.n), dim3(256), 0, st>>>(a); }
-    else if (wide && !q8 && a.n >= 2048 && (yarn ? rope_chunk_launch_f32<true, 1, false>(a, st) : rope_chunk_launch_f32<false, 1, false>(a, st))) {}
-    else if (wide && q8 && a.n >= 2048 && (yarn ? rope_chunk_launch_f32<true, 1, true>(a, st) : rope_chunk_launch_f32<false, 1, true>(a, st))) {}
+    else if (wide && !q8 && chunk && (yarn ? rope_chunk_launch_f32<true, 1, false>(a, st) : rope_chunk_launch_f32<false, 1, false>(a, st))) {}
+    else if (wide && q8 && chunk_q8 && (yarn ? rope_chunk_launch_f32<true, 1, true>(a, st) : rope_chunk_launch_f32<false, 1, true>(a, st))) {}
     else if (wide && a.n >= 2048) {               // fp32 rows of a prefill chunk: the same kernel, three wave steps (48 heads) per pass
         const dim3 g4((a.n + 3) / 4);
         if (q8) { if (yarn) qk_rope_wide_tokens<true, 4, true, 3, true><<<g4, dim3(256), 0, st>>>(a); else qk_rope_wide_tokens<false, 4, true, 3, true><<<g4, dim3(256), 0, st>>>(a); }

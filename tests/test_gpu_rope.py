@@ -283,3 +283,39 @@ def test_qk_rope_paged_at_chunk_size_equals_the_small_batch_kernel(q8, yarn):
     written = np.zeros(n_pages * page, bool); written[rows[ok]] = True
     assert (got[~written] == 0x3c).all() and not (got[written] == 0x3c).all(axis=1).any()
     assert host(qa, np.uint16)[[7, 900, 1300, 2000]].any(axis=(1, 2)).all()
+
+
+@pytest.mark.parametrize('n', [257, 700, 2048])
+@pytest.mark.parametrize('yarn', [0, 1])
+def test_a_tokens_bits_do_not_depend_on_the_batch(n, yarn):
+    """from these counts on a batch takes the chunk kernels (bf16 and fp32 rows; through a page table; Q8 rows): the same bits as the same
+    tokens in batches of at most 199, which the token kernels take, and not a byte behind the last token"""
+    rng = np.random.default_rng(n + yarn)
+    page, pages = 256, 16
+
+    def run(bf16, q8, paged, step):
+        nh, nkv = (16, 8) if bf16 else (12, 4)
+        ldq, M = (nh + 2 * nkv) * 128, nkv * 128
+        row = 2 * (M // 32) * 34 if q8 else 4 * M
+        g = torch.Generator(device='cuda'); g.manual_seed(n)
+        qkv = torch.randn(n, ldq, generator=g, device='cuda'); qkv = qkv.bfloat16() if bf16 else qkv
+        par = torch.cat([1 + 0.1 * torch.randn(256, generator=g, device='cuda'), torch.tensor([0.8, 1e-6], device='cuda'), torch.rand(65, generator=g, device='cuda')])
+        order = torch.randperm(page * pages, generator=g, device='cuda')[:n].to(torch.int32)
+        pos, pt = (order % page).contiguous(), torch.zeros(n, 2, dtype=torch.int32, device='cuda')
+        pt[:, 0] = order // page
+        q16 = torch.full((n + 1, nh, 128), 7, dtype=torch.int16, device='cuda'); cache = torch.full((page * pages + n + 8, row), 9, dtype=torch.uint8, device='cuda')
+        err = torch.zeros(1, dtype=torch.int32, device='cuda')
+        for lo in range(0, n, step):
+            m = min(step, n - lo)
+            if paged:
+                call('camx_qk_rope_paged', ptr(qkv[lo:]), I(ldq), I(nh), I(nkv), ptr(par), ptr(pos[lo:]), ptr(q16[lo:]), ptr(cache), ptr(err), ptr(pt[lo:]), I(2), I(page), I(pages),
+                     I(m), I(yarn), I(int(q8)))
+            elif bf16: call('camx_qk_rope_bf16', ptr(qkv[lo:]), I(ldq), I(nh), I(nkv), ptr(par), I(3 + lo), ptr(q16[lo:]), ptr(cache), I(m), I(yarn))
+            elif q8: call('camx_q3p_qk_rope_q8', ptr(qkv[lo:]), I(ldq), I(nh), I(nkv), ptr(par), I(3 + lo), ptr(q16[lo:]), ptr(cache), ptr(err), I(m), I(yarn))
+            else: call('camx_q3p_qk_rope', ptr(qkv[lo:]), I(ldq), I(nh), I(nkv), ptr(par), I(3 + lo), ptr(q16[lo:]), ptr(cache), I(m), I(yarn))
+        torch.cuda.synchronize()
+        return q16, cache, err
+    for bf16, q8, paged in ((True, False, False), (False, False, False), (False, True, False), (False, False, True), (False, True, True)):
+        whole, parts = run(bf16, q8, paged, n), run(bf16, q8, paged, 199)
+        assert all(torch.equal(a, b) for a, b in zip(whole, parts)), (bf16, q8, paged)
+        assert int(whole[2]) == 0 and bool((whole[0][n:] == 7).all())
