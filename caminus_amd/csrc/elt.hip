@@ -171,28 +171,43 @@ __global__ void __launch_bounds__(256) op_gdn_conv_k(const float * __restrict__ 
         }
     }
 }
-// Prefill chunks: a lane owns VW consecutive channels and walks TR consecutive tokens, with the rows of the next eight tokens
-// always in flight (a ring of eight 128-bit loads that is refilled as it is consumed) and the four-tap window in registers;
-// one wave per workgroup, so the grid's (channel groups x token ranges) waves spread evenly over the chip.
+// Prefill chunks: a lane owns VW consecutive channels, a wave TPW consecutive tokens whose rows (and the three before them) are all
+// requested before the first one is used; a workgroup's four waves take consecutive token groups, so three of four find their neighbour's
+// rows in the caches.
 // L2: the L2 norm of the q / k heads (the first heads * 128 channels) in the same pass, from the values as they are stored: qk
 // [T][heads][128]. A head is 16 lanes x 8 channels (bf16 rows) or 32 lanes x 4 (fp32 rows, the lanes in slot order), whole heads per
 // wave (C % 128 == 0), so every lane of a head is present.
+// commit (T >= 3): the state's buffer, which the wave of the first tokens, the only reader of its channels, leaves holding the last three inputs.
 CAMX_DEV void l2_head_w8(const float (&v)[8], float (&o)[8], float rs);
 CAMX_DEV f32x4 l2_head_l4(f32x4 v, int lane, float rs);
-template <bool BF16, bool L2 = false>
-__global__ void __launch_bounds__(64) gdn_conv_stream(const void * __restrict__ x, const float * __restrict__ w, const float * __restrict__ st,
-                                                      void * __restrict__ y, int C, int T, int ldx, int ldy, int TR,
-                                                      void * __restrict__ qk = nullptr, int heads = 0, float rs = 0.0f) {
-    constexpr int VW = BF16 ? 8 : 4, P = 8;
-    const int lane_l2 = slot_of(threadIdx.x);
-    const int cv = blockIdx.x * 64 + (L2 && !BF16 ? lane_l2 : (int)threadIdx.x);
-    if (cv * VW >= C) return;
-    const int c0 = cv * VW, t0 = blockIdx.y * TR, t1 = T < t0 + TR ? T : t0 + TR;
-    auto row = [&](int t) {                                            // (a row index past the batch is clamped: the load is harmless and never used)
-        const int tc = t < T - 1 ? t : T - 1;
-        return BF16 ? __builtin_nontemporal_load((const u32x4 *)((const uint16_t *)x + (size_t)tc * ldx + c0))
-                    : __builtin_nontemporal_load((const u32x4 *)((const float *)x + (size_t)tc * ldx + c0));
+template <bool BF16, bool L2, int TPW, bool STREAM>
+__global__ void __launch_bounds__(256) gdn_conv_rows(const void * __restrict__ x, const float * __restrict__ w, const float * st,
+                                                     void * __restrict__ y, int C, int T, int ldx, int ldy,
+                                                     void * __restrict__ qk, int heads, float rs, float * commit) {
+    constexpr int VW = BF16 ? 8 : 4;
+    const int lane_l2 = slot_of(threadIdx.x & 63), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int cv = blockIdx.x * 64 + (L2 && !BF16 ? lane_l2 : (int)(threadIdx.x & 63));
+    const int c0 = cv * VW, t0 = (blockIdx.y * 4 + wave) * TPW;
+    if (c0 >= C || t0 >= T) return;
+    u32x4 raw[TPW + 3];                                                // row t0 - 3 + j (clamped: before the chunk the state stands in, behind it nothing is stored)
+    auto at = [&](int j) {
+        const int tj = t0 - 3 + j, tc = tj < 0 ? 0 : tj < T ? tj : T - 1;
+        return (const u32x4 *)(BF16 ? (const void *)((const uint16_t *)x + (size_t)tc * ldx + c0) : (const void *)((const float *)x + (size_t)tc * ldx + c0));
     };
+    if constexpr (STREAM) {                                            // the first and last three rows are another wave's too
+#pragma unroll
+        for (int j = 0; j < 3; j++) raw[j] = *at(j);
+#pragma unroll
+        for (int j = 3; j < TPW; j++) raw[j] = __builtin_nontemporal_load(at(j));
+#pragma unroll
+        for (int j = TPW; j < TPW + 3; j++) raw[j] = *at(j);
+    } else {
+#pragma unroll
+        for (int j = 0; j < TPW + 3; j++) raw[j] = *at(j);
+    }
+    f32x4 w4[VW];
+#pragma unroll
+    for (int k = 0; k < VW; k++) w4[k] = *(const f32x4 *)(w + (size_t)(c0 + k) * 4);
     auto widen = [&](float (&o)[VW], u32x4 r) {
         if (BF16) {
 #pragma unroll
@@ -202,82 +217,80 @@ __global__ void __launch_bounds__(64) gdn_conv_stream(const void * __restrict__ 
             for (int p = 0; p < 4; p++) { const uint32_t b = r[p]; o[p % VW] = __builtin_bit_cast(float, b); }
         }
     };
-    u32x4 halo[3];                                                     // the three rows before the range (another wave's tokens; clamped when the state stands in)
-#pragma unroll
-    for (int j = 0; j < 3; j++) {
-        const int tj = t0 - 3 + j < 0 ? 0 : t0 - 3 + j;
-        halo[j] = BF16 ? *(const u32x4 *)((const uint16_t *)x + (size_t)tj * ldx + c0) : *(const u32x4 *)((const float *)x + (size_t)tj * ldx + c0);
-    }
-    u32x4 ring[P];
-#pragma unroll
-    for (int u = 0; u < P; u++) ring[u] = row(t0 + u);
-    f32x4 w4[VW];
-#pragma unroll
-    for (int k = 0; k < VW; k++) w4[k] = *(const f32x4 *)(w + (size_t)(c0 + k) * 4);
     float win[4][VW];                                                  // token t0 - 3 + j sits in slot j & 3
 #pragma unroll
-    for (int j = 0; j < 3; j++) {
-        const int tj = t0 - 3 + j;
-        if (tj < 0) {
+    for (int j = 0; j < 3; j++) widen(win[j], raw[j]);
+    if (t0 == 0) {                                                     // (uniform)
 #pragma unroll
-            for (int k = 0; k < VW; k++) win[j][k] = st[(size_t)(c0 + k) * 3 + 3 + tj];
-        } else widen(win[j], halo[j]);
+        for (int j = 0; j < 3; j++)
+#pragma unroll
+            for (int k = 0; k < VW; k++) win[j][k] = st[(size_t)(c0 + k) * 3 + j];
     }
-    auto emit = [&](int tt, int u) {                                   // token tt's output from window slots u .. u + 3 (mod 4)
+#pragma unroll
+    for (int u = 0; u < TPW; u++) {
+        const int tt = t0 + u;
+        widen(win[(u + 3) & 3], raw[u + 3]);
         float r[VW];
 #pragma unroll
         for (int k = 0; k < VW; k++) {
             float sumf = 0.0f;
             sumf = __builtin_fmaf(win[u & 3][k], w4[k].x, sumf); sumf = __builtin_fmaf(win[(u + 1) & 3][k], w4[k].y, sumf);
             sumf = __builtin_fmaf(win[(u + 2) & 3][k], w4[k].z, sumf); sumf = __builtin_fmaf(win[(u + 3) & 3][k], w4[k].w, sumf);
-            r[k] = BF16 ? silu_fast(sumf) : silu_f(sumf);
+            r[k] = BF16 ? silu_fast(sumf) : sumf;
         }
-        const size_t o = (size_t)tt * ldy + c0;
-        if (BF16) {
-            const u32x2 lo = pack_bf16x4_rne((f32x4){r[0], r[1], r[2], r[3]}), hi = pack_bf16x4_rne((f32x4){r[4 % VW], r[5 % VW], r[6 % VW], r[7 % VW]});
-            if (!L2 || y) __builtin_nontemporal_store((u32x4){lo.x, lo.y, hi.x, hi.y}, (u32x4 *)((uint16_t *)y + o));     // (on cold lines: 38.5 us against 42.2 with plain stores, 4096 x 10240)
-            if constexpr (L2) {
-                const f32x4 a = unpack_bf16x4(lo), b = unpack_bf16x4(hi);
-                const float v8[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-                float o8[8];
-                l2_head_w8(v8, o8, rs);
-                if (c0 < heads * 128) {
-                    const u32x2 pa = pack_bf16x4_rne((f32x4){o8[0], o8[1], o8[2], o8[3]}), pb = pack_bf16x4_rne((f32x4){o8[4], o8[5], o8[6], o8[7]});
-                    __builtin_nontemporal_store((u32x4){pa.x, pa.y, pb.x, pb.y}, (u32x4 *)((uint16_t *)qk + (size_t)tt * heads * 128 + c0));
+        if (!BF16) silu_group<VW>(r);
+        if (tt < T) {                                                  // (uniform)
+            const size_t o = (size_t)tt * ldy + c0;
+            if (BF16) {
+                const u32x2 lo = pack_bf16x4_rne((f32x4){r[0], r[1], r[2], r[3]}), hi = pack_bf16x4_rne((f32x4){r[4 % VW], r[5 % VW], r[6 % VW], r[7 % VW]});
+                if (!L2 || y) __builtin_nontemporal_store((u32x4){lo.x, lo.y, hi.x, hi.y}, (u32x4 *)((uint16_t *)y + o));     // (on cold lines: 38.5 us against 42.2 with plain stores, 4096 x 10240)
+                if constexpr (L2) {
+                    const f32x4 a = unpack_bf16x4(lo), b = unpack_bf16x4(hi);
+                    const float v8[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+                    float o8[8];
+                    l2_head_w8(v8, o8, rs);
+                    if (c0 < heads * 128) {
+                        const u32x2 pa = pack_bf16x4_rne((f32x4){o8[0], o8[1], o8[2], o8[3]}), pb = pack_bf16x4_rne((f32x4){o8[4], o8[5], o8[6], o8[7]});
+                        __builtin_nontemporal_store((u32x4){pa.x, pa.y, pb.x, pb.y}, (u32x4 *)((uint16_t *)qk + (size_t)tt * heads * 128 + c0));
+                    }
+                }
+            } else {
+                if (!L2 || y) __builtin_nontemporal_store((f32x4){r[0], r[1], r[2], r[3]}, (f32x4 *)((float *)y + o));
+                if constexpr (L2) {
+                    const f32x4 q4 = l2_head_l4((f32x4){r[0], r[1], r[2], r[3]}, lane_l2, rs);
+                    if (c0 < heads * 128) __builtin_nontemporal_store(q4, (f32x4 *)((float *)qk + (size_t)tt * heads * 128 + c0));
                 }
             }
-        } else {
-            if (!L2 || y) __builtin_nontemporal_store((f32x4){r[0], r[1], r[2], r[3]}, (f32x4 *)((float *)y + o));
-            if constexpr (L2) {
-                const f32x4 q4 = l2_head_l4((f32x4){r[0], r[1], r[2], r[3]}, lane_l2, rs);
-                if (c0 < heads * 128) __builtin_nontemporal_store(q4, (f32x4 *)((float *)qk + (size_t)tt * heads * 128 + c0));
-            }
         }
-    };
-    int t = t0;
-    // No row past the wave's range is requested: it is another wave's, and would come from HBM twice (with eight rows requested ahead
-    // regardless, 4096 x 10240 read 34 % more than its input, 16384 tokens 17 %). The last group asks for the range's last row again
-    // instead, which is still on its way or in L2 (+ 3 % of reads); a branch around the request would do without that, but with it the
-    // compiler keeps all eight tokens of a group live at once (fp32 rows: 404 registers instead of 92).
-    for (; t + P <= t1; t += P) {                                      // whole groups of eight tokens
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (commit && t0 == 0) {                                           // (uniform)
 #pragma unroll
-        for (int u = 0; u < P; u++) {
-            // the whole row is widened before its ring slot is requested again: left to itself the compiler widens half of it later,
-            // keeps that half in a copy, and hoists the copies of all eight slots (and the waits for their loads) to the top of the loop
-            widen(win[(u + 3) & 3], ring[u]);
-            if constexpr (BF16) {
+        for (int j = 0; j < 3; j++) {
+            float v[VW];
+            widen(v, BF16 ? *(const u32x4 *)((const uint16_t *)x + (size_t)(T - 3 + j) * ldx + c0) : *(const u32x4 *)((const float *)x + (size_t)(T - 3 + j) * ldx + c0));
 #pragma unroll
-                for (int k = 0; k < VW; k++) asm volatile("" : "+v"(win[(u + 3) & 3][k]));
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            ring[u] = row(t + u + P < t1 ? t + u + P : t1 - 1);
-            if constexpr (BF16) __builtin_amdgcn_sched_barrier(0);
-            emit(t + u, u);
+            for (int k = 0; k < VW; k++) commit[(size_t)(c0 + k) * 3 + j] = v[k];
         }
     }
-#pragma unroll
-    for (int u = 0; u < P; u++)                                        // the last, partial group
-        if (t + u < t1) { widen(win[(u + 3) & 3], ring[u]); emit(t + u, u); __builtin_amdgcn_sched_barrier(0); }
+}
+template <bool L2>
+static void launch_conv_rows(const void * x, const float * w, const float * state, void * y, int C, int T, int ldx, int ldy, int bf16, void * qk, int heads, float rs,
+                             float * commit, hipStream_t st) {
+    // Tokens per wave. From 2^24 values on a chunk comes from HBM: eight tokens, the rows that no other wave reads past the caches; below, its rows
+    // were just written and the chip wants more waves: four. fp32 / bf16 x 10240 channels: 200 tokens 4.9 / 4.5 us (eight 5.5 / 5.0; a wave that walked 32
+    // tokens with the next eight rows in flight 12.5 / 11.4), 3001 tokens 40.1 / 25.8 (four 42.6 / 24.7, walking 49.3 / 27.8), 16384 tokens 219.7 /
+    // 109.6 (four 218.6 / 132.9, walking 250 / 130); with the L2 norm at 4096 tokens 70.0 / 42.5 (walking 91.0 / 49.2).
+    const bool big = (long)T * C >= (1L << 24);
+    const int tpw = big ? 8 : 4, per = bf16 ? 8 : 4;
+    const dim3 grid((unsigned)((C / per + 63) / 64), (unsigned)((T + 4 * tpw - 1) / (4 * tpw))), block(256);
+    if (bf16) {
+        if (big) gdn_conv_rows<true, L2, 8, true><<<grid, block, 0, st>>>(x, w, state, y, C, T, ldx, ldy, qk, heads, rs, commit);
+        else gdn_conv_rows<true, L2, 4, false><<<grid, block, 0, st>>>(x, w, state, y, C, T, ldx, ldy, qk, heads, rs, commit);
+    } else {
+        if (big) gdn_conv_rows<false, L2, 8, true><<<grid, block, 0, st>>>(x, w, state, y, C, T, ldx, ldy, qk, heads, rs, commit);
+        else gdn_conv_rows<false, L2, 4, false><<<grid, block, 0, st>>>(x, w, state, y, C, T, ldx, ldy, qk, heads, rs, commit);
+    }
 }
 
 template <bool BF16>
@@ -804,18 +817,14 @@ int camx_gate_mul(const void * a, const void * gt, void * y, long N, int D, int 
     else gate_mul_k<2><<<grid, block, 0, st>>>(a, gt, y, N, D, stride, off);
     CAMX_LAUNCH_RET();
 }
+// the chunk kernel takes the convolution (a decode / verify batch: the one-value-per-thread kernel)
+static bool conv_streams(const void * x, const void * y, int C, int T, int ldx, int ldy, int bf16) {
+    const int vw = bf16 ? 8 : 4;
+    return (long)T * C >= (1L << 20) && C % vw == 0 && ldx % vw == 0 && ldy % vw == 0 && !(((uintptr_t)x | (uintptr_t)y) & 15);
+}
 int camx_pf_gdn_conv(const void * x, const float * w, const float * state, void * y, int C, int T, int ldx, int ldy, int bf16, hipStream_t st) {
     if (!x || !w || !state || !y || C < 1 || T < 1 || ldx < C || ldy < C || ((uintptr_t)w & 15)) return CAMX_EINVAL;
-    const int vw = bf16 ? 8 : 4;
-    if ((long)T * C >= (1L << 20) && C % vw == 0 && ldx % vw == 0 && ldy % vw == 0 && !(((uintptr_t)x | (uintptr_t)y) & 15)) {
-        // tokens per wave: at 4096 tokens 16 and 64 measured 15 % slower than 32 (halo re-reads; too few waves); from 16384 tokens on there
-        // are waves enough for 64, and the three halo rows a wave re-reads are 5 % of its reads instead of 9 % (a decode / verify batch
-        // takes the one-value-per-thread kernel below)
-        const int tr = T >= 16384 ? 64 : 32;
-        const dim3 gs((unsigned)((C / vw + 63) / 64), (unsigned)((T + tr - 1) / tr)), bs(64);
-        if (bf16) gdn_conv_stream<true><<<gs, bs, 0, st>>>(x, w, state, y, C, T, ldx, ldy, tr); else gdn_conv_stream<false><<<gs, bs, 0, st>>>(x, w, state, y, C, T, ldx, ldy, tr);
-        CAMX_LAUNCH_RET();
-    }
+    if (conv_streams(x, y, C, T, ldx, ldy, bf16)) { launch_conv_rows<false>(x, w, state, y, C, T, ldx, ldy, bf16, nullptr, 0, 0.0f, nullptr, st); CAMX_LAUNCH_RET(); }
     const dim3 grid((unsigned)(((long)T * C + 255) / 256)), block(256);
     if (bf16) gdn_conv_k<true><<<grid, block, 0, st>>>(x, w, state, y, C, T, ldx, ldy);
     else gdn_conv_k<false><<<grid, block, 0, st>>>(x, w, state, y, C, T, ldx, ldy);
@@ -837,6 +846,15 @@ int camx_pf_conv_state(const void * x, float * state, int C, int T, int ldx, int
     if (bf16) conv_state_k<true><<<grid, block, 0, st>>>(x, state, C, T, ldx);
     else conv_state_k<false><<<grid, block, 0, st>>>(x, state, C, T, ldx);
     CAMX_LAUNCH_RET();
+}
+// camx_pf_gdn_conv, then camx_pf_conv_state on the same rows, in one launch where the chunk kernel takes them
+int camx_pf_gdn_conv_commit(const void * x, const float * w, float * state, void * y, int C, int T, int ldx, int ldy, int bf16, hipStream_t st) {
+    if (x && w && state && y && C >= 1 && T >= 3 && ldx >= C && ldy >= C && !((uintptr_t)w & 15) && conv_streams(x, y, C, T, ldx, ldy, bf16)) {
+        launch_conv_rows<false>(x, w, state, y, C, T, ldx, ldy, bf16, nullptr, 0, 0.0f, state, st);
+        CAMX_LAUNCH_RET();
+    }
+    const int rc = camx_pf_gdn_conv(x, w, state, y, C, T, ldx, ldy, bf16, st);
+    return rc ? rc : camx_pf_conv_state(x, state, C, T, ldx, bf16, st);
 }
 int camx_pf_gdn_l2(const void * x, void * y, int heads, int K, int ldx, float rs, int T, int bf16, hipStream_t st) {
     if (!x || !y || heads < 1 || K < 1 || K > 512 || T < 0 || ldx < heads * K) return CAMX_EINVAL;
@@ -869,10 +887,7 @@ int camx_gdn_conv_l2(const void * x, const float * w, const float * state, void 
     if (!x || !w || !state || !qk || C < 128 || (C & 127) || T < 1 || ldx < C || (y && ldy < C) || heads < 1 || heads > C / 128 || (ldx % vw) || (y && ldy % vw) ||
         ((uintptr_t)w & 15) || (((uintptr_t)x | (uintptr_t)y | (uintptr_t)qk) & 15)) return CAMX_EINVAL;
     if ((long)T * C >= (1L << 20)) {
-        const int tr = T >= 16384 ? 64 : 32;
-        const dim3 gs((unsigned)((C / vw + 63) / 64), (unsigned)((T + tr - 1) / tr)), bs(64);
-        if (bf16) gdn_conv_stream<true, true><<<gs, bs, 0, st>>>(x, w, state, y, C, T, ldx, ldy, tr, qk, heads, rs);
-        else gdn_conv_stream<false, true><<<gs, bs, 0, st>>>(x, w, state, y, C, T, ldx, ldy, tr, qk, heads, rs);
+        launch_conv_rows<true>(x, w, state, y, C, T, ldx, ldy, bf16, qk, heads, rs, nullptr, st);
         CAMX_LAUNCH_RET();
     }
     const dim3 grid((unsigned)(((long)T * (C >> 7) + 7) / 8)), block(256);

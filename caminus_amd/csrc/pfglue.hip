@@ -362,59 +362,73 @@ __global__ void __launch_bounds__(256) ple_conv_k(const float * __restrict__ x, 
     if (y) y[i] = o;
     if (res) { const float ab = a[i] + o; res[i] = res[i] + ab; }
 }
-// the same for C % 4 == 0, D % 4 == 0 and 16-byte aligned operands: the token in blockIdx.y (no division of an element index), four
-// channels per thread (their sixteen fp16 weights in two 16-byte loads), streamed outputs non-temporal
-__global__ void __launch_bounds__(256) ple_conv_rows(const float * __restrict__ x, const float * __restrict__ xscl, const float * __restrict__ xw,
-                                                     const uint16_t * __restrict__ w, const float * __restrict__ hist, float * __restrict__ y,
-                                                     const float * __restrict__ a, float * __restrict__ res, int C, int D, int dil) {
-    // workgroup i runs on XCD i mod 8, each with its own L2: an XCD takes a contiguous range of tokens, so that the three earlier rows a
-    // token reads were fetched into the same L2 by its neighbours a moment ago (with tokens dealt round-robin every row crossed the fabric
-    // four times: 67 MB read for 17 MB of input at 4096 x 1024)
-    int t = blockIdx.y, bx = blockIdx.x;
-    const int total = gridDim.x * gridDim.y;
-    if ((total & 7) == 0) {
-        const int lin = blockIdx.x + gridDim.x * blockIdx.y, nw = (lin & 7) * (total >> 3) + (lin >> 3);
-        t = nw / gridDim.x; bx = nw - t * gridDim.x;
+// The same for C % 4 == 0, D % 4 == 0 and 16-byte aligned operands: a lane owns four channels, a wave TPW tokens dil apart (t0, t0 + dil, ..), whose rows
+// and the three before them, every one a tap of four of its tokens, are all requested before the first is used: (TPW + 3) / TPW rows
+// requested per token, where a thread per token requested four (x 10240, dilation 3, caller's buffers in rotation: 777 tokens 22.6 -> 11.5 us, 2048
+// tokens 49.7 -> 30.8, 4096 102 -> 58; floor 9.8, 25.8, 51.6; eight tokens a wave 11.8, 31.5, 59.2). Streamed outputs are non-temporal.
+// commit (T >= 3 dil): hist's buffer, which the waves of the first tokens leave holding the last 3 dil inputs: the wave of token r < dil is the only
+// reader of the entries r, r + dil, r + 2 dil of its channels, and the one that writes them.
+template <int TPW>
+__global__ void __launch_bounds__(256) ple_conv_taps(const float * __restrict__ x, const float * __restrict__ xscl, const float * __restrict__ xw,
+                                                     const uint16_t * __restrict__ w, const float * hist, float * __restrict__ y,
+                                                     const float * __restrict__ a, float * __restrict__ res, int C, int T, int D, int dil, float * commit) {
+    const int gw = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), block = gw / dil, t0 = block * dil * TPW + gw - block * dil;
+    const int c = 4 * (blockIdx.x * 64 + (threadIdx.x & 63)), hl = 3 * dil;
+    if (c >= C || t0 >= T) return;
+    f32x4 in[TPW + 3];                                   // the row of token t0 + (j - 3) dil (clamped: before the chunk the history stands in, behind it nothing is stored)
+    float sc[TPW + 3];
+#pragma unroll
+    for (int j = 0; j < TPW + 3; j++) {
+        const int tj = t0 + (j - 3) * dil, tc = tj < 0 ? 0 : tj < T ? tj : T - 1;
+        in[j] = *(const f32x4 *)(x + (size_t)tc * C + c);
+        sc[j] = xscl ? xscl[(size_t)tc * (C / D) + c / D] : 1.0f;
     }
-    const int c = 4 * (bx * 256 + threadIdx.x), hl = 3 * dil;
-    if (c >= C) return;
     const u32x4 w0 = *(const u32x4 *)(w + (size_t)c * 4), w1 = *(const u32x4 *)(w + (size_t)c * 4 + 8);
-    const uint32_t ww[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};      // channel j's taps: halves 4 j .. 4 j + 3
-    f32x4 xwv = {1.0f, 1.0f, 1.0f, 1.0f};
-    if (xscl) xwv = *(const f32x4 *)(xw + c);
-    float conv[4];
+    float tap[4][4];                                     // [channel][tap]
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const int back = (3 - k) * dil;
-        float xv[4];
-        if (back <= t) {
-            const int tb = t - back;
-            const f32x4 v = *(const f32x4 *)(x + (size_t)tb * C + c);
-            xv[0] = v.x; xv[1] = v.y; xv[2] = v.z; xv[3] = v.w;
-            if (xscl) {
-                const float sc = xscl[tb * (C / D) + c / D];
-                xv[0] = (xv[0] * sc) * xwv.x; xv[1] = (xv[1] * sc) * xwv.y; xv[2] = (xv[2] * sc) * xwv.z; xv[3] = (xv[3] * sc) * xwv.w;
-            }
-        } else {
+    for (int j = 0; j < 4; j++) {
+        const uint32_t lo = j < 2 ? w0[2 * j] : w1[2 * j - 4], hi = j < 2 ? w0[2 * j + 1] : w1[2 * j - 3];
+        tap[j][0] = h2f_bits((uint16_t)lo); tap[j][1] = h2f_bits((uint16_t)(lo >> 16)); tap[j][2] = h2f_bits((uint16_t)hi); tap[j][3] = h2f_bits((uint16_t)(hi >> 16));
+    }
+    if (xscl) {                                          // (uniform)
+        const f32x4 xwv = *(const f32x4 *)(xw + c);
 #pragma unroll
-            for (int j = 0; j < 4; j++) xv[j] = hist[(size_t)(c + j) * hl + hl - (back - t)];
-        }
+        for (int j = 0; j < TPW + 3; j++) { in[j].x = (in[j].x * sc[j]) * xwv.x; in[j].y = (in[j].y * sc[j]) * xwv.y; in[j].z = (in[j].z * sc[j]) * xwv.z; in[j].w = (in[j].w * sc[j]) * xwv.w; }
+    }
+    if (block == 0) {                                    // (uniform)
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) in[j][k] = hist[(size_t)(c + k) * hl + t0 + j * dil];
+    }
+#pragma unroll
+    for (int u = 0; u < TPW; u++) {
+        const int t = t0 + u * dil;
+        float conv[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const uint32_t pair = ww[2 * j + (k >> 1)];
-            const float term = xv[j] * h2f_bits((uint16_t)((k & 1) ? pair >> 16 : pair & 0xffffu));
-            conv[j] = k == 0 ? term : conv[j] + term;
+            const float p0 = in[u][j] * tap[j][0], p1 = in[u + 1][j] * tap[j][1], p2 = in[u + 2][j] * tap[j][2], p3 = in[u + 3][j] * tap[j][3];
+            conv[j] = ((p0 + p1) + p2) + p3;
+        }
+        silu_group<4>(conv);
+        if (t < T) {                                     // (uniform)
+            const size_t i = (size_t)t * C + c;
+            const f32x4 o = {conv[0], conv[1], conv[2], conv[3]};
+            if (y) __builtin_nontemporal_store(o, (f32x4 *)(y + i));
+            if (res) {
+                const f32x4 av = __builtin_nontemporal_load((const f32x4 *)(a + i)), rv = __builtin_nontemporal_load((const f32x4 *)(res + i));
+                f32x4 r; r.x = rv.x + (av.x + o.x); r.y = rv.y + (av.y + o.y); r.z = rv.z + (av.z + o.z); r.w = rv.w + (av.w + o.w);
+                __builtin_nontemporal_store(r, (f32x4 *)(res + i));
+            }
         }
     }
-    f32x4 o;
-    o.x = conv[0] / (1.0f + expf(-conv[0])); o.y = conv[1] / (1.0f + expf(-conv[1]));
-    o.z = conv[2] / (1.0f + expf(-conv[2])); o.w = conv[3] / (1.0f + expf(-conv[3]));
-    const size_t i = (size_t)t * C + c;
-    if (y) __builtin_nontemporal_store(o, (f32x4 *)(y + i));
-    if (res) {
-        const f32x4 av = __builtin_nontemporal_load((const f32x4 *)(a + i)), rv = __builtin_nontemporal_load((const f32x4 *)(res + i));
-        f32x4 r; r.x = rv.x + (av.x + o.x); r.y = rv.y + (av.y + o.y); r.z = rv.z + (av.z + o.z); r.w = rv.w + (av.w + o.w);
-        __builtin_nontemporal_store(r, (f32x4 *)(res + i));
+    if (commit && block == 0) {                          // (uniform)
+#pragma unroll
+        for (int m = 0; m < 3; m++) {
+            const int j = t0 + m * dil, tj = T - hl + j;
+#pragma unroll
+            for (int k = 0; k < 4; k++) commit[(size_t)(c + k) * hl + j] = ple_x(x, xscl, xw, tj, c + k, C, D);
+        }
     }
 }
 // hist[c] = the last 3 dil inputs of [hist[c], x[0 .. T - 1][c]]; 3 dil <= 32
@@ -584,15 +598,23 @@ int camx_pf_ple_gate(const float * kn, const float * q, const float * qscl, cons
     ple_gate_k<<<dim3(T), dim3(256), 0, st>>>(kn, q, qscl, qw, val, ldv, gated, gate_out, HC, D);
     CAMX_LAUNCH_RET();
 }
+#define PLE_TPW 4
+static long ple_waves(int T, int dil) { const long per = (long)dil * PLE_TPW; return (T + per - 1) / per * dil; }
+static bool ple_taps(const float * x, const float * xw, const uint16_t * w, const float * y, const float * a, const float * res, int C, int T, int D, int dil) {
+    return C % 4 == 0 && D % 4 == 0 && dil <= 65535 && (ple_waves(T, dil) + 3) / 4 <= 65535 &&
+           !(((uintptr_t)x | (uintptr_t)xw | (uintptr_t)w | (uintptr_t)y | (uintptr_t)a | (uintptr_t)res) & 15);
+}
+static void launch_ple_taps(const float * x, const float * xscl, const float * xw, const uint16_t * w, const float * hist, float * y, const float * a, float * res,
+                            int C, int T, int D, int dil, float * commit, hipStream_t st) {
+    const dim3 grid((unsigned)((C / 4 + 63) / 64), (unsigned)((ple_waves(T, dil) + 3) / 4));
+    ple_conv_taps<PLE_TPW><<<grid, dim3(256), 0, st>>>(x, xscl, xw, w, hist, y, a, res, C, T, D, dil, commit);
+}
 int camx_pf_ple_conv(const float * x, const float * xscl, const float * xw, const uint16_t * w, const float * hist, float * y, const float * a, float * res,
                      int C, int T, int D, int dil, hipStream_t st) {
     if (!x || !w || !hist || (!y && !res) || (res && !a) || C < 1 || T < 0 || D < 1 || C % D || dil < 1 || ((xscl == nullptr) != (xw == nullptr))) return CAMX_EINVAL;
     if (T == 0) return CAMX_OK;
     if ((long)T * C >= 0x7fffffffL * 256) return CAMX_EINVAL;
-    if (C % 4 == 0 && D % 4 == 0 && T <= 65535 && !(((uintptr_t)x | (uintptr_t)xw | (uintptr_t)w | (uintptr_t)y | (uintptr_t)a | (uintptr_t)res) & 15)) {
-        ple_conv_rows<<<dim3((unsigned)((C / 4 + 255) / 256), (unsigned)T), dim3(256), 0, st>>>(x, xscl, xw, w, hist, y, a, res, C, D, dil);
-        CAMX_LAUNCH_RET();
-    }
+    if (ple_taps(x, xw, w, y, a, res, C, T, D, dil)) { launch_ple_taps(x, xscl, xw, w, hist, y, a, res, C, T, D, dil, nullptr, st); CAMX_LAUNCH_RET(); }
     ple_conv_k<<<dim3((unsigned)(((long)T * C + 255) / 256)), dim3(256), 0, st>>>(x, xscl, xw, w, hist, y, a, res, C, T, D, dil);
     CAMX_LAUNCH_RET();
 }
@@ -600,6 +622,18 @@ int camx_pf_ple_hist(const float * x, const float * xscl, const float * xw, floa
     if (!x || !hist || C < 1 || T < 0 || D < 1 || C % D || dil < 1 || 3 * dil > 32 || ((xscl == nullptr) != (xw == nullptr))) return CAMX_EINVAL;
     ple_hist_k<<<dim3((unsigned)((C + 255) / 256)), dim3(256), 0, st>>>(x, xscl, xw, hist, C, T, D, dil);
     CAMX_LAUNCH_RET();
+}
+
+// camx_pf_ple_conv, then camx_pf_ple_hist on the same rows, in one launch where a chunk reaches past the history
+int camx_pf_ple_conv_commit(const float * x, const float * xscl, const float * xw, const uint16_t * w, float * hist, float * y, const float * a, float * res,
+                            int C, int T, int D, int dil, hipStream_t st) {
+    if (x && w && hist && (y || res) && !(res && !a) && C >= 1 && D >= 1 && C % D == 0 && dil >= 1 && 3 * dil <= 32 && T >= 3 * dil && (xscl == nullptr) == (xw == nullptr) &&
+        ple_taps(x, xw, w, y, a, res, C, T, D, dil)) {
+        launch_ple_taps(x, xscl, xw, w, hist, y, a, res, C, T, D, dil, hist, st);
+        CAMX_LAUNCH_RET();
+    }
+    const int rc = camx_pf_ple_conv(x, xscl, xw, w, hist, y, a, res, C, T, D, dil, st);
+    return rc ? rc : camx_pf_ple_hist(x, xscl, xw, hist, C, T, D, dil, st);
 }
 
 }   // extern "C"

@@ -166,6 +166,8 @@ def _glue(K):
             'pf_hc_post': _plain('camx_pf_hc_post'), 'pf_hc_mean': _plain('camx_pf_hc_mean'),
             'pf_gdn_conv': ('camx_pf_gdn_conv', lambda g, b, v: list(v) + [I(0)]),
             'pf_conv_state': ('camx_pf_conv_state', lambda g, b, v: list(v) + [I(0)]),
+            # not symbols of the reference: each a launch of its own followed by the one that advances its history, in one
+            'pf_gdn_conv_commit': ('camx_pf_gdn_conv_commit', lambda g, b, v: list(v) + [I(0)]), 'pf_ple_conv_commit': _plain('camx_pf_ple_conv_commit'),
             'pf_add_sum': ('camx_pf_add_sum', lambda g, b, v: [v[0], v[1], v[2], L64(_val(v[3]))]),
             'pf_silu_bf16': _plain('camx_pf_silu_bf16'), 'pf_to_bf16': _plain('camx_pf_to_bf16'),
             'pf_ple_gate': _rows('camx_pf_ple_gate'), 'pf_ple_conv': _plain('camx_pf_ple_conv'), 'pf_ple_hist': _plain('camx_pf_ple_hist')}

@@ -7,6 +7,7 @@ import ctypes
 import torch
 
 from ..device.bufcheck import LaunchCheck
+from ..device import hip
 from ..device.hip import Module
 
 GLUE_MODULES = {'prefill_glue': 2560, 'prefill_glue_q35': 2048, 'prefill_glue_q35d': 5120}     # module -> row length
@@ -87,8 +88,12 @@ class Glue:
             raise ValueError(f'gdn_conv: C {C} T {T} ldx {ldx} ldy {ldy}')
         _check(self.dev, 'gdn_conv', dict(x=(x, F32, (T - 1) * ldx + C), w=(w, F32, C * 4), state=(state, F32, C * 3), y=(y, F32, (T - 1) * ldy + C)),
                ('y', 'state'))
-        self._go('pf_gdn_conv', T * C, x, w, state, y, ctypes.c_int(C), ctypes.c_int(T), ctypes.c_int(ldx), ctypes.c_int(ldy))
-        self._go('pf_conv_state', C, x, state, ctypes.c_int(C), ctypes.c_int(T), ctypes.c_int(ldx))
+        I = ctypes.c_int
+        if hip.RECORD is None:
+            self._go('pf_gdn_conv_commit', T * C, x, w, state, y, I(C), I(T), I(ldx), I(ldy))
+        else:                                     # a recorder sees the reference's two launches
+            self._go('pf_gdn_conv', T * C, x, w, state, y, I(C), I(T), I(ldx), I(ldy))
+            self._go('pf_conv_state', C, x, state, I(C), I(T), I(ldx))
 
     def ple_gate(self, kn, qn, val, gated, gate, T, HC, D=None, ldv=None, qscale=None, qw=None):
         """per token and stream: gate = sigmoid(sgn(s) sqrt(max(|s|, 1e-6))), s = kn . qn / sqrt(D); gated = val * gate.
@@ -124,9 +129,12 @@ class Glue:
         bufs = dict(x=(x, F32, T * C), xscale=(xscale, F32, T * (C // D)), xw=(xw, F32, C), w=wspec, hist=(hist, F32, C * 3 * dil), y=(y, F32, T * C),
                     a=(a, F32, T * C), res=(res, F32, T * C))
         _check(self.dev, 'ple_conv', bufs, ('hist', 'y', 'res'), opt=('xscale', 'xw', 'y', 'a', 'res'))
-        n = self._nul
-        self._go('pf_ple_conv', T * C, x, n(xscale), n(xw), w_f16, hist, n(y), n(a), n(res), ctypes.c_int(C), ctypes.c_int(T), ctypes.c_int(D), ctypes.c_int(dil))
-        self._go('pf_ple_hist', C, x, n(xscale), n(xw), hist, ctypes.c_int(C), ctypes.c_int(T), ctypes.c_int(D), ctypes.c_int(dil))
+        n, tail = self._nul, (ctypes.c_int(C), ctypes.c_int(T), ctypes.c_int(D), ctypes.c_int(dil))
+        if hip.RECORD is None:
+            self._go('pf_ple_conv_commit', T * C, x, n(xscale), n(xw), w_f16, hist, n(y), n(a), n(res), *tail)
+        else:                                     # a recorder sees the reference's two launches
+            self._go('pf_ple_conv', T * C, x, n(xscale), n(xw), w_f16, hist, n(y), n(a), n(res), *tail)
+            self._go('pf_ple_hist', C, x, n(xscale), n(xw), hist, *tail)
 
     def add_sum(self, a, b, y, n):
         """y += a + b (y may be a or b exactly)"""

@@ -322,6 +322,8 @@ int camx_pf_gdn_conv(const void * x, const float * w, const float * state, void 
                      camx_stream_t stream);
 /* pf_conv_state (kernels/prefill_glue.hip:334-341): state[c] = the last 3 inputs of [state[c], x[0 .. T-1][c]]. */
 int camx_pf_conv_state(const void * x, float * state, int C, int T, int ldx, int bf16, camx_stream_t stream);
+/* camx_pf_gdn_conv, then camx_pf_conv_state on the same rows (one launch where the chunk kernel takes them); x does not overlap y or state. */
+int camx_pf_gdn_conv_commit(const void * x, const float * w, float * state, void * y, int C, int T, int ldx, int ldy, int bf16, camx_stream_t stream);
 /* pf_gdn_l2 (kernels/prefill_gdn.hip:66-78) = OP_GDN_L2 (kernels/k3_q35_ops.h:181-194): per head of K <= 512 values
  * y = (scale * x) * (1 / sqrt(K)), scale = 1 / sqrt(sum x^2 / K + rs); head h of token t at x + t * ldx + h * K. */
 int camx_pf_gdn_l2(const void * x, void * y, int heads, int K, int ldx, float rs, int T, int bf16, camx_stream_t stream);
@@ -377,6 +379,9 @@ int camx_pf_ple_gate(const float * kn, const float * q, const float * qscl, cons
 int camx_pf_ple_conv(const float * x, const float * xscl, const float * xw, const uint16_t * w, const float * hist, float * y, const float * a,
                      float * res, int C, int T, int D, int dil, camx_stream_t stream);
 int camx_pf_ple_hist(const float * x, const float * xscl, const float * xw, float * hist, int C, int T, int D, int dil, camx_stream_t stream);
+/* camx_pf_ple_conv, then camx_pf_ple_hist on the same rows (3 dil <= 32; one launch where T >= 3 dil); x overlaps neither hist nor an output. */
+int camx_pf_ple_conv_commit(const float * x, const float * xscl, const float * xw, const uint16_t * w, float * hist, float * y, const float * a,
+                            float * res, int C, int T, int D, int dil, camx_stream_t stream);
 
 /* ---- activation fake-quant, forward (kernels/actq.hip) ------------------------------------------------------------------------------ */
 /* actq_fwd_{f32,bf16} and actq_fwd_codes_{f32,bf16} (kernels/actq.hip:96-132, 315-326): M rows of K values (K % 128 == 0,

@@ -204,3 +204,53 @@ def test_op_gdn_conv_lazy_commit(C, T):
         yc = dev(np.zeros((T, C), np.float32))                      # the chunk kernel from the committed state: the same bits
         call('camx_pf_gdn_conv', ptr(dev(x2)), ptr(wd), ptr(std), ptr(yc), I(C), I(T), I(C), I(C), I(0))
         assert bits_equal(host(yc), host(y2))
+
+
+def _same(a, b):
+    import torch
+    return bool(((a == b) | (torch.isnan(a) & torch.isnan(b))).all())
+
+
+@pytest.mark.parametrize('T', [128, 129, 131, 257, 2047, 2048, 2049, 2053])
+@pytest.mark.parametrize('bf16', [0, 1])
+def test_gdn_conv_tokens_do_not_depend_on_the_chunk(T, bf16):
+    """the chunk kernel (from 2^20 values, more tokens a wave from 2^24) against the same tokens in pieces of 64, which the kernel of one value a
+    thread takes, its state advanced by camx_pf_conv_state; the committing entry's y and state against both; chunks that end inside a
+    wave's tokens and inside a workgroup; values beyond the exponential's short form, infinities and a NaN; nothing behind the last row"""
+    import torch
+    C, ldx, ldy = 8192, 8200, 8208
+    g = torch.Generator(device='cuda'); g.manual_seed(T)
+    x = torch.randn(T, ldx, generator=g, device='cuda')
+    x[::7, 5::11] *= 300; x[T // 2, 17] = float('inf'); x[3, 40] = float('nan'); x[T - 1, 8191] = -float('inf'); x[5, :16] = 0
+    w = torch.randn(C, 4, generator=g, device='cuda'); st0 = torch.randn(C, 3, generator=g, device='cuda')
+    dt = torch.bfloat16 if bf16 else torch.float32
+    x = x.to(dt)
+    parts, st = torch.empty(T, ldy, device='cuda', dtype=dt), st0.clone()
+    for lo in range(0, T, 64):
+        m = min(64, T - lo)
+        call('camx_pf_gdn_conv', ptr(x[lo:]), ptr(w), ptr(st), ptr(parts[lo:]), I(C), I(m), I(ldx), I(ldy), I(bf16))
+        call('camx_pf_conv_state', ptr(x[lo:]), ptr(st), I(C), I(m), I(ldx), I(bf16))
+    for entry in ('camx_pf_gdn_conv', 'camx_pf_gdn_conv_commit'):
+        y, st1 = torch.full((T + 1, ldy), 7.0, device='cuda', dtype=dt), st0.clone()
+        call(entry, ptr(x), ptr(w), ptr(st1), ptr(y), I(C), I(T), I(ldx), I(ldy), I(bf16))
+        torch.cuda.synchronize()
+        assert _same(y[:T, :C], parts[:, :C]) and bool((y[T] == 7).all()) and bool((y[:, C:] == 7).all())
+        assert _same(st1, st if entry.endswith('commit') else st0)
+    y, qk, qk2 = torch.empty(T, C, device='cuda', dtype=dt), torch.empty(T * 16, 128, device='cuda', dtype=dt), torch.empty(T * 16, 128, device='cuda', dtype=dt)
+    call('camx_gdn_conv_l2', ptr(x), ptr(w), ptr(st0), ptr(y), ptr(qk), I(C), I(T), I(ldx), I(C), I(16), F(1e-8), I(bf16))
+    call('camx_pf_gdn_l2', ptr(y), ptr(qk2), I(16), I(128), I(C), F(1e-8), I(T), I(bf16))
+    torch.cuda.synchronize()
+    assert _same(y, parts[:, :C]) and _same(qk, qk2)
+
+
+@pytest.mark.parametrize('T,C', [(1, 64), (2, 8192), (3, 64), (130, 8200), (200, 6000)])
+def test_gdn_conv_commit_is_the_two_launches(T, C):
+    """chunks shorter than the state, below the chunk kernel's size, and channels it does not take"""
+    import torch
+    g = torch.Generator(device='cuda'); g.manual_seed(T)
+    x = torch.randn(T, C, generator=g, device='cuda'); w = torch.randn(C, 4, generator=g, device='cuda'); a = torch.randn(C, 3, generator=g, device='cuda'); b = a.clone()
+    ya, yb = torch.empty(T, C, device='cuda'), torch.empty(T, C, device='cuda')
+    call('camx_pf_gdn_conv', ptr(x), ptr(w), ptr(a), ptr(ya), I(C), I(T), I(C), I(C), I(0)); call('camx_pf_conv_state', ptr(x), ptr(a), I(C), I(T), I(C), I(0))
+    call('camx_pf_gdn_conv_commit', ptr(x), ptr(w), ptr(b), ptr(yb), I(C), I(T), I(C), I(C), I(0))
+    torch.cuda.synchronize()
+    assert torch.equal(ya, yb) and torch.equal(a, b)

@@ -199,3 +199,37 @@ def test_host_wrappers_of_the_new_ops():
     assert np.allclose(host(out), O.gdn_gates(al, be, dt, Aa), rtol=1e-5, atol=1e-6) and bits_equal(host(ya), O.hc_avg(r))
     assert close_16(host(y16.view(torch.int16), np.uint16), O.gdn_norm(o, w, z, 1e-6, silu=True)[1], 'f16')
     assert bits_equal(host(cache.view(torch.int16), np.uint16), O.kv_append16(k, v, M, np.zeros((T + 4, 2 * M), np.uint16), 2)[0]) and int(host(err)[0]) == 0
+
+
+@pytest.mark.parametrize('T,dil', [(1, 3), (8, 3), (9, 3), (11, 3), (12, 3), (13, 3), (36, 3), (50, 1), (51, 2), (301, 3), (77, 10), (30, 10)])
+@pytest.mark.parametrize('rec', [False, True])
+def test_ple_conv_tokens_do_not_depend_on_the_chunk(T, dil, rec):
+    """the kernel of four tokens a wave against the kernel of one value a thread (reached with D = 2), and the committing entry, whose history
+    matches camx_pf_ple_hist's: chunks shorter than the history, of exactly its length, and that end inside a wave's tokens; rows given
+    or recomputed from their scales; large values, infinities and a NaN; nothing behind the last row"""
+    import torch
+    C, D = 1028, 4
+    g = torch.Generator(device='cuda'); g.manual_seed(T + dil)
+    x = torch.randn(T, C, generator=g, device='cuda'); x[T // 2, 7::13] *= 400; x[0, 3] = float('inf'); x[T - 1, 900] = float('nan'); x[T // 3, 64:96] = -0.0
+    w = (torch.randn(C, 4, generator=g, device='cuda') * 0.5).half(); hist = torch.randn(C, 3 * dil, generator=g, device='cuda')
+    # (a scale per row and D channels: the same value for every pair of channels of a group, so that D = 2 reads the same numbers)
+    scl4 = 0.5 + torch.rand(T, C // 4, generator=g, device='cuda'); scl2 = scl4.repeat_interleave(2, 1).contiguous(); xw = torch.randn(C, generator=g, device='cuda')
+    a, res = torch.randn(T, C, generator=g, device='cuda'), torch.randn(T, C, generator=g, device='cuda')
+
+    def same(p, q): return bool(((p == q) | (torch.isnan(p) & torch.isnan(q))).all())
+
+    def run(entry, d, h):
+        y, r = torch.full((T + 1, C), 5.0, device='cuda'), torch.cat([res, torch.full((1, C), 5.0, device='cuda')])
+        sc, sw = (ptr(scl4 if d == 4 else scl2), ptr(xw)) if rec else (NULL, NULL)
+        call(entry, ptr(x), sc, sw, ptr(w), ptr(h), ptr(y), ptr(a), ptr(r), I(C), I(T), I(d), I(dil))
+        torch.cuda.synchronize()
+        assert bool((y[T] == 5).all()) and bool((r[T] == 5).all())
+        return y[:T], r[:T]
+    h0, h1, h2 = hist.clone(), hist.clone(), hist.clone()
+    y0, r0 = run('camx_pf_ple_conv', 2, h0)
+    y1, r1 = run('camx_pf_ple_conv', 4, h1)
+    y2, r2 = run('camx_pf_ple_conv_commit', 4, h2)
+    assert same(y0, y1) and same(r0, r1) and same(y0, y2) and same(r0, r2) and torch.equal(h1, hist) and torch.equal(h0, hist)
+    call('camx_pf_ple_hist', ptr(x), ptr(scl4) if rec else NULL, ptr(xw) if rec else NULL, ptr(h1), I(C), I(T), I(D), I(dil))
+    torch.cuda.synchronize()
+    assert same(h1, h2)
