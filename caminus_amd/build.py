@@ -9,10 +9,12 @@ import glob
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, 'csrc')
 LIB = os.path.join(HERE, 'libcamx.so')
+LAUNCH = os.path.join(HERE, 'device', '_launch.so')          # the Python side's launches (plain C: no device code)
 HIPCC = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
 FLAGS = ['--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC', '-shared', '-ffp-contract=off', '-fno-fast-math',
          '-fhip-fp32-correctly-rounded-divide-sqrt', '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops',
@@ -41,6 +43,8 @@ def build(verbose=False):
         if p.returncode: bad = True; print(f'FAILED: {src}', file=sys.stderr)
     if bad: raise RuntimeError('hipcc failed')
     subprocess.run([HIPCC, '--offload-arch=gfx950', '-shared', '-fPIC', '-o', LIB] + objs, check=True)
+    subprocess.run([os.environ.get('CC', 'gcc'), '-O2', '-Wall', '-Wextra', '-shared', '-fPIC', '-I', sysconfig.get_paths()['include'], '-o', LAUNCH,
+                    os.path.join(CSRC, 'launch.c')], check=True)
     return LIB
 
 

@@ -272,3 +272,65 @@ def test_entry_points_accept_empty_batches_and_refuse_bad_arguments():
         for pos, val in bad:
             args = list(good); args[pos] = val
             assert fn(*args, ST) == 1, (name, pos)
+
+
+# ---- the launch extension (caminus_amd/csrc/launch.c): every entry point's call goes through its one prototype -----------------------------
+
+def _launch_target(types):
+    """a C function of these argument types that keeps what it was given"""
+    got = []
+    fn = ctypes.CFUNCTYPE(ctypes.c_int, *types)(lambda *a: got.append(a) or 7)
+    return got, fn, ctypes.cast(fn, ctypes.c_void_p).value
+
+
+@pytest.mark.parametrize('n_int,n_float', [(0, 0), (1, 0), (0, 1), (6, 8), (7, 3), (16, 8), (17, 2), (40, 8)])
+def test_launch_extension_passes_what_ctypes_passes(n_int, n_float):
+    """bind() and call() against the same C function with its declared types: integers in registers and on the stack, floats between them,
+    values reduced to their width, tensors and None as addresses"""
+    from caminus_amd.device import hip
+    native = hip._load_native()
+    t = torch.zeros(4)
+    kinds = [('i', ctypes.c_int), ('p', ctypes.c_void_p), ('l', ctypes.c_long), ('a', ctypes.c_void_p)]
+    order, ni, nf = [], 0, 0
+    while ni < n_int or nf < n_float:                       # a float after every second integer
+        if nf < n_float and (ni >= n_int or ni >= 2 * nf + 1): order.append(('f', ctypes.c_float)); nf += 1
+        else: order.append(kinds[ni % 4]); ni += 1
+    values = {'i': [3, -1, 2 ** 31 + 5, np.int64(9), True], 'p': [t, None], 'l': [2 ** 40 + 1, -(2 ** 40)], 'a': [2 ** 47 - 8, 16], 'f': [0.1, -2, np.float32(3.5)]}
+    args = [values[s][k % len(values[s])] for k, (s, _) in enumerate(order)]
+    got, keep, address = _launch_target([c for _, c in order])
+    typed = [ctypes.c_void_p(a.data_ptr() if a is t else a) if s in 'pa' else c(a) for (s, c), a in zip(order, args)]
+    want = tuple(v.value for v in typed)
+    assert native.bind(address, ''.join(s for s, _ in order))(*args) == 7 and got.pop() == want
+    if any(s == 'p' for s, _ in order): typed[next(k for k, (s, _) in enumerate(order) if s == 'p' and args[k] is t)] = t
+    assert native.call(address, *typed) == 7 and got.pop() == want
+
+
+def test_launch_extension_refuses_before_it_calls():
+    from caminus_amd.device import hip
+    native = hip._load_native()
+    got, keep, address = _launch_target([ctypes.c_int, ctypes.c_float])
+    entry = native.bind(address, 'if')
+    for bad in ((1.5, 1.0), ('1', 1.0), (1, 'x'), (1,), (1, 1.0, 2), (None, 1.0)):
+        with pytest.raises(TypeError): entry(*bad)
+    with pytest.raises(TypeError): entry(1, 1.0, k=2)
+    with pytest.raises(AttributeError): native.bind(address, 'pf')(5, 1.0)
+    for sig in ('x', 'i\0', 'f' * 9, 'i' * 41):
+        with pytest.raises(ValueError): native.bind(address, sig)
+    with pytest.raises(ValueError): native.bind(0, 'i')
+    # arguments without a type of their own are left to ctypes: nothing is called
+    for a in (1, 1.0, np.float32(1), torch.nn.Parameter(torch.zeros(1)), ctypes.c_uint(1), 'x'):
+        assert native.call(address, a, ctypes.c_float(1)) is NotImplemented
+    assert native.call(address, *[ctypes.c_int(1)] * 41) is NotImplemented and native.call(address, *[ctypes.c_float(1)] * 9) is NotImplemented
+    assert got == []
+
+
+def test_tape_signatures_are_the_headers():
+    """the one prototype checks nothing: every signature the tape binds is the entry point's declaration, the stream last"""
+    text = re.sub(r'/\*.*?\*/|//[^\n]*', '', open(os.path.join(ROOT, 'include', 'camx.h')).read(), flags=re.S)
+    declared = {n: re.sub(r'\s+', ' ', a).split(',') for n, a in re.findall(r'\bint (camx_[a-z0-9_]+)\s*\(([^)]*)\)', text)}
+    kind = lambda a: 'p' if '*' in a else 'a' if 'stream' in a.lower() else 'f' if 'float' in a else 'i' if re.match(r'\s*(const )?(int|int32_t|unsigned) ', a) else '?'
+    bound = re.findall(r"_go\('(camx_\w+)', '([a-z]+)'", open(os.path.join(ROOT, 'caminus_amd', 'engine', 'k3.py')).read())
+    assert len(bound) >= 20
+    for name, sig in bound:
+        want = ''.join(kind(a) for a in declared[name])
+        assert sig[:-1] == want[:-1] and sig[-1] == 'a' and 'stream' in declared[name][-1], (name, sig, want)
