@@ -595,7 +595,7 @@ struct SinkSiluMul {
         dgp = pack_f2bf_x4(dg); dup = pack_f2bf_x4(du);
     }
     // (the gates and multipliers are read a second time here: held in registers since the source fetched them they cost 48 more,
-    // two waves per SIMD instead of three, and 8192 x 2048 takes 65 us instead of 62)
+    // two waves per SIMD instead of three: 8192 x 2048 65 us instead of 62 in the layout of four values a lane, 41.6 in this one)
     CAMX_DEV void st8(int row, int k, const float (&v)[8], u32x4 keep, bool stream) const {
         const f32x4 a = {v[0], v[1], v[2], v[3]}, b = {v[4], v[5], v[6], v[7]};
         const uint16_t * r = gu + (size_t)row * ld + k;
