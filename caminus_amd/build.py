@@ -7,14 +7,17 @@ default), packed-fp32 instruction selection off.
 """
 import glob
 import os
+import platform
+import shutil
 import subprocess
 import sys
 import sysconfig
 
+from .device.kernels import launch_extension
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, 'csrc')
 LIB = os.path.join(HERE, 'libcamx.so')
-LAUNCH = os.path.join(HERE, 'device', '_launch.so')          # the Python side's launches (plain C: no device code)
 HIPCC = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
 FLAGS = ['--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC', '-shared', '-ffp-contract=off', '-fno-fast-math',
          '-fhip-fp32-correctly-rounded-divide-sqrt', '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops',
@@ -43,9 +46,21 @@ def build(verbose=False):
         if p.returncode: bad = True; print(f'FAILED: {src}', file=sys.stderr)
     if bad: raise RuntimeError('hipcc failed')
     subprocess.run([HIPCC, '--offload-arch=gfx950', '-shared', '-fPIC', '-o', LIB] + objs, check=True)
-    subprocess.run([os.environ.get('CC', 'gcc'), '-O2', '-Wall', '-Wextra', '-shared', '-fPIC', '-I', sysconfig.get_paths()['include'], '-o', LAUNCH,
-                    os.path.join(CSRC, 'launch.c')], check=True)
+    build_launch()
     return LIB
+
+
+def build_launch():
+    """the Python side's launch extension for the running interpreter (plain C: no device code). Where it cannot be built, launches go through ctypes"""
+    out, cc, include = launch_extension(), os.environ.get('CC', 'gcc'), sysconfig.get_paths()['include']
+    if os.path.exists(out): os.remove(out)               # (never one of another source)
+    lacks = ([f'an x86-64 machine (this one: {platform.machine()})'] if platform.machine() not in ('x86_64', 'AMD64') else []) + \
+            ([f'the compiler {cc}'] if not shutil.which(cc.split()[0]) else []) + ([f"{include}/Python.h"] if not os.path.isfile(os.path.join(include, 'Python.h')) else [])
+    if lacks:
+        print(f"launch extension not built, it needs {', '.join(lacks)}: launches go through ctypes", file=sys.stderr)
+        return None
+    subprocess.run(cc.split() + ['-O2', '-Wall', '-Wextra', '-shared', '-fPIC', '-I', include, '-o', out, os.path.join(CSRC, 'launch.c')], check=True)
+    return out
 
 
 if __name__ == '__main__':

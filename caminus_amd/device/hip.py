@@ -13,6 +13,9 @@ shape arguments where the reference kernel would have read them.
 There is no fallback path: a missing library is a FileNotFoundError, an unknown symbol an AttributeError.
 """
 import ctypes
+import importlib.util
+import os
+import warnings
 
 import torch
 
@@ -45,19 +48,24 @@ def stream_handle():
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
-_native = None       # the extension that calls the C entry points (csrc/launch.c); loaded with the library
+_native = None       # the extension that calls the C entry points (csrc/launch.c), or False where there is none for this interpreter; set with the library
 _bound = {}
 
 
 def _load_native():
     global _native
     if _native is None:
-        try:
-            from . import _launch
-        except ImportError as e:
-            raise FileNotFoundError(f'caminus_amd.device._launch is not built ({e}); run python -m caminus_amd.build') from None
-        _launch.setup(torch.Tensor, ctypes.c_int, ctypes.c_long, ctypes.c_float, ctypes.c_void_p)
-        _native = _launch
+        path, ext = _kernels.launch_extension(), False
+        if os.path.isfile(path):
+            try:
+                spec = importlib.util.spec_from_file_location(__package__ + '._launch', path)
+                ext = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(ext)
+                ext.setup(torch.Tensor, ctypes.c_int, ctypes.c_long, ctypes.c_float, ctypes.c_void_p)
+            except ImportError as e:
+                warnings.warn(f'{path} does not load ({e}): launches go through ctypes')
+                ext = False
+        _native = ext
     return _native
 
 
@@ -65,12 +73,27 @@ def _address(fn):
     return ctypes.cast(fn, ctypes.c_void_p).value
 
 
+_CONVERT = {'p': lambda a: ctypes.c_void_p(None if a is None else a.data_ptr()), 'i': ctypes.c_int, 'l': ctypes.c_long, 'f': ctypes.c_float, 'a': ctypes.c_void_p}
+
+
+def _ctypes_entry(fn, sig):
+    """what the extension's bind() gives, through ctypes"""
+    convert = [_CONVERT[c] for c in sig]
+
+    def entry(*args):
+        if len(args) != len(convert):
+            raise TypeError(f'this entry point takes {len(convert)} positional arguments ({len(args)} given)')
+        return fn(*[c(a) for c, a in zip(convert, args)])
+    return entry
+
+
 def bound(name, sig):
     """the C entry point as a callable that converts its arguments natively: sig has 'p' for a tensor or None, 'i' / 'l' for an int / long, 'f' for a
     float, 'a' for an address. 0.5 to 0.9 us for 4 to 25 arguments, where a ctypes object per argument cost 1.2 to 3.1"""
     f = _bound.get(name)
     if f is None:
-        f = _bound[name] = _load_native().bind(_address(getattr(_lib.load(), name)), sig)
+        fn, native = getattr(_lib.load(), name), _load_native()
+        f = _bound[name] = native.bind(_address(fn), sig) if native else _ctypes_entry(fn, sig)
     return f
 
 
@@ -245,7 +268,7 @@ class Kernel:
     def __call__(self, grid, block, *args, shmem=0, stream=None):
         r = RECORD
         grid, block = _dim3(grid), _dim3(block)
-        if r is None and self._addr is not None:            # no recorder wants the converted values: the arguments go on as they are
+        if r is None and self._addr is not None and _native:            # no recorder wants the converted values: the arguments go on as they are
             err = _native.call(self._addr, *self._adapt(grid, block, args), ctypes.c_void_p(stream_handle() if stream is None else stream))
             if err is not NotImplemented:                   # (an argument of another type: ctypes converts or refuses it below)
                 return check(err)

@@ -5,6 +5,7 @@ CAMINUS_KERNEL_DIR environment variable first, else the package's own directory 
 implementation: a missing library is a FileNotFoundError naming how to build it.
 """
 import os
+import sysconfig
 
 ARCH = 'gfx950'
 LIBNAME = 'libcamx.so'
@@ -27,6 +28,12 @@ def kernel_dir():
 def library_path():
     d, _ = kernel_dir()
     return os.path.join(d, LIBNAME)
+
+
+def launch_extension():
+    """the Python side's launch extension (csrc/launch.c) for the running interpreter: part of the package, whatever CAMINUS_KERNEL_DIR names, and
+    optional (device/hip.py launches through ctypes without it)"""
+    return os.path.join(PKG, 'device', '_launch' + sysconfig.get_config_var('EXT_SUFFIX'))
 
 
 def missing_message(name, d, where):

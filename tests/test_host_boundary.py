@@ -324,6 +324,46 @@ def test_launch_extension_refuses_before_it_calls():
     assert got == []
 
 
+@pytest.fixture
+def no_extension(monkeypatch, tmp_path):
+    """a package whose launch extension is not built for this interpreter; another's beside it under its plain name"""
+    from caminus_amd.device import hip
+    path = str(tmp_path / os.path.basename(kernels.launch_extension()))
+    open(tmp_path / '_launch.so', 'wb').write(b'another interpreter')
+    monkeypatch.setattr(kernels, 'launch_extension', lambda: path)
+    monkeypatch.setattr(hip, '_native', None)
+    monkeypatch.setattr(hip, '_bound', {})
+    return path
+
+
+def test_launch_extension_belongs_to_its_interpreter():
+    import importlib.machinery
+    assert os.path.basename(kernels.launch_extension()) == '_launch' + importlib.machinery.EXTENSION_SUFFIXES[0] != '_launch.so'
+
+
+def test_library_alone_serves_every_launch(no_extension, monkeypatch, tmp_path):
+    """a deployment of libcamx.so in CAMINUS_KERNEL_DIR without the launch extension: modules load and their calls reach the entry points (which
+    refuse these null operands, so nothing is launched)"""
+    from caminus_amd.device import hip
+    if not os.path.isfile(kernels.library_path()): pytest.skip('libcamx.so is not built in this checkout (python -m caminus_amd.build)')
+    monkeypatch.setattr(hip, 'RECORD', None)
+    I, null = ctypes.c_int, ctypes.c_void_p(0)
+    m = hip.Module('camx')
+    assert hip._native is False
+    with pytest.raises(RuntimeError, match='HIP error 1'):
+        m.camx_op_add_sum((1,), (256,), null, null, null, I(4), stream=0)
+    assert hip.bound('camx_op_add_sum', 'pppia')(None, None, None, 4, 0) == 1
+    with pytest.raises(TypeError): hip.bound('camx_op_add_sum', 'pppia')(None, None, None, 4)
+    with pytest.raises(TypeError): hip.bound('camx_op_add_sum', 'pppia')(None, None, None, 1.5, 0)
+
+
+def test_launch_extension_that_does_not_load_is_left_out(no_extension):
+    from caminus_amd.device import hip
+    open(no_extension, 'wb').write(b'not a library')
+    with pytest.warns(UserWarning, match='does not load'):
+        assert hip._load_native() is False
+
+
 def test_tape_signatures_are_the_headers():
     """the one prototype checks nothing: every signature the tape binds is the entry point's declaration, the stream last"""
     text = re.sub(r'/\*.*?\*/|//[^\n]*', '', open(os.path.join(ROOT, 'include', 'camx.h')).read(), flags=re.S)
