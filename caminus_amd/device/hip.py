@@ -90,10 +90,10 @@ def _ctypes_entry(fn, sig):
 def bound(name, sig):
     """the C entry point as a callable that converts its arguments natively: sig has 'p' for a tensor or None, 'i' / 'l' for an int / long, 'f' for a
     float, 'a' for an address. 0.5 to 0.9 us for 4 to 25 arguments, where a ctypes object per argument cost 1.2 to 3.1"""
-    f = _bound.get(name)
+    f = _bound.get((name, sig))
     if f is None:
         fn, native = getattr(_lib.load(), name), _load_native()
-        f = _bound[name] = native.bind(_address(fn), sig) if native else _ctypes_entry(fn, sig)
+        f = _bound[name, sig] = native.bind(_address(fn), sig) if native else _ctypes_entry(fn, sig)
     return f
 
 

@@ -364,6 +364,18 @@ def test_launch_extension_that_does_not_load_is_left_out(no_extension):
         assert hip._load_native() is False
 
 
+def test_bound_entry_points_are_kept_by_their_signature_too(monkeypatch):
+    """the same entry point under another signature converts by that one"""
+    from caminus_amd.device import hip, lib
+    got, keep, address = _launch_target([ctypes.c_int, ctypes.c_int])
+    monkeypatch.setattr(hip, '_bound', {})
+    monkeypatch.setattr(lib, '_lib', type('L', (), {'camx_probe': keep}))
+    assert hip.bound('camx_probe', 'ii')(-1, 2) == 7 and got.pop() == (-1, 2)
+    with pytest.raises(TypeError): hip.bound('camx_probe', 'if')('x', 2.0)
+    with pytest.raises(TypeError): hip.bound('camx_probe', 'i')(1, 2)
+    assert hip.bound('camx_probe', 'ii') is hip.bound('camx_probe', 'ii') and got == []
+
+
 def test_tape_signatures_are_the_headers():
     """the one prototype checks nothing: every signature the tape binds is the entry point's declaration, the stream last"""
     text = re.sub(r'/\*.*?\*/|//[^\n]*', '', open(os.path.join(ROOT, 'include', 'camx.h')).read(), flags=re.S)
