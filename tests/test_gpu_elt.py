@@ -243,6 +243,30 @@ def test_gdn_conv_tokens_do_not_depend_on_the_chunk(T, bf16):
     assert _same(y, parts[:, :C]) and _same(qk, qk2)
 
 
+@pytest.mark.parametrize('T,C,bf16', [(16 * 65535 + 5, 8, 1), (16 * 65535 + 21, 4, 0), (32 * 65535 + 77, 128, 1)])
+def test_gdn_conv_past_65535_groups_of_tokens(T, C, bf16):
+    """more token groups than a grid has workgroups in y: the same rows in slices through the one-value kernel"""
+    import torch
+    g = torch.Generator(device='cuda'); g.manual_seed(C)
+    dt = torch.bfloat16 if bf16 else torch.float32
+    x = torch.randn(T, C, generator=g, device='cuda').to(dt); w = torch.randn(C, 4, generator=g, device='cuda'); st0 = torch.randn(C, 3, generator=g, device='cuda')
+    want, st, n = torch.empty_like(x), st0.clone(), (1 << 20) // C - 1
+    for lo in range(0, T, n):
+        m = min(n, T - lo)
+        call('camx_pf_gdn_conv', ptr(x[lo:]), ptr(w), ptr(st), ptr(want[lo:]), I(C), I(m), I(C), I(C), I(bf16))
+        call('camx_pf_conv_state', ptr(x[lo:]), ptr(st), I(C), I(m), I(C), I(bf16))
+    y, st1 = torch.full_like(x, 7.0), st0.clone()
+    call('camx_pf_gdn_conv_commit', ptr(x), ptr(w), ptr(st1), ptr(y), I(C), I(T), I(C), I(C), I(bf16))
+    torch.cuda.synchronize()
+    assert _same(y, want) and _same(st1, st)
+    if C % 128 == 0:
+        y.fill_(7.0); qk, qk2 = torch.empty(T, 128, device='cuda', dtype=dt), torch.empty(T, 128, device='cuda', dtype=dt)
+        call('camx_gdn_conv_l2', ptr(x), ptr(w), ptr(st0), ptr(y), ptr(qk), I(C), I(T), I(C), I(C), I(1), F(1e-8), I(bf16))
+        call('camx_pf_gdn_l2', ptr(want), ptr(qk2), I(1), I(128), I(C), F(1e-8), I(T), I(bf16))
+        torch.cuda.synchronize()
+        assert _same(y, want) and _same(qk, qk2)
+
+
 @pytest.mark.parametrize('T,C', [(1, 64), (2, 8192), (3, 64), (130, 8200), (200, 6000)])
 def test_gdn_conv_commit_is_the_two_launches(T, C):
     """chunks shorter than the state, below the chunk kernel's size, and channels it does not take"""
