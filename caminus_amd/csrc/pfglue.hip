@@ -362,7 +362,59 @@ __global__ void __launch_bounds__(256) ple_conv_k(const float * __restrict__ x, 
     if (y) y[i] = o;
     if (res) { const float ab = a[i] + o; res[i] = res[i] + ab; }
 }
-// The same for C % 4 == 0, D % 4 == 0 and 16-byte aligned operands: a lane owns four channels, a wave TPW tokens dil apart (t0, t0 + dil, ..), whose rows
+// The same for C % 4 == 0, D % 4 == 0 and 16-byte aligned operands, small batches (bound by the launch and one chain of loads): the token
+// in blockIdx.y (no division of an element index), four channels per thread (their sixteen fp16 weights in two 16-byte loads), streamed
+// outputs non-temporal
+__global__ void __launch_bounds__(256) ple_conv_rows(const float * __restrict__ x, const float * __restrict__ xscl, const float * __restrict__ xw,
+                                                     const uint16_t * __restrict__ w, const float * __restrict__ hist, float * __restrict__ y,
+                                                     const float * __restrict__ a, float * __restrict__ res, int C, int D, int dil) {
+    // workgroup i runs on XCD i mod 8, each with its own L2: an XCD takes a contiguous range of tokens, so that the three earlier rows a
+    // token reads were fetched into the same L2 by its neighbours a moment ago (with tokens dealt round-robin every row crossed the fabric
+    // four times: 67 MB read for 17 MB of input at 4096 x 1024)
+    const int total = gridDim.x * gridDim.y, lin = blockIdx.x + gridDim.x * blockIdx.y, xcd = lin & 7;
+    const int nw = xcd * (total >> 3) + min(xcd, total & 7) + (lin >> 3), t = nw / gridDim.x, bx = nw - t * gridDim.x;
+    const int c = 4 * (bx * 256 + threadIdx.x), hl = 3 * dil;
+    if (c >= C) return;
+    const u32x4 w0 = *(const u32x4 *)(w + (size_t)c * 4), w1 = *(const u32x4 *)(w + (size_t)c * 4 + 8);
+    const uint32_t ww[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};      // channel j's taps: halves 4 j .. 4 j + 3
+    f32x4 xwv = {1.0f, 1.0f, 1.0f, 1.0f};
+    if (xscl) xwv = *(const f32x4 *)(xw + c);
+    float conv[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int back = (3 - k) * dil;
+        float xv[4];
+        if (back <= t) {
+            const int tb = t - back;
+            const f32x4 v = *(const f32x4 *)(x + (size_t)tb * C + c);
+            xv[0] = v.x; xv[1] = v.y; xv[2] = v.z; xv[3] = v.w;
+            if (xscl) {
+                const float sc = xscl[tb * (C / D) + c / D];
+                xv[0] = (xv[0] * sc) * xwv.x; xv[1] = (xv[1] * sc) * xwv.y; xv[2] = (xv[2] * sc) * xwv.z; xv[3] = (xv[3] * sc) * xwv.w;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) xv[j] = hist[(size_t)(c + j) * hl + hl - (back - t)];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t pair = ww[2 * j + (k >> 1)];
+            const float term = xv[j] * h2f_bits((uint16_t)((k & 1) ? pair >> 16 : pair & 0xffffu));
+            conv[j] = k == 0 ? term : conv[j] + term;
+        }
+    }
+    f32x4 o;
+    o.x = conv[0] / (1.0f + expf(-conv[0])); o.y = conv[1] / (1.0f + expf(-conv[1]));
+    o.z = conv[2] / (1.0f + expf(-conv[2])); o.w = conv[3] / (1.0f + expf(-conv[3]));
+    const size_t i = (size_t)t * C + c;
+    if (y) __builtin_nontemporal_store(o, (f32x4 *)(y + i));
+    if (res) {
+        const f32x4 av = __builtin_nontemporal_load((const f32x4 *)(a + i)), rv = __builtin_nontemporal_load((const f32x4 *)(res + i));
+        f32x4 r; r.x = rv.x + (av.x + o.x); r.y = rv.y + (av.y + o.y); r.z = rv.z + (av.z + o.z); r.w = rv.w + (av.w + o.w);
+        __builtin_nontemporal_store(r, (f32x4 *)(res + i));
+    }
+}
+// Larger batches: a lane owns four channels, a wave TPW tokens dil apart (t0, t0 + dil, ..), whose rows
 // and the three before them, every one a tap of four of its tokens, are all requested before the first is used: (TPW + 3) / TPW rows
 // requested per token, where a thread per token requested four (x 10240, dilation 3, caller's buffers in rotation: 777 tokens 22.6 -> 11.5 us, 2048
 // tokens 49.7 -> 30.8, 4096 102 -> 58; floor 9.8, 25.8, 51.6; eight tokens a wave 11.8, 31.5, 59.2). Streamed outputs are non-temporal.
@@ -600,9 +652,21 @@ int camx_pf_ple_gate(const float * kn, const float * q, const float * qscl, cons
 }
 #define PLE_TPW 4
 static long ple_waves(int T, int dil) { const long per = (long)dil * PLE_TPW; return (T + per - 1) / per * dil; }
+static bool ple_vec(const float * x, const float * xw, const uint16_t * w, const float * y, const float * a, const float * res, int C, int D) {
+    return C % 4 == 0 && D % 4 == 0 && !(((uintptr_t)x | (uintptr_t)xw | (uintptr_t)w | (uintptr_t)y | (uintptr_t)a | (uintptr_t)res) & 15);
+}
 static bool ple_taps(const float * x, const float * xw, const uint16_t * w, const float * y, const float * a, const float * res, int C, int T, int D, int dil) {
-    return C % 4 == 0 && D % 4 == 0 && dil <= 65535 && (ple_waves(T, dil) + 3) / 4 <= 65535 &&
-           !(((uintptr_t)x | (uintptr_t)xw | (uintptr_t)w | (uintptr_t)y | (uintptr_t)a | (uintptr_t)res) & 15);
+    return ple_vec(x, xw, w, y, a, res, C, D) && dil <= 65535 && (ple_waves(T, dil) + 3) / 4 <= 65535;
+}
+// A thread per token while its waves are resident at once, thirty-two a CU, or where the waves above have no grid. Its history reads are scattered (a lane's
+// channels lie 3 dil floats apart, up to a line each), so the tokens that read it count for more. This form / the waves above, dilation 3: 16 x 10240 3.3 / 4.2 us,
+// 64 x 2560 3.2 / 4.3, 256 x 1024 3.2 / 4.2, 640 x 2560 5.4 / 5.5, 2048 x 1024 5.6 / 6.2; 2560 x 1024 7.7 / 6.8, 128 x 10240 5.6 / 5.2; dilation 8: 2048 x 256
+// 3.6 / 5.2, 4096 x 256 4.6 / 5.7, 640 x 2560 8.0 / 6.5. (The committing entry keeps the waves at every size: one launch instead of this form and the history's.)
+static bool ple_rows(const float * x, const float * xw, const uint16_t * w, const float * y, const float * a, const float * res, int C, int T, int D, int dil) {
+    if (!ple_vec(x, xw, w, y, a, res, C, D) || T > 65535) return false;
+    if (dil > 65535) return true;
+    const long past = T < 3 * dil ? T : 3 * dil;
+    return (T + 4L * dil * past) * ((C + 255) / 256) < 9000;
 }
 static void launch_ple_taps(const float * x, const float * xscl, const float * xw, const uint16_t * w, const float * hist, float * y, const float * a, float * res,
                             int C, int T, int D, int dil, float * commit, hipStream_t st) {
@@ -614,6 +678,10 @@ int camx_pf_ple_conv(const float * x, const float * xscl, const float * xw, cons
     if (!x || !w || !hist || (!y && !res) || (res && !a) || C < 1 || T < 0 || D < 1 || C % D || dil < 1 || ((xscl == nullptr) != (xw == nullptr))) return CAMX_EINVAL;
     if (T == 0) return CAMX_OK;
     if ((long)T * C >= 0x7fffffffL * 256) return CAMX_EINVAL;
+    if (ple_rows(x, xw, w, y, a, res, C, T, D, dil)) {
+        ple_conv_rows<<<dim3((unsigned)((C / 4 + 255) / 256), (unsigned)T), dim3(256), 0, st>>>(x, xscl, xw, w, hist, y, a, res, C, D, dil);
+        CAMX_LAUNCH_RET();
+    }
     if (ple_taps(x, xw, w, y, a, res, C, T, D, dil)) { launch_ple_taps(x, xscl, xw, w, hist, y, a, res, C, T, D, dil, nullptr, st); CAMX_LAUNCH_RET(); }
     ple_conv_k<<<dim3((unsigned)(((long)T * C + 255) / 256)), dim3(256), 0, st>>>(x, xscl, xw, w, hist, y, a, res, C, T, D, dil);
     CAMX_LAUNCH_RET();

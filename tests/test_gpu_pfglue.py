@@ -233,3 +233,9 @@ def test_ple_conv_tokens_do_not_depend_on_the_chunk(T, dil, rec):
     call('camx_pf_ple_hist', ptr(x), ptr(scl4) if rec else NULL, ptr(xw) if rec else NULL, ptr(h1), I(C), I(T), I(D), I(dil))
     torch.cuda.synchronize()
     assert same(h1, h2)
+
+
+@pytest.mark.parametrize('T,dil', [(1691, 3), (1692, 3), (1697, 3), (76, 7), (1211, 7), (1212, 7), (1787, 1), (1788, 1), (1793, 1)])
+def test_ple_conv_at_the_line_between_its_kernels(T, dil):
+    """camx_pf_ple_conv on both sides of the batch size from which a wave takes four tokens (1028 channels, five waves a token: T + 4 dil 3 dil = 1800)"""
+    test_ple_conv_tokens_do_not_depend_on_the_chunk(T, dil, bool(T & 1))
