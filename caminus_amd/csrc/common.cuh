@@ -199,16 +199,11 @@ CAMX_DEV void pf_q8_0_emit(f32x4 xv, uint8_t * blk, int sub, bool active) {     
     if (sub == 0) *(uint16_t *)blk = f2h_bits(d);
 }
 
-// ---- x / (1 + expf(-x)) of N values: the library exponential's and the IEEE division's bits in two thirds of their issue cycles ----------
-// For |x| <= 80 the exponential needs no range checks (the library's own steps without them) and the division no scaling: rcp(den) is good
-// enough that one residual step gives the correctly rounded quotient (all inputs of that range compared on the card: the same bits but for
-// the sign of -0, which is copied). A lane with a larger value, an infinity or a NaN takes the plain form.
-CAMX_DEV float one_plus_exp_neg(float x) {                        // 1 + expf(-x), |x| <= 80
-    const float l2e = -1.44269502162933349609f, l2e_low = -1.92596303256e-8f;          // -log2(e) in two parts
-    const float t = x * l2e, n = __builtin_rintf(t);
-    const float low = __builtin_fmaf(x, l2e_low, __builtin_fmaf(x, l2e, -t));
-    return 1.0f + __builtin_ldexpf(__builtin_amdgcn_exp2f((t - n) + low), (int)n);
-}
+// ---- x / (1 + expf(-x)) of N values with the IEEE division's bits in half of its issue cycles ---------------------------------------------
+// For |x| <= 80 no step of the division leaves the range of normal numbers, so it needs no scaling: v_rcp_f32 and one residual step (Markstein, IBM J.
+// Res. Dev. 34, 1990; the sign of -0 is copied). A lane with a larger value, an infinity or a NaN divides. The kernels for small batches divide in
+// any case, and a token's bits must not depend on the batch it came in: with a reciprocal an ulp off the step is exact for every input of this range and not
+// in general, which test_silu_of_every_finite_value checks by comparing the two kernels over all finite inputs.
 template <int N>
 CAMX_DEV void silu_group(float (&v)[N]) {
     float most = 0.0f, in[N];
@@ -219,7 +214,7 @@ CAMX_DEV void silu_group(float (&v)[N]) {
     for (int k = 0; k < N; k += 2) nan |= __builtin_isunordered(v[k], v[(k + 1) % N]);
 #pragma unroll
     for (int k = 0; k < N; k++) {
-        const float den = one_plus_exp_neg(in[k]), r = __builtin_amdgcn_rcpf(den), q = in[k] * r;
+        const float den = 1.0f + expf(-in[k]), r = __builtin_amdgcn_rcpf(den), q = in[k] * r;
         v[k] = __builtin_copysignf(__builtin_fmaf(__builtin_fmaf(-den, q, in[k]), r, q), in[k]);
     }
     if (__builtin_expect(most > 80.0f || nan, 0)) {

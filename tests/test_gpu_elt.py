@@ -278,3 +278,27 @@ def test_gdn_conv_commit_is_the_two_launches(T, C):
     call('camx_pf_gdn_conv_commit', ptr(x), ptr(w), ptr(b), ptr(yb), I(C), I(T), I(C), I(C), I(0))
     torch.cuda.synchronize()
     assert torch.equal(ya, yb) and torch.equal(a, b)
+
+
+@pytest.mark.parametrize('entry', ['gdn', 'ple'])
+@pytest.mark.parametrize('part', range(4))
+def test_silu_of_every_finite_value(entry, part):
+    """a token's bits do not depend on the batch it came in: the convolutions' chunk kernels (their own division up to 80) against the kernels
+    for small batches (the IEEE division), the last tap alone, over all finite fp32 inputs, 2^28 at a time"""
+    import torch
+    T, C = 32768, 8192
+    w = torch.zeros(C, 4, device='cuda'); w[:, 3] = 1.0; st = torch.zeros(C, 3, device='cuda'); w16 = w.half()
+
+    def conv(x, y, n):
+        if entry == 'gdn': call('camx_pf_gdn_conv', ptr(x), ptr(w), ptr(st), ptr(y), I(C), I(n), I(C), I(C), I(0))
+        else: call('camx_pf_ple_conv', ptr(x), NULL, NULL, ptr(w16), ptr(st), ptr(y), NULL, NULL, I(C), I(n), I(C), I(1))
+    for k in range(4 * part, 4 * part + 4):
+        first = (k << 28) - (1 << 31)
+        bits = torch.arange(1 << 28, dtype=torch.int32, device='cuda') + first
+        bits[(bits & 0x7f800000) == 0x7f800000] = 0
+        x = bits.view(torch.float32).view(T, C)
+        y, z = torch.empty_like(x), torch.empty_like(x)
+        conv(x, y, T)
+        for lo in range(0, T, 127): conv(x[lo:], z[lo:], min(127, T - lo))          # (127 x 8192 values: below every chunk kernel's batch)
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int32), z.view(torch.int32)), k
