@@ -180,7 +180,7 @@ __global__ void __launch_bounds__(256) op_gdn_conv_k(const float * __restrict__ 
 // commit (T >= 3): the state's buffer, which the wave of the first tokens, the only reader of its channels, leaves holding the last three inputs.
 CAMX_DEV void l2_head_w8(const float (&v)[8], float (&o)[8], float rs);
 CAMX_DEV f32x4 l2_head_l4(f32x4 v, int lane, float rs);
-constexpr int CONV_GRID_Y = 65535;                                     // workgroups in y; more token groups go on in z
+constexpr int CONV_GROUPS = 65535;                                     // workgroups in y
 template <bool BF16, bool L2, int TPW, bool STREAM>
 __global__ void __launch_bounds__(256) gdn_conv_rows(const void * __restrict__ x, const float * __restrict__ w, const float * st,
                                                      void * __restrict__ y, int C, int T, int ldx, int ldy,
@@ -188,9 +188,8 @@ __global__ void __launch_bounds__(256) gdn_conv_rows(const void * __restrict__ x
     constexpr int VW = BF16 ? 8 : 4;
     const int lane_l2 = slot_of(threadIdx.x & 63), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int cv = blockIdx.x * 64 + (L2 && !BF16 ? lane_l2 : (int)(threadIdx.x & 63));
-    const long tl = (((long)blockIdx.z * CONV_GRID_Y + blockIdx.y) * 4 + wave) * TPW;
-    const int c0 = cv * VW, t0 = (int)tl;
-    if (c0 >= C || tl >= T) return;
+    const int c0 = cv * VW, t0 = (blockIdx.y * 4 + wave) * TPW;
+    if (c0 >= C || t0 >= T) return;
     u32x4 raw[TPW + 3];                                                // row t0 - 3 + j (clamped: before the chunk the state stands in, behind it nothing is stored)
     auto at = [&](int j) {
         const int tj = t0 - 3 + j, tc = tj < 0 ? 0 : tj < T ? tj : T - 1;
@@ -280,13 +279,12 @@ template <bool L2>
 static void launch_conv_rows(const void * x, const float * w, const float * state, void * y, int C, int T, int ldx, int ldy, int bf16, void * qk, int heads, float rs,
                              float * commit, hipStream_t st) {
     // Tokens per wave. From 2^24 values on a chunk comes from HBM: eight tokens, the rows that no other wave reads past the caches; below, its rows
-    // were just written and the chip wants more waves: four. fp32 / bf16 x 10240 channels: 200 tokens 4.9 / 4.5 us (eight 5.5 / 5.0; a wave that walked 32
+    // were just written and the chip wants more waves: four (as many groups of those as a grid holds). fp32 / bf16 x 10240 channels: 200 tokens 4.9 / 4.5 us (eight 5.5 / 5.0; a wave that walked 32
     // tokens with the next eight rows in flight 12.5 / 11.4), 3001 tokens 40.1 / 25.8 (four 42.6 / 24.7, walking 49.3 / 27.8), 16384 tokens 219.7 /
     // 109.6 (four 218.6 / 132.9, walking 250 / 130); with the L2 norm at 4096 tokens 70.0 / 42.5 (walking 91.0 / 49.2).
-    const bool big = (long)T * C >= (1L << 24);
+    const bool big = (long)T * C >= (1L << 24) || T > 16 * CONV_GROUPS;
     const int tpw = big ? 8 : 4, per = bf16 ? 8 : 4;
-    const long groups = ((long)T + 4 * tpw - 1) / (4 * tpw);
-    const dim3 grid((unsigned)((C / per + 63) / 64), (unsigned)(groups < CONV_GRID_Y ? groups : CONV_GRID_Y), (unsigned)((groups + CONV_GRID_Y - 1) / CONV_GRID_Y)), block(256);
+    const dim3 grid((unsigned)((C / per + 63) / 64), (unsigned)((T + 4 * tpw - 1) / (4 * tpw))), block(256);
     if (bf16) {
         if (big) gdn_conv_rows<true, L2, 8, true><<<grid, block, 0, st>>>(x, w, state, y, C, T, ldx, ldy, qk, heads, rs, commit);
         else gdn_conv_rows<true, L2, 4, false><<<grid, block, 0, st>>>(x, w, state, y, C, T, ldx, ldy, qk, heads, rs, commit);
@@ -820,8 +818,8 @@ int camx_gate_mul(const void * a, const void * gt, void * y, long N, int D, int 
     else gate_mul_k<2><<<grid, block, 0, st>>>(a, gt, y, N, D, stride, off);
     CAMX_LAUNCH_RET();
 }
-// the chunk kernel takes the convolution (a decode / verify batch: the one-value-per-thread kernel). A wave counts up to eleven tokens past T in an int
-static bool conv_chunk(int C, int T) { return (long)T * C >= (1L << 20) && T <= 0x7fffffff - 16; }
+// the chunk kernel takes the convolution (a decode / verify batch, and more tokens than a grid has workgroups for: the one-value-per-thread kernel)
+static bool conv_chunk(int C, int T) { return (long)T * C >= (1L << 20) && T <= 32 * CONV_GROUPS; }
 static bool conv_streams(const void * x, const void * y, int C, int T, int ldx, int ldy, int bf16) {
     const int vw = bf16 ? 8 : 4;
     return conv_chunk(C, T) && C % vw == 0 && ldx % vw == 0 && ldy % vw == 0 && !(((uintptr_t)x | (uintptr_t)y) & 15);

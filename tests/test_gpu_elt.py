@@ -243,9 +243,9 @@ def test_gdn_conv_tokens_do_not_depend_on_the_chunk(T, bf16):
     assert _same(y, parts[:, :C]) and _same(qk, qk2)
 
 
-@pytest.mark.parametrize('T,C,bf16', [(16 * 65535 + 5, 8, 1), (16 * 65535 + 21, 4, 0), (32 * 65535 + 77, 128, 1)])
+@pytest.mark.parametrize('T,C,bf16', [(16 * 65535 + 5, 8, 1), (16 * 65535 + 21, 4, 0), (32 * 65535, 8, 0), (32 * 65535 + 77, 128, 1)])
 def test_gdn_conv_past_65535_groups_of_tokens(T, C, bf16):
-    """more token groups than a grid has workgroups in y: the same rows in slices through the one-value kernel"""
+    """more token groups than a grid has workgroups in y (eight tokens a wave, then the one-value kernel): the same rows in slices through that kernel"""
     import torch
     g = torch.Generator(device='cuda'); g.manual_seed(C)
     dt = torch.bfloat16 if bf16 else torch.float32
