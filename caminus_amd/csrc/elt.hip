@@ -278,11 +278,13 @@ __global__ void __launch_bounds__(256) gdn_conv_rows(const void * __restrict__ x
 template <bool L2>
 static void launch_conv_rows(const void * x, const float * w, const float * state, void * y, int C, int T, int ldx, int ldy, int bf16, void * qk, int heads, float rs,
                              float * commit, hipStream_t st) {
-    // Tokens per wave. From 2^24 values on a chunk comes from HBM: eight tokens, the rows that no other wave reads past the caches; below, its rows
-    // were just written and the chip wants more waves: four (as many groups of those as a grid holds). fp32 / bf16 x 10240 channels: 200 tokens 4.9 / 4.5 us (eight 5.5 / 5.0; a wave that walked 32
-    // tokens with the next eight rows in flight 12.5 / 11.4), 3001 tokens 40.1 / 25.8 (four 42.6 / 24.7, walking 49.3 / 27.8), 16384 tokens 219.7 /
-    // 109.6 (four 218.6 / 132.9, walking 250 / 130); with the L2 norm at 4096 tokens 70.0 / 42.5 (walking 91.0 / 49.2).
-    const bool big = (long)T * C >= (1L << 24) || T > 16 * CONV_GROUPS;
+    // Tokens per wave. From 2^24 fp32 or 3 x 2^21 bf16 values on (768 workgroups of four tokens a wave, three a CU) a chunk comes from HBM: eight tokens, the rows
+    // that no other wave reads past the caches; below, its rows were just written and the chip wants more waves: four (as many groups of those as a grid holds).
+    // fp32 / bf16 x 10240 channels: 200 tokens on warm lines 4.9 / 4.5 us (eight 5.5 / 5.0; a wave that walked 32 tokens with the next eight rows in flight 12.5 /
+    // 11.4); on cold lines 3001 tokens 40.9 / 26.1 (four 42.6 / 29.1, walking 49.3 / 27.8), 16384 tokens 219.7 / 109.6 (four 218.6 / 132.9, walking 250 / 130);
+    // bf16 777 x 8192 8.8 (four 10.2), 1600 x 10240 16.0 (18.2), 3001 x 2048, below the line, 8.5 (eight 8.9); with the L2 norm 2048 x 2048 8.2 (eight 9.2),
+    // 4096 tokens of 10240 68.9 / 42.9 (walking 91.0 / 49.2).
+    const bool big = (long)T * C >= (bf16 ? 3L << 21 : 1L << 24) || T > 16 * CONV_GROUPS;
     const int tpw = big ? 8 : 4, per = bf16 ? 8 : 4;
     const dim3 grid((unsigned)((C / per + 63) / 64), (unsigned)((T + 4 * tpw - 1) / (4 * tpw))), block(256);
     if (bf16) {

@@ -214,7 +214,7 @@ def _same(a, b):
 @pytest.mark.parametrize('T', [128, 129, 131, 257, 2047, 2048, 2049, 2053])
 @pytest.mark.parametrize('bf16', [0, 1])
 def test_gdn_conv_tokens_do_not_depend_on_the_chunk(T, bf16):
-    """the chunk kernel (from 2^20 values, more tokens a wave from 2^24) against the same tokens in pieces of 64, which the kernel of one value a
+    """the chunk kernel (from 2^20 values, more tokens a wave from 2^24 fp32 or 3 x 2^21 bf16) against the same tokens in pieces of 64, which the kernel of one value a
     thread takes, its state advanced by camx_pf_conv_state; the committing entry's y and state against both; chunks that end inside a
     wave's tokens and inside a workgroup; values beyond the exponential's short form, infinities and a NaN; nothing behind the last row"""
     import torch
