@@ -37,21 +37,22 @@ struct NormArgs {
 // OUT != 0 is the chunk form for batches that stream from HBM: the set of copies is fixed at compile time (NORM_* bits, so
 // no branch stands in the store loop either), every access is non-temporal, the requests of a row leave a short pause apart,
 // and gamma waits in LDS instead of registers: GL == 1 one copy per workgroup (one gamma row for all), GL == 2 one row per
-// wave (row r uses gamma row r % wr). A wave past the last row repeats it and stores nothing (as a launch of its own the last rows
-// cost 4 to 10 us: 777 x 5120 14.3 us in two launches).
+// wave (row r uses gamma row r % wr). RAGGED: the rows are no whole number of workgroups, a wave past the last row repeats it and stores nothing (as a
+// launch of its own the last rows cost 4 to 10 us: 777 x 5120 14.3 us in two launches). An instance of its own: its branches cost a whole batch of 2048 rows
+// of 2048 9.1 -> 9.6 us and the hyper-connections' update and norm of 32768 rows of 2560 140.8 -> 142.9.
 enum { NORM_H = 1, NORM_H16 = 2, NORM_HBF = 4, NORM_Q8 = 8, NORM_SCL = 16 };
 #define CAMX_ISSUE_GAP() do { if (OUT) { __builtin_amdgcn_sched_barrier(0); __builtin_amdgcn_s_sleep(1); __builtin_amdgcn_sched_barrier(0); } } while (0)
 // SPLIT (a batch too small to fill the chip, with a q8_1 copy): a workgroup per row. Every wave loads the row and walks the same
 // sum of squares (the same operations on the same values: the same bits in all four), but writes the residual and the copies of
 // the slabs j = wave (mod 4) only: the serial part behind the reduction, eight q8_1 slabs for a 2048-wide row, is a quarter as long.
-template <int NI_MAX, int ADD, bool EXACT, int OUT = 0, int GL = 0, bool SPLIT = false>
+template <int NI_MAX, int ADD, bool EXACT, int OUT = 0, int GL = 0, bool SPLIT = false, bool RAGGED = false>
 __global__ void __launch_bounds__(256) add_rms_rows(NormArgs a) {
-    static_assert(OUT == 0 ? GL == 0 : (EXACT && !SPLIT), "the chunk form is straight-line code");
+    static_assert(OUT == 0 ? GL == 0 && !RAGGED : (EXACT && !SPLIT), "the chunk form is straight-line code");
     extern __shared__ __attribute__((aligned(16))) float gsh[];
     const int lraw = threadIdx.x & 63, lane = slot_of(lraw), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int row_raw = SPLIT ? blockIdx.x : blockIdx.x * 4 + wave;
     if (!OUT && row_raw >= a.rows) return;
-    const bool live = !OUT || row_raw < a.rows;              // (wave-uniform)
+    const bool live = !RAGGED || row_raw < a.rows;           // (wave-uniform)
     const int row = live ? row_raw : a.rows - 1;
     auto mine = [&](int j) { return !SPLIT || (j & 3) == wave; };
     const int N = EXACT ? NI_MAX * 256 : a.N, ni = EXACT ? NI_MAX : N >> 8;
@@ -178,7 +179,7 @@ __global__ void __launch_bounds__(256) add_rms_rows(NormArgs a) {
         __builtin_amdgcn_s_waitcnt(0x0f70);       // vmcnt(0): this wave's gamma pieces have landed in LDS (they were first in the queue)
         if (GL == 1) __syncthreads();
     }
-    if (OUT && !live) return;
+    if (!live) return;
     const float * gl = gsh + (GL == 2 ? wave * N : 0);
     // (two copies of the loop, chosen once: with the choice inside it the stores of a long row were no longer issued back to back)
     auto emit = [&](auto nt, auto redo) {
@@ -284,7 +285,7 @@ __global__ void __launch_bounds__(256) add_rms_rows_any(NormArgs a) {
 // stores its part of the residual as soon as its own loads are back. The sum of squares keeps its order: logical thread 4 lane + k chains
 // its elements slab by slab, so the lane's four partial sums go from wave to wave through LDS (part p continues where part p - 1 stopped)
 // and the last part forms the row's total with the same tree. Gamma comes straight into registers (a wave needs NS slabs of it).
-template <int NS, int W, int ADD, int OUT>
+template <int NS, int W, int ADD, int OUT, bool RAGGED = false>
 __global__ void __launch_bounds__(256) add_rms_rows_div(NormArgs a) {
     static_assert(ADD != ADD_HC, "the addends of the row kernels");
     constexpr int N = NS * W * 256, RPW = 4 / W;
@@ -292,7 +293,7 @@ __global__ void __launch_bounds__(256) add_rms_rows_div(NormArgs a) {
     __shared__ float totsh[RPW];
     const int lraw = threadIdx.x & 63, lane = slot_of(lraw), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int rw = wave / W, part = wave % W;
-    const bool live = (int)(blockIdx.x * RPW) + rw < a.rows;     // (wave-uniform)
+    const bool live = !RAGGED || (int)(blockIdx.x * RPW) + rw < a.rows;      // (wave-uniform)
     const int row = live ? blockIdx.x * RPW + rw : a.rows - 1;
     const int e0 = part * (NS * 256) + 4 * lane;                        // this lane's first element of the row
     float * xr = a.x + (size_t)row * N + e0;
@@ -412,7 +413,10 @@ static bool launch_norm_div(const NormArgs & a, hipStream_t st) {
         switch (ni) {
         case 4: add_rms_rows_div<1, 4, ADD, OUT><<<grid, block, 0, st>>>(a); return true;
         case 8: add_rms_rows_div<2, 4, ADD, OUT><<<grid, block, 0, st>>>(a); return true;
-        case 10: add_rms_rows_div<5, 2, ADD, OUT><<<grid, block, 0, st>>>(a); return true;
+        case 10:
+            if (a.rows & 1) add_rms_rows_div<5, 2, ADD, OUT, true><<<grid, block, 0, st>>>(a);
+            else add_rms_rows_div<5, 2, ADD, OUT><<<grid, block, 0, st>>>(a);
+            return true;
         case 16: add_rms_rows_div<4, 4, ADD, OUT><<<grid, block, 0, st>>>(a); return true;
         case 20: add_rms_rows_div<5, 4, ADD, OUT><<<grid, block, 0, st>>>(a); return true;
         }
@@ -428,13 +432,17 @@ static bool launch_norm_chunk(const NormArgs & a, hipStream_t st) {
     const dim3 grid((a.rows + 3) / 4), block(256);
     const size_t lds = (size_t)(gl == 1 ? 1 : 4) * a.N * sizeof(float);
     switch (ni) {
+#define CAMX_NORM_ROWS(NI, GL) \
+        if (a.rows & 3) add_rms_rows<NI, ADD, true, OUT, GL, false, true><<<grid, block, lds, st>>>(a); \
+        else add_rms_rows<NI, ADD, true, OUT, GL><<<grid, block, lds, st>>>(a)
 #define CAMX_NORM_CHUNK(NI) case NI: \
-        if (gl == 1) add_rms_rows<NI, ADD, true, OUT, 1><<<grid, block, lds, st>>>(a); \
-        else if constexpr (ADD == ADD_NONE || ADD == ADD_HC) { if constexpr (NI <= 10) add_rms_rows<NI, ADD, true, OUT, 2><<<grid, block, lds, st>>>(a); } \
+        if (gl == 1) { CAMX_NORM_ROWS(NI, 1); } \
+        else if constexpr (ADD == ADD_NONE || ADD == ADD_HC) { if constexpr (NI <= 10) { CAMX_NORM_ROWS(NI, 2); } } \
         else return false; \
         return true;
         CAMX_NORM_CHUNK(4) CAMX_NORM_CHUNK(8) CAMX_NORM_CHUNK(10) CAMX_NORM_CHUNK(16) CAMX_NORM_CHUNK(20)
 #undef CAMX_NORM_CHUNK
+#undef CAMX_NORM_ROWS
     }
     return false;
 }

@@ -177,3 +177,9 @@ def test_hc_glue(T, HC, N):
     call('camx_pf_hc_mean', ptr(xn), NULL, NULL, ptr(dev(g)), ptr(out), I(T), I(HC), I(N), F(0.25))
     call('camx_pf_hc_mean', ptr(rd), ptr(scl), ptr(wd), ptr(dev(g)), ptr(out2), I(T), I(HC), I(N), F(0.25))
     assert close_fp32(host(out), O.hc_mean(gxn, g)) and bits_equal(host(out2), host(out))
+
+
+@pytest.mark.parametrize('T,HC,N', [(102, 4, 2560), (103, 4, 2560), (137, 3, 2560), (255, 4, 2560), (341, 3, 2560), (257, 1, 5120), (515, 1, 4096), (1023, 1, 2048)])
+def test_hc_glue_between_256_and_chunk_rows(T, HC, N):
+    """batches that the chunk form takes below its 1024 rows, from 2^20 values: whole and ragged last workgroups, a gamma row per workgroup and per wave"""
+    test_hc_glue(T, HC, N)
