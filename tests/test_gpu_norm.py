@@ -119,6 +119,21 @@ def test_norm_forms_between_256_and_chunk_rows(n, N):
     assert tail_ok(xd, np.float32) and tail_ok(h, np.float32) and tail_ok(h16, np.uint16)
 
 
+@pytest.mark.parametrize('n,N', [(512, 5120), (513, 5120), (513, 2560), (514, 4096), (768, 2048), (769, 2048), (1024, 2048), (1025, 2048)])
+def test_norm_forms_at_their_lines(n, N):
+    """the last batch that divides its rows over waves and the first that does not, whole and ragged; one slot addend at its own lines"""
+    test_norm_forms_between_256_and_chunk_rows(n, N)
+    if N > 2048: return
+    rng = np.random.default_rng(n)
+    x, d = outliers(rng, (n, N)), outliers(rng, (n, 1, N)); nw = (1 + 0.1 * rng.standard_normal(N)).astype(np.float32)
+    ref = O.add_rms16(x, nw, 1e-6, d=d, S=1)
+    for want_h in (False, True):
+        xd, h, h16 = dev(x), dev(np.zeros((n, N), np.float32)), dev(np.zeros((n + 1, N), np.uint16))
+        call('camx_q3p_add_rms16', ptr(xd), ptr(dev(d)), NULL, I(1), ptr(dev(nw)), F(1e-6), ptr(h) if want_h else NULL, ptr(h16), I(N), I(n))
+        assert bits_equal(host(xd), ref['x']) and bits_equal(host(h16, np.uint16)[:n], ref['h16']) and not host(h16, np.uint16)[n].any()
+        if want_h: assert bits_equal(host(h), ref['h'])
+
+
 @pytest.mark.parametrize('R,K,wr', [(8, 2560, 4), (3, 2048, 1), (5, 100, 1), (2, 896, 2), (516, 3072, 4), (512, 5120, 1), (1028, 2560, 4), (1029, 2560, 1), (1026, 2048, 1), (1024, 5120, 4), (16388, 2048, 4)])
 def test_rms_mul_and_rmsnorm(R, K, wr):
     rng = np.random.default_rng(R * K)
