@@ -234,7 +234,7 @@ __global__ void __launch_bounds__(256) actq_fwd_k(Src src, uint16_t * y, float *
 // order as above. What a value costs is counted in issue cycles, measured on the card: an add, subtract, multiply, bit operation or
 // multiply-add that reads at most two vector registers takes 2.3 per wave and SIMD, everything else (shifts, converts, maxima,
 // compares, row moves, an operand in a scalar register) 4.2. Hence rounds of eight values that live as packed bf16 words between the
-// passes, maxima of packed words, and checks that a row settles once. bf16 rows, forward / backward, against four lanes a chunk with 32
+// passes, and maxima of packed words. bf16 rows, forward / backward, against four lanes a chunk with 32
 // values each (up to 2048) and a workgroup per row: 32768 x 512 35.6 -> 20.1 / 65.4 -> 27.2 us, 32768 x 1024 38.6 -> 29.4 / 69.4 -> 44.0,
 // 16384 x 2048 27.6 -> 26.5 / 44.5 -> 37.0 (floor 20.6 / 31.0: bytes at 6.5 TB/s), 8192 x 4096 30.9 -> 25.5 / 50.8 -> 38.6; at 32768 x 2048
 // the forward is bound by its bytes either way (49 us for 268 MB).
@@ -393,40 +393,21 @@ CAMX_DEV void lds_table_copy(const void * src, void * dst, int bytes) {         
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)((const uint8_t *)src + 1024 * j + 16 * lane),
                                          (__attribute__((address_space(3))) void *)((uint8_t *)dst + 1024 * j), 16, 0, 0);
 }
-// Whether rintf(u * rcp) is the row's quantizer for every value: no NaN, the largest quotient below 16 and not rounding above qmax (so
-// nothing is clamped), and no bf16 value whose quotient lies within 2e-5 of a half-integer (see RowScale: 1e-5 would do). The bf16
-// values next to the half-integers' products with s are few enough to be looked at once per row, a half-integer per lane (1 to 2 % of
-// rows hold one), in place of a subtraction and a maximum per value.
-CAMX_DEV bool row_is_tame(const RowScale & rs, float amax, bool nan) {
-    const float p = amax * rs.rcp;
-    if (nan || !(p < 16.0f && p < rs.hi + 0.499f && rs.s < 0x1p100f)) return false;            // (uniform; an infinite amax gives a NaN)
-    const int lane = threadIdx.x & 63;
-    const float hs = ((float)lane + 0.5f) * rs.s, near = bf_lo(hw_pk_bf16(hs, 0.0f));
-    return __builtin_amdgcn_ballot_w64((float)lane < rs.hi && fabsf(near - hs) < 2e-5f * rs.s) == 0;
-}
 // the values and codes of a row (or a wave's part of it) from its packed rotated words; y, codes: the row's, or null
 template <int R, int W>
-CAMX_DEV void quantize_row_w(const u32x4 (&uw)[R], float amax, bool nan, float s, int qmax, int e0, bool last_on, uint16_t * y, uint16_t * codes, bool stream) {
+CAMX_DEV void quantize_row_w(const u32x4 (&uw)[R], float amax, float s, int qmax, int e0, bool last_on, uint16_t * y, uint16_t * codes, bool stream) {
     const RowScale rs(s, amax, qmax);
-    const bool tame = row_is_tame(rs, amax, nan);
 #pragma unroll
     for (int j = 0; j < R; j++) {
         if (j == R - 1 && !last_on) break;
         float q[8];
         unpack8(uw[j], q);
-        if (__builtin_expect(tame, 1)) {
-#pragma unroll
-            for (int k = 0; k < 8; k++) q[k] = rintf(q[k] * rs.rcp);
-        } else {
-            const f32x4 a = rs.quant4((f32x4){q[0], q[1], q[2], q[3]}), b = rs.quant4((f32x4){q[4], q[5], q[6], q[7]});
-            q[0] = a.x; q[1] = a.y; q[2] = a.z; q[3] = a.w; q[4] = b.x; q[5] = b.y; q[6] = b.z; q[7] = b.w;
-        }
+        const f32x4 a = rs.quant4((f32x4){q[0], q[1], q[2], q[3]}), b = rs.quant4((f32x4){q[4], q[5], q[6], q[7]});
         const int e = e0 + 512 * W * j;
-        if (codes) *(u32_a2 *)(codes + (e >> 2)) = rs.nibbles4((f32x4){q[0], q[1], q[2], q[3]}) | (rs.nibbles4((f32x4){q[4], q[5], q[6], q[7]}) << 16);
+        if (codes) *(u32_a2 *)(codes + (e >> 2)) = rs.nibbles4(a) | (rs.nibbles4(b) << 16);
         if (y) {
-#pragma unroll
-            for (int k = 0; k < 8; k++) q[k] *= s;
-            store16(__builtin_expect(tame, 1) ? pack8_any(q) : pack8_canon(q), y + e, stream);   // (a tame row's products are numbers)
+            const float v[8] = {a.x * s, a.y * s, a.z * s, a.w * s, b.x * s, b.y * s, b.z * s, b.w * s};
+            store16(pack8_canon(v), y + e, stream);
         }
     }
 }
@@ -460,7 +441,7 @@ __global__ void __launch_bounds__(256) actq_fwd_wave_k(Src src, uint16_t * __res
     if (W > 1 && row >= M) return;
     const float s = fmaxf(amax * clip / (float)qmax, 1e-8f);
     if (lane == 0 && part == 0 && s_out) s_out[row] = s;
-    quantize_row_w<R, W>(uw, amax, nan, s, qmax, e0, last_on, y ? y + (size_t)row * K : nullptr, codes ? codes + (size_t)row * (K / 4) : nullptr, stream);
+    quantize_row_w<R, W>(uw, amax, s, qmax, e0, last_on, y ? y + (size_t)row * K : nullptr, codes ? codes + (size_t)row * (K / 4) : nullptr, stream);
 }
 
 // ---- backward ----------------------------------------------------------------------------------------------------------------
@@ -885,18 +866,11 @@ CAMX_DEV void entry_row_fwd(const u32x2 (&hb)[NR], int lane, int row, bool store
     const float amax = entry_rotate<NR>(hb, lane, u, nan);
     const float s = fmaxf(amax * clip / (float)qmax, 1e-8f);
     const RowScale rs(s, amax, qmax);
-    const bool tame = row_is_tame(rs, amax, nan);
     if (!stored) return;                                 // (wave-uniform)
-    if (__builtin_expect(tame, 1)) {
-#pragma unroll
-        for (int c = 0; c < NR; c++) u[c] = (f32x4){rintf(u[c].x * rs.rcp), rintf(u[c].y * rs.rcp), rintf(u[c].z * rs.rcp), rintf(u[c].w * rs.rcp)};
-    } else {
-#pragma unroll
-        for (int c = 0; c < NR; c++) u[c] = rs.quant4(u[c]);
-    }
 #pragma unroll
     for (int c = 0; c < NR; c++) {
         const int k = 256 * c + 4 * lane;
+        u[c] = rs.quant4(u[c]);
         if (c < NR - 1 || k < d) {
             if (y) store8(pack_f2bf_x4((f32x4){u[c].x * s, u[c].y * s, u[c].z * s, u[c].w * s}), y + (size_t)row * d + k, stream);
             if (codes) codes[((size_t)row * d + k) >> 2] = (uint16_t)rs.nibbles4(u[c]);
@@ -1204,7 +1178,7 @@ __global__ void __launch_bounds__(512, 6) block_entry_fwd_rows16(const float * _
         const float amax = row_absmax_w<R>(uw, most, nan);
         const float s = fmaxf(amax * clip / (float)qmax, 1e-8f);
         if (row < M) {                                   // (wave-uniform)
-            quantize_row_w<R, 1>(uw, amax, nan, s, qmax, e0, last_on, y ? y + (size_t)row * d : nullptr, codes ? codes + (size_t)row * (d / 4) : nullptr, stream);
+            quantize_row_w<R, 1>(uw, amax, s, qmax, e0, last_on, y ? y + (size_t)row * d : nullptr, codes ? codes + (size_t)row * (d / 4) : nullptr, stream);
             if (lraw == 0) { if (s_out) s_out[row] = s; if (rstd_out) rstd_out[row] = i ? rstd[1] : rstd[0]; }
         }
     }
