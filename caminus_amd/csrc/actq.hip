@@ -234,10 +234,10 @@ __global__ void __launch_bounds__(256) actq_fwd_k(Src src, uint16_t * y, float *
 // order as above. What a value costs is counted in issue cycles, measured on the card: an add, subtract, multiply, bit operation or
 // multiply-add that reads at most two vector registers takes 2.3 per wave and SIMD, everything else (shifts, converts, maxima,
 // compares, row moves, an operand in a scalar register) 4.2. Hence rounds of eight values that live as packed bf16 words between the
-// passes, and maxima of packed words. bf16 rows, forward / backward, against four lanes a chunk with 32
-// values each (up to 2048) and a workgroup per row: 32768 x 512 35.6 -> 20.1 / 65.4 -> 27.2 us, 32768 x 1024 38.6 -> 29.4 / 69.4 -> 44.0,
-// 16384 x 2048 27.6 -> 26.5 / 44.5 -> 37.0 (floor 20.6 / 31.0: bytes at 6.5 TB/s), 8192 x 4096 30.9 -> 25.5 / 50.8 -> 38.6; at 32768 x 2048
-// the forward is bound by its bytes either way (49 us for 268 MB).
+// passes, and maxima of packed words. bf16 rows, forward / backward, against four lanes a chunk with 32 values each (up to 2048) and a
+// workgroup per row, buffers cold: 32768 x 512 40.3 -> 17.0 / 66.1 -> 27.0 us, 32768 x 1024 43.5 -> 27.1 / 69.4 -> 43.0, 16384 x 2048 35.7 ->
+// 28.4 / 44.5 -> 39.0 (floor 20.6 / 31.0: bytes at 6.5 TB/s), 32768 x 2048 64.6 -> 48.6 / 81.2 -> 77.0, 8192 x 4096 35.3 -> 27.8 / 51.7 ->
+// 38.7; the SiLU-fused pair at 16384 x 2048 47.2 -> 42.3 / 92.1 -> 77.2 (floor 34 / 52).
 CAMX_DEV void bfly(float & a, float & b) { const float s = a + b, d = a - b; a = s; b = d; }
 CAMX_DEV float bf_lo(uint32_t v) { return __builtin_bit_cast(float, v << 16); }
 CAMX_DEV float bf_hi(uint32_t v) { return __builtin_bit_cast(float, v & 0xffff0000u); }
@@ -254,7 +254,7 @@ CAMX_DEV u32x4 unknown_words(u32x4 w) {
 // eight values to packed bf16 by the hardware convert: a NaN stays one (see rbf4_any)
 CAMX_DEV u32x4 pack8_any(const float (&v)[8]) { return (u32x4){hw_pk_bf16(v[0], v[1]), hw_pk_bf16(v[2], v[3]), hw_pk_bf16(v[4], v[5]), hw_pk_bf16(v[6], v[7])}; }
 // A batch of 2^20 values or more streams: its bf16 outputs leave past the caches as whole lines (the wave's round is 1 KiB without a gap:
-// 16384 x 2048 forward 31.4 -> 26.3 us, backward 40.1 -> 36.3 with g read past them too). fp32 gradients stay plain: a lane's eight values
+// 16384 x 2048 forward 31.4 -> 26.3 us, backward 40.1 -> 36.3 with g read past them too, buffers warm). fp32 gradients stay plain: a lane's eight values
 // are two half lines, which only the cache puts together (61 -> 85 us).
 typedef u32x4 u32x4_a8 __attribute__((aligned(8)));                      // (the block entry's operands are 8-byte aligned, its codes 2)
 typedef uint32_t u32_a2 __attribute__((aligned(2)));
@@ -376,13 +376,19 @@ CAMX_DEV u16x2 actq_rotate_w(const Src & src, const u32x4 (&raw)[R][Src::NW], co
     }
     return most;
 }
+// A chunk behind the row reads the row's first one and is replaced afterwards: a load under a condition ends in a copy of its result, and so in a wait for
+// everything requested so far, before the next request goes out.
 template <int R, int W, typename Src>
 CAMX_DEV void fetch_row_w(const Src & src, int row, int e0, bool last_on, u32x4 (&raw)[R][Src::NW]) {
 #pragma unroll
-    for (int j = 0; j < R; j++) {
+    for (int j = 0; j < R; j++) src.fetch(row, j < R - 1 || last_on ? e0 + 512 * W * j : e0 & 127, raw[j]);
+}
+template <int R, typename Src>
+CAMX_DEV void absent_chunk_w(const Src &, bool last_on, u32x4 (&raw)[R][Src::NW]) {
 #pragma unroll
-        for (int w = 0; w < Src::NW; w++) raw[j][w] = Src::absent(w);
-        if (j < R - 1 || last_on) src.fetch(row, e0 + 512 * W * j, raw[j]);
+    for (int w = 0; w < Src::NW; w++) {
+        const u32x4 none = Src::absent(w);
+        raw[R - 1][w] = (u32x4){last_on ? raw[R - 1][w].x : none.x, last_on ? raw[R - 1][w].y : none.y, last_on ? raw[R - 1][w].z : none.z, last_on ? raw[R - 1][w].w : none.w};
     }
 }
 
@@ -432,6 +438,7 @@ __global__ void __launch_bounds__(256) actq_fwd_wave_k(Src src, uint16_t * __res
         if (W == 1 && row >= M) return;
     }
     __shared__ float xch[4];
+    absent_chunk_w<R>(src, last_on, raw);
     const Lanes16 ln(slot);
     u32x4 uw[R], keep[R];                                // (keep: only the backward uses it)
     const u16x2 most = actq_rotate_w<R>(src, raw, ln, uw, keep);
@@ -770,10 +777,7 @@ __global__ void __launch_bounds__(256) actq_bwd_wave_k(Src src, const uint16_t *
     u32x4 raw[R][Src::NW], gw[R];
     fetch_row_w<R, W>(src, row, e0, last_on, raw);
 #pragma unroll
-    for (int j = 0; j < R; j++) {
-        gw[j] = (u32x4){0u, 0u, 0u, 0u};
-        if (j < R - 1 || last_on) gw[j] = __builtin_nontemporal_load((const u32x4 *)(g + (size_t)row * K + e0 + 512 * W * j));
-    }
+    for (int j = 0; j < R; j++) gw[j] = __builtin_nontemporal_load((const u32x4 *)(g + (size_t)row * K + (j < R - 1 || last_on ? e0 + 512 * W * j : e0 & 127)));
     if (Src::lds_tables) {                               // the gates' tables, shared by the workgroup's rows
         __shared__ __attribute__((aligned(16))) uint16_t small[SWS_TAB];
         __shared__ __attribute__((aligned(16))) float dsmall[SWS_TAB];
@@ -785,6 +789,8 @@ __global__ void __launch_bounds__(256) actq_bwd_wave_k(Src src, const uint16_t *
         if (W == 1 && row_raw >= M) return;
     }
     __shared__ PairShare share;
+    absent_chunk_w<R>(src, last_on, raw);
+    gw[R - 1] = (u32x4){last_on ? gw[R - 1].x : 0u, last_on ? gw[R - 1].y : 0u, last_on ? gw[R - 1].z : 0u, last_on ? gw[R - 1].w : 0u};
     const Lanes16 ln(slot);
     u32x4 uw[R], keep[R];
     const u16x2 most = actq_rotate_w<R>(src, raw, ln, uw, keep);
@@ -896,7 +902,7 @@ CAMX_DEV void entry_row_bwd(const u32x2 (&hb)[NR], const u32x2 (&gy)[NR], int la
 #pragma unroll
     for (int c = 0; c < NR; c++) {
         const bool on = c < NR - 1 || 256 * c + 4 * lane < d;
-        gv[c] = unpack_bf16x4(gy[c]);
+        gv[c] = unpack_bf16x4((u32x2){on ? gy[c].x : 0u, on ? gy[c].y : 0u});
         const f32x4 t = rd.div4(u[c], on);
         f32x4 v = {rintf(t.x) - t.x, rintf(t.y) - t.y, rintf(t.z) - t.z, rintf(t.w) - t.w};
         const float most = fmaxf(fmaxf(fabsf(u[c].x), fabsf(u[c].y)), fmaxf(fabsf(u[c].z), fabsf(u[c].w)));
@@ -948,15 +954,22 @@ CAMX_DEV float entry_rstd(const f32x4 (&xk)[NR], int d, float eps) {
     }
     return rsqrt_exact(wave_groups_in_order(group32_sum(acc)) / (float)d + eps);
 }
-// a lane's rounds of an fp32 row, zeros behind it
-template <int NR>
-CAMX_DEV void entry_load(const float * row, int d, int lane, bool stream, f32x4 (&v)[NR]) {
+// A lane's rounds of an fp32 row. Behind the row it reads the row's first values, which entry_zero replaces once they are there (see fetch_row_w). NT: past the
+// caches (of two loads chosen by a run-time flag the compiler makes a plain one).
+template <bool NT, int NR>
+CAMX_DEV void entry_load(const float * row, int d, int lane, f32x4 (&v)[NR]) {
 #pragma unroll
     for (int c = 0; c < NR; c++) {
-        const int k = 256 * c + 4 * lane;
-        v[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-        if (c < NR - 1 || k < d) v[c] = stream ? __builtin_nontemporal_load((const f32x4 *)(row + k)) : *(const f32x4 *)(row + k);
+        const int k = c < NR - 1 || 256 * c + 4 * lane < d ? 256 * c + 4 * lane : 0;
+        if constexpr (NT) v[c] = __builtin_nontemporal_load((const f32x4 *)(row + k));
+        else v[c] = *(const f32x4 *)(row + k);
     }
+}
+template <int NR>
+CAMX_DEV void entry_zero(f32x4 (&v)[NR], int d, int lane) {
+    const bool on = 256 * (NR - 1) + 4 * lane < d;
+    f32x4 & e = v[NR - 1];
+    e = (f32x4){on ? e.x : 0.0f, on ? e.y : 0.0f, on ? e.z : 0.0f, on ? e.w : 0.0f};
 }
 template <int NR>
 CAMX_DEV void entry_pack(const f32x4 (&xk)[NR], const f32x4 (&wk)[NR], float rstd, int d, int lane, u32x2 (&hb)[NR]) {
@@ -972,8 +985,9 @@ __global__ void __launch_bounds__(64) block_entry_fwd_wave(const float * x, cons
                                                            int d, float clip, int qmax, bool stream) {
     const int row = blockIdx.x, lane = slot_of(threadIdx.x);
     f32x4 xk[NR], wk[NR];
-    entry_load<NR>(x + (size_t)row * d, d, lane, true, xk);
-    entry_load<NR>(nw, d, lane, false, wk);
+    entry_load<true, NR>(x + (size_t)row * d, d, lane, xk);
+    entry_load<false, NR>(nw, d, lane, wk);
+    entry_zero<NR>(xk, d, lane);
     const float rstd = entry_rstd<NR>(xk, d, eps);
     u32x2 hb[NR];
     entry_pack<NR>(xk, wk, rstd, d, lane, hb);
@@ -1039,8 +1053,8 @@ __global__ void __launch_bounds__(256) block_entry_fwd_k(const float * x, const 
 
 // ---- block entry with projections, rows of at most 1024 values: a wave per row, four rows share the projections on the matrix cores ----
 // Bound by instruction issue: with the projections as vector multiply-adds of a row's own wave, they, the conversions of wab and sixteen
-// reductions of 256 logical threads were two thirds of a row's instructions (32768 rows x 1024 values, 16 projections: 114 us, this
-// kernel 84; 512 rows: 11.6 and 7.0; large batches with more than four projections: block_entry_fwd_rows16). A K = 1 matrix instruction
+// reductions of 256 logical threads were two thirds of a row's instructions (32768 rows x 1024 values, 16 projections: 117 us, this
+// kernel 86; 512 rows: 12.0 and 7.7; large batches with more than four projections: block_entry_fwd_rows16). A K = 1 matrix instruction
 // (v_mfma_f32_4x4x1: 16 blocks of 4 x 4 single multiply-adds, each rounded like fmaf) computes for 16 logical threads t the terms of
 // 4 rows x 4 projections, so a thread's chain over its elements t, t + 256, .. is a chain of NR such instructions in the same order.
 // A workgroup's four waves own a row each and hand bf16(h) on through LDS; then wave w takes projections 4 w .. 4 w + 3 of all four rows.
@@ -1060,8 +1074,9 @@ __global__ void __launch_bounds__(256, 4) block_entry_fwd_quad(const float * __r
     const int Q = lraw >> 2, odd = Q & 1, jp = odd ? 3 - (lraw & 3) : lraw & 3;      // the lane's block and its projection of the wave's four
     const int r0 = 4 * blockIdx.x, row = r0 + wave;
     f32x4 xk[NR], wk[NR];
-    entry_load<NR>(x + (size_t)min(row, M - 1) * d, d, lane, true, xk);
-    entry_load<NR>(nw, d, lane, false, wk);
+    entry_load<true, NR>(x + (size_t)min(row, M - 1) * d, d, lane, xk);
+    entry_load<false, NR>(nw, d, lane, wk);
+    entry_zero<NR>(xk, d, lane);
     const float rstd = entry_rstd<NR>(xk, d, eps);
     u32x2 hb[NR];
     entry_pack<NR>(xk, wk, rstd, d, lane, hb);
@@ -1127,9 +1142,9 @@ __global__ void __launch_bounds__(256, 4) block_entry_fwd_quad(const float * __r
 // 32 w + 8 b + e. A lane's eight elements of a step are 16 bytes of LDS (rows) and of device memory (projections), converted once for
 // sixteen rows. The tree's first steps (t ^ 16, 8) pair blocks, which are registers of the result, the others (t ^ 4, 2, 1) instructions;
 // the eight group sums meet in LDS, where a thread adds them in order.
-// 32768 x 1024 with 16 projections 56.0 us, with 8 54.8; as four rows and four projections a wave 84 and 64. A barrier for the whole
-// workgroup costs what the matrix instructions save where there are four projections (57 us either way) and few workgroups
-// (512 rows: 10.2 us, four rows a workgroup 7.0).
+// 32768 x 1024 with 16 projections 53 us, with 8 52; as four rows and four projections a wave 86 and 65. A barrier for the whole
+// workgroup costs more than the matrix instructions save where there are few projections (4096 x 1024 with 4: 11.9 us, four rows a
+// workgroup 11.5) and few workgroups (512 rows with 16: 10.2 and 7.6).
 CAMX_DEV float bf_half(uint32_t v, int odd) { return odd ? bf_hi(v) : bf_lo(v); }
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 CAMX_DEV void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier(); __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront"); }
@@ -1153,11 +1168,12 @@ __global__ void __launch_bounds__(512, 6) block_entry_fwd_rows16(const float * _
     const int r0 = 16 * blockIdx.x;
     f32x4 xk[2][NR], wk[NR];
 #pragma unroll
-    for (int i = 0; i < 2; i++) entry_load<NR>(x + (size_t)min(r0 + 2 * wave + i, M - 1) * d, d, la, true, xk[i]);
-    entry_load<NR>(nw, d, la, false, wk);
+    for (int i = 0; i < 2; i++) entry_load<true, NR>(x + (size_t)min(r0 + 2 * wave + i, M - 1) * d, d, la, xk[i]);
+    entry_load<false, NR>(nw, d, la, wk);
     float rstd[2];
 #pragma unroll
     for (int i = 0; i < 2; i++) {
+        entry_zero<NR>(xk[i], d, la);
         rstd[i] = entry_rstd<NR>(xk[i], d, eps);
         u32x2 hb[NR];
         entry_pack<NR>(xk[i], wk, rstd[i], d, la, hb);
@@ -1202,7 +1218,7 @@ __global__ void __launch_bounds__(512, 6) block_entry_fwd_rows16(const float * _
         for (int c = 0; c < NR; c++) {
             const uint32_t av = A[c][e >> 1], bv = B[c][e >> 1];
             a = __builtin_amdgcn_mfma_f32_16x16x1f32(bf_half(av, e & 1), bf_half(bv, e & 1), a, 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);           // (one chain at a time: 80 registers, six waves per SIMD; 110 and 63.4 us otherwise)
+            __builtin_amdgcn_sched_barrier(0);           // (one chain at a time: 80 registers, six waves per SIMD)
         }
 #pragma unroll
         for (int r = 0; r < 4; r++) t[e][r] = (a[r] + a[8 + r]) + (a[4 + r] + a[12 + r]);            // t ^ 16, t ^ 8
@@ -1254,15 +1270,11 @@ CAMX_DEV void rms_bwd_row(const f32x4 (&xk)[NR], const f32x4 (&wk)[NR], float rs
         }
     }
 }
-// a lane's rounds of a bf16 row, zeros behind it
+// a lane's rounds of a bf16 row; behind the row its first values, for which entry_row_bwd puts zeros
 template <int NR>
 CAMX_DEV void entry_load16(const uint16_t * row, int d, int lane, u32x2 (&v)[NR]) {
 #pragma unroll
-    for (int c = 0; c < NR; c++) {
-        const int k = 256 * c + 4 * lane;
-        v[c] = (u32x2){0u, 0u};
-        if (c < NR - 1 || k < d) v[c] = __builtin_nontemporal_load((const u32x2 *)(row + k));
-    }
+    for (int c = 0; c < NR; c++) v[c] = __builtin_nontemporal_load((const u32x2 *)(row + (c < NR - 1 || 256 * c + 4 * lane < d ? 256 * c + 4 * lane : 0)));
 }
 // dh = actq backward of dy, plus the two projection groups' input gradients (wab rows [0, nab / 2) and [nab / 2, nab), each
 // group's sum rounded to bf16); then the RMSNorm backward. d <= 1024. One wave per row, NR = ceil(d / 256) rounds: the lane's elements are
@@ -1273,23 +1285,24 @@ __global__ void __launch_bounds__(64) block_entry_bwd_k(const float * x, const f
     const float rstd = rstd_in[row];
     f32x4 xk[NR], wk[NR], dh[NR];
     u32x2 gy[NR], hb[NR];
-    entry_load<NR>(x + (size_t)row * d, d, la, true, xk);
-    entry_load<NR>(nw, d, la, false, wk);
+    entry_load<true, NR>(x + (size_t)row * d, d, la, xk);
+    entry_load<false, NR>(nw, d, la, wk);
     entry_load16<NR>(dy + (size_t)row * d, d, la, gy);
+    __builtin_amdgcn_sched_barrier(0);
     entry_pack<NR>(xk, wk, rstd, d, la, hb);
     entry_row_bwd<NR>(hb, gy, la, dh, d, clip, qmax);
     rms_bwd_row<NR>(xk, wk, rstd, dh, dx + (size_t)row * d, d, la, stream);
 }
 
 // The same for nab > 0 with the projections' part on the matrix cores (as vector multiply-adds of the row's own wave 143 us at 32768 x
-// 1024 with 16 projections, 90): a workgroup's four waves own a row each and first compute a quarter
+// 1024 with 16 projections, here 84): a workgroup's four waves own a row each and first compute a quarter
 // of that part for all four rows, one of the two groups for half of the column blocks of 256 (32768 x 256 with 4 projections 31.8 us, as
 // one wave per column block 36.4, with vector multiply-adds 34.3). A K = 1 instruction adds one j's term dab[row][j] wab[j][column]
 // (rounded like fmaf) for 4 rows x 64 columns: block Q's four columns are its lanes' own, so with A = dab (lane 4 Q + i: row i) and B = a
 // lane's column of wab, D holds a lane's column with a word per row. The two groups' sums, rounded to bf16, reach the rows' owners
 // through LDS. Loads return in order: rows of more than 512 values ask for what the projections need first (it comes from the caches) and for
-// the row and its gradient behind it, so that the projections run while those are on their way (115 -> 101 us at 32768 x 1024; 49.6 -> 52.2 at 32768 x 512); shorter
-// rows have too little to do meanwhile and ask for the row first.
+// the row and its gradient behind it, so that the projections run while those are on their way (87.8 -> 84.9 us
+// at 32768 x 1024 with 16); shorter rows ask for the row first.
 template <int NR>
 __global__ void __launch_bounds__(256, 4) block_entry_bwd_quad(const float * x, const float * __restrict__ nw, const float * __restrict__ rstd_in, const uint16_t * __restrict__ wab,
                                                                int nab, const uint16_t * __restrict__ dy, const uint16_t * __restrict__ dab, float * dx, int d, float clip, int qmax, int M, bool stream) {
@@ -1300,7 +1313,7 @@ __global__ void __launch_bounds__(256, 4) block_entry_bwd_quad(const float * x, 
     constexpr bool LATE = NR >= 3;
     f32x4 xk[NR], wk[NR];
     u32x2 gy[NR];
-    if (!LATE) { entry_load<NR>(nw, d, la, false, wk); entry_load<NR>(x + (size_t)row * d, d, la, true, xk); }
+    if (!LATE) { entry_load<false, NR>(nw, d, la, wk); entry_load<true, NR>(x + (size_t)row * d, d, la, xk); }
     // wave w: group w & 1 of column blocks (w >> 1) and (w >> 1) + 2; of a single block words w >> 1 of each lane's two
     constexpr int NT = (2 * NR + 3) / 4, NP = NR == 1 ? 1 : 2;
     const int h = wave & 1, c0 = NR == 1 ? 0 : wave >> 1, p0 = NR == 1 ? wave >> 1 : 0;
@@ -1308,21 +1321,19 @@ __global__ void __launch_bounds__(256, 4) block_entry_bwd_quad(const float * x, 
     float av[8];
     const uint16_t * ar = dab + (size_t)min(r0 + (lraw & 3), M - 1) * nab + h * half;
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        av[j] = 0.0f;
-        if (j < half) av[j] = bf2f(ar[j]);               // (uniform)
-    }
+    for (int j = 0; j < 8; j++) av[j] = bf2f(ar[min(j, half - 1)]);       // (no condition: see fetch_row_w; the terms from half on are not added)
 #pragma unroll
-    for (int j = 0; j < 8; j++)
+    for (int j = 0; j < 8; j++) {
+        if (j > 0 && j >= half) break;                   // (uniform)
 #pragma unroll
         for (int t = 0; t < NT; t++) {
-            const int k = 256 * (c0 + 2 * t) + 4 * la;
-            const uint16_t * b = wab + (size_t)(h * half + j) * d + k;
-            const bool on = j < half && k < d;
-            if (NP == 1) B[t][j][0] = on ? ((const uint32_t *)b)[p0] : 0u;
-            else { u32x2 v = {0u, 0u}; if (on) v = *(const u32x2 *)b; B[t][j][0] = v.x; B[t][j][NP - 1] = v.y; }
+            const int k = 256 * (c0 + 2 * t) + 4 * la;   // (a column behind the row takes the first one's: its result is not stored)
+            const uint16_t * b = wab + (size_t)(h * half + j) * d + (k < d ? k : 0);
+            if (NP == 1) B[t][j][0] = ((const uint32_t *)b)[p0];
+            else { const u32x2 v = *(const u32x2 *)b; B[t][j][0] = v.x; B[t][j][NP - 1] = v.y; }
         }
-    if (LATE) { entry_load<NR>(x + (size_t)row * d, d, la, true, xk); entry_load<NR>(nw, d, la, false, wk); entry_load16<NR>(dy + (size_t)row * d, d, la, gy); }
+    }
+    if (LATE) { entry_load<true, NR>(x + (size_t)row * d, d, la, xk); entry_load<false, NR>(nw, d, la, wk); entry_load16<NR>(dy + (size_t)row * d, d, la, gy); }
     const float rstd = rstd_in[row];
     f32x4 acc[NT][2 * NP];                               // (half >= 1: the first term opens the sums)
 #pragma unroll
