@@ -1300,9 +1300,9 @@ __global__ void __launch_bounds__(64) block_entry_bwd_k(const float * x, const f
 // one wave per column block 36.4, with vector multiply-adds 34.3). A K = 1 instruction adds one j's term dab[row][j] wab[j][column]
 // (rounded like fmaf) for 4 rows x 64 columns: block Q's four columns are its lanes' own, so with A = dab (lane 4 Q + i: row i) and B = a
 // lane's column of wab, D holds a lane's column with a word per row. The two groups' sums, rounded to bf16, reach the rows' owners
-// through LDS. Loads return in order: rows of more than 512 values ask for what the projections need first (it comes from the caches) and for
-// the row and its gradient behind it, so that the projections run while those are on their way (87.8 -> 84.9 us
-// at 32768 x 1024 with 16); shorter rows ask for the row first.
+// through LDS. Loads return in order: rows of more than 256 values ask for what the projections need first (it comes from the caches) and for
+// the row and its gradient behind it, so that the projections run while those are on their way (16 projections, 32768 x 1024 87.8 -> 84.9 us,
+// 32768 x 512 48.6 -> 47.8, 512 x 512 8 % less); shorter rows are as fast either way (2048 x 256 1 % slower) and ask for the row first.
 template <int NR>
 __global__ void __launch_bounds__(256, 4) block_entry_bwd_quad(const float * x, const float * __restrict__ nw, const float * __restrict__ rstd_in, const uint16_t * __restrict__ wab,
                                                                int nab, const uint16_t * __restrict__ dy, const uint16_t * __restrict__ dab, float * dx, int d, float clip, int qmax, int M, bool stream) {
@@ -1310,7 +1310,7 @@ __global__ void __launch_bounds__(256, 4) block_entry_bwd_quad(const float * x, 
     const int lraw = threadIdx.x & 63, la = slot_of(lraw), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = nab / 2;
     const int r0 = 4 * blockIdx.x;
     const int row = min(r0 + wave, M - 1);               // (a wave past the end repeats the last row and stores nothing)
-    constexpr bool LATE = NR >= 3;
+    constexpr bool LATE = NR >= 2;
     f32x4 xk[NR], wk[NR];
     u32x2 gy[NR];
     if (!LATE) { entry_load<false, NR>(nw, d, la, wk); entry_load<true, NR>(x + (size_t)row * d, d, la, xk); }
