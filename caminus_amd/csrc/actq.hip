@@ -1431,6 +1431,15 @@ static int actq_check(int K, int qmax, int M) { return (K < 128 || K % 128 || K 
         case 7: { constexpr int NR = 7; CALL; } break; default: { constexpr int NR = 8; CALL; } break;                  \
     }
 
+// Sixteen rows share the projections, whatever their number, or four rows in steps of four projections. A workgroup of sixteen rows takes a CU's time
+// once for every 4096 rows or part of them (16 projections x 1024: 4096 rows 11.9 us, 5120 17.3, 8192 18.6, 9216 23.8), one of four rows a quarter of
+// them (14.3, 18.1, 25.4, 29.2). r: a row's time with four rows a workgroup over one's with sixteen, in sixteenths, from 32768 rows: 5 to 8 projections 1.19
+// at 1024 values, 1.10 at 768, 1.00 at 256; 13 to 16 1.62, 1.43, 1.22 (an odd number of rounds of 256 leaves half a round of 512 empty).
+static bool entry_rows16(int M, int d, int nab) {
+    const int groups = (nab + 3) / 4, nr = (d + 255) / 256, r = nr == 1 ? 2 * groups + 11 : nr == 3 ? 3 * groups + 11 : 3 * groups + 12;
+    return nab > 4 && M >= 4096 && (long)M * r >= (((long)M + 4095) / 4096) << 16;
+}
+
 extern "C" {
 
 // actq_fwd_{f32,bf16} and actq_fwd_codes_{f32,bf16}: y bf16 [M][K] (optional when codes are written), s [M] (optional),
@@ -1474,10 +1483,7 @@ int camx_block_entry_fwd(const float * x, const float * nw, const uint16_t * wab
             case 3: KERNEL<3><<<dim3((unsigned)(GRID)), dim3(BLOCK), 0, st>>>(__VA_ARGS__); break;                      \
             default: KERNEL<4><<<dim3((unsigned)(GRID)), dim3(BLOCK), 0, st>>>(__VA_ARGS__); break;                     \
         }
-        // sixteen rows share the projections, whatever their number, or four rows in steps of four projections; a sixteen-row workgroup has to
-        // come often enough to fill the chip. 16 projections at 4096 x 1024: 12.5 us, four rows a workgroup 14.5, at 2048 rows 10.9 and 9.6; 8 at
-        // 8192 x 1024 19.6 and 20.9, at 4096 x 640 10.4 and 9.9; 4 at 32768 x 1024 58 and 57
-        if (nab > 4 && M >= (nab > 8 ? 4096 : 8192)) { ENTRY_ROUNDS(block_entry_fwd_rows16, ((long)M + 15) / 16, 512, x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax, M, stream) }
+        if (entry_rows16(M, d, nab)) { ENTRY_ROUNDS(block_entry_fwd_rows16, ((long)M + 15) / 16, 512, x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax, M, stream) }
         else if (nab > 0) { ENTRY_ROUNDS(block_entry_fwd_quad, ((long)M + 3) / 4, 256, x, nw, wab, nab, eps, y, s, codes, ab, rstd_out, d, clip, qmax, M, stream) }
         else { ENTRY_ROUNDS(block_entry_fwd_wave, M, 64, x, nw, eps, y, s, codes, rstd_out, d, clip, qmax, stream) }
         CAMX_LAUNCH_RET();

@@ -391,3 +391,9 @@ def test_actq_fwd_and_bwd_four_million_values(bf):
     dx = dev(np.zeros((M, K), np.uint16 if bf else np.float32))
     call('camx_actq_bwd', ptr(xd), I(int(bf)), ptr(dev(g)), ptr(dx), I(K), F(0.95), I(7), I(M))
     assert bits_equal(host(dx, np.uint16) if bf else host(dx), O.actq_bwd(src, g, clip=0.95, qmax=7, bf16=bf))
+
+
+@pytest.mark.parametrize('M,d,nab,eps', [(8177, 1024, 16, 1e-6), (8191, 384, 10, 0.0), (4096, 896, 5, 1e-6), (12284, 640, 13, 0.0), (8192, 512, 8, 1e-6), (8190, 128, 13, 0.0)])
+def test_block_entry_fwd_sixteen_rows_from_a_full_chip(M, d, nab, eps):
+    """batches just below whole multiples of 4096 rows, which sixteen rows a workgroup take: last workgroups of 1, 15, 16, 12, 16 and 14 rows"""
+    test_block_entry_fwd_sixteen_rows_a_workgroup(M, d, nab, eps)
