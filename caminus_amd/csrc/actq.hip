@@ -4,10 +4,10 @@
 // 96-218, 247-333).
 //
 // Rows of at most 4096 values with 16-byte aligned operands, forward and backward, plain and SiLU-fused: one wave per row, two above 2048
-// (actq_fwd_wave_k, actq_bwd_wave_k), the fused forms with the gates' tables in LDS. The RMSNorm-fused block entry of rows of at most
+// (actq_fwd_wave_k, actq_bwd_wave_k; two waves only in batches that fill the chip), the fused forms with the gates' tables in LDS. The RMSNorm-fused block entry of rows of at most
 // 1024 values: a wave per row as well, four or sixteen rows sharing the projections (block_entry_fwd_quad, block_entry_fwd_rows16,
 // block_entry_bwd_quad). Everything else
-// (longer rows, unaligned operands):
+// (longer rows, unaligned operands, small batches of rows above 2048 values):
 // One 256-thread workgroup per row. A half-wave (32 lanes) transforms one 128-chunk: lane l holds elements 4l .. 4l + 3,
 // butterfly stages 1-2 in registers, 4 .. 64 across lanes; half-wave h takes chunks h, h + 8, ... (the reference's wave h of
 // 32), NR = ceil(K / 1024) rounds of them stay in registers across the row-wide reductions. Kernels are instantiated per
@@ -1408,7 +1408,13 @@ __attribute__((visibility("hidden"))) int dsilu_luts_init(hipStream_t st) {     
 // the wave-per-row kernels: rows of at most 4096 values (longer ones would need more registers than a wave has, or sums handed from wave
 // to wave), operands aligned for 16-byte loads and 16- / 4-byte stores
 static bool actq_wave_ok(int K, uintptr_t x, uintptr_t y, uintptr_t codes) { return K <= 4096 && !((x | y) & 15) && !(codes & 3); }
-// one instance per number of rounds of 512 values, from 2048 on two waves a row
+// Two waves a row (above 2048 values) from the batch that fills the chip with them; smaller ones are a chain of latencies, which a workgroup a row halves.
+// bf16 / fp32 / SiLU forward at 3072 values, in turn: 64 rows 3.9 / 4.0 / 5.1 us (two waves 4.3 / 4.7 / 5.7), 256 rows 4.7 / 4.4 / 5.5 (4.9 / 5.1 / 6.1), 1024
+// rows 7.3 / 8.1 / 10.2 (6.4 / 7.7 / 9.1); backward fp32 / SiLU 1 row 4.6 / 6.6 (4.9 / 7.5), 256 rows 6.3 / 8.7 (6.4 / 9.2), 512 rows 8.4 / 10.5 (8.2 / 9.7);
+// bf16 256 rows 6.8 (6.2).
+static bool actq_fwd_waves(int K, int M, bool bf16_rows) { return K <= 2048 || M >= (bf16_rows ? 512 : 1024); }
+static bool actq_bwd_waves(int K, int M, bool bf16_rows) { return K <= 2048 || bf16_rows || M >= 512; }
+// one instance per number of rounds of 512 values, above 2048 values two waves a row
 #define ACTQ_WAVES(K, M, CALL)                                                                                          \
     {                                                                                                                   \
         const bool stream = (long)(M) * (K) >= (1L << 20);                                                              \
@@ -1447,7 +1453,7 @@ extern "C" {
 int camx_actq_fwd(const void * x, int is_bf16, uint16_t * y, float * s, uint16_t * codes, int K, float clip, int qmax, int M, hipStream_t st) {
     if (!x || (!y && !codes) || actq_check(K, qmax, M) || ((uintptr_t)x & (is_bf16 ? 7 : 15)) || ((uintptr_t)y & 7) || ((uintptr_t)codes & 1)) return CAMX_EINVAL;
     if (M == 0) return CAMX_OK;
-    if (actq_wave_ok(K, (uintptr_t)x, (uintptr_t)y, (uintptr_t)codes)) {
+    if (actq_wave_ok(K, (uintptr_t)x, (uintptr_t)y, (uintptr_t)codes) && actq_fwd_waves(K, M, is_bf16)) {
         if (is_bf16) ACTQ_WAVES(K, M, (actq_fwd_wave_k<PlainBF16, R, W><<<grid, block, 0, st>>>(PlainBF16{(const uint16_t *)x, K}, y, s, codes, K, clip, qmax, M, stream)))
         else ACTQ_WAVES(K, M, (actq_fwd_wave_k<PlainF32, R, W><<<grid, block, 0, st>>>(PlainF32{(const float *)x, K}, y, s, codes, K, clip, qmax, M, stream)))
         CAMX_LAUNCH_RET();
@@ -1462,7 +1468,7 @@ int camx_silu_mul_actq_fwd(const uint16_t * gu, int ld, int F, uint16_t * y, flo
     const uint16_t * lut = nullptr, * small = nullptr;
     const int rc = silu_luts_get(st, &lut, &small);
     if (rc) return rc;
-    if (!(ld & 7) && actq_wave_ok(F, (uintptr_t)gu, (uintptr_t)y, (uintptr_t)codes)) {
+    if (!(ld & 7) && actq_wave_ok(F, (uintptr_t)gu, (uintptr_t)y, (uintptr_t)codes) && actq_fwd_waves(F, M, false)) {
         ACTQ_WAVES(F, M, (actq_fwd_wave_k<SiluMulSrc, R, W><<<grid, block, 0, st>>>(SiluMulSrc{gu, ld, F, lut, nullptr}, y, s, codes, F, clip, qmax, M, stream, small)))
         CAMX_LAUNCH_RET();
     }
@@ -1496,7 +1502,7 @@ int camx_block_entry_fwd(const float * x, const float * nw, const uint16_t * wab
 int camx_actq_bwd(const void * x, int is_bf16, const uint16_t * g, void * dx, int K, float clip, int qmax, int M, hipStream_t st) {
     if (!x || !g || !dx || actq_check(K, qmax, M) || ((uintptr_t)x & (is_bf16 ? 7 : 15)) || ((uintptr_t)dx & (is_bf16 ? 7 : 15)) || ((uintptr_t)g & 7)) return CAMX_EINVAL;
     if (M == 0) return CAMX_OK;
-    if (actq_wave_ok(K, (uintptr_t)x | (uintptr_t)g, (uintptr_t)dx, 0)) {
+    if (actq_wave_ok(K, (uintptr_t)x | (uintptr_t)g, (uintptr_t)dx, 0) && actq_bwd_waves(K, M, is_bf16)) {
         if (is_bf16) ACTQ_WAVES(K, M, (actq_bwd_wave_k<PlainBF16, SinkBF16, R, W><<<grid, block, 0, st>>>(PlainBF16{(const uint16_t *)x, K}, g, SinkBF16{(uint16_t *)dx, K}, K, clip, qmax, M, stream)))
         else ACTQ_WAVES(K, M, (actq_bwd_wave_k<PlainF32, SinkF32, R, W><<<grid, block, 0, st>>>(PlainF32{(const float *)x, K}, g, SinkF32{(float *)dx, K}, K, clip, qmax, M, stream)))
         CAMX_LAUNCH_RET();
@@ -1514,7 +1520,7 @@ int camx_silu_mul_actq_bwd(const uint16_t * gu, int ld, int F, const uint16_t * 
     int rc = silu_luts_get(st, &lut, &small);
     if (!rc) rc = dsilu_luts_get(st, &dlut, &dsmall);
     if (rc) return rc;
-    if (!(ld & 7) && actq_wave_ok(F, (uintptr_t)gu | (uintptr_t)g, (uintptr_t)dgu, 0)) {
+    if (!(ld & 7) && actq_wave_ok(F, (uintptr_t)gu | (uintptr_t)g, (uintptr_t)dgu, 0) && actq_bwd_waves(F, M, false)) {
         ACTQ_WAVES(F, M, (actq_bwd_wave_k<SiluMulSrc, SinkSiluMul, R, W><<<grid, block, 0, st>>>(SiluMulSrc{gu, ld, F, lut, nullptr}, g, SinkSiluMul{gu, ld, F, dgu, dlut, nullptr}, F, clip, qmax, M, stream, small, dsmall)))
         CAMX_LAUNCH_RET();
     }

@@ -393,6 +393,62 @@ def test_actq_fwd_and_bwd_four_million_values(bf):
     assert bits_equal(host(dx, np.uint16) if bf else host(dx), O.actq_bwd(src, g, clip=0.95, qmax=7, bf16=bf))
 
 
+@pytest.mark.parametrize('M', [511, 513, 1023, 1025])
+@pytest.mark.parametrize('K', [2176, 3072, 3200, 4096])
+def test_actq_two_waves_of_a_row(M, K):
+    """rows of 2049 to 4096 values on both sides of the batch sizes that give them two waves (512 and 1024), plain and SiLU-fused, forward and backward,
+    odd row counts: a NaN or an infinity in one wave's chunks only (chunks 0 .. 3 and 4 .. 7 of every 8 are the first and the second wave's), zeros,
+    maxima in either half. Bit for bit against the same rows in batches that a workgroup a row takes, and the ordinary rows against the oracle"""
+    import torch
+    rng = np.random.default_rng(K + M)
+    x = outliers(rng, (M, K)); g = O.f2bf(rng.standard_normal((M, K)).astype(np.float32))
+    gate = (rng.standard_normal((M, K)) * 2).astype(np.float32); gate[rng.random((M, K)) < 1e-3] *= 200
+    for a in (x, gate):
+        a[0, 5] = np.nan; a[1, 5 * 128 + 3] = np.nan; a[2, 3] = np.inf; a[3, 6 * 128] = -np.inf; a[M - 1, K - 1] = np.nan; a[M - 2, 0] = np.inf
+        a[4] = 0; a[5] = -0.0; a[6] = 0; a[6, 7] = 3.0; a[7] = 0; a[7, 4 * 128 + 7] = 3.0; a[8, 128:256] *= 100; a[9, 4 * 128:5 * 128] *= 100
+    gu = O.f2bf(np.concatenate([gate, x], axis=1))
+    plain = [4, 5, 6, 7, 8, 9, 10, M // 2, M - 3]                 # rows without a NaN or an infinity
+    gd, n = dev(g), 255
+
+    def equal(a, b):
+        nan = torch.isnan(a) & torch.isnan(b)
+        return bool(((a.view(torch.int16) == b.view(torch.int16)) if a.dtype == torch.bfloat16 else (a.view(torch.int32) == b.view(torch.int32))).logical_or(nan).all())
+
+    def buffers(dt, width): return [torch.full((M + 1, width), 5.0, device='cuda', dtype=dt) for _ in range(2)]
+
+    def both(run):                                                # the whole batch, then 255 rows at a time
+        run(0, 0, M)
+        for lo in range(0, M, n): run(1, lo, min(n, M - lo))
+        torch.cuda.synchronize()
+
+    for form in ('f32', 'bf16', 'silu'):
+        src = dev(x) if form == 'f32' else dev(O.f2bf(x)).view(torch.bfloat16) if form == 'bf16' else dev(gu).view(torch.bfloat16)
+        y, s = buffers(torch.bfloat16, K), [torch.full((M + 1,), 5.0, device='cuda') for _ in range(2)]
+        c = [torch.full((M + 1, K // 2), 5, device='cuda', dtype=torch.uint8) for _ in range(2)]
+        d = buffers(torch.float32 if form == 'f32' else torch.bfloat16, 2 * K if form == 'silu' else K)
+
+        def forward(i, lo, m):
+            a = (ptr(y[i][lo:]), ptr(s[i][lo:]), ptr(c[i][lo:]))
+            if form == 'silu': call('camx_silu_mul_actq_fwd', ptr(src[lo:]), I(2 * K), I(K), *a, F(1.0), I(7), I(m))
+            else: call('camx_actq_fwd', ptr(src[lo:]), I(int(form == 'bf16')), *a, I(K), F(1.0), I(7), I(m))
+
+        def backward(i, lo, m):
+            if form == 'silu': call('camx_silu_mul_actq_bwd', ptr(src[lo:]), I(2 * K), I(K), ptr(gd[lo:]), ptr(d[i][lo:]), F(1.0), I(7), I(m))
+            else: call('camx_actq_bwd', ptr(src[lo:]), I(int(form == 'bf16')), ptr(gd[lo:]), ptr(d[i][lo:]), I(K), F(1.0), I(7), I(m))
+        both(forward); both(backward)
+        for a, b in (y, [t.view(M + 1, 1) for t in s], d): assert equal(a, b), form
+        assert torch.equal(c[0], c[1]), form
+        for t in (y[0], s[0], c[0], d[0]): assert bool((t[M] == 5).all()), form
+        rows = np.array(plain)
+        if form == 'silu': (ry, rs, rc), want = O.silu_mul_actq_fwd(gu[rows]), O.silu_mul_actq_bwd(gu[rows], g[rows], table=True)
+        else:
+            a = O.f2bf(x[rows]) if form == 'bf16' else x[rows]
+            (ry, rs, rc), want = O.actq_fwd(a, bf16=form == 'bf16'), O.actq_bwd(a, g[rows], bf16=form == 'bf16')
+        got = host(d[0][:M].view(torch.int16), np.uint16) if d[0].dtype == torch.bfloat16 else host(d[0][:M])
+        assert bits_equal(host(y[0][:M].view(torch.int16), np.uint16)[rows], ry) and bits_equal(host(s[0])[rows], rs) and bits_equal(host(c[0])[rows], rc), form
+        assert bits_equal(got[rows], want), form
+
+
 @pytest.mark.parametrize('M,d,nab,eps', [(8177, 1024, 16, 1e-6), (8191, 384, 10, 0.0), (4096, 896, 5, 1e-6), (12284, 640, 13, 0.0), (8192, 512, 8, 1e-6), (8190, 128, 13, 0.0)])
 def test_block_entry_fwd_sixteen_rows_from_a_full_chip(M, d, nab, eps):
     """batches just below whole multiples of 4096 rows, which sixteen rows a workgroup take: last workgroups of 1, 15, 16, 12, 16 and 14 rows"""
