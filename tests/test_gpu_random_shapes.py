@@ -24,8 +24,8 @@ def _generators(r):
         return ch([1, 2, 3, 5, 8, 17, 64, 255, 256, 257, 300, 515, 1023, 1024, 1025, 1026, 1030])
 
     def silu_actq():
-        m, f = ri(2, 40), 128 * ri(1, 24)
-        return m, f, 2 * f + 4 * ri(0, 8)                      # strides for the wave-per-row form (16-byte rows) and the workgroup form
+        m, f = ch([ri(2, 40), ri(2, 40), ri(500, 1030)]), 128 * ri(1, 33)
+        return m, f, 2 * f + 4 * ri(0, 8)                      # strides for the wave-per-row forms (16-byte rows; two waves from 512 rows above 2048 values) and the workgroup form
 
     def rms_mul():
         wr = ch([1, 1, 2, 4])
@@ -41,7 +41,7 @@ def _generators(r):
         (A.test_block_entry_bwd, lambda: (ri(1, 200), 128 * ri(1, 8), 2 * ri(0, 8))),
         (A.test_block_entry_fwd, lambda: (ri(1, 200), 128 * ch([ri(1, 8), ri(1, 8), ri(9, 64)]), ri(0, 16))),
         (A.test_silu_mul_actq_bwd, silu_actq),
-        (A.test_silu_mul_actq_fwd, lambda: (ri(2, 300), 128 * ri(1, 24))),
+        (A.test_silu_mul_actq_fwd, lambda: (ch([ri(2, 300), ri(2, 300), ri(1000, 1100)]), 128 * ri(1, 33))),
         (E.test_swiglu, lambda: (ri(1, 70000),)),
         (E.test_silu_mul_bf16, lambda: (ri(1, 300), ri(6, 3000))),
         (E.test_gdn_conv, lambda: (ri(1, 600), ch([6, 64, 100, 256, 512, 1000, 4096, 8200, 10240]))),
