@@ -3,11 +3,11 @@
 // actq_fwd_codes_{f32,bf16}, actq_bwd_{f32,bf16}, silu_mul_actq_{fwd,bwd} and block_entry_{fwd,bwd} (kernels/actq.hip:40-53,
 // 96-218, 247-333).
 //
-// Rows of at most 4096 values with 16-byte aligned operands, forward and backward, plain and SiLU-fused: one wave per row, two above 2048
-// (actq_fwd_wave_k, actq_bwd_wave_k; two waves only in batches that fill the chip), the fused forms with the gates' tables in LDS. The RMSNorm-fused block entry of rows of at most
-// 1024 values: a wave per row as well, four or sixteen rows sharing the projections (block_entry_fwd_quad, block_entry_fwd_rows16,
-// block_entry_bwd_quad). Everything else
-// (longer rows, unaligned operands, small batches of rows above 2048 values):
+// Rows of at most 4096 values with 16-byte aligned operands, forward and backward, plain and SiLU-fused: one wave per row, above 2048
+// values two, in batches that fill the chip (actq_fwd_wave_k, actq_bwd_wave_k), the fused forms with the gates' tables in LDS. The
+// RMSNorm-fused block entry of rows of at most 1024 values: a wave per row as well, four or sixteen rows sharing the projections
+// (block_entry_fwd_quad, block_entry_fwd_rows16, block_entry_bwd_quad). Everything else (longer rows, unaligned operands, small batches
+// of rows above 2048 values):
 // One 256-thread workgroup per row. A half-wave (32 lanes) transforms one 128-chunk: lane l holds elements 4l .. 4l + 3,
 // butterfly stages 1-2 in registers, 4 .. 64 across lanes; half-wave h takes chunks h, h + 8, ... (the reference's wave h of
 // 32), NR = ceil(K / 1024) rounds of them stay in registers across the row-wide reductions. Kernels are instantiated per

@@ -1252,7 +1252,8 @@ static int rope_launch(const RopeArgs & a, int yarn, bool q8, hipStream_t st, bo
     const bool aligned = (a.ldq & (bf16in ? 7 : 3)) == 0 && ((uintptr_t)a.qkv & 15) == 0 && ((uintptr_t)a.q16 & 15) == 0 && ((uintptr_t)a.cache & 15) == 0;
     const bool wide = (!q8 || !bf16in) && !a.page_table && aligned;
     // A token per workgroup with all its loads first, from a batch that covers the chip (80 bf16 heads, 300 tokens 5.2 us, 777 tokens 7.6, 1500 tokens
-    // 10.5: the token kernel 6.2, 8.7, 14.6; 40 fp32 heads 5.0, 6.9, 9.2 and 5.7, 8.1, 12.1). The Q8 rows are bound by their arithmetic, which
+    // 10.5: the token kernel 6.2, 8.7, 14.6; 40 fp32 heads 5.0, 6.9, 9.2 and 5.7, 8.1, 12.1; 12 bf16 heads 257 tokens 3.5 and 4.7, 2047 tokens 5.5 and 10.8; of 8 to
+    // 72 heads none slower). The Q8 rows are bound by their arithmetic, which
     // the token kernel spreads over more waves: 777 tokens 9.5 us, chunk 9.9, 1800 tokens 15.9 and 16.4, 2048 tokens 20.5 and 17.6; through a page table, where a token's row
     // address is a chain of loads that the chunk kernel starts early, 512 tokens 7.5 and 8.0, 777 tokens 10.4 and 10.1, 1500 tokens 15.5 and 13.6.
     const bool chunk = a.n > 256, chunk_q8 = a.n >= 2048, chunk_paged = a.n >= 700;
