@@ -405,11 +405,13 @@ static bool launch_norm_div(const NormArgs & a, hipStream_t st) {
         // q3p_add_rms16 at 4096 x 2048 is slower this way (26.7 -> 28.3 us) and keeps the wave per row. Batches whose rows as a wave each
         // leave the chip half empty: 5120-wide rows with a bf16 addend 512 rows 6.4 us (a wave per row: chunk form 7.7, general form 9.9), 640 rows 8.9
         // (8.2, 10.8); with fp32 addend and copies 8.0 (9.7, 10.9) and 12.3 (10.6, 12.0); eight slots of 2048 512 rows 9.7 (15.2, 11.8), 1023 rows
-        // 16.4 (-, 17.6), 1024 rows 17.0 (19.8, -), 2048 rows 33.6 (32.6). One or no slot: the chunk form where its workgroups of four rows nearly fill
-        // the last round of 256 CUs (777 x 2048 6.1 us, divided 6.4; 1024 6.4 and 6.7; 1027 8.8 and 7.6; 1536 10.3 and 9.6; 2047 11.0 and 11.9). Other addends divided
-        // to two workgroups a CU: 512 rows of 5120 with fp32 copies 8.7 us (chunk form 10.0), 520 rows 10.9 (10.1).
-        const int ni = a.N >> 8;
-        const bool slots = ADD == ADD_F32_SLOTS && a.rows < 2048 && (a.S > 1 || ((1024 - (a.rows & 1023)) & 1023) >= 256);
+        // 16.4 (-, 17.6), 1024 rows 17.0 (19.8, -), 2048 rows 33.6 (32.6). One or no slot: the chunk form where its workgroups of four rows
+        // nearly fill the last round of 256 CUs (with the fp16 copy alone 777 x 2048 5.8 us, divided 6.3, 1024 6.4 and 6.7, 1536 10.4 and 9.5, 2047 10.9 and 11.8;
+        // with both copies, where a wave that ends late has more to write, in the second round only: 777 6.1 and 6.4 but 1024 7.3 and 6.9, 1400 11.7 and 11.1,
+        // 1700 11.5 and 12.9, 2047 12.7 and 14.7). Other addends divided to two workgroups a CU: 512 rows of 5120 with fp32 copies 8.7 us (chunk form 10.0),
+        // 520 rows 10.9 (10.1).
+        const int ni = a.N >> 8, idle = -a.rows & 1023, fill = !(OUT & NORM_H) ? 256 : a.rows > 1024 ? 512 : 0;
+        const bool slots = ADD == ADD_F32_SLOTS && a.rows < 2048 && (a.S > 1 || idle >= fill);
         if (!((OUT & NORM_Q8) || ni == 10 || a.rows >= 16384 || a.rows <= 512 || slots)) return false;
         const int w = ni == 10 ? 2 : 4, rpw = 4 / w;
         const dim3 grid((a.rows + rpw - 1) / rpw), block(256);
