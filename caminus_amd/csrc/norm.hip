@@ -409,10 +409,11 @@ static bool launch_norm_div(const NormArgs & a, hipStream_t st) {
         // nearly fill the last round of 256 CUs (with the fp16 copy alone 777 x 2048 5.8 us, divided 6.3, 1024 6.4 and 6.7, 1536 10.4 and 9.5, 2047 10.9 and 11.8;
         // with both copies, where a wave that ends late has more to write, in the second round only: 777 6.1 and 6.4 but 1024 7.3 and 6.9, 1400 11.7 and 11.1,
         // 1700 11.5 and 12.9, 2047 12.7 and 14.7). Other addends divided to two workgroups a CU: 512 rows of 5120 with fp32 copies 8.7 us (chunk form 10.0),
-        // 520 rows 10.9 (10.1).
+        // 520 rows 10.9 (10.1); of 2048 a little longer (bf16 copy alone 599 rows 4.5 us, chunk form 4.8; with the fp32 copy 544 rows 5.0 and 5.2, 599 5.7 and 5.4).
         const int ni = a.N >> 8, idle = -a.rows & 1023, fill = !(OUT & NORM_H) ? 256 : a.rows > 1024 ? 512 : 0;
+        const int few = a.N > 2048 ? 512 : OUT & NORM_H ? 560 : 599;
         const bool slots = ADD == ADD_F32_SLOTS && a.rows < 2048 && (a.S > 1 || idle >= fill);
-        if (!((OUT & NORM_Q8) || ni == 10 || a.rows >= 16384 || a.rows <= 512 || slots)) return false;
+        if (!((OUT & NORM_Q8) || ni == 10 || a.rows >= 16384 || a.rows <= few || slots)) return false;
         const int w = ni == 10 ? 2 : 4, rpw = 4 / w;
         const dim3 grid((a.rows + rpw - 1) / rpw), block(256);
         switch (ni) {
@@ -570,10 +571,10 @@ __global__ void __launch_bounds__(256) add_rms_bf16_chunk(float * __restrict__ x
         }
     }
 }
-// Whether the chunk form applies: an addend, a bf16 copy and no fp32 copy, more than 512 rows (up to there, a row is divided over four waves:
-// launch_norm_div) of 256 NI values for the NI below, 16-byte aligned. A batch of less than 2^20 values stays in the caches.
+// Whether the chunk form applies: an addend, a bf16 copy and no fp32 copy, more than 512 rows, 599 of up to 2048 values (up to there, a row is
+// divided over four waves: launch_norm_div) of 256 NI values for the NI below, 16-byte aligned. A batch of less than 2^20 values stays in the caches.
 static bool launch_add_rms_bf16_chunk(float * x, const uint16_t * d, const float * nw, float eps, uint16_t * hbf, int N, int n, hipStream_t st) {
-    if (!d || !hbf || n <= 512 || (n < 1024 && (long)n * N < (1L << 20)) || (N & 255) || (((uintptr_t)x | (uintptr_t)d | (uintptr_t)nw | (uintptr_t)hbf) & 15)) return false;
+    if (!d || !hbf || n <= (N > 2048 ? 512 : 599) || (n < 1024 && (long)n * N < (1L << 20)) || (N & 255) || (((uintptr_t)x | (uintptr_t)d | (uintptr_t)nw | (uintptr_t)hbf) & 15)) return false;
     const dim3 grid((n + 3) / 4), block(256);
     switch (N >> 8) {
 #define CAMX_CHUNK(NI) case NI: \

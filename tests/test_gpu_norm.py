@@ -119,7 +119,7 @@ def test_norm_forms_between_256_and_chunk_rows(n, N):
     assert tail_ok(xd, np.float32) and tail_ok(h, np.float32) and tail_ok(h16, np.uint16)
 
 
-@pytest.mark.parametrize('n,N', [(512, 5120), (513, 5120), (513, 2560), (514, 4096), (768, 2048), (769, 2048), (1024, 2048), (1025, 2048), (1536, 2048), (1537, 2048), (1792, 1024), (1793, 1024)])
+@pytest.mark.parametrize('n,N', [(512, 5120), (513, 5120), (513, 2560), (514, 4096), (560, 2048), (561, 2048), (599, 2048), (600, 2048), (768, 2048), (769, 2048), (1024, 2048), (1025, 2048), (1536, 2048), (1537, 2048), (1792, 1024), (1793, 1024)])
 def test_norm_forms_at_their_lines(n, N):
     """the last batch that divides its rows over waves and the first that does not, whole and ragged; one slot addend at its own lines"""
     test_norm_forms_between_256_and_chunk_rows(n, N)
