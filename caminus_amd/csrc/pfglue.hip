@@ -658,15 +658,13 @@ static bool ple_vec(const float * x, const float * xw, const uint16_t * w, const
 static bool ple_taps(const float * x, const float * xw, const uint16_t * w, const float * y, const float * a, const float * res, int C, int T, int D, int dil) {
     return ple_vec(x, xw, w, y, a, res, C, D) && dil <= 65535 && (ple_waves(T, dil) + 3) / 4 <= 65535;
 }
-// A thread per token while its waves are resident at once, thirty-two a CU, or where the waves above have no grid. Its history reads are scattered (a lane's
+// A thread per token while its waves are resident at once, thirty-two a CU (which also keeps its 32-bit indexes in range). Its history reads are scattered (a lane's
 // channels lie 3 dil floats apart, up to a line each), so the tokens that read it count for more. This form / the waves above, dilation 3: 16 x 10240 3.3 / 4.2 us,
 // 64 x 2560 3.2 / 4.3, 256 x 1024 3.2 / 4.2, 640 x 2560 5.4 / 5.5, 2048 x 1024 5.6 / 6.2; 2560 x 1024 7.7 / 6.8, 128 x 10240 5.6 / 5.2; dilation 8: 2048 x 256
 // 3.6 / 5.2, 4096 x 256 4.6 / 5.7, 640 x 2560 8.0 / 6.5. (The committing entry keeps the waves at every size: one launch instead of this form and the history's.)
 static bool ple_rows(const float * x, const float * xw, const uint16_t * w, const float * y, const float * a, const float * res, int C, int T, int D, int dil) {
-    if (!ple_vec(x, xw, w, y, a, res, C, D) || T > 65535) return false;
-    if (dil > 65535) return true;
-    const long past = T < 3 * dil ? T : 3 * dil;
-    return (T + 4L * dil * past) * ((C + 255) / 256) < 9000;
+    const long past = T < 3L * dil ? T : 3L * dil;
+    return ple_vec(x, xw, w, y, a, res, C, D) && (T + 4L * dil * past) * ((C + 255) / 256) < 9000;
 }
 static void launch_ple_taps(const float * x, const float * xscl, const float * xw, const uint16_t * w, const float * hist, float * y, const float * a, float * res,
                             int C, int T, int D, int dil, float * commit, hipStream_t st) {
